@@ -88,6 +88,16 @@ struct GridView {
      * grid exceeds VT_PACKED_MAX_EXTENT */
     const uint64_t* occr;
     int32_t wide;               /* padded masks span 4 GiB or more (byte offsets need 64 bits) */
+    /* 2-bit empty-cube codes of the jump march, 16 per word, over the grid's
+     * cells of 2^cg voxels padded by one cell on every side, linear order
+     * (cx + ccx*(cy + ccy*cz)): 0 = some voxel of the cell is occupied or
+     * outside the grid, c = 1..3 = the aligned cube of (byte c of cedge) + 1
+     * voxels an edge around the cell is empty and inside the grid */
+    const uint32_t* codes;
+    uint32_t code_words;
+    uint32_t ccx, ccy;          /* padded cell extents in x and y */
+    uint32_t cg, cedge;
+    float jc0;                  /* 2^-24 (2 max extent + 32): the jump march's error bound at distance 0 */
     int32_t n_emissive;
     const int32_t* emissive;    /* linear voxel indices */
     const int4* lights;         /* per emissive entry: voxel x, y, z and its material slot */
@@ -699,6 +709,229 @@ __device__ __forceinline__ int DdaState::advance_wave_packed(const GridView& g, 
     if (marching) return steps >= g.max_steps ? 2 : 0;
     return inside ? 1 : 2;
 }
+
+/* ---- jump march ------------------------------------------------------------------------
+ * The voxel at which the DDA of dda.h:7-61 stops, without its step count:
+ * the traversal of renders that collect no statistics.
+ *
+ * The DDA visits voxels in the order of three sequences, one per axis: X_0 =
+ * dis.x and X_{k+1} = fl(X_k + a.x) (a = |1/d|), the value at which the k-th
+ * x step is taken, and the same for y and z.  Each iteration takes the axes
+ * whose next value is the smallest, so the position after all values <= m
+ * depends on m alone: x0 + #{k: X_k <= m}, and so on.  While the ray is inside an
+ * aligned cube of empty voxels the visited voxels need no test, and the whole
+ * passage is one jump: m = the smallest of the three values at which an axis
+ * steps out of the cube, then the three counts.
+ *
+ * Values and counts are evaluated on the real line X_0 + k a.  Every add of
+ * the FP32 sums is off by at most half an ulp, so with M the largest count
+ * (m, as a >= 0.99) the two sequences that a decision compares are together
+ * off their lines by at most 2^-24 (M^2 + 3M) steps, and the evaluation itself
+ * by 2^-24 (3M + 2 extent + 8); del = 2^-24 (1.06 (M + 4)^2 + 2 extent + 32)
+ * covers both.  With q the real-valued position (an integer where an axis
+ * steps), floor(q + del) is the exact position unless q lies within del of an
+ * integer; on the axis that leaves the cube it always does, and it is then
+ * right as well.  When a second axis is that near an integer the order of the
+ * two steps is undecided (0.1-0.3 % of the jumps): jump() leaves the position
+ * unchanged and resolve() compares the FP32 sums themselves.
+ *
+ * Axes are mirrored (x ^ -1) so that every step is +1 and the far face of an
+ * aligned cube is x | (edge - 1).  A ray whose set-up leaves the ranges the
+ * bound was derived for (non-finite or very unnormalised directions) is
+ * marched step by step instead.
+ *
+ * Full-shading scene (256^3, 99 DDA steps a ray): 12 iterations a ray, 99.9 %
+ * of the rays within 69 (the steps: 580). */
+#define VT_JUMP_A_MIN 0.99f
+#define VT_JUMP_A_MAX 2.0e5f
+#define VT_ULP24 5.9604644775390625e-8f   /* 2^-24 */
+/* 1.03 * 2^-12 and 4 times that: (m * W1 + W4)^2 = 1.06 * 2^-24 (m + 4)^2 */
+#define VT_JUMP_W1 2.5146484375e-4f
+#define VT_JUMP_W4 1.005859375e-3f
+
+/* The sum X + a + a + ... of n FP32 adds, exactly.  Inside one binade every
+ * add rounds a to the same multiple of the ulp (once the sum is the result of
+ * an add there, which settles the parity of ties), so a run of adds that stays
+ * below the binade's end is one exact multiply-add. */
+__device__ __forceinline__ float sum_steps(float X, float a, float ia, int32_t n)
+{
+    while (n > 0) {
+        const float p = X + a;
+        if (--n == 0) return p;
+        X = p + a;
+        --n;
+        const uint32_t ub = __float_as_uint(X) & 0x7f800000u;
+        if (n > 0 && ub == (__float_as_uint(p) & 0x7f800000u)) {
+            const float end = __uint_as_float(ub + 0x00800000u);
+            /* three steps short of the end: covers the rounding of the quotient and of a */
+            int32_t r = (int32_t)((end - X) * ia) - 3;
+            r = r < n ? r : n;
+            if (r > 0) {
+                X = __builtin_fmaf((float)r, (X + a) - X, X);
+                n -= r;
+            }
+        }
+    }
+    return X;
+}
+
+struct JumpState {
+    int32_t x, y, z;            /* mirrored position */
+    int32_t x0, y0, z0;         /* mirrored start */
+    int32_t fx, fy, fz;         /* 0, or -1 on a mirrored axis */
+    float X0, Y0, Z0, ax, ay, az, ix, iy, iz, qx, qy, qz;
+
+    enum { OUTSIDE = 0, READY = 1, STEPWISE = 2 };
+
+    /* DdaState::init's arithmetic; STEPWISE when the bound does not hold. */
+    __device__ __forceinline__ int init(const GridView& g, const PreRay& r)
+    {
+        const float vox = ((r.o.x - g.bmin[0]) * g.ext[0]) * g.rx;
+        const float voy = ((r.o.y - g.bmin[1]) * g.ext[1]) * g.ry;
+        const float voz = ((r.o.z - g.bmin[2]) * g.ext[2]) * g.rz;
+        const float bx = floorf(vox), by = floorf(voy), bz = floorf(voz);
+        if (bx < 0.0f || by < 0.0f || bz < 0.0f || bx >= g.rx || by >= g.ry || bz >= g.rz) return OUTSIDE;
+        X0 = (((bx - vox) + 0.5f) + (float)r.sx * 0.5f) * r.inv.x;
+        Y0 = (((by - voy) + 0.5f) + (float)r.sy * 0.5f) * r.inv.y;
+        Z0 = (((bz - voz) + 0.5f) + (float)r.sz * 0.5f) * r.inv.z;
+        ax = vt_absf(r.inv.x); ay = vt_absf(r.inv.y); az = vt_absf(r.inv.z);
+        const float lo = min3f(ax, ay, az);
+        const bool sane = lo >= VT_JUMP_A_MIN && ax <= VT_JUMP_A_MAX && ay <= VT_JUMP_A_MAX && az <= VT_JUMP_A_MAX &&
+                          X0 >= 0.0f && Y0 >= 0.0f && Z0 >= 0.0f && X0 <= ax * 1.001f && Y0 <= ay * 1.001f &&
+                          Z0 <= az * 1.001f;
+        if (!sane) return STEPWISE;
+        fx = r.sx < 0 ? -1 : 0; fy = r.sy < 0 ? -1 : 0; fz = r.sz < 0 ? -1 : 0;
+        x = x0 = (int32_t)bx ^ fx; y = y0 = (int32_t)by ^ fy; z = z0 = (int32_t)bz ^ fz;
+        ix = __builtin_amdgcn_rcpf(ax); iy = __builtin_amdgcn_rcpf(ay); iz = __builtin_amdgcn_rcpf(az);
+        qx = __builtin_fmaf(-X0, ix, (float)(x0 + 1));
+        qy = __builtin_fmaf(-Y0, iy, (float)(y0 + 1));
+        qz = __builtin_fmaf(-Z0, iz, (float)(z0 + 1));
+        return READY;
+    }
+
+    /* Edge minus one of the empty aligned cube around the position, 0 for a
+     * single voxel; false when the voxel is occupied or outside the grid.
+     * FINE: cells are the 4x4x4 blocks.  UNI: one grid for the whole wave. */
+    template <bool FINE, bool UNI>
+    __device__ __forceinline__ bool lookup(const GridView& g, const uint32_t* __restrict__ codes, int32_t& edge) const
+    {
+        const uint32_t cg = FINE ? 2u : g.cg;
+        const uint32_t pad = 1u << cg;
+        const uint32_t ux = xor_add<UNI>(x, fx, pad), uy = xor_add<UNI>(y, fy, pad), uz = xor_add<UNI>(z, fz, pad);
+        const uint32_t ci = index3<UNI>(ux >> cg, uy >> cg, uz >> cg, g.ccx, g.ccy);
+        const uint32_t c = field<2, false>(codes[ci >> 4], ci << 1);
+        edge = (int32_t)field<8, UNI>(g.cedge, c << 3);
+        if (c == 0u) {
+            uint32_t bi = ci;
+            if (!FINE) {
+                const uint32_t k = pad - 4u;
+                bi = index3<UNI>((ux - k) >> 2, (uy - k) >> 2, (uz - k) >> 2, g.bxp, g.byp);
+            }
+            const uint64_t m = g.occp[bi];
+            if (m == 0ull) {
+                edge = 3;
+            } else {
+                const uint32_t bit = (ux & 3u) | ((uy & 3u) << 2) | ((uz & 3u) << 4);
+                if ((m >> bit) & 1ull) return false;
+            }
+        }
+        return true;
+    }
+
+    /* (a ^ b) + c in one instruction; c is wave-uniform with UNI */
+    template <bool UNI>
+    static __device__ __forceinline__ uint32_t xor_add(int32_t a, int32_t b, uint32_t c)
+    {
+        uint32_t r;
+        if constexpr (UNI) asm("v_xad_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+        else asm("v_xad_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+        return r;
+    }
+    /* W bits of v from bit (at & 31); v is wave-uniform with UNI */
+    template <uint32_t W, bool UNI>
+    static __device__ __forceinline__ uint32_t field(uint32_t v, uint32_t at)
+    {
+        uint32_t r;
+        if constexpr (UNI) asm("v_bfe_u32 %0, %1, %2, %3" : "=v"(r) : "s"(v), "v"(at), "n"(W));
+        else asm("v_bfe_u32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(at), "n"(W));
+        return r;
+    }
+    /* x + ex (y + ey z) on 24-bit operands */
+    template <bool UNI>
+    static __device__ __forceinline__ uint32_t index3(uint32_t ix, uint32_t iy, uint32_t iz, uint32_t ex, uint32_t ey)
+    {
+        uint32_t r;
+        if constexpr (UNI) {
+            asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(iz), "s"(ey), "v"(iy));
+            asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(r), "s"(ex), "v"(ix));
+        } else {
+            asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(iz), "v"(ey), "v"(iy));
+            asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(r), "v"(ex), "v"(ix));
+        }
+        return r;
+    }
+
+    /* Leave the cube of lookup(); false, with the position unchanged, when
+     * the order of two steps is undecided. */
+    __device__ __forceinline__ bool jump(const GridView& g, int32_t edge)
+    {
+        const int32_t bx = x | edge, by = y | edge, bz = z | edge;
+        const float m = min3f(__builtin_fmaf((float)(bx - x0), ax, X0), __builtin_fmaf((float)(by - y0), ay, Y0),
+                              __builtin_fmaf((float)(bz - z0), az, Z0));
+        const float w = __builtin_fmaf(m, VT_JUMP_W1, VT_JUMP_W4);
+        const float del = __builtin_fmaf(w, w, g.jc0);
+        const float px = __builtin_fmaf(m, ix, qx) + del, py = __builtin_fmaf(m, iy, qy) + del,
+                    pz = __builtin_fmaf(m, iz, qz) + del;
+        if (__builtin_amdgcn_fmed3f(__builtin_amdgcn_fractf(px), __builtin_amdgcn_fractf(py),
+                                    __builtin_amdgcn_fractf(pz)) < del + del)
+            return false;
+        x = floor_i32(px); y = floor_i32(py); z = floor_i32(pz);
+        return true;
+    }
+
+    static __device__ __forceinline__ int32_t floor_i32(float v)
+    {
+        int32_t r;
+        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+        return r;
+    }
+
+    /* The jump that jump() left undecided: the values of the near axes' steps
+     * as the FP32 sums they are; a step is taken when its value is not above
+     * the smallest one that leaves the cube. */
+    __device__ __forceinline__ void resolve(const GridView& g, int32_t edge)
+    {
+        const int32_t b[3] = { x | edge, y | edge, z | edge };
+        const float m = min3f(__builtin_fmaf((float)(b[0] - x0), ax, X0), __builtin_fmaf((float)(b[1] - y0), ay, Y0),
+                              __builtin_fmaf((float)(b[2] - z0), az, Z0));
+        const float w = __builtin_fmaf(m, VT_JUMP_W1, VT_JUMP_W4);
+        const float del = __builtin_fmaf(w, w, g.jc0);
+        const float p[3] = { __builtin_fmaf(m, ix, qx) + del, __builtin_fmaf(m, iy, qy) + del,
+                             __builtin_fmaf(m, iz, qz) + del };
+        const int32_t at[3] = { x, y, z }, s0[3] = { x0, y0, z0 };
+        const float S0[3] = { X0, Y0, Z0 }, a[3] = { ax, ay, az }, ia[3] = { ix, iy, iz };
+        int32_t to[3];
+        float v[3], me = __uint_as_float(0x7f800000u);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            to[k] = floor_i32(p[k]);
+            v[k] = 0.0f;
+            /* a near axis whose step is still ahead */
+            if (__builtin_amdgcn_fractf(p[k]) < del + del && to[k] > at[k]) {
+                v[k] = sum_steps(S0[k], a[k], ia[k], to[k] - 1 - s0[k]);
+                if (to[k] > b[k] && v[k] < me) me = v[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (v[k] > me) to[k] -= 1;
+        x = to[0]; y = to[1]; z = to[2];
+    }
+
+    __device__ __forceinline__ int32_t gx() const { return x ^ fx; }
+    __device__ __forceinline__ int32_t gy() const { return y ^ fy; }
+    __device__ __forceinline__ int32_t gz() const { return z ^ fz; }
+};
 
 /* ---- 3D-DDA (dda.h:7-61) -----------------------------------------------------------
  * Returns 1 on hit, 0 when the march ended without a hit (position written),

@@ -23,7 +23,7 @@ struct TraceArgs {
     uint32_t* tile_counter;
     int32_t tiles_x, n_tiles;
     int32_t lds_bits;            /* stage occupancy bits in LDS */
-    int32_t lds_bits_p;          /* wavefront traversal: stage the padded block bits in LDS */
+    int32_t lds_bits_p;          /* wavefront traversal with statistics: stage the padded block bits in LDS */
     int32_t cdfv_lds_bytes;
     int32_t dda_budget;          /* wavefront traversal: DDA steps between refill checks */
     int32_t refill_min;          /* wavefront traversal: idle lanes that trigger a refill */
@@ -191,6 +191,13 @@ hipError_t launch_brick_from_ids(const BrickDims& d, const uint8_t* dense, const
  * set. */
 hipError_t launch_block_masks(const BrickDims& d, const uint8_t* bricks, uint64_t* occ64, uint32_t* bits,
                               uint64_t* occp, uint32_t* bitsp, uint64_t* occr, hipStream_t s);
+/* The jump march's codes (GridView::codes) from the padded masks: one byte
+ * per cell of 2^cg voxels in `cells` (padded by one cell, whose bytes stay
+ * zero; n_cells bytes, readable up to the next multiple of 16), then 16
+ * two-bit codes per word.  The largest coded cube has 2^top cells an edge
+ * (top 2 or 3), the next 2, the smallest 1. */
+hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint8_t* cells,
+                             uint64_t n_cells, uint32_t* codes, hipStream_t s);
 /* Bricked slots -> dense int32 offsets via slot_off[256]. */
 hipError_t launch_dense_from_bricks(const BrickDims& d, const uint8_t* bricks, const int32_t* slot_off, int32_t* dense,
                                     hipStream_t s);

@@ -134,6 +134,59 @@ __global__ __launch_bounds__(256) void block_masks_reversed_kernel(const uint64_
         occr[i] = __builtin_bitreverse64(occp[i]);
 }
 
+/* Bytes of the jump march's codes: one workgroup per aligned cube of the
+ * largest size (2^T cells an edge), one thread per cell, eight consecutive
+ * threads per 2x2x2 cells.  A cell is taken as occupied when any of its
+ * voxels is occupied or lies outside the grid (occp has those bits set), so
+ * no coded cube reaches past the grid.  codes bytes: see GridView::codes. */
+template <int T>
+__global__ __launch_bounds__(1 << (3 * T)) void cell_codes_kernel(BrickDims d, const uint64_t* __restrict__ occp,
+                                                                  uint32_t cg, int32_t ncx, int32_t ncy, int32_t ncz,
+                                                                  uint8_t* __restrict__ cells)
+{
+    const uint32_t t = threadIdx.x;
+    /* local cell: bit k of each coordinate from bits 3k, 3k+1, 3k+2 of the thread */
+    int32_t l[3] = { 0, 0, 0 };
+#pragma unroll
+    for (int k = 0; k < T; ++k)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) l[c] |= (int32_t)((t >> (3 * k + c)) & 1u) << k;
+    const int32_t cx = (int32_t)(blockIdx.x << T) + l[0], cy = (int32_t)(blockIdx.y << T) + l[1],
+                  cz = (int32_t)(blockIdx.z << T) + l[2];
+    const bool in = cx < ncx && cy < ncy && cz < ncz;
+    bool full = true;
+    if (in) {
+        const int32_t e = 1 << (cg - 2u);     /* 4x4x4 blocks per cell edge */
+        const int32_t x0 = cx * e, y0 = cy * e, z0 = cz * e;
+        full = x0 + e > d.kx || y0 + e > d.ky || z0 + e > d.kz;
+        const uint64_t px = (uint64_t)(d.kx + 2), py = (uint64_t)(d.ky + 2);
+        for (int32_t z = z0; z < z0 + e && !full; ++z)
+            for (int32_t y = y0; y < y0 + e && !full; ++y)
+                for (int32_t x = x0; x < x0 + e; ++x)
+                    full = full || occp[(uint64_t)(x + 1) + px * ((uint64_t)(y + 1) + py * (uint64_t)(z + 1))] != 0ull;
+    }
+    const unsigned long long m = __ballot(full);
+    const bool oct_full = ((m >> (t & 56u)) & 0xffull) != 0ull;
+    const bool top_full = T == 2 ? m != 0ull : __syncthreads_or(full) != 0;
+    if (in)
+        cells[(uint64_t)(cx + 1) + (uint64_t)(ncx + 2) * ((uint64_t)(cy + 1) + (uint64_t)(ncy + 2) * (uint64_t)(cz + 1))] =
+            full ? 0 : !top_full ? 3 : !oct_full ? 2 : 1;
+}
+
+/* 16 cell bytes -> one word of two-bit codes. */
+__global__ __launch_bounds__(256) void pack_codes_kernel(const uint4* __restrict__ cells, uint32_t n_words,
+                                                         uint32_t* __restrict__ codes)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_words) return;
+    const uint4 v = cells[i];
+    const uint32_t wd[4] = { v.x, v.y, v.z, v.w };
+    uint32_t out = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) out |= ((wd[k >> 2] >> (8 * (k & 3))) & 3u) << (2 * k);
+    codes[i] = out;
+}
+
 __global__ __launch_bounds__(256) void dense_from_bricks_kernel(BrickDims d, const uint8_t* __restrict__ bricks,
                                                                 const int32_t* __restrict__ slot_off,
                                                                 int32_t* __restrict__ dense)
@@ -204,6 +257,22 @@ hipError_t launch_block_masks(const BrickDims& d, const uint8_t* bricks, uint64_
     block_masks_padded_kernel<<<grid_for(np), 256, 0, s>>>(d, occ64, occp);
     block_bits_kernel<<<grid_for((np + 31) / 32), 256, 0, s>>>(np, occp, bitsp);
     if (occr) block_masks_reversed_kernel<<<grid_for(np), 256, 0, s>>>(occp, occr, np);
+    return hipGetLastError();
+}
+
+hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint8_t* cells,
+                             uint64_t n_cells, uint32_t* codes, hipStream_t s)
+{
+    const int32_t e = 1 << cg;
+    const int32_t nx = (d.nx + e - 1) / e, ny = (d.ny + e - 1) / e, nz = (d.nz + e - 1) / e;
+    const uint32_t c = 1u << top;
+    const dim3 grid(((uint32_t)nx + c - 1) / c, ((uint32_t)ny + c - 1) / c, ((uint32_t)nz + c - 1) / c);
+    if (top == 2u)
+        cell_codes_kernel<2><<<grid, 64, 0, s>>>(d, occp, cg, nx, ny, nz, cells);
+    else
+        cell_codes_kernel<3><<<grid, 512, 0, s>>>(d, occp, cg, nx, ny, nz, cells);
+    const uint32_t words = (uint32_t)((n_cells + 15) / 16);
+    pack_codes_kernel<<<(words + 255) / 256, 256, 0, s>>>((const uint4*)cells, words, codes);
     return hipGetLastError();
 }
 
