@@ -10,6 +10,7 @@
 #include "../../include/vt_api.h"
 #include "vt_kernels.h"
 #include "vt_cache.h"
+#include "vt_staging.h"
 #include "../host/vt_host_algos.h"
 
 #include <algorithm>
@@ -137,6 +138,28 @@ int noalloc_lookup(int device)
 }
 }  // namespace
 
+/* Staging rings (vt_staging.h) and the contexts that share them, per device.
+ * A ring object is never destroyed, only emptied: the process may end with
+ * contexts alive. */
+namespace {
+std::mutex g_ring_lock;
+vt::StagingRing* g_ring[VT_MAX_DEVICES] = {};
+int g_ring_users[VT_MAX_DEVICES] = {};
+
+void ring_join(int device)
+{
+    std::lock_guard<std::mutex> lk(g_ring_lock);
+    if (!g_ring[device]) g_ring[device] = new vt::StagingRing();
+    ++g_ring_users[device];
+}
+
+void ring_leave(int device)
+{
+    std::lock_guard<std::mutex> lk(g_ring_lock);
+    if (--g_ring_users[device] == 0) g_ring[device]->release();
+}
+}  // namespace
+
 struct vt_context {
     /* batches and caches built on this context; destroying the context
      * releases their device memory and leaves them unusable (their own
@@ -144,6 +167,7 @@ struct vt_context {
     std::vector<vt_batch*> batches;
     std::vector<vt_cache*> caches;
     int device = 0;
+    vt::StagingRing* ring = nullptr;   /* the device's, for large copies */
     int cus = 0;
     size_t lds_limit = 65536;       /* dynamic LDS per workgroup */
     hipStream_t stream = nullptr;
@@ -217,6 +241,21 @@ struct vt_context {
 };
 
 namespace {
+
+/* Copies between the caller's memory and the device, on the context's
+ * stream: device memory to host, complete on return; host memory to device,
+ * the host memory free on return. */
+hipError_t to_host(vt_context* c, void* dst, const void* src, size_t bytes)
+{
+    if (bytes >= vt::StagingRing::MIN_BYTES) return c->ring->read(dst, src, bytes, c->stream);
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
+    return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
+}
+hipError_t to_device(vt_context* c, void* dst, const void* src, size_t bytes)
+{
+    if (bytes >= vt::StagingRing::MIN_BYTES) return c->ring->write(dst, src, bytes, c->stream);
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream);
+}
 
 float mat_at(const std::vector<float>& m, int64_t i) { return (i < 0 || i >= (int64_t)m.size()) ? 0.0f : m[(size_t)i]; }
 
@@ -537,8 +576,10 @@ int vt_create(int device, vt_context** out)
         if (int r = noalloc_lookup(device)) return r;
         vt_context* c = new vt_context();
         c->device = device;
+        ring_join(device);
+        c->ring = g_ring[device];
         hipDeviceProp_t prop;
-        if (hipGetDeviceProperties(&prop, device) != hipSuccess) { delete c; return fail(VT_ERR_HIP, "device query failed"); }
+        if (hipGetDeviceProperties(&prop, device) != hipSuccess) { ring_leave(device); delete c; return fail(VT_ERR_HIP, "device query failed"); }
         c->cus = prop.multiProcessorCount;
         c->lds_limit = prop.sharedMemPerBlock;
         if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
@@ -586,6 +627,7 @@ void vt_destroy(vt_context* c)
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     for (hipEvent_t e : c->lt_ev) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    ring_leave(c->device);
     delete c;
 }
 
@@ -637,7 +679,7 @@ int vt_set_volume(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const int32
         VT_HIP(hipMalloc(&d_dense.p, (size_t)nvox * 4u));
         VT_HIP(hipMalloc(&d_lut.p, lut.size()));
         VT_HIP(hipMalloc(&d_bad.p, 4));
-        VT_HIP(hipMemcpyAsync(d_dense.p, offsets, (size_t)nvox * 4u, hipMemcpyHostToDevice, c->stream));
+        VT_HIP(to_device(c, d_dense.p, offsets, (size_t)nvox * 4u));
         VT_HIP(hipMemcpyAsync(d_lut.p, lut.data(), lut.size(), hipMemcpyHostToDevice, c->stream));
         VT_HIP(vt::launch_fill_u32(d_bad.p, 1, 0u, c->stream));
         VT_HIP(vt::launch_brick_from_offsets(c->dims, d_dense.p, d_lut.p, mat_size, c->d_bricks, d_bad.p, c->stream));
@@ -682,7 +724,7 @@ int vt_set_volume_u8(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const ui
         DevTmp<uint8_t> d_remap;
         VT_HIP(hipMalloc(&d_dense.p, (size_t)nvox));
         VT_HIP(hipMalloc(&d_remap.p, 256));
-        VT_HIP(hipMemcpyAsync(d_dense.p, ids, (size_t)nvox, hipMemcpyHostToDevice, c->stream));
+        VT_HIP(to_device(c, d_dense.p, ids, (size_t)nvox));
         VT_HIP(hipMemcpyAsync(d_remap.p, remap, 256, hipMemcpyHostToDevice, c->stream));
         VT_HIP(vt::launch_brick_from_ids(c->dims, d_dense.p, d_remap.p, c->d_bricks, c->stream));
         VT_HIP(hipStreamSynchronize(c->stream));
@@ -719,8 +761,7 @@ int vt_read_volume(vt_context* c, int32_t* offsets)
         VT_HIP(hipMalloc(&d_table.p, sizeof(table)));
         VT_HIP(hipMemcpyAsync(d_table.p, table, sizeof(table), hipMemcpyHostToDevice, c->stream));
         VT_HIP(vt::launch_dense_from_bricks(c->dims, c->d_bricks, d_table.p, d_dense.p, c->stream));
-        VT_HIP(hipMemcpyAsync(offsets, d_dense.p, (size_t)nvox * 4u, hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
+        VT_HIP(to_host(c, offsets, d_dense.p, (size_t)nvox * 4u));
         return VT_OK;
     });
 }
@@ -785,8 +826,8 @@ int vt_set_environment(vt_context* c, const vt_environment* env)
             if (he == hipSuccess) he = hipMalloc(&cdfu, nu * 4);
             if (he == hipSuccess) he = hipMalloc(&cdfv, (size_t)e.cdf_v_n * 4);
             if (he == hipSuccess) he = hipMalloc(&quad, (size_t)(e.image_w + 1) * (size_t)(e.image_h + 1) * 64);
-            if (he == hipSuccess) he = hipMemcpyAsync(img, e.image_rgb, ni * 4, hipMemcpyHostToDevice, c->stream);
-            if (he == hipSuccess) he = hipMemcpyAsync(cdfu, e.cdf_u, nu * 4, hipMemcpyHostToDevice, c->stream);
+            if (he == hipSuccess) he = to_device(c, img, e.image_rgb, ni * 4);
+            if (he == hipSuccess) he = to_device(c, cdfu, e.cdf_u, nu * 4);
             if (he == hipSuccess)
                 he = hipMemcpyAsync(cdfv, e.cdf_v, (size_t)e.cdf_v_n * 4, hipMemcpyHostToDevice, c->stream);
             if (he == hipSuccess) he = vt::launch_env_quads(img, e.image_w, e.image_h, quad, c->stream);
@@ -1514,8 +1555,8 @@ int cache_upload_samples(vt_cache* c, int64_t n, const float* raw, const float* 
         VT_HIP(hipMalloc(&c->d_tgt, (size_t)n * vt::MLP_OUT * 4));
         c->cap = n;
     }
-    VT_HIP(hipMemcpyAsync(c->d_raw, raw, (size_t)n * vt::MLP_RAW * 4, hipMemcpyHostToDevice, s));
-    VT_HIP(hipMemcpyAsync(c->d_tgt, target, (size_t)n * vt::MLP_OUT * 4, hipMemcpyHostToDevice, s));
+    VT_HIP(to_device(c->ctx, c->d_raw, raw, (size_t)n * vt::MLP_RAW * 4));
+    VT_HIP(to_device(c->ctx, c->d_tgt, target, (size_t)n * vt::MLP_OUT * 4));
     VT_HIP(vt::launch_fill_u32(c->d_nsamp, 1, (uint32_t)n, s));
     return VT_OK;
 }
@@ -1710,10 +1751,9 @@ int vt_cache_infer(vt_cache* c, int64_t n, const float* raw, float* out)
             VT_HIP(hipMalloc(&c->d_iout, (size_t)n * vt::MLP_OUT * 4));
             c->icap = n;
         }
-        VT_HIP(hipMemcpyAsync(c->d_iraw, raw, (size_t)n * vt::MLP_RAW * 4, hipMemcpyHostToDevice, s));
+        VT_HIP(to_device(c->ctx, c->d_iraw, raw, (size_t)n * vt::MLP_RAW * 4));
         VT_HIP(vt::launch_mlp_infer(c->d_pack, c->d_bias, c->d_iraw, c->d_iout, n, c->ctx->cus, s));
-        VT_HIP(hipMemcpyAsync(out, c->d_iout, (size_t)n * vt::MLP_OUT * 4, hipMemcpyDeviceToHost, s));
-        VT_HIP(hipStreamSynchronize(s));
+        VT_HIP(to_host(c->ctx, out, c->d_iout, (size_t)n * vt::MLP_OUT * 4));
         return VT_OK;
     });
 }
@@ -1967,8 +2007,7 @@ int vt_read_accum(vt_context* c, float* rgba)
         if (!c || !rgba) return fail(VT_ERR_ARG, "null argument");
         if (!c->d_accum) return fail(VT_ERR_STATE, "no frame");
         VT_HIP(hipSetDevice(c->device));
-        VT_HIP(hipMemcpyAsync(rgba, c->d_accum, (size_t)c->W * c->H * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
+        VT_HIP(to_host(c, rgba, c->d_accum, (size_t)c->W * c->H * sizeof(float4)));
         return VT_OK;
     });
 }
@@ -1979,8 +2018,7 @@ int vt_read_sum64(vt_context* c, double* rgb)
         if (!c || !rgb) return fail(VT_ERR_ARG, "null argument");
         if (!c->d_sum64) return fail(VT_ERR_STATE, "frame has no FP64 sums");
         VT_HIP(hipSetDevice(c->device));
-        VT_HIP(hipMemcpyAsync(rgb, c->d_sum64, (size_t)c->W * c->H * 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
+        VT_HIP(to_host(c, rgb, c->d_sum64, (size_t)c->W * c->H * 3 * sizeof(double)));
         return VT_OK;
     });
 }
@@ -1991,7 +2029,7 @@ int vt_write_accum(vt_context* c, const float* rgba)
         if (!c || !rgba) return fail(VT_ERR_ARG, "null argument");
         if (!c->d_accum) return fail(VT_ERR_STATE, "no frame");
         VT_HIP(hipSetDevice(c->device));
-        VT_HIP(hipMemcpyAsync(c->d_accum, rgba, (size_t)c->W * c->H * sizeof(float4), hipMemcpyHostToDevice, c->stream));
+        VT_HIP(to_device(c, c->d_accum, rgba, (size_t)c->W * c->H * sizeof(float4)));
         VT_HIP(hipStreamSynchronize(c->stream));
         return VT_OK;
     });
@@ -2003,7 +2041,7 @@ int vt_write_sum64(vt_context* c, const double* rgb)
         if (!c || !rgb) return fail(VT_ERR_ARG, "null argument");
         if (!c->d_sum64) return fail(VT_ERR_STATE, "frame has no FP64 sums");
         VT_HIP(hipSetDevice(c->device));
-        VT_HIP(hipMemcpyAsync(c->d_sum64, rgb, (size_t)c->W * c->H * 3 * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        VT_HIP(to_device(c, c->d_sum64, rgb, (size_t)c->W * c->H * 3 * sizeof(double)));
         VT_HIP(hipStreamSynchronize(c->stream));
         return VT_OK;
     });
@@ -2043,8 +2081,7 @@ int vt_trace_first_hit(vt_context* c, uint64_t seed, uint32_t frame, int32_t* re
         DevTmp<int32_t> d;
         VT_HIP(hipMalloc(&d.p, bytes));
         VT_HIP(vt::launch_first_hit(a, d.p, c->stream));
-        VT_HIP(hipMemcpyAsync(rec, d.p, bytes, hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
+        VT_HIP(to_host(c, rec, d.p, bytes));
         return VT_OK;
     });
 }
@@ -2063,11 +2100,10 @@ int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, in
         VT_HIP(hipMalloc(&d_o.p, (size_t)n * 12));
         VT_HIP(hipMalloc(&d_d.p, (size_t)n * 12));
         VT_HIP(hipMalloc(&d_r.p, (size_t)n * 32));
-        VT_HIP(hipMemcpyAsync(d_o.p, o, (size_t)n * 12, hipMemcpyHostToDevice, c->stream));
-        VT_HIP(hipMemcpyAsync(d_d.p, dir, (size_t)n * 12, hipMemcpyHostToDevice, c->stream));
+        VT_HIP(to_device(c, d_o.p, o, (size_t)n * 12));
+        VT_HIP(to_device(c, d_d.p, dir, (size_t)n * 12));
         VT_HIP(vt::launch_trace_rays(a, n, d_o.p, d_d.p, d_r.p, c->stream));
-        VT_HIP(hipMemcpyAsync(rec, d_r.p, (size_t)n * 32, hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
+        VT_HIP(to_host(c, rec, d_r.p, (size_t)n * 32));
         return VT_OK;
     });
 }
@@ -2138,8 +2174,8 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
         if (ntri > 0) {
             VT_HIP(hipMalloc(&d_v.p, (size_t)nv * 12));
             VT_HIP(hipMalloc(&d_i.p, (size_t)ntri * 12));
-            VT_HIP(hipMemcpyAsync(d_v.p, verts, (size_t)nv * 12, hipMemcpyHostToDevice, c->stream));
-            VT_HIP(hipMemcpyAsync(d_i.p, idx, (size_t)ntri * 12, hipMemcpyHostToDevice, c->stream));
+            VT_HIP(to_device(c, d_v.p, verts, (size_t)nv * 12));
+            VT_HIP(to_device(c, d_i.p, idx, (size_t)ntri * 12));
         }
         if (occupancy) {
             VT_HIP(hipMalloc(&d_occ.p, (size_t)nvox));
@@ -2165,7 +2201,7 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
             int r = refresh_occupancy(c);
             if (r != VT_OK) return r;
         }
-        if (occupancy) VT_HIP(hipMemcpyAsync(occupancy, d_occ.p, (size_t)nvox, hipMemcpyDeviceToHost, c->stream));
+        if (occupancy) VT_HIP(to_host(c, occupancy, d_occ.p, (size_t)nvox));
         VT_HIP(hipStreamSynchronize(c->stream));
         return VT_OK;
     });

@@ -1,0 +1,276 @@
+/*
+ * vt_staging.h - large copies between pageable host memory and the device.
+ *
+ * The runtime's own pageable copy moves 1 MiB at a time through a staging
+ * buffer, one thread copying while the device waits and the device copying
+ * while the thread waits (about 90 us a MiB on an MI355X host: 20 us on the
+ * link, 70 us in memcpy and page faults).  Here a ring of pinned chunks keeps
+ * the link busy while several threads move the chunks to or from the caller's
+ * memory.  The link is driven by a copy kernel over the pinned chunk: 2 MiB at
+ * a time it moves 52 GB/s either way, the runtime's copies 24 GB/s to the
+ * device and 46 GB/s from it (56 GB/s in one piece).
+ *
+ * One ring and its threads per device, shared by the device's contexts: made
+ * by the first large copy, given back when the last context is destroyed.  A
+ * copy that finds the ring in use by another thread, or whose ring could not
+ * be made, takes the runtime's path.
+ */
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <stdint.h>
+
+#include <atomic>
+#include <condition_variable>
+#include <cstring>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace vt {
+
+/* Copy kernel between device memory and a pinned chunk, both 16-byte aligned
+ * (vt_volume.hip). */
+hipError_t launch_copy_chunk(const void* src, void* dst, size_t bytes, hipStream_t s);
+
+class StagingRing {
+public:
+    static constexpr size_t CHUNK = 2u << 20;      /* one transfer of the link */
+    static constexpr size_t PIECE = 128u << 10;    /* one thread's copy */
+    static constexpr int SLOTS = 6;
+    static constexpr int WORKERS = 3;              /* besides the calling thread */
+    static constexpr size_t MIN_BYTES = 1u << 20;  /* smaller copies take the runtime's path */
+
+    static constexpr int PIECES = (int)(CHUNK / PIECE);
+
+    /* Device to host; complete when it returns. */
+    hipError_t read(void* dst, const void* src, size_t bytes, hipStream_t s)
+    {
+        std::unique_lock<std::mutex> lk(use_, std::try_to_lock);
+        if (!lk.owns_lock() || !make()) {
+            const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+            return e != hipSuccess ? e : hipStreamSynchronize(s);
+        }
+        hipError_t err = settle();
+        if (err != hipSuccess) return err;
+        begin((char*)dst, bytes, false);
+        const int n = chunks_;
+        int issued = 0, arrived = 0;
+        while (arrived < n && err == hipSuccess) {
+            /* a slot is free again once its last chunk is out of it */
+            while (issued < n && err == hipSuccess && (issued < SLOTS || copied_[issued % SLOTS].load(std::memory_order_acquire) ==
+                                                                             goal(issued - SLOTS))) {
+                const size_t off = (size_t)issued * CHUNK;
+                if (issued >= SLOTS) copied_[issued % SLOTS].store(0, std::memory_order_relaxed);
+                err = launch_copy_chunk((const char*)src + off, slot_[issued % SLOTS], length(issued), s);
+                if (err == hipSuccess) err = hipEventRecord(ev_[issued % SLOTS], s);
+                if (err == hipSuccess) ++issued;
+            }
+            if (err == hipSuccess && arrived < issued) {
+                err = hipEventSynchronize(ev_[arrived % SLOTS]);
+                if (err == hipSuccess) open_.store(++arrived, std::memory_order_release);
+            } else if (err == hipSuccess) {
+                help();
+            }
+        }
+        if (err != hipSuccess) abandon_.store(true, std::memory_order_release);
+        finish();
+        if (err != hipSuccess) (void)hipStreamSynchronize(s);
+        return err;
+    }
+
+    /* Host to device, ordered on the stream; the host memory is free again
+     * when it returns. */
+    hipError_t write(void* dst, const void* src, size_t bytes, hipStream_t s)
+    {
+        std::unique_lock<std::mutex> lk(use_, std::try_to_lock);
+        if (!lk.owns_lock() || !make()) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+        hipError_t err = settle();
+        if (err != hipSuccess) return err;
+        begin((char*)const_cast<void*>(src), bytes, true);
+        const int n = chunks_;
+        int issued = 0, drained = 0;
+        open_.store(n < SLOTS ? n : SLOTS, std::memory_order_release);
+        while (issued < n && err == hipSuccess) {
+            if (issued < open_.load(std::memory_order_relaxed) &&
+                copied_[issued % SLOTS].load(std::memory_order_acquire) == goal(issued)) {
+                err = launch_copy_chunk(slot_[issued % SLOTS], (char*)dst + (size_t)issued * CHUNK, length(issued), s);
+                if (err == hipSuccess) err = hipEventRecord(ev_[issued % SLOTS], s);
+                if (err == hipSuccess) ++issued;
+            } else if (drained < issued && open_.load(std::memory_order_relaxed) < n &&
+                       hipEventQuery(ev_[drained % SLOTS]) == hipSuccess) {
+                copied_[drained % SLOTS].store(0, std::memory_order_relaxed);
+                ++drained;
+                open_.store(drained + SLOTS < n ? drained + SLOTS : n, std::memory_order_release);
+            } else {
+                (void)hipGetLastError();   /* hipErrorNotReady of the query */
+                help();
+            }
+        }
+        if (err != hipSuccess) abandon_.store(true, std::memory_order_release);
+        finish();
+        in_flight_ = true;
+        return err;
+    }
+
+    /* Ends the threads and frees the ring; no copy may be running. */
+    void release()
+    {
+        std::lock_guard<std::mutex> lk(use_);
+        if (!made_) return;
+        (void)settle();
+        {
+            std::lock_guard<std::mutex> g(wake_lock_);
+            quit_ = true;
+        }
+        wake_.notify_all();
+        for (std::thread& t : threads_) t.join();
+        threads_.clear();
+        quit_ = false;
+        free_slots();
+        made_ = false;
+    }
+
+private:
+    size_t length(int chunk) const
+    {
+        const size_t off = (size_t)chunk * CHUNK;
+        return total_ - off < CHUNK ? total_ - off : CHUNK;
+    }
+    int goal(int chunk) const { return (int)((length(chunk) + PIECE - 1) / PIECE); }
+
+    bool make()
+    {
+        if (made_) return true;
+        for (int k = 0; k < SLOTS; ++k) {
+            if (hipHostMalloc(&slot_[k], CHUNK, hipHostMallocDefault) != hipSuccess ||
+                hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                free_slots();
+                return false;
+            }
+        }
+        try {
+            for (int k = 0; k < WORKERS; ++k) threads_.emplace_back([this] { work(); });
+        } catch (...) {
+            /* fewer threads copy, the caller at least */
+        }
+        made_ = true;
+        return true;
+    }
+
+    void free_slots()
+    {
+        for (int k = 0; k < SLOTS; ++k) {
+            if (slot_[k]) (void)hipHostFree(slot_[k]);
+            if (ev_[k]) (void)hipEventDestroy(ev_[k]);
+            slot_[k] = nullptr;
+            ev_[k] = nullptr;
+        }
+    }
+
+    /* the last write's chunks have left the ring */
+    hipError_t settle()
+    {
+        if (!in_flight_) return hipSuccess;
+        in_flight_ = false;
+        for (int k = 0; k < SLOTS; ++k) {
+            const hipError_t e = hipEventSynchronize(ev_[k]);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+
+    void begin(char* host, size_t bytes, bool to_ring)
+    {
+        host_ = host;
+        total_ = bytes;
+        to_ring_ = to_ring;
+        chunks_ = (int)((bytes + CHUNK - 1) / CHUNK);
+        pieces_ = (int64_t)((bytes + PIECE - 1) / PIECE);
+        for (int k = 0; k < SLOTS; ++k) copied_[k].store(0, std::memory_order_relaxed);
+        next_.store(0, std::memory_order_relaxed);
+        done_.store(0, std::memory_order_relaxed);
+        open_.store(0, std::memory_order_relaxed);
+        abandon_.store(false, std::memory_order_relaxed);
+        {
+            std::lock_guard<std::mutex> g(wake_lock_);
+            ++job_;
+            active_.store(true, std::memory_order_release);
+        }
+        wake_.notify_all();
+    }
+
+    /* One piece of an open chunk; false when there is none now. */
+    bool help()
+    {
+        int64_t p = next_.load(std::memory_order_relaxed);
+        for (;;) {
+            if (p >= pieces_ || p / PIECES >= open_.load(std::memory_order_acquire)) return false;
+            if (next_.compare_exchange_weak(p, p + 1, std::memory_order_acq_rel)) break;
+        }
+        const int chunk = (int)(p / PIECES);
+        const size_t off = (size_t)p * PIECE;
+        const size_t len = total_ - off < PIECE ? total_ - off : PIECE;
+        char* ring = (char*)slot_[chunk % SLOTS] + (off - (size_t)chunk * CHUNK);
+        if (to_ring_) std::memcpy(ring, host_ + off, len);
+        else std::memcpy(host_ + off, ring, len);
+        copied_[chunk % SLOTS].fetch_add(1, std::memory_order_acq_rel);
+        done_.fetch_add(1, std::memory_order_acq_rel);
+        return true;
+    }
+
+    /* every piece that was taken is copied (all of them, unless abandoned),
+     * and no thread looks at the job any more */
+    void finish()
+    {
+        while (!abandon_.load(std::memory_order_acquire) && done_.load(std::memory_order_acquire) < pieces_) help();
+        active_.store(false, std::memory_order_release);
+        while (busy_.load(std::memory_order_acquire) != 0) std::this_thread::yield();
+    }
+
+    void work()
+    {
+        uint64_t seen = 0;
+        for (;;) {
+            {
+                std::unique_lock<std::mutex> g(wake_lock_);
+                wake_.wait(g, [&] { return quit_ || job_ != seen; });
+                if (quit_) return;
+                seen = job_;
+                busy_.fetch_add(1, std::memory_order_acq_rel);
+            }
+            /* a copy is at most some milliseconds long: look for pieces until
+             * all are taken (a thread that wakes late finds no active job, or
+             * the next one, which waits for it as well) */
+            while (active_.load(std::memory_order_acquire) && !abandon_.load(std::memory_order_acquire) &&
+                   next_.load(std::memory_order_relaxed) < pieces_)
+                if (!help()) std::this_thread::yield();
+            busy_.fetch_sub(1, std::memory_order_acq_rel);
+        }
+    }
+
+    std::mutex use_;
+    bool made_ = false, in_flight_ = false;
+    void* slot_[SLOTS] = {};
+    hipEvent_t ev_[SLOTS] = {};
+    std::vector<std::thread> threads_;
+    /* the copy in progress */
+    char* host_ = nullptr;
+    size_t total_ = 0;
+    bool to_ring_ = false;
+    int chunks_ = 0;
+    int64_t pieces_ = 0;
+    std::atomic<int> copied_[SLOTS];
+    std::atomic<int64_t> next_{ 0 }, done_{ 0 };
+    std::atomic<int> open_{ 0 };
+    std::atomic<bool> abandon_{ false }, active_{ false };
+    std::atomic<int> busy_{ 0 };
+    std::mutex wake_lock_;
+    std::condition_variable wake_;
+    uint64_t job_ = 0;
+    bool quit_ = false;
+};
+
+}  // namespace vt
