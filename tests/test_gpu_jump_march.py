@@ -49,7 +49,7 @@ def workload_of(shape, lens, width, height, rng):
 # 16 and 32; cells of 8 (too many of 4 for the LDS); one cell; slabs
 @pytest.mark.parametrize("shape,lens", [((4, 4, 4), 0), ((5, 3, 9), 1), ((33, 31, 32), 0), ((64, 17, 65), 2),
                                         ((21, 45, 224), 1), ((37, 16, 229), 0), ((256, 40, 255), 2),
-                                        ((1, 64, 64), 0), ((264, 264, 266), 0), ((272, 270, 275), 1)])
+                                        ((1, 64, 64), 0), ((264, 264, 266), 0), ((272, 270, 275), 1), ((6, 7, 4096), 0)])
 def test_jump_march_equals_step_by_step(ctx, shape, lens):
     from voxeltoy_amd import workloads
     rng = np.random.default_rng(sum(shape) + lens)

@@ -1,7 +1,8 @@
 """CPU emulation of the jump march (JumpState in voxeltoy_amd/csrc/vt_device.h)
 against the oracle's raymarch (src/shaders/shared/dda.h:7-61): empty-cube codes
 built as cell_codes_kernel builds them, positions from the real-line values
-with the error bound, undecided jumps from the exact FP32 sums.  Every table
+with the error bound, undecided jumps by the voxels they could skip and else
+from the exact FP32 sums.  Every table
 read must fall inside its table, the voxel a ray stops in must be the
 oracle's, and every jump must move."""
 import numpy as np
@@ -63,7 +64,7 @@ def sum_steps(X, a, ia, n):
         ub = int(X.view(np.uint32)) & 0x7F800000
         if n > 0 and ub == (int(p.view(np.uint32)) & 0x7F800000):
             end = np.uint32(ub + 0x00800000).view(F)
-            r = min(int(F(F(end - X) * F(ia))) - 3, n)
+            r = min(int(F(F(end - X) * F(ia))) - 2, n)
             if r > 0:
                 X = fma(F(r), F(F(X + a) - X), X)
                 n -= r
@@ -82,9 +83,9 @@ def march(occ, tables, cg, res, bmin, bmax, o, d):
     dc = [F(1e-5) if F(1e-5) >= abs(F(v)) else F(v) for v in d]
     inc = [F(1.0) / v for v in dc]
     sg = [1 if v > 0 else -1 for v in dc]
-    X0 = [F(F(F(F(vp[i] - vo[i]) + F(0.5)) + F(F(sg[i]) * F(0.5))) * inc[i]) for i in range(3)]
     a = [F(abs(v)) for v in inc]
-    if not all(F(0.99) <= a[i] <= F(2e5) and 0 <= X0[i] <= F(a[i] * F(1.001)) for i in range(3)):
+    X0 = [F(F(abs(F(F(F(vp[i] - vo[i]) + F(0.5)) + F(F(sg[i]) * F(0.5))))) * a[i]) for i in range(3)]
+    if not all(F(2.0 ** -10) <= a[i] <= F(2e5) and X0[i] <= F(2e5) for i in range(3)):
         return "stepwise", 0
     ia = [F(1.0) / v for v in a]
     f = [-1 if s < 0 else 0 for s in sg]
@@ -92,6 +93,7 @@ def march(occ, tables, cg, res, bmin, bmax, o, d):
     p0 = list(p)
     q = [fma(-X0[i], ia[i], F(p0[i] + 1)) for i in range(3)]
     c0 = F(ULP24 * F(2 * max(res) + 32))
+    w1 = F(W1 * max(ia))
     undecided = 0
     for _ in range(sum(res) + 8):
         u = [p[i] ^ f[i] for i in range(3)]
@@ -109,28 +111,48 @@ def march(occ, tables, cg, res, bmin, bmax, o, d):
                 return tuple(u), undecided
         b = [v | edge for v in p]
         m = min(fma(F(b[i] - p0[i]), a[i], X0[i]) for i in range(3))
-        w = fma(m, W1, W4)
+        w = fma(m, w1, W4)
         dl = fma(w, w, c0)
         pq = [F(fma(m, ia[i], q[i]) + dl) for i in range(3)]
         fr = [F(v - F(np.floor(v))) for v in pq]
         to = [int(np.floor(v)) for v in pq]
         if sorted(fr)[1] < dl + dl:
-            undecided += 1
-            v = [F(0)] * 3
-            me = F(np.inf)
-            for i in range(3):
-                if fr[i] < dl + dl and to[i] > p[i]:
-                    v[i] = sum_steps(X0[i], a[i], ia[i], to[i] - 1 - p0[i])
-                    if to[i] > b[i]:
-                        me = min(me, v[i])
-            to = [to[i] - 1 if v[i] > me else to[i] for i in range(3)]
+            d2 = dl + dl
+            near = [fr[i] < d2 and to[i] > p[i] for i in range(3)]
+            sums = all(near)
+            if sum(near) == 2:
+                am = max(a[i] for i in range(3) if near[i])
+                e = [F(d2 * fma(am, ia[i], F(1))) for i in range(3)]
+                sums = not max(e) < F(0.4) or any(
+                    not near[i] and ((to[i] > p[i] and fr[i] < e[i]) or fr[i] > F(1) - e[i]) for i in range(3))
+                for i in range(3):
+                    if near[i] and not sums:
+                        v = [(to[j] - (j == i)) ^ f[j] for j in range(3)]
+                        bi = [(c + 4) >> 2 for c in v]
+                        assert all(0 <= bi[j] < masks.shape[2 - j] for j in range(3))
+                        sums = masks[bi[2], bi[1], bi[0]][(v[0] & 3) | ((v[1] & 3) << 2) | ((v[2] & 3) << 4)]
+            if sums:
+                undecided += 1
+                t = [fma(F(b[i] - p0[i]), a[i], X0[i]) for i in range(3)]
+                first = a[t.index(m)]
+                cand = [i for i in range(3) if F(t[i] - m) <= F(d2 * F(a[i] + first))]
+                m = min(sum_steps(X0[i], a[i], ia[i], b[i] - p0[i]) for i in cand)
+                w = fma(m, w1, W4)
+                dl = fma(w, w, c0)
+                for i in range(3):
+                    pv = F(fma(m, ia[i], q[i]) + dl)
+                    to[i] = int(np.floor(pv))
+                    if F(pv - F(np.floor(pv))) < dl + dl:
+                        while to[i] > p[i] and sum_steps(X0[i], a[i], ia[i], to[i] - 1 - p0[i]) > m:
+                            to[i] -= 1
         assert to != p and all(p[i] <= to[i] <= b[i] + 1 for i in range(3))
         p = to
     raise AssertionError("the march did not stop")
 
 
 @pytest.mark.parametrize("shape,cg,top", [((16, 16, 16), 2, 2), ((20, 33, 65), 2, 2), ((7, 9, 230), 2, 3),
-                                          ((48, 24, 64), 3, 2), ((40, 96, 33), 4, 2), ((1, 1, 5), 2, 2)])
+                                          ((48, 24, 64), 3, 2), ((40, 96, 33), 4, 2), ((1, 1, 5), 2, 2),
+                                          ((2, 6, 4096), 2, 3)])
 def test_jump_march_stops_where_the_oracle_does(orc, shape, cg, top):
     nz, ny, nx = shape
     res = (nx, ny, nz)
@@ -152,7 +174,14 @@ def test_jump_march_stops_where_the_oracle_does(orc, shape, cg, top):
     o[80:140] = lo + rng.integers(0, np.array(res) + 1, (60, 3)) * vs             # from voxel corners
     o[200:, 1] = hi[1] - 1e-3 * vs[1]
     d[200:, 1] = -np.abs(d[200:, 1])
+    # past voxel edges at distances from 1e-7 to 1e-3 voxels, half of them along steep axes
+    near = (rng.integers(0, np.array(res) + 1, (60, 3)) + rng.normal(0, 1, (60, 3)) * 10.0 ** rng.uniform(-7, -3, (60, 1)))
+    near[np.arange(60), rng.integers(0, 3, 60)] += 0.37
+    d[140:200] = rng.standard_normal((60, 3))
+    d[np.arange(140, 200), rng.integers(0, 3, 60)] *= 10.0 ** rng.uniform(-3.5, 0, 60)
+    o[140:200] = lo + near * vs - d[140:200] / np.abs(d[140:200]).max(1, keepdims=True) * rng.uniform(0, 0.6, (60, 1)) * (hi - lo)
     d /= np.linalg.norm(d, axis=1, keepdims=True)
+    d[::9] *= rng.choice([0.3, 4.0, 50.0], (len(d[::9]), 1))           # not unit
     o, d = o.astype(np.float32), d.astype(np.float32)
     want = sc.trace_rays(o, d)
     undecided = stepwise = 0

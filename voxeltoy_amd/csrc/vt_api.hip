@@ -513,7 +513,7 @@ vt::TraceArgs trace_args(const vt_context* c)
     a.cdfv_lds_bytes = c->env.use_image ? ((c->env.cdf_v_n * 4 + 15) / 16) * 16 : 0;
     const size_t base = 256 * sizeof(vt::MatRec) + (size_t)a.cdfv_lds_bytes;
     a.lds_bits = (base + (size_t)c->bit_words * 4u <= c->lds_limit) ? 1 : 0;
-    a.lds_bits_p = ((size_t)c->bit_words_p * 4u <= c->lds_limit) ? 1 : 0;
+    a.lds_bits_p = ((size_t)c->bit_words_p * 4u + 16u <= c->lds_limit) ? 1 : 0;   /* and the list counter */
     a.dda_budget = c->dda_budget;
     a.refill_min = c->refill_min;
     a.refill_chunk = c->refill_chunk;

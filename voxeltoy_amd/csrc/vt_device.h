@@ -724,28 +724,33 @@ __device__ __forceinline__ int DdaState::advance_wave_packed(const GridView& g, 
  * steps out of the cube, then the three counts.
  *
  * Values and counts are evaluated on the real line X_0 + k a.  Every add of
- * the FP32 sums is off by at most half an ulp, so with M the largest count
- * (m, as a >= 0.99) the two sequences that a decision compares are together
- * off their lines by at most 2^-24 (M^2 + 3M) steps, and the evaluation itself
- * by 2^-24 (3M + 2 extent + 8); del = 2^-24 (1.06 (M + 4)^2 + 2 extent + 32)
- * covers both.  With q the real-valued position (an integer where an axis
+ * the FP32 sums is off by at most half an ulp, so with M = m / (smallest a) the
+ * two sequences that a decision compares are together off their lines by at
+ * most 2^-24 (M^2 + 3M) steps, and the evaluation itself by 2^-24 (3M + 2
+ * extent + 8); del = 2^-24 (1.06 (M + 4)^2 + 2 extent + 32) covers both.  With q the real-valued position (an integer where an axis
  * steps), floor(q + del) is the exact position unless q lies within del of an
  * integer; on the axis that leaves the cube it always does, and it is then
  * right as well.  When a second axis is that near an integer the order of the
- * two steps is undecided (0.1-0.3 % of the jumps): jump() leaves the position
+ * two steps is undecided (0.1-0.3 % of the jumps).  Both orders and a common
+ * step end in the same voxel, by way of one of the two voxels where one of the
+ * steps is still missing: if both are empty the ray passes and the order does
+ * not matter.  That holds when no other step can fall between the two, which
+ * are at most 2 del a apart (a: the longer step of the two axes): the third
+ * axis must be 2 del (1 + a / its step) from an integer on either side.
+ * Otherwise (10-19 % of the undecided jumps) jump() leaves the position
  * unchanged and resolve() compares the FP32 sums themselves.
  *
  * Axes are mirrored (x ^ -1) so that every step is +1 and the far face of an
- * aligned cube is x | (edge - 1).  A ray whose set-up leaves the ranges the
- * bound was derived for (non-finite or very unnormalised directions) is
- * marched step by step instead.
+ * aligned cube is x | (edge - 1).  A ray whose set-up leaves the range of the
+ * limits below (non-finite or far from unit directions) is marched step by
+ * step instead.
  *
  * Full-shading scene (256^3, 99 DDA steps a ray): 12 iterations a ray, 99.9 %
  * of the rays within 69 (the steps: 580). */
-#define VT_JUMP_A_MIN 0.99f
+#define VT_JUMP_A_MIN 9.765625e-4f        /* 2^-10 */
 #define VT_JUMP_A_MAX 2.0e5f
 #define VT_ULP24 5.9604644775390625e-8f   /* 2^-24 */
-/* 1.03 * 2^-12 and 4 times that: (m * W1 + W4)^2 = 1.06 * 2^-24 (m + 4)^2 */
+/* 1.03 * 2^-12 and 4 times that: (m / a W1 + W4)^2 = 1.06 * 2^-24 (m / a + 4)^2 */
 #define VT_JUMP_W1 2.5146484375e-4f
 #define VT_JUMP_W4 1.005859375e-3f
 
@@ -763,8 +768,9 @@ __device__ __forceinline__ float sum_steps(float X, float a, float ia, int32_t n
         const uint32_t ub = __float_as_uint(X) & 0x7f800000u;
         if (n > 0 && ub == (__float_as_uint(p) & 0x7f800000u)) {
             const float end = __uint_as_float(ub + 0x00800000u);
-            /* three steps short of the end: covers the rounding of the quotient and of a */
-            int32_t r = (int32_t)((end - X) * ia) - 3;
+            /* two steps short of the end: covers the rounding of the quotient
+             * and, over at most 4096 adds, of a */
+            int32_t r = (int32_t)((end - X) * ia) - 2;
             r = r < n ? r : n;
             if (r > 0) {
                 X = __builtin_fmaf((float)r, (X + a) - X, X);
@@ -779,33 +785,49 @@ struct JumpState {
     int32_t x, y, z;            /* mirrored position */
     int32_t x0, y0, z0;         /* mirrored start */
     int32_t fx, fy, fz;         /* 0, or -1 on a mirrored axis */
-    float X0, Y0, Z0, ax, ay, az, ix, iy, iz, qx, qy, qz;
+    float X0, Y0, Z0, ax, ay, az, ix, iy, iz, q_x, q_y, q_z;
+    float w1;                   /* W1 over the smallest a */
+
+    /* the error bound at value m, in steps */
+    __device__ __forceinline__ float bound(const GridView& g, float m) const
+    {
+        const float w = __builtin_fmaf(m, w1, VT_JUMP_W4);
+        return __builtin_fmaf(w, w, g.jc0);
+    }
 
     enum { OUTSIDE = 0, READY = 1, STEPWISE = 2 };
 
-    /* DdaState::init's arithmetic; STEPWISE when the bound does not hold. */
-    __device__ __forceinline__ int init(const GridView& g, const PreRay& r)
+    /* DdaState::init's arithmetic from a queue entry (queue_a, queue_b): the
+     * distance to the first step is |1/d| times the part of the voxel that is
+     * left along the ray, in [0, 1].  STEPWISE when the bound does not hold;
+     * compared as integers, a NaN exceeds every limit. */
+    __device__ __forceinline__ int init(const GridView& g, float4 qa, float2 qb)
     {
-        const float vox = ((r.o.x - g.bmin[0]) * g.ext[0]) * g.rx;
-        const float voy = ((r.o.y - g.bmin[1]) * g.ext[1]) * g.ry;
-        const float voz = ((r.o.z - g.bmin[2]) * g.ext[2]) * g.rz;
+        const float vox = ((qa.x - g.bmin[0]) * g.ext[0]) * g.rx;
+        const float voy = ((qa.y - g.bmin[1]) * g.ext[1]) * g.ry;
+        const float voz = ((qa.z - g.bmin[2]) * g.ext[2]) * g.rz;
         const float bx = floorf(vox), by = floorf(voy), bz = floorf(voz);
-        if (bx < 0.0f || by < 0.0f || bz < 0.0f || bx >= g.rx || by >= g.ry || bz >= g.rz) return OUTSIDE;
-        X0 = (((bx - vox) + 0.5f) + (float)r.sx * 0.5f) * r.inv.x;
-        Y0 = (((by - voy) + 0.5f) + (float)r.sy * 0.5f) * r.inv.y;
-        Z0 = (((bz - voz) + 0.5f) + (float)r.sz * 0.5f) * r.inv.z;
-        ax = vt_absf(r.inv.x); ay = vt_absf(r.inv.y); az = vt_absf(r.inv.z);
-        const float lo = min3f(ax, ay, az);
-        const bool sane = lo >= VT_JUMP_A_MIN && ax <= VT_JUMP_A_MAX && ay <= VT_JUMP_A_MAX && az <= VT_JUMP_A_MAX &&
-                          X0 >= 0.0f && Y0 >= 0.0f && Z0 >= 0.0f && X0 <= ax * 1.001f && Y0 <= ay * 1.001f &&
-                          Z0 <= az * 1.001f;
-        if (!sane) return STEPWISE;
-        fx = r.sx < 0 ? -1 : 0; fy = r.sy < 0 ? -1 : 0; fz = r.sz < 0 ? -1 : 0;
-        x = x0 = (int32_t)bx ^ fx; y = y0 = (int32_t)by ^ fy; z = z0 = (int32_t)bz ^ fz;
+        /* saturating, a NaN gives 0 and is found below */
+        const int32_t jx = floor_i32(vox), jy = floor_i32(voy), jz = floor_i32(voz);
+        if ((uint32_t)jx >= (uint32_t)g.nx || (uint32_t)jy >= (uint32_t)g.ny || (uint32_t)jz >= (uint32_t)g.nz)
+            return OUTSIDE;
+        ax = vt_absf(qa.w); ay = vt_absf(qb.x); az = vt_absf(qb.y);
+        X0 = vt_absf(((bx - vox) + 0.5f) + __builtin_copysignf(0.5f, qa.w)) * ax;
+        Y0 = vt_absf(((by - voy) + 0.5f) + __builtin_copysignf(0.5f, qb.x)) * ay;
+        Z0 = vt_absf(((bz - voz) + 0.5f) + __builtin_copysignf(0.5f, qb.y)) * az;
+        const uint32_t ua = __float_as_uint(ax), ub = __float_as_uint(ay), uc = __float_as_uint(az);
+        const uint32_t u0 = __float_as_uint(X0), u1 = __float_as_uint(Y0), u2 = __float_as_uint(Z0);
+        const uint32_t lo = min(min(ua, ub), uc), hi = max(max(ua, ub), uc), h0 = max(max(u0, u1), u2);
+        if (lo < __float_as_uint(VT_JUMP_A_MIN) || max(hi, h0) > __float_as_uint(VT_JUMP_A_MAX)) return STEPWISE;
+        fx = (int32_t)__float_as_uint(qa.w) >> 31;
+        fy = (int32_t)__float_as_uint(qb.x) >> 31;
+        fz = (int32_t)__float_as_uint(qb.y) >> 31;
+        x = x0 = jx ^ fx; y = y0 = jy ^ fy; z = z0 = jz ^ fz;
         ix = __builtin_amdgcn_rcpf(ax); iy = __builtin_amdgcn_rcpf(ay); iz = __builtin_amdgcn_rcpf(az);
-        qx = __builtin_fmaf(-X0, ix, (float)(x0 + 1));
-        qy = __builtin_fmaf(-Y0, iy, (float)(y0 + 1));
-        qz = __builtin_fmaf(-Z0, iz, (float)(z0 + 1));
+        w1 = VT_JUMP_W1 * fmaxf(fmaxf(ix, iy), iz);
+        q_x = __builtin_fmaf(-X0, ix, (float)(x0 + 1));
+        q_y = __builtin_fmaf(-Y0, iy, (float)(y0 + 1));
+        q_z = __builtin_fmaf(-Z0, iz, (float)(z0 + 1));
         return READY;
     }
 
@@ -819,7 +841,8 @@ struct JumpState {
         const uint32_t pad = 1u << cg;
         const uint32_t ux = xor_add<UNI>(x, fx, pad), uy = xor_add<UNI>(y, fy, pad), uz = xor_add<UNI>(z, fz, pad);
         const uint32_t ci = index3<UNI>(ux >> cg, uy >> cg, uz >> cg, g.ccx, g.ccy);
-        const uint32_t c = field<2, false>(codes[ci >> 4], ci << 1);
+        const uint32_t word = UNI ? codes[ci >> 4] : ((const __attribute__((address_space(1))) uint32_t*)codes)[ci >> 4];
+        const uint32_t c = field<2, false>(word, ci << 1);
         edge = (int32_t)field<8, UNI>(g.cedge, c << 3);
         if (c == 0u) {
             uint32_t bi = ci;
@@ -827,15 +850,33 @@ struct JumpState {
                 const uint32_t k = pad - 4u;
                 bi = index3<UNI>((ux - k) >> 2, (uy - k) >> 2, (uz - k) >> 2, g.bxp, g.byp);
             }
-            const uint64_t m = g.occp[bi];
-            if (m == 0ull) {
-                edge = 3;
-            } else {
-                const uint32_t bit = (ux & 3u) | ((uy & 3u) << 2) | ((uz & 3u) << 4);
-                if ((m >> bit) & 1ull) return false;
-            }
+            const uint64_t m = load_mask(g.occp, bi);
+            if (voxel_bit(m, ux, uy, uz)) return false;
+            if (!FINE && m == 0ull) edge = 3;
         }
         return true;
+    }
+
+    static __device__ __forceinline__ uint64_t load_mask(const uint64_t* occp, uint32_t i)
+    {
+        return ((const __attribute__((address_space(1))) uint64_t*)occp)[i];
+    }
+    /* bit (x & 3) + 4 (y & 3) + 16 (z & 3) of m */
+    static __device__ __forceinline__ bool voxel_bit(uint64_t m, uint32_t vx, uint32_t vy, uint32_t vz)
+    {
+        uint32_t b = vy << 2;
+        asm("v_bfi_b32 %0, 3, %1, %2" : "=v"(b) : "v"(vx), "v"(b));
+        uint32_t c = vz << 4;
+        asm("v_bfi_b32 %0, 15, %1, %2" : "=v"(c) : "v"(b), "v"(c));
+        return ((m >> (c & 63u)) & 1ull) != 0ull;
+    }
+    /* Whether the voxel at mirrored (px, py, pz), inside the grid or one past
+     * it, is occupied or outside the grid. */
+    template <bool UNI>
+    __device__ __forceinline__ bool blocked(const GridView& g, int32_t px, int32_t py, int32_t pz) const
+    {
+        const uint32_t vx = xor_add<false>(px, fx, 4u), vy = xor_add<false>(py, fy, 4u), vz = xor_add<false>(pz, fz, 4u);
+        return voxel_bit(load_mask(g.occp, index3<UNI>(vx >> 2, vy >> 2, vz >> 2, g.bxp, g.byp)), vx, vy, vz);
     }
 
     /* (a ^ b) + c in one instruction; c is wave-uniform with UNI */
@@ -872,20 +913,39 @@ struct JumpState {
     }
 
     /* Leave the cube of lookup(); false, with the position unchanged, when
-     * the order of two steps is undecided. */
+     * the order of two steps is undecided and matters. */
+    template <bool UNI>
     __device__ __forceinline__ bool jump(const GridView& g, int32_t edge)
     {
         const int32_t bx = x | edge, by = y | edge, bz = z | edge;
         const float m = min3f(__builtin_fmaf((float)(bx - x0), ax, X0), __builtin_fmaf((float)(by - y0), ay, Y0),
                               __builtin_fmaf((float)(bz - z0), az, Z0));
-        const float w = __builtin_fmaf(m, VT_JUMP_W1, VT_JUMP_W4);
-        const float del = __builtin_fmaf(w, w, g.jc0);
-        const float px = __builtin_fmaf(m, ix, qx) + del, py = __builtin_fmaf(m, iy, qy) + del,
-                    pz = __builtin_fmaf(m, iz, qz) + del;
-        if (__builtin_amdgcn_fmed3f(__builtin_amdgcn_fractf(px), __builtin_amdgcn_fractf(py),
-                                    __builtin_amdgcn_fractf(pz)) < del + del)
-            return false;
-        x = floor_i32(px); y = floor_i32(py); z = floor_i32(pz);
+        const float del = bound(g, m);
+        const float px = __builtin_fmaf(m, ix, q_x) + del, py = __builtin_fmaf(m, iy, q_y) + del,
+                    pz = __builtin_fmaf(m, iz, q_z) + del;
+        const float rx = __builtin_amdgcn_fractf(px), ry = __builtin_amdgcn_fractf(py), rz = __builtin_amdgcn_fractf(pz);
+        const float del2 = del + del;
+        const int32_t tx = floor_i32(px), ty = floor_i32(py), tz = floor_i32(pz);
+        if (__builtin_amdgcn_fmed3f(rx, ry, rz) < del2) {
+            /* steps ahead only: one that is behind was taken before */
+            const bool mx = tx > x, my = ty > y, mz = tz > z;
+            const bool nx = rx < del2 && mx, ny = ry < del2 && my, nz = rz < del2 && mz;
+            if (nx && ny && nz) return false;
+            if ((nx && ny) || (ny && nz) || (nz && nx)) {
+                const float am = fmaxf(fmaxf(nx ? ax : 0.0f, ny ? ay : 0.0f), nz ? az : 0.0f);
+                const float ex = del2 * __builtin_fmaf(am, ix, 1.0f), ey = del2 * __builtin_fmaf(am, iy, 1.0f),
+                            ez = del2 * __builtin_fmaf(am, iz, 1.0f);
+                if (!(fmaxf(fmaxf(ex, ey), ez) < 0.4f)) return false;
+                if ((!nx && ((mx && rx < ex) || rx > 1.0f - ex)) || (!ny && ((my && ry < ey) || ry > 1.0f - ey)) ||
+                    (!nz && ((mz && rz < ez) || rz > 1.0f - ez)))
+                    return false;
+                /* the voxels where one of the two steps is missing */
+                if (nx && blocked<UNI>(g, tx - 1, ty, tz)) return false;
+                if (ny && blocked<UNI>(g, tx, ty - 1, tz)) return false;
+                if (nz && blocked<UNI>(g, tx, ty, tz - 1)) return false;
+            }
+        }
+        x = tx; y = ty; z = tz;
         return true;
     }
 
@@ -896,35 +956,37 @@ struct JumpState {
         return r;
     }
 
-    /* The jump that jump() left undecided: the values of the near axes' steps
-     * as the FP32 sums they are; a step is taken when its value is not above
-     * the smallest one that leaves the cube. */
+    /* The jump that jump() left undecided: the smallest value that leaves the
+     * cube from the FP32 sums, then on each axis the steps up to it, the last
+     * one checked against its sum where the real line leaves it open. */
     __device__ __forceinline__ void resolve(const GridView& g, int32_t edge)
     {
-        const int32_t b[3] = { x | edge, y | edge, z | edge };
-        const float m = min3f(__builtin_fmaf((float)(b[0] - x0), ax, X0), __builtin_fmaf((float)(b[1] - y0), ay, Y0),
-                              __builtin_fmaf((float)(b[2] - z0), az, Z0));
-        const float w = __builtin_fmaf(m, VT_JUMP_W1, VT_JUMP_W4);
-        const float del = __builtin_fmaf(w, w, g.jc0);
-        const float p[3] = { __builtin_fmaf(m, ix, qx) + del, __builtin_fmaf(m, iy, qy) + del,
-                             __builtin_fmaf(m, iz, qz) + del };
         const int32_t at[3] = { x, y, z }, s0[3] = { x0, y0, z0 };
-        const float S0[3] = { X0, Y0, Z0 }, a[3] = { ax, ay, az }, ia[3] = { ix, iy, iz };
-        int32_t to[3];
-        float v[3], me = __uint_as_float(0x7f800000u);
+        const float S0[3] = { X0, Y0, Z0 }, a[3] = { ax, ay, az }, ia[3] = { ix, iy, iz }, q[3] = { q_x, q_y, q_z };
+        float t[3], m = __uint_as_float(0x7f800000u);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            to[k] = floor_i32(p[k]);
-            v[k] = 0.0f;
-            /* a near axis whose step is still ahead */
-            if (__builtin_amdgcn_fractf(p[k]) < del + del && to[k] > at[k]) {
-                v[k] = sum_steps(S0[k], a[k], ia[k], to[k] - 1 - s0[k]);
-                if (to[k] > b[k] && v[k] < me) me = v[k];
-            }
+            t[k] = __builtin_fmaf((float)((at[k] | edge) - s0[k]), a[k], S0[k]);
+            m = fminf(m, t[k]);
         }
+        /* an axis further behind than both errors leaves later */
+        const float m0 = m, d0 = 2.0f * bound(g, m);
+        const float first = m0 == t[0] ? a[0] : m0 == t[1] ? a[1] : a[2];
+        m = __uint_as_float(0x7f800000u);
 #pragma unroll
         for (int k = 0; k < 3; ++k)
-            if (v[k] > me) to[k] -= 1;
+            if (t[k] - m0 <= d0 * (a[k] + first)) m = fminf(m, sum_steps(S0[k], a[k], ia[k], (at[k] | edge) - s0[k]));
+        const float del = bound(g, m);
+        int32_t to[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float p = __builtin_fmaf(m, ia[k], q[k]) + del;
+            to[k] = floor_i32(p);
+            /* at most one step too far unless the bound is above 1/2 (more
+             * than 2800 steps) */
+            if (__builtin_amdgcn_fractf(p) < del + del)
+                while (to[k] > at[k] && sum_steps(S0[k], a[k], ia[k], to[k] - 1 - s0[k]) > m) to[k] -= 1;
+        }
         x = to[0]; y = to[1]; z = to[2];
     }
 

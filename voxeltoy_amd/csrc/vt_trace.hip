@@ -603,13 +603,17 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * takes about 13 ns an update.  Workgroups of 1024 threads share one
  * LDS copy of the empty-cube codes (of the block occupancy bits with STATS).
  *
- * Bound by vector issue (1.0 wave-instructions a CU and cycle, 44 % of the
- * lanes at work, full-shading scene).  That scene at 1024^2, 16 passes, 8
- * bounces (90 M rays, 9 launches): 10.1 ms stepping voxel by voxel, 7.0 ms
- * with the jump march and one queue counter (of that, 4.6 ms at least in the
- * counter's 352 k updates), 5.3 ms dealt; one pass at 1920x1080: 3.15, 2.4,
- * 1.1 ms; 512^3 mesh scene at 1920x1080, 8 passes: 5.26, 2.9, 2.05 ms. */
+ * Bound by vector issue (0.86 wave-instructions a CU and cycle, 48 % of the
+ * lanes at work, full-shading scene) and, in the later launches, by the chain
+ * of its longest rays (up to 160 jumps of about a microsecond).  That scene at
+ * 1024^2, 16 passes, 8 bounces (90 M rays, 9 launches): 10.1 ms stepping voxel
+ * by voxel, 7.0 ms with the jump march and one queue counter (of that, 4.6 ms
+ * at least in the counter's 352 k updates), 5.3 ms dealt, 4.5 ms with the
+ * undecided steps settled by the voxels they could skip; one pass at
+ * 1920x1080: 3.15, 2.4, 1.1, 0.81 ms; 512^3 mesh scene at 1920x1080, 8 passes:
+ * 5.26, 2.9, 2.05, 1.45 ms. */
 #define WF_TRAVERSE_THREADS 1024
+#define WF_TAKEN_BYTES 16u      /* LDS of a traversal workgroup's list counter */
 
 /* SGPRs are allocated in steps of 16.  A build of this kernel whose
  * allocation rose from 80 to 96 SGPRs, with its hot loop unchanged
@@ -618,24 +622,28 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * workgroups per CU need all 8): the cap keeps the allocation at 80. */
 #define WF_TRAVERSE_SGPRS 80
 
-/* Idle lanes that trigger a refill of the jump march: a.refill_min times this */
+/* Idle lanes that trigger a refill of the jump march: a.refill_min times this
+ * (swept from 6 to 42 lanes: within 2 % from 18 on) */
 #define VT_JUMP_REFILL 3u
-/* undecided lanes of a wave that are worth a resolve while others march */
-#define VT_JUMP_RESOLVE 6u
 
 /* The jump march of the calling lanes: at most `jumps` jumps, until fewer than
- * `keep` of them still march. */
-enum { JM_MARCHING = 0, JM_STOPPED = 1, JM_UNDECIDED = 2 };
+ * `keep` of them still march.  `stop`: the position is the ray's last voxel;
+ * `und`: its next jump needs a resolve. */
 template <bool FINE, bool UNI>
-__device__ __forceinline__ int jump_march(JumpState& J, const GridView& g, const uint32_t* __restrict__ codes,
-                                          int jumps, int keep)
+__device__ __forceinline__ void jump_march(JumpState& J, const GridView& g, const uint32_t* __restrict__ codes,
+                                           int jumps, int keep, bool& stop, bool& und)
 {
     do {
         int32_t edge;
-        if (!J.lookup<FINE, UNI>(g, codes, edge)) return JM_STOPPED;
-        if (!J.jump(g, edge)) return JM_UNDECIDED;
+        if (!J.lookup<FINE, UNI>(g, codes, edge)) {
+            stop = true;
+            break;
+        }
+        if (!J.jump<UNI>(g, edge)) {
+            und = true;
+            break;
+        }
     } while (--jumps > 0 && __popcll(__builtin_amdgcn_ballot_w64(true)) >= keep);
-    return JM_MARCHING;
 }
 
 /* A ray marched step by step (DdaState::advance): hit record. */
@@ -671,14 +679,14 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
     if (blockIdx.x >= n_seg) return;
     /* entries of the workgroup's own list, its segments one after another */
     const uint32_t mine = ((n_seg - blockIdx.x + gridDim.x - 1u) / gridDim.x) << seg_log;
-    __shared__ uint32_t taken;     /* of the workgroup's list */
-    if (threadIdx.x == 0) taken = 0u;
     /* the march reads the padded block bits, or the codes */
     constexpr bool STAGE = !BATCH && (LDSB || !STATS);
     const uint32_t* bits = STATS ? a.g.bitsp : a.g.codes;
+    const uint32_t words = !STAGE ? 0u : STATS ? a.g.bit_words_p : a.g.code_words;
+    uint32_t* taken = (uint32_t*)smem + words;     /* of the workgroup's list; after the table, whose reads then need no base */
+    if (threadIdx.x == 0) *taken = 0u;
     if (STAGE) {
         uint32_t* sb = (uint32_t*)smem;
-        const uint32_t words = STATS ? a.g.bit_words_p : a.g.code_words;
         for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) sb[i] = bits[i];
         bits = sb;
     }
@@ -693,7 +701,6 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
     const int budget = a.dda_budget;
     DdaState D;
     JumpState J;
-    bool und = false;              /* the lane's jump waits for a resolve */
     GridView gl;                   /* the lane's scene grid (batch only) */
     const GridView& G = BATCH ? gl : a.g;
     uint32_t jq = 0;               /* queue position of the lane's ray (hits are stored there) */
@@ -704,8 +711,8 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
         const uint32_t n_idle = (uint32_t)__popcll(idle);
         if (!done && n_idle >= refill_min) {
             uint32_t v = 0;
-            if (lane == 0) v = atomicAdd(&taken, n_idle);
-            v = __shfl(v, 0, 64);
+            if (lane == 0) v = atomicAdd(taken, n_idle);
+            v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
             done = v + n_idle >= mine;
             if (!has) {
                 v += (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
@@ -723,15 +730,15 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
                     asm volatile("" : "+v"(o.x), "+v"(o.y), "+v"(o.z), "+v"(o.w), "+v"(d.x), "+v"(d.y));
                     jq = j;
                     if (BATCH) gl = B.tab[qt[j]].g;
-                    const PreRay r = unpack_ray(o, d);
                     if constexpr (STATS) {
-                        has = D.init(G, r);
+                        has = D.init(G, unpack_ray(o, d));
                         if (!has) P.hit[j] = pack_hit(0, 0, 0, KIND_MISS);
                     } else {
-                        const int st = J.init(G, r);
+                        const int st = J.init(G, o, d);
                         has = st == JumpState::READY;
                         if (!has)
-                            P.hit[j] = st == JumpState::OUTSIDE ? pack_hit(0, 0, 0, KIND_MISS) : stepwise_hit(G, r);
+                            P.hit[j] = st == JumpState::OUTSIDE ? pack_hit(0, 0, 0, KIND_MISS)
+                                                                : stepwise_hit(G, unpack_ray(o, d));
                     }
                 }
             }
@@ -761,23 +768,17 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
                 }
             }
         } else {
-            /* Undecided lanes wait until several of them share the exact sums
-             * (or nothing else is left to march). */
-            const unsigned long long um = __ballot(und);
-            if (um && ((uint32_t)__popcll(um) >= VT_JUMP_RESOLVE || __ballot(has && !und) == 0ull)) {
+            if (has) {
+                /* march on until a refill is due, or to the end */
+                const int keep = done ? 1 : 65 - (int)refill_min;
+                bool stop = false, und = false;
+                jump_march<LDSB, !BATCH>(J, G, BATCH ? G.codes : bits, budget, keep, stop, und);
                 if (und) {
                     int32_t edge;
                     (void)J.lookup<LDSB, !BATCH>(G, BATCH ? G.codes : bits, edge);
                     J.resolve(G, edge);
-                    und = false;
                 }
-            }
-            if (has && !und) {
-                /* march on until a refill is due, or to the end */
-                const int keep = done ? 1 : 65 - (int)refill_min;
-                const int status = jump_march<LDSB, !BATCH>(J, G, BATCH ? G.codes : bits, budget, keep);
-                und = status == JM_UNDECIDED;
-                if (status == JM_STOPPED) {
+                if (stop) {
                     const int32_t x = J.gx(), y = J.gy(), z = J.gz();
                     const bool inside = (uint32_t)x < (uint32_t)G.nx && (uint32_t)y < (uint32_t)G.ny &&
                                         (uint32_t)z < (uint32_t)G.nz;
@@ -1043,7 +1044,8 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
                          uint64_t n_pixels, int rounds, int cus, hipStream_t s, const LaunchTimer* timer = nullptr,
                          hipEvent_t acc_wait = nullptr)
 {
-    const size_t lds_t = BATCH ? 0u : STATS ? (LDSB ? (size_t)a.g.bit_words_p * 4u : 0u) : (size_t)a.g.code_words * 4u;
+    const size_t lds_t = WF_TAKEN_BYTES + (BATCH ? 0u : STATS ? (LDSB ? (size_t)a.g.bit_words_p * 4u : 0u)
+                                                          : (size_t)a.g.code_words * 4u);
     const size_t lds_s = BATCH ? 0 : 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
     const int bt = blocks_per_cu(wf_traverse_kernel<STATS, LDSB, BATCH>, WF_TRAVERSE_THREADS, lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<STATS, PH_PRIMARY, BATCH>, WF_SHADE_THREADS, lds_s);
@@ -1137,7 +1139,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
                                 const float* bias, int cus, hipStream_t s)
 {
     const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0 };
-    const size_t lds_t = (size_t)a.g.code_words * 4u;
+    const size_t lds_t = WF_TAKEN_BYTES + (size_t)a.g.code_words * 4u;
     const size_t lds_s = 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
     const int bt = blocks_per_cu(wf_traverse_kernel<false, LDSB, false>, WF_TRAVERSE_THREADS, lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<false, PH_PRIMARY, false, true>, WF_SHADE_THREADS, lds_s);
