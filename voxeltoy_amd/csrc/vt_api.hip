@@ -58,6 +58,7 @@ int no_throw(F&& f) noexcept
 #define VT_DEFAULT_DDA_BUDGET 32
 #define VT_DEFAULT_REFILL_MIN 8
 #define VT_DEFAULT_REFILL_CHUNK 256
+#define VT_WORK_KEEP (256ull << 20)  /* workspace kept on a context */
 #define VT_CODE_LDS_BYTES 80640ull  /* half a CU's LDS but one 1280-byte allocation unit */
 /* (x, y) columns above which the voxelizer gives a triangle a whole wave */
 #define VT_VOX_BIG_AREA 32
@@ -190,20 +191,20 @@ struct vt_context {
     vt::BrickDims dims{};
     float bmin[3] = { 0, 0, 0 }, bmax[3] = { 0, 0, 0 }, vs[3] = { 0, 0, 0 };
     uint8_t* d_bricks = nullptr;
-    uint64_t* d_occ64 = nullptr;
-    uint32_t* d_bits = nullptr;
-    uint32_t bit_words = 0;
-    uint64_t* d_occp = nullptr;     /* padded levels of the wave march */
+    uint64_t* d_occp = nullptr;     /* padded block masks */
     uint64_t* d_occr = nullptr;     /* padded masks with reversed bits, for the packed march */
     uint32_t* d_bitsp = nullptr;
     uint32_t bit_words_p = 0;
-    uint8_t* d_cells = nullptr;     /* the jump march's codes, a byte per cell and packed */
-    uint32_t* d_codes = nullptr;
-    uint64_t n_cells = 0;
+    uint32_t* d_codes = nullptr;    /* the jump march's codes */
+    uint32_t code_words = 0;
     uint32_t cell_shift = 2, code_top = 2, cell_ex = 0, cell_ey = 0;
     int32_t* d_emissive = nullptr;
     int32_t n_emissive = 0;
     int4* d_lights = nullptr;       /* emissive entries decoded: x, y, z, slot */
+    int32_t emissive_cap = 0, lights_cap = 0;   /* entries allocated */
+    std::mutex work_lock;           /* the kept workspace is one call's at a time (WorkSpace) */
+    uint8_t* d_work = nullptr;
+    size_t work_cap = 0;
     std::vector<float> mat;
     int32_t slot_off[256];
     int32_t n_slots = 0;            /* slots 1..n_slots used */
@@ -286,25 +287,57 @@ int upload_records(vt_context* c)
     return VT_OK;
 }
 
-/* Rebuild both occupancy levels from the slot bytes. */
 vt::TraceArgs trace_args(const vt_context* c);
 
-/* After any change of the bricks or the emissive list: block occupancy and
- * the emissive light table. */
-int refresh_occupancy(vt_context* c)
+/* After any change of the block levels or the emissive list: the jump march's
+ * codes and the emissive light table. */
+int refresh_codes(vt_context* c)
 {
-    VT_HIP(vt::launch_block_masks(c->dims, c->d_bricks, c->d_occ64, c->d_bits, c->d_occp, c->d_bitsp, c->d_occr,
-                                  c->stream));
-    VT_HIP(vt::launch_cell_codes(c->dims, c->d_occp, c->cell_shift, c->code_top, c->d_cells, c->n_cells, c->d_codes,
+    VT_HIP(vt::launch_cell_codes(c->dims, c->d_occp, c->cell_shift, c->code_top, c->cell_ex, c->cell_ey, c->d_codes,
                                  c->stream));
-    dfree(c->d_lights);
     if (c->n_emissive > 0 && c->d_emissive) {
-        VT_HIP(hipMalloc(&c->d_lights, (size_t)c->n_emissive * 16u));
+        if (c->lights_cap < c->n_emissive) {
+            dfree(c->d_lights);
+            c->lights_cap = 0;
+            VT_HIP(hipMalloc(&c->d_lights, (size_t)c->n_emissive * 16u));
+            c->lights_cap = c->n_emissive;
+        }
         const vt::TraceArgs a = trace_args(c);
         VT_HIP(vt::launch_light_table(a.g, c->d_lights, c->stream));
     }
     return VT_OK;
 }
+
+vt::BlockLevels block_levels(const vt_context* c) { return { c->d_occp, c->d_occr, c->d_bitsp }; }
+
+/* Device workspace of one call, which waits for its work before it returns.
+ * The context keeps up to VT_WORK_KEEP bytes for the next call; a larger one,
+ * or one of a second thread that meets the context busy, is allocated for the
+ * call and freed with it. */
+struct WorkSpace {
+    uint8_t* p = nullptr;
+    int take(vt_context* c, size_t bytes)
+    {
+        if (bytes <= VT_WORK_KEEP) lock = std::unique_lock<std::mutex>(c->work_lock, std::try_to_lock);
+        if (!lock.owns_lock()) {
+            VT_HIP(hipMalloc(&own.p, bytes));
+            p = own.p;
+            return VT_OK;
+        }
+        if (c->work_cap < bytes) {
+            dfree(c->d_work);
+            c->work_cap = 0;
+            VT_HIP(hipMalloc(&c->d_work, bytes));
+            c->work_cap = bytes;
+        }
+        p = c->d_work;
+        return VT_OK;
+    }
+private:
+    std::unique_lock<std::mutex> lock;
+    DevTmp<uint8_t> own;
+};
+size_t aligned(size_t bytes) { return (bytes + 255u) & ~(size_t)255u; }
 
 vt::BrickDims make_dims(int32_t nx, int32_t ny, int32_t nz)
 {
@@ -317,7 +350,8 @@ vt::BrickDims make_dims(int32_t nx, int32_t ny, int32_t nz)
     d.bdim = p;
     d.n_bricks = (uint64_t)p * p * p;
     d.kx = (nx + 3) / 4; d.ky = (ny + 3) / 4; d.kz = (nz + 3) / 4;
-    d.n_blocks = (uint64_t)d.kx * d.ky * d.kz;
+    d.px = (d.kx + 5) / 4 * 4; d.py = d.ky + 2; d.pz = d.kz + 2;
+    d.n_padded = (uint64_t)d.px * d.py * d.pz;
     return d;
 }
 
@@ -347,13 +381,13 @@ void choose_cells(vt_context* c)
     for (;; ++cg) {
         const uint64_t e = 1ull << cg;
         ex = ((uint64_t)d.nx + e - 1) / e; ey = ((uint64_t)d.ny + e - 1) / e; ez = ((uint64_t)d.nz + e - 1) / e;
-        if ((ex + 2) * (ey + 2) * (ez + 2) <= VT_CODE_LDS_BYTES * 4u) break;
+        if (((ex + 5) / 4 * 4) * (ey + 2) * (ez + 2) <= VT_CODE_LDS_BYTES * 4u) break;
     }
     c->cell_shift = cg;
     c->code_top = std::max(ex, std::max(ey, ez)) > 56 && cg < 6 ? 3u : 2u;   /* an edge of at most 256: cedge holds bytes */
-    c->cell_ex = (uint32_t)ex + 2;
+    c->cell_ex = (uint32_t)((ex + 5) / 4 * 4);      /* rows of whole bytes; dims.px for cells of one block */
     c->cell_ey = (uint32_t)ey + 2;
-    c->n_cells = (ex + 2) * (ey + 2) * (ez + 2);
+    c->code_words = (uint32_t)(((uint64_t)c->cell_ex * c->cell_ey * (ez + 2) + 15) / 16);
 }
 
 int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const float* mat_data, int32_t mat_size,
@@ -364,15 +398,17 @@ int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const
     if (mat_size < 0 || (mat_size > 0 && !mat_data)) return fail(VT_ERR_ARG, "bad material data");
     const vt::BrickDims d = make_dims(nx, ny, nz);
     c->has_volume = false;
-    dfree(c->d_bricks);
-    dfree(c->d_occ64);
-    dfree(c->d_bits);
-    dfree(c->d_occp);
-    dfree(c->d_bitsp);
-    dfree(c->d_occr);
-    dfree(c->d_cells);
-    dfree(c->d_codes);
-    dfree(c->d_emissive);
+    /* a grid of the same extents keeps its buffers */
+    const bool keep = c->d_bricks && c->d_occp && c->d_bitsp && c->d_codes && c->dims.nx == nx && c->dims.ny == ny &&
+                      c->dims.nz == nz;
+    if (!keep) {
+        dfree(c->d_bricks);
+        dfree(c->d_occp);
+        dfree(c->d_bitsp);
+        dfree(c->d_occr);
+        dfree(c->d_codes);
+    }
+    c->n_emissive = 0;
     c->dims = d;
     if (bmin && bmax) {
         for (int k = 0; k < 3; ++k) { c->bmin[k] = bmin[k]; c->bmax[k] = bmax[k]; }
@@ -384,52 +420,58 @@ int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const
     c->mat.assign(mat_data, mat_data + mat_size);
     for (int i = 0; i < 256; ++i) c->slot_off[i] = -1;
     c->n_slots = 0;
-    VT_HIP(hipMalloc(&c->d_bricks, d.n_bricks * 512u));
-    VT_HIP(hipMalloc(&c->d_occ64, d.n_blocks * 8u));
-    c->bit_words = (uint32_t)((d.n_blocks + 31) / 32);
-    VT_HIP(hipMalloc(&c->d_bits, (size_t)c->bit_words * 4u));
-    const uint64_t np = (uint64_t)(d.kx + 2) * (uint64_t)(d.ky + 2) * (uint64_t)(d.kz + 2);
-    VT_HIP(hipMalloc(&c->d_occp, np * 8u));
-    c->bit_words_p = (uint32_t)((np + 31) / 32);
-    VT_HIP(hipMalloc(&c->d_bitsp, (size_t)c->bit_words_p * 4u));
-    if (nx <= VT_PACKED_MAX_EXTENT && ny <= VT_PACKED_MAX_EXTENT && nz <= VT_PACKED_MAX_EXTENT)
-        VT_HIP(hipMalloc(&c->d_occr, np * 8u));
-    choose_cells(c);
-    VT_HIP(hipMalloc(&c->d_cells, (c->n_cells + 15) / 16 * 16));
-    VT_HIP(hipMalloc(&c->d_codes, (c->n_cells + 15) / 16 * 4));
-    VT_HIP(vt::launch_fill_u8(c->d_cells, (c->n_cells + 15) / 16 * 16, 0, c->stream));
-    VT_HIP(vt::launch_fill_u8(c->d_bricks, d.n_bricks * 512u, 0, c->stream));
+    if (!keep) {
+        VT_HIP(hipMalloc(&c->d_bricks, d.n_bricks * 512u));
+        const uint64_t np = d.n_padded;
+        VT_HIP(hipMalloc(&c->d_occp, np * 8u));
+        c->bit_words_p = (uint32_t)((np + 31) / 32);
+        VT_HIP(hipMalloc(&c->d_bitsp, (size_t)c->bit_words_p * 4u));
+        if (nx <= VT_PACKED_MAX_EXTENT && ny <= VT_PACKED_MAX_EXTENT && nz <= VT_PACKED_MAX_EXTENT)
+            VT_HIP(hipMalloc(&c->d_occr, np * 8u));
+        choose_cells(c);
+        VT_HIP(hipMalloc(&c->d_codes, (size_t)c->code_words * 4u));
+        /* what the conversions never write: the bricks' voxels outside the
+         * grid and the codes' padding */
+        VT_HIP(vt::launch_fill_u8((uint8_t*)c->d_codes, (uint64_t)c->code_words * 4u, 0, c->stream));
+        VT_HIP(vt::launch_fill_u8(c->d_bricks, d.n_bricks * 512u, 0, c->stream));
+    }
     return VT_OK;
 }
 
-int finish_volume(vt_context* c, const int32_t* emissive, int32_t n_emissive, const std::vector<uint8_t>& occupied_of_linear,
-                  bool have_occ)
+/* The emissive list onto the device (its voxels are checked there). */
+int upload_emissive(vt_context* c, const int32_t* emissive, int32_t n)
 {
-    (void)occupied_of_linear;
-    (void)have_occ;
-    c->n_emissive = n_emissive;
-    if (n_emissive > 0) {
-        VT_HIP(hipMalloc(&c->d_emissive, (size_t)n_emissive * 4u));
-        VT_HIP(hipMemcpyAsync(c->d_emissive, emissive, (size_t)n_emissive * 4u, hipMemcpyHostToDevice, c->stream));
+    if (n <= 0 || !emissive) return VT_OK;
+    if (c->emissive_cap < n) {
+        dfree(c->d_emissive);
+        c->emissive_cap = 0;
+        VT_HIP(hipMalloc(&c->d_emissive, (size_t)n * 4u));
+        c->emissive_cap = n;
     }
-    int r = refresh_occupancy(c);
+    VT_HIP(to_device(c, c->d_emissive, emissive, (size_t)n * 4u));
+    return VT_OK;
+}
+
+/* The error of the list's first bad entry, as launch_check_emissive found it
+ * (`bad`: its index, or all ones). */
+int emissive_error(const int32_t* emissive, int32_t n, int64_t nvox, uint32_t bad)
+{
+    if (n < 0 || (n > 0 && !emissive)) return fail(VT_ERR_ARG, "bad emissive list");
+    if (bad >= (uint32_t)n) return VT_OK;
+    if (emissive[bad] < 0 || (int64_t)emissive[bad] >= nvox)
+        return fail(VT_ERR_ARG, "emissive voxel index out of range at " + std::to_string(bad));
+    return fail(VT_ERR_ARG, "emissive voxel " + std::to_string(emissive[bad]) + " is empty");
+}
+
+/* Codes, lights and records of a converted grid; waits for all of it. */
+int finish_volume(vt_context* c, int32_t n_emissive)
+{
+    c->n_emissive = n_emissive;
+    int r = refresh_codes(c);
     if (r != VT_OK) return r;
     r = upload_records(c);
     if (r != VT_OK) return r;
-    VT_HIP(hipStreamSynchronize(c->stream));
     c->has_volume = true;
-    return VT_OK;
-}
-
-int check_emissive(const int32_t* emissive, int32_t n, int64_t nvox, const std::vector<uint8_t>& occ)
-{
-    if (n < 0 || (n > 0 && !emissive)) return fail(VT_ERR_ARG, "bad emissive list");
-    for (int32_t i = 0; i < n; ++i) {
-        if (emissive[i] < 0 || (int64_t)emissive[i] >= nvox)
-            return fail(VT_ERR_ARG, "emissive voxel index out of range at " + std::to_string(i));
-        if (!occ[(size_t)emissive[i]])
-            return fail(VT_ERR_ARG, "emissive voxel " + std::to_string(emissive[i]) + " is empty");
-    }
     return VT_OK;
 }
 
@@ -451,20 +493,15 @@ vt::GridView grid_view(const vt_context* c)
         g.ext[k] = 1.0f / (c->bmax[k] - c->bmin[k]);
     }
     g.bricks = c->d_bricks;
-    g.bx4 = (uint32_t)c->dims.kx;
-    g.by4 = (uint32_t)c->dims.ky;
-    g.occ64 = c->d_occ64;
-    g.bits = c->d_bits;
-    g.bit_words = c->bit_words;
-    g.bxp = (uint32_t)c->dims.kx + 2u;
+    g.bxp = (uint32_t)c->dims.px;
     g.byp = (uint32_t)c->dims.ky + 2u;
     g.occp = c->d_occp;
     g.bitsp = c->d_bitsp;
     g.bit_words_p = c->bit_words_p;
     g.occr = c->d_occr;
-    g.wide = ((uint64_t)(c->dims.kx + 2) * (uint64_t)(c->dims.ky + 2) * (uint64_t)(c->dims.kz + 2)) > (1ull << 29);
+    g.wide = c->dims.n_padded > (1ull << 29);
     g.codes = c->d_codes;
-    g.code_words = (uint32_t)((c->n_cells + 15) / 16);
+    g.code_words = c->code_words;
     g.ccx = c->cell_ex;
     g.ccy = c->cell_ey;
     g.cg = c->cell_shift;
@@ -512,7 +549,7 @@ vt::TraceArgs trace_args(const vt_context* c)
     a.n_tiles = a.tiles_x * ((c->H + 7) / 8);
     a.cdfv_lds_bytes = c->env.use_image ? ((c->env.cdf_v_n * 4 + 15) / 16) * 16 : 0;
     const size_t base = 256 * sizeof(vt::MatRec) + (size_t)a.cdfv_lds_bytes;
-    a.lds_bits = (base + (size_t)c->bit_words * 4u <= c->lds_limit) ? 1 : 0;
+    a.lds_bits = (base + (size_t)c->bit_words_p * 4u <= c->lds_limit) ? 1 : 0;
     a.lds_bits_p = ((size_t)c->bit_words_p * 4u + 16u <= c->lds_limit) ? 1 : 0;   /* and the list counter */
     a.dda_budget = c->dda_budget;
     a.refill_min = c->refill_min;
@@ -614,7 +651,7 @@ void vt_destroy(vt_context* c)
     while (!c->batches.empty()) batch_release(c->batches.back());
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    dfree(c->d_bricks); dfree(c->d_occ64); dfree(c->d_bits); dfree(c->d_occp); dfree(c->d_bitsp); dfree(c->d_occr); dfree(c->d_cells); dfree(c->d_codes); dfree(c->d_emissive); dfree(c->d_lights); dfree(c->d_recs);
+    dfree(c->d_bricks); dfree(c->d_occp); dfree(c->d_bitsp); dfree(c->d_occr); dfree(c->d_codes); dfree(c->d_work); dfree(c->d_emissive); dfree(c->d_lights); dfree(c->d_recs);
     dfree(c->d_img); dfree(c->d_quad); dfree(c->d_cdfu); dfree(c->d_cdfv);
     dfree(c->d_accum); dfree(c->d_sum64); dfree(c->d_tile); dfree(c->d_stats);
     free_wavefront(c);
@@ -651,43 +688,48 @@ int vt_set_volume(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const int32
         int r = common_volume_setup(c, nx, ny, nz, mat_data, mat_size, bmin, bmax);
         if (r != VT_OK) return r;
         const int64_t nvox = (int64_t)nx * ny * nz;
+        const size_t lut_n = (size_t)std::max(mat_size, 1);
+        /* workspace: dense grid, offsets in use, LUT, {first bad voxel, first bad emissive entry} */
+        WorkSpace ws;
+        const size_t used_at = aligned((size_t)nvox * 4u), bad_at = used_at + aligned(lut_n), lut_at = bad_at + 256;
+        r = ws.take(c, lut_at + lut_n);
+        if (r != VT_OK) return r;
+        uint8_t* const work = ws.p;
+        const int32_t* d_dense = (const int32_t*)work;
+        unsigned long long* d_bad = (unsigned long long*)(work + bad_at);
+        VT_HIP(to_device(c, work, offsets, (size_t)nvox * 4u));
+        VT_HIP(vt::launch_fill_u8(work + used_at, aligned(lut_n), 0, c->stream));
+        VT_HIP(vt::launch_fill_u8(work + bad_at, 16, 0xff, c->stream));
+        r = upload_emissive(c, emissive, n_emissive);
+        if (r != VT_OK) return r;
+        VT_HIP(vt::launch_scan_offsets(d_dense, (uint64_t)nvox, mat_size, work + used_at, d_bad, c->stream));
+        if (n_emissive > 0 && emissive)
+            VT_HIP(vt::launch_check_emissive(c->d_emissive, n_emissive, (uint64_t)nvox, d_dense, nullptr, nullptr,
+                                             (uint32_t*)(d_bad + 1), c->stream));
+        std::vector<uint8_t> back(bad_at - used_at + 16);
+        VT_HIP(to_host(c, back.data(), work + used_at, back.size()));
+        uint64_t bad_voxel;
+        uint32_t bad_entry;
+        std::memcpy(&bad_voxel, back.data() + (bad_at - used_at), 8);
+        std::memcpy(&bad_entry, back.data() + (bad_at - used_at) + 8, 4);
+        if (bad_voxel != ~0ull)
+            return fail(VT_ERR_ARG, "material offset " + std::to_string(offsets[bad_voxel]) + " outside material data");
         /* distinct occupied offsets -> slots, in increasing offset order */
-        std::vector<uint8_t> used((size_t)std::max(mat_size, 1), 0);
-        std::vector<uint8_t> occ((size_t)nvox, 0);
-        for (int64_t i = 0; i < nvox; ++i) {
-            const int32_t o = offsets[i];
-            if (o < 0) continue;
-            if (o >= mat_size) return fail(VT_ERR_ARG, "material offset " + std::to_string(o) + " outside material data");
-            used[(size_t)o] = 1;
-            occ[(size_t)i] = 1;
-        }
-        std::vector<uint8_t> lut((size_t)std::max(mat_size, 1), 0);
+        std::vector<uint8_t> lut(lut_n, 0);
         int32_t ns = 0;
         for (int32_t o = 0; o < mat_size; ++o) {
-            if (!used[(size_t)o]) continue;
+            if (!back[(size_t)o]) continue;
             if (ns == 255) return fail(VT_ERR_LIMIT, "more than 255 distinct material offsets in the grid");
             ++ns;
             lut[(size_t)o] = (uint8_t)ns;
             c->slot_off[ns] = o;
         }
         c->n_slots = ns;
-        r = check_emissive(emissive, n_emissive, nvox, occ);
+        r = emissive_error(emissive, n_emissive, nvox, bad_entry);
         if (r != VT_OK) return r;
-        DevTmp<int32_t> d_dense;
-        DevTmp<uint8_t> d_lut;
-        DevTmp<uint32_t> d_bad;
-        VT_HIP(hipMalloc(&d_dense.p, (size_t)nvox * 4u));
-        VT_HIP(hipMalloc(&d_lut.p, lut.size()));
-        VT_HIP(hipMalloc(&d_bad.p, 4));
-        VT_HIP(to_device(c, d_dense.p, offsets, (size_t)nvox * 4u));
-        VT_HIP(hipMemcpyAsync(d_lut.p, lut.data(), lut.size(), hipMemcpyHostToDevice, c->stream));
-        VT_HIP(vt::launch_fill_u32(d_bad.p, 1, 0u, c->stream));
-        VT_HIP(vt::launch_brick_from_offsets(c->dims, d_dense.p, d_lut.p, mat_size, c->d_bricks, d_bad.p, c->stream));
-        uint32_t bad = 0;
-        VT_HIP(hipMemcpyAsync(&bad, d_bad.p, 4, hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
-        if (bad) return fail(VT_ERR_ARG, "grid conversion found an unmapped material offset");
-        return finish_volume(c, emissive, n_emissive, occ, true);
+        VT_HIP(to_device(c, work + lut_at, lut.data(), lut_n));
+        VT_HIP(vt::launch_blocks_from_offsets(c->dims, d_dense, work + lut_at, c->d_bricks, block_levels(c), c->stream));
+        return finish_volume(c, n_emissive);
     });
 }
 
@@ -713,22 +755,26 @@ int vt_set_volume_u8(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const ui
         }
         c->n_slots = ns;
         const int64_t nvox = (int64_t)nx * ny * nz;
-        std::vector<uint8_t> occ;
-        if (n_emissive > 0) {
-            occ.assign((size_t)nvox, 0);
-            for (int64_t i = 0; i < nvox; ++i) occ[(size_t)i] = remap[ids[i]] != 0;
-        }
-        r = check_emissive(emissive, n_emissive, nvox, occ);
+        WorkSpace ws;
+        const size_t remap_at = aligned((size_t)nvox), bad_at = remap_at + 256;
+        r = ws.take(c, bad_at + 4);
         if (r != VT_OK) return r;
-        DevTmp<uint8_t> d_dense;
-        DevTmp<uint8_t> d_remap;
-        VT_HIP(hipMalloc(&d_dense.p, (size_t)nvox));
-        VT_HIP(hipMalloc(&d_remap.p, 256));
-        VT_HIP(to_device(c, d_dense.p, ids, (size_t)nvox));
-        VT_HIP(hipMemcpyAsync(d_remap.p, remap, 256, hipMemcpyHostToDevice, c->stream));
-        VT_HIP(vt::launch_brick_from_ids(c->dims, d_dense.p, d_remap.p, c->d_bricks, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
-        return finish_volume(c, emissive, n_emissive, occ, false);
+        uint8_t* const work = ws.p;
+        VT_HIP(to_device(c, work, ids, (size_t)nvox));
+        VT_HIP(to_device(c, work + remap_at, remap, 256));
+        uint32_t bad_entry = 0xffffffffu;
+        if (n_emissive > 0 && emissive) {
+            r = upload_emissive(c, emissive, n_emissive);
+            if (r != VT_OK) return r;
+            VT_HIP(vt::launch_fill_u32((uint32_t*)(work + bad_at), 1, 0xffffffffu, c->stream));
+            VT_HIP(vt::launch_check_emissive(c->d_emissive, n_emissive, (uint64_t)nvox, nullptr, work, work + remap_at,
+                                             (uint32_t*)(work + bad_at), c->stream));
+            VT_HIP(to_host(c, &bad_entry, work + bad_at, 4));
+        }
+        r = emissive_error(emissive, n_emissive, nvox, bad_entry);
+        if (r != VT_OK) return r;
+        VT_HIP(vt::launch_blocks_from_ids(c->dims, work, work + remap_at, c->d_bricks, block_levels(c), c->stream));
+        return finish_volume(c, n_emissive);
     });
 }
 
@@ -755,13 +801,14 @@ int vt_read_volume(vt_context* c, int32_t* offsets)
         int32_t table[256];
         table[0] = -1;
         for (int s = 1; s < 256; ++s) table[s] = c->slot_off[s];
-        DevTmp<int32_t> d_dense;
-        DevTmp<int32_t> d_table;
-        VT_HIP(hipMalloc(&d_dense.p, (size_t)nvox * 4u));
-        VT_HIP(hipMalloc(&d_table.p, sizeof(table)));
-        VT_HIP(hipMemcpyAsync(d_table.p, table, sizeof(table), hipMemcpyHostToDevice, c->stream));
-        VT_HIP(vt::launch_dense_from_bricks(c->dims, c->d_bricks, d_table.p, d_dense.p, c->stream));
-        VT_HIP(to_host(c, offsets, d_dense.p, (size_t)nvox * 4u));
+        WorkSpace ws;
+        const size_t table_at = aligned((size_t)nvox * 4u);
+        const int r = ws.take(c, table_at + sizeof(table));
+        if (r != VT_OK) return r;
+        uint8_t* const work = ws.p;
+        VT_HIP(to_device(c, work + table_at, table, sizeof(table)));
+        VT_HIP(vt::launch_dense_from_bricks(c->dims, c->d_bricks, (const int32_t*)(work + table_at), (int32_t*)work, c->stream));
+        VT_HIP(to_host(c, offsets, work, (size_t)nvox * 4u));
         return VT_OK;
     });
 }
@@ -2078,10 +2125,12 @@ int vt_trace_first_hit(vt_context* c, uint64_t seed, uint32_t frame, int32_t* re
         vt::TraceArgs a = trace_args(c);
         a.seed = seed; a.n0 = frame;
         const size_t bytes = (size_t)c->W * c->H * 8 * 4;
-        DevTmp<int32_t> d;
-        VT_HIP(hipMalloc(&d.p, bytes));
-        VT_HIP(vt::launch_first_hit(a, d.p, c->stream));
-        VT_HIP(to_host(c, rec, d.p, bytes));
+        WorkSpace ws;
+        const int r = ws.take(c, bytes);
+        if (r != VT_OK) return r;
+        uint8_t* const work = ws.p;
+        VT_HIP(vt::launch_first_hit(a, (int32_t*)work, c->stream));
+        VT_HIP(to_host(c, rec, work, bytes));
         return VT_OK;
     });
 }
@@ -2094,16 +2143,16 @@ int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, in
         if (n == 0) return VT_OK;
         VT_HIP(hipSetDevice(c->device));
         vt::TraceArgs a = trace_args(c);
-        DevTmp<float> d_o;
-        DevTmp<float> d_d;
-        DevTmp<int32_t> d_r;
-        VT_HIP(hipMalloc(&d_o.p, (size_t)n * 12));
-        VT_HIP(hipMalloc(&d_d.p, (size_t)n * 12));
-        VT_HIP(hipMalloc(&d_r.p, (size_t)n * 32));
-        VT_HIP(to_device(c, d_o.p, o, (size_t)n * 12));
-        VT_HIP(to_device(c, d_d.p, dir, (size_t)n * 12));
-        VT_HIP(vt::launch_trace_rays(a, n, d_o.p, d_d.p, d_r.p, c->stream));
-        VT_HIP(to_host(c, rec, d_r.p, (size_t)n * 32));
+        WorkSpace ws;
+        const size_t dir_at = aligned((size_t)n * 12), rec_at = 2 * dir_at;
+        const int r = ws.take(c, rec_at + (size_t)n * 32);
+        if (r != VT_OK) return r;
+        uint8_t* const work = ws.p;
+        VT_HIP(to_device(c, work, o, (size_t)n * 12));
+        VT_HIP(to_device(c, work + dir_at, dir, (size_t)n * 12));
+        VT_HIP(vt::launch_trace_rays(a, n, (const float*)work, (const float*)(work + dir_at), (int32_t*)(work + rec_at),
+                                     c->stream));
+        VT_HIP(to_host(c, rec, work + rec_at, (size_t)n * 32));
         return VT_OK;
     });
 }
@@ -2144,8 +2193,9 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
             return fail(VT_ERR_ARG, "bad argument");
         if (mode != 0 && mode != 1) return fail(VT_ERR_ARG, "mode must be 0 (THIN) or 1 (FAT)");
         if (!c->has_volume) return fail(VT_ERR_STATE, "no volume: call vt_set_volume first");
-        for (int64_t i = 0; i < 3 * ntri; ++i)
-            if ((int64_t)idx[i] >= nv) return fail(VT_ERR_ARG, "triangle index out of range");
+        uint32_t top = 0;              /* largest index, without a branch per index */
+        for (int64_t i = 0; i < 3 * ntri; ++i) top = idx[i] > top ? idx[i] : top;
+        if (ntri > 0 && (int64_t)top >= nv) return fail(VT_ERR_ARG, "triangle index out of range");
         if (material_offset < 0 || material_offset >= (int32_t)c->mat.size())
             return fail(VT_ERR_ARG, "material offset outside material data");
         int slot = 0;
@@ -2167,28 +2217,29 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
         a.mode = mode;
         a.slot = (uint8_t)slot;
         a.bricks = c->d_bricks;
-        DevTmp<float> d_v;
-        DevTmp<uint32_t> d_i;
-        DevTmp<uint8_t> d_occ;
         const int64_t nvox = (int64_t)c->dims.nx * c->dims.ny * c->dims.nz;
-        if (ntri > 0) {
-            VT_HIP(hipMalloc(&d_v.p, (size_t)nv * 12));
-            VT_HIP(hipMalloc(&d_i.p, (size_t)ntri * 12));
-            VT_HIP(to_device(c, d_v.p, verts, (size_t)nv * 12));
-            VT_HIP(to_device(c, d_i.p, idx, (size_t)ntri * 12));
+        /* workspace: vertices, indices, the list of large triangles (a wave
+         * each) and its counter, the dense occupancy */
+        WorkSpace ws;
+        const size_t idx_at = aligned((size_t)nv * 12), big_at = idx_at + aligned((size_t)ntri * 12),
+                     occ_at = big_at + aligned(((size_t)ntri + 1) * 4);
+        {
+            const int r = ws.take(c, occ_at + (occupancy ? (size_t)nvox : 0u));
+            if (r != VT_OK) return r;
         }
-        if (occupancy) {
-            VT_HIP(hipMalloc(&d_occ.p, (size_t)nvox));
-            VT_HIP(vt::launch_fill_u8(d_occ.p, (uint64_t)nvox, 0, c->stream));
-        }
-        a.verts = d_v.p; a.idx = d_i.p; a.occ = d_occ.p;
-        /* the list of large triangles (a wave each) and its counter */
-        DevTmp<uint32_t> d_big;
+        uint8_t* const work = ws.p;
         if (ntri > 0) {
-            VT_HIP(hipMalloc(&d_big.p, ((size_t)ntri + 1) * 4));
-            VT_HIP(vt::launch_fill_u32(d_big.p + ntri, 1, 0u, c->stream));
-            a.big = d_big.p;
-            a.big_count = d_big.p + ntri;
+            VT_HIP(to_device(c, work, verts, (size_t)nv * 12));
+            VT_HIP(to_device(c, work + idx_at, idx, (size_t)ntri * 12));
+        }
+        if (occupancy) VT_HIP(vt::launch_fill_u8(work + occ_at, (uint64_t)nvox, 0, c->stream));
+        a.verts = (const float*)work;
+        a.idx = (const uint32_t*)(work + idx_at);
+        a.occ = occupancy ? work + occ_at : nullptr;
+        if (ntri > 0) {
+            a.big = (uint32_t*)(work + big_at);
+            a.big_count = a.big + ntri;
+            VT_HIP(vt::launch_fill_u32(a.big_count, 1, 0u, c->stream));
             a.big_cap = (uint32_t)std::min<int64_t>(ntri, 0x7fffffff);   /* beyond it, triangles keep their thread */
             a.big_area = VT_VOX_BIG_AREA;
         }
@@ -2197,11 +2248,12 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
         VT_HIP(hipEventRecord(c->ev1, c->stream));
         c->timed = true;           /* vt_get_stats: kernel_ms of the voxelizer launch */
         c->stats_valid = false;
+        VT_HIP(vt::launch_blocks_from_bricks(c->dims, c->d_bricks, block_levels(c), c->stream));
         {
-            int r = refresh_occupancy(c);
+            int r = refresh_codes(c);
             if (r != VT_OK) return r;
         }
-        if (occupancy) VT_HIP(to_host(c, occupancy, d_occ.p, (size_t)nvox));
+        if (occupancy) VT_HIP(to_host(c, occupancy, work + occ_at, (size_t)nvox));
         VT_HIP(hipStreamSynchronize(c->stream));
         return VT_OK;
     });

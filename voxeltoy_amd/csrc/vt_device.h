@@ -10,11 +10,12 @@
  * read only at a hit.
  *
  * The traversal reads two occupancy levels over the 4x4x4 blocks, both in
- * linear block order (bx + BX*(by + BY*bz), BX = ceil(nx/4), ...): one bit
- * per block (set when any voxel of the block is occupied), staged in LDS when
- * it fits, and one 64-bit voxel mask per block (bit x + 4y + 16z for local
- * voxel (x, y, z)).  Entering a block costs one bit test; only non-empty
- * blocks load their 8-byte mask.
+ * linear order over the padded block grid (bxp, byp below): one bit per block
+ * (set when any voxel of the block is occupied or outside the grid), staged in
+ * LDS when it fits, and one 64-bit voxel mask per block (bit x + 4y + 16z for
+ * local voxel (x, y, z)).  Entering a block costs one bit test; only non-empty
+ * blocks load their 8-byte mask.  Renders without statistics read codes of
+ * empty cubes instead of the bits (the jump march, below).
  *
  * The traversal replays the reference 3D-DDA (src/shaders/shared/dda.h:7-100)
  * step by step: `dis` is a running FP32 sum, so empty space skips the loads
@@ -71,14 +72,11 @@ struct GridView {
     float rx, ry, rz;           /* resolution as float */
     float bmin[3], bmax[3], vs[3], ext[3];
     const uint8_t* bricks;      /* Morton bricks of 512 bytes */
-    uint32_t bx4, by4;          /* 4x4x4 block grid extents in x and y */
-    const uint64_t* occ64;      /* per-block voxel masks, linear block order */
-    const uint32_t* bits;       /* per-block non-empty bits (global copy) */
-    uint32_t bit_words;
-    /* the same two levels over the block grid padded by one block on every
-     * side (grid block (bx, by, bz) is padded block (bx+1, by+1, bz+1)), in
-     * which every voxel outside the grid reads as occupied: the wave march
-     * stops at the first voxel outside the grid without a bounds test */
+    /* per-block voxel masks and non-empty bits, linear order over the block
+     * grid padded by one block on every side, rows to a multiple of four
+     * blocks (grid block (bx, by, bz) is padded block (bx+1, by+1, bz+1)), in
+     * which every voxel outside the grid reads as occupied: the wave marches
+     * stop at the first voxel outside the grid without a bounds test */
     uint32_t bxp, byp;          /* padded block extents in x and y */
     const uint64_t* occp;
     const uint32_t* bitsp;
@@ -89,8 +87,9 @@ struct GridView {
     const uint64_t* occr;
     int32_t wide;               /* padded masks span 4 GiB or more (byte offsets need 64 bits) */
     /* 2-bit empty-cube codes of the jump march, 16 per word, over the grid's
-     * cells of 2^cg voxels padded by one cell on every side, linear order
-     * (cx + ccx*(cy + ccy*cz)): 0 = some voxel of the cell is occupied or
+     * cells of 2^cg voxels padded by one cell on every side (rows to a multiple
+     * of four cells, so that they begin at a byte; cells of one block are
+     * numbered as the padded blocks), linear order (cx + ccx*(cy + ccy*cz)): 0 = some voxel of the cell is occupied or
      * outside the grid, c = 1..3 = the aligned cube of (byte c of cedge) + 1
      * voxels an edge around the cell is empty and inside the grid */
     const uint32_t* codes;
@@ -156,8 +155,6 @@ __device__ __forceinline__ uint32_t local_morton(uint32_t x, uint32_t y, uint32_
 {
     return spread3_3(x & 7u) | (spread3_3(y & 7u) << 1) | (spread3_3(z & 7u) << 2);
 }
-/* Linear index of the 4x4x4 block holding in-grid voxel (x, y, z); fits
- * 24-bit multiplies since block extents are at most 1024. */
 /* a * b + c on 24-bit operands as one full-rate instruction (the compiler
  * otherwise may pick a 64-bit multiply-add) */
 __device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c)
@@ -165,16 +162,6 @@ __device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c)
     uint32_t r;
     asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
-}
-
-__device__ __forceinline__ uint32_t block_index(const GridView& g, uint32_t x, uint32_t y, uint32_t z)
-{
-    return mad24(mad24(z >> 2, g.by4, y >> 2), g.bx4, x >> 2);
-}
-/* Bit of voxel (x, y, z) in its 4x4x4 block mask. */
-__device__ __forceinline__ uint32_t block_bit(uint32_t x, uint32_t y, uint32_t z)
-{
-    return (x & 3u) | ((y & 3u) << 2) | ((z & 3u) << 4);
 }
 
 /* ---- rayAABBIntersection (aabb.h:1-32) -------------------------------------------- */
@@ -204,12 +191,6 @@ __device__ __forceinline__ float min3f(float a, float b, float c)
     float r;
     asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
-}
-
-/* Key of the 4x4x4 block of an in-grid voxel (10 bits per axis). */
-__device__ __forceinline__ uint32_t block_key(int32_t x, int32_t y, int32_t z)
-{
-    return ((uint32_t)x >> 2) | (((uint32_t)y >> 2) << 10) | (((uint32_t)z >> 2) << 20);
 }
 
 /* The grid-independent part of raymarch's set-up (dda.h:7-35): origin
@@ -307,18 +288,18 @@ struct DdaState {
         const int32_t limit = budget < g.max_steps - steps ? steps + budget : g.max_steps;
         bool done = false;
         /* block-grid strides held in vector registers across the loop */
-        uint32_t bx4 = g.bx4, by4 = g.by4;
-        asm volatile("" : "+v"(bx4), "+v"(by4));
+        uint32_t bxp = g.bxp, byp = g.byp, first = 1u + g.bxp + g.bxp * g.byp;   /* padded index of block (0, 0, 0) */
+        asm volatile("" : "+v"(bxp), "+v"(byp), "+v"(first));
         for (;;) {
             const bool inside = (uint32_t)x < (uint32_t)g.nx && (uint32_t)y < (uint32_t)g.ny &&
                                 (uint32_t)z < (uint32_t)g.nz;
             const bool more = steps < limit;
             /* the block's linear index doubles as its key (meaningful for
              * in-grid voxels only, the only ones that reload) */
-            const uint32_t bk = mad24(mad24((uint32_t)z >> 2, by4, (uint32_t)y >> 2), bx4, (uint32_t)x >> 2);
+            const uint32_t bk = mad24(mad24((uint32_t)z >> 2, byp, (uint32_t)y >> 2), bxp, (uint32_t)x >> 2) + first;
             if (inside && bk != key) {
                 key = bk;
-                mask = ((bits[bk >> 5] >> (bk & 31u)) & 1u) ? g.occ64[bk] : 0ull;
+                mask = ((bits[bk >> 5] >> (bk & 31u)) & 1u) ? g.occp[bk] : 0ull;
             }
             /* the voxel test only when some lane's block has an occupied voxel
              * (a wave-uniform branch: rays in empty space skip it) */

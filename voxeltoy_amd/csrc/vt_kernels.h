@@ -173,31 +173,43 @@ struct BrickDims {
     int32_t bdim;                /* power-of-two cube edge in bricks (Morton range) */
     uint64_t n_bricks;           /* bdim^3 */
     int32_t kx, ky, kz;          /* 4x4x4 blocks per axis (ceil(n/4)) */
-    uint64_t n_blocks;           /* kx*ky*kz */
+    /* the block grid padded by one block on every side, rows to a multiple of
+     * four blocks (rows of the jump march's codes are whole bytes, and with
+     * cells of one block both have one index) */
+    int32_t px, py, pz;
+    uint64_t n_padded;           /* px*py*pz */
 };
 
-/* Dense int32 offsets -> bricked slots via lut[offset] (offset in
- * [0, lut_n)), -1 (or any negative) -> slot 0.  Out-of-range offsets set
- * *bad. */
-hipError_t launch_brick_from_offsets(const BrickDims& d, const int32_t* dense, const uint8_t* lut, int32_t lut_n,
-                                     uint8_t* bricks, uint32_t* bad, hipStream_t s);
-/* Dense uint8 ids -> bricked slots via remap[256]. */
-hipError_t launch_brick_from_ids(const BrickDims& d, const uint8_t* dense, const uint8_t* remap, uint8_t* bricks,
-                                 hipStream_t s);
-/* Per 4x4x4 block voxel masks in linear block order (occ64 holds n_blocks
- * words) and the per-block non-empty bits ((n_blocks+31)/32 words); then
- * the same over the block grid padded by one block on every side
- * ((kx+2)(ky+2)(kz+2) words in occp), where voxels outside the grid are
- * set. */
-hipError_t launch_block_masks(const BrickDims& d, const uint8_t* bricks, uint64_t* occ64, uint32_t* bits,
-                              uint64_t* occp, uint32_t* bitsp, uint64_t* occr, hipStream_t s);
-/* The jump march's codes (GridView::codes) from the padded masks: one byte
- * per cell of 2^cg voxels in `cells` (padded by one cell, whose bytes stay
- * zero; n_cells bytes, readable up to the next multiple of 16), then 16
- * two-bit codes per word.  The largest coded cube has 2^top cells an edge
- * (top 2 or 3), the next 2, the smallest 1. */
-hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint8_t* cells,
-                             uint64_t n_cells, uint32_t* codes, hipStream_t s);
+/* Which material offsets a dense int32 grid uses: used[o] = 1 for every o in
+ * [0, lut_n) that occurs (used zero at launch); *bad = the smallest index of
+ * an offset >= lut_n (all ones at launch). */
+hipError_t launch_scan_offsets(const int32_t* dense, uint64_t n, int32_t lut_n, uint8_t* used, unsigned long long* bad,
+                               hipStream_t s);
+/* *bad = the smallest i whose emissive[i] lies outside [0, n_vox) or is an
+ * empty voxel of the dense grid (offsets, or ids with their remap; the other
+ * null); all ones at launch. */
+hipError_t launch_check_emissive(const int32_t* emissive, int32_t n, uint64_t n_vox, const int32_t* offsets,
+                                 const uint8_t* ids, const uint8_t* remap, uint32_t* bad, hipStream_t s);
+/* The block levels (GridView: masks occp, their bit-reversed copy occr unless
+ * null, bits bitsp) of the padded block grid.  From the bricks, or from a
+ * dense grid (offsets with lut, or ids with remap), which also writes the
+ * bricks. */
+struct BlockLevels {
+    uint64_t* occp;
+    uint64_t* occr;
+    uint32_t* bitsp;
+};
+hipError_t launch_blocks_from_bricks(const BrickDims& d, const uint8_t* bricks, const BlockLevels& L, hipStream_t s);
+hipError_t launch_blocks_from_offsets(const BrickDims& d, const int32_t* dense, const uint8_t* lut, uint8_t* bricks,
+                                      const BlockLevels& L, hipStream_t s);
+hipError_t launch_blocks_from_ids(const BrickDims& d, const uint8_t* dense, const uint8_t* remap, uint8_t* bricks,
+                                  const BlockLevels& L, hipStream_t s);
+/* The jump march's codes (GridView::codes) from the padded masks, for cells of
+ * 2^cg voxels in rows of ccx and layers of ccx ccy cells.  The largest coded
+ * cube has 2^top cells an edge (top 2 or 3), the next 2, the smallest 1.  The
+ * codes of the padding are not written (zero). */
+hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint32_t ccx,
+                             uint32_t ccy, uint32_t* codes, hipStream_t s);
 /* Bricked slots -> dense int32 offsets via slot_off[256]. */
 hipError_t launch_dense_from_bricks(const BrickDims& d, const uint8_t* bricks, const int32_t* slot_off, int32_t* dense,
                                     hipStream_t s);

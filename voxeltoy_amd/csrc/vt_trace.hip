@@ -244,10 +244,10 @@ __device__ __forceinline__ void stage_lds(const TraceArgs& a, uint8_t* smem, Mat
     cdfv = cv;
     if (LDSB) {
         uint32_t* sb = (uint32_t*)(smem + 256 * sizeof(MatRec) + a.cdfv_lds_bytes);
-        for (uint32_t i = threadIdx.x; i < a.g.bit_words; i += blockDim.x) sb[i] = a.g.bits[i];
+        for (uint32_t i = threadIdx.x; i < a.g.bit_words_p; i += blockDim.x) sb[i] = a.g.bitsp[i];
         bits = sb;
     } else {
-        bits = a.g.bits;
+        bits = a.g.bitsp;
     }
     __syncthreads();
 }
@@ -654,7 +654,7 @@ __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r
     /* with no finite distance the ray never moves: its start voxel decides */
     const bool stuck = D.disx != D.disx && D.disy != D.disy && D.disz != D.disz;
     uint32_t dummy = 0;
-    const int status = D.advance<false>(g, g.bits, stuck ? 1 : g.max_steps, dummy);
+    const int status = D.advance<false>(g, g.bitsp, stuck ? 1 : g.max_steps, dummy);
     return pack_hit(D.x, D.y, D.z, status == 1 ? KIND_VOXEL : (D.y < 0 ? KIND_GROUND : KIND_MISS));
 }
 
@@ -910,7 +910,7 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
             const TraceArgs& a = BATCH ? B.tab[sid] : a0;
             const MatRec* recs = BATCH ? a.recs : recs0;
             const float* cdfv = BATCH ? a.e.cdfv : cdfv0;
-            const uint32_t* bits = BATCH ? a.g.bits : bits0;
+            const uint32_t* bits = BATCH ? a.g.bitsp : bits0;
             const uint32_t slot1 = CACHE ? me.w : 0u;   /* training slot + 1 */
             Hit h;
             h.steps = 0;
@@ -1199,7 +1199,7 @@ __global__ __launch_bounds__(256) void light_table_kernel(GridView g, int4* __re
         idx -= z * dz;
         const int32_t y = idx / dy;
         idx -= y * dy;
-        out[i] = make_int4(idx, y, z, (int32_t)fetch_slot(g, g.bits, idx, y, z));
+        out[i] = make_int4(idx, y, z, (int32_t)fetch_slot(g, g.bitsp, idx, y, z));
     }
 }
 
@@ -1246,7 +1246,7 @@ __global__ __launch_bounds__(256) void first_hit_kernel(TraceArgs a, int32_t* ou
         for (int k = 0; k < 8; ++k) rec[k] = 0;
         return;
     }
-    hit_record(g, g.bits, o + d * t, d, o, rec);
+    hit_record(g, g.bitsp, o + d * t, d, o, rec);
 }
 
 __global__ __launch_bounds__(256) void trace_rays_kernel(TraceArgs a, int32_t n, const float* orig, const float* dir,
@@ -1256,7 +1256,7 @@ __global__ __launch_bounds__(256) void trace_rays_kernel(TraceArgs a, int32_t n,
     if (i >= n) return;
     const f3 o = mk(orig[3 * i], orig[3 * i + 1], orig[3 * i + 2]);
     const f3 d = mk(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]);
-    hit_record(a.g, a.g.bits, o, d, o, out + 8 * (size_t)i);
+    hit_record(a.g, a.g.bitsp, o, d, o, out + 8 * (size_t)i);
 }
 
 __global__ void reset_counter_kernel(uint32_t* c, unsigned long long* stats)
@@ -1289,7 +1289,7 @@ __global__ void device_math_kernel(int32_t fn, int32_t n, const float* a, const 
 /* ---- launchers ------------------------------------------------------------------ */
 size_t render_lds_bytes(const TraceArgs& a)
 {
-    return 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes + (a.lds_bits ? (size_t)a.g.bit_words * 4u : 0u);
+    return 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes + (a.lds_bits ? (size_t)a.g.bit_words_p * 4u : 0u);
 }
 
 static void (*render_ptr(bool stats, bool ldsb))(TraceArgs)

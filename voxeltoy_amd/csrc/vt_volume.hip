@@ -19,173 +19,215 @@ __device__ __forceinline__ uint64_t brick_byte(int32_t x, int32_t y, int32_t z)
            local_morton((uint32_t)x, (uint32_t)y, (uint32_t)z);
 }
 
-__global__ __launch_bounds__(256) void brick_from_offsets_kernel(BrickDims d, const int32_t* __restrict__ dense,
-                                                                 const uint8_t* __restrict__ lut, int32_t lut_n,
-                                                                 uint8_t* __restrict__ bricks, uint32_t* bad)
+/* One coalesced pass over the offsets (64 MB in 17 us).  With the conversion
+ * below it replaces three loops over the grid on one host thread: loading a
+ * 256^3 grid of offsets and rendering 960x540 from it went from 7.7 to 2.2 ms,
+ * 1.3 of them the link. */
+__global__ __launch_bounds__(256) void scan_offsets_kernel(const int32_t* __restrict__ dense, uint64_t n, int32_t lut_n,
+                                                           uint8_t* used, unsigned long long* bad)
 {
-    const int64_t n = (int64_t)d.nx * d.ny * d.nz;
+    const uint64_t n4 = n / 4u;
+    int32_t last = -1;                       /* neighbours mostly share an offset or are empty */
+    uint64_t first_bad = ~0ull;
+    auto look = [&](int32_t o, uint64_t i) {
+        if (o < 0 || o == last) return;
+        last = o;
+        if (o >= lut_n) first_bad = i < first_bad ? i : first_bad, last = -1;
+        else if (!used[o]) used[o] = 1u;
+    };
+    for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n4; q += (uint64_t)gridDim.x * blockDim.x) {
+        const int4 v = ((const int4*)dense)[q];
+        look(v.x, 4u * q);
+        look(v.y, 4u * q + 1u);
+        look(v.z, 4u * q + 2u);
+        look(v.w, 4u * q + 3u);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3u)) look(dense[4u * n4 + threadIdx.x], 4u * n4 + threadIdx.x);
+    if (first_bad != ~0ull) atomicMin(bad, (unsigned long long)first_bad);
+}
+
+__global__ __launch_bounds__(256) void check_emissive_kernel(const int32_t* __restrict__ emissive, int32_t n,
+                                                             uint64_t n_vox, const int32_t* __restrict__ offsets,
+                                                             const uint8_t* __restrict__ ids,
+                                                             const uint8_t* __restrict__ remap, uint32_t* bad)
+{
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t x = (int32_t)(i % d.nx);
-        const int64_t r = i / d.nx;
-        const int32_t y = (int32_t)(r % d.ny), z = (int32_t)(r / d.ny);
-        const int32_t off = dense[i];
-        uint8_t slot = 0;
-        if (off >= 0) {
-            if (off < lut_n && lut[off] != 0) slot = lut[off];
-            else atomicOr(bad, 1u);
-        }
-        bricks[brick_byte(x, y, z)] = slot;
+        const int32_t e = emissive[i];
+        const bool ok = e >= 0 && (uint64_t)e < n_vox && (offsets ? offsets[e] >= 0 : remap[ids[e]] != 0u);
+        if (!ok) atomicMin(bad, (uint32_t)i);
     }
 }
 
-__global__ __launch_bounds__(256) void brick_from_ids_kernel(BrickDims d, const uint8_t* __restrict__ dense,
-                                                             const uint8_t* __restrict__ remap,
-                                                             uint8_t* __restrict__ bricks)
+/* Four flags (bits 0..3) of the non-zero bytes of v. */
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v)
 {
-    const int64_t n = (int64_t)d.nx * d.ny * d.nz;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t x = (int32_t)(i % d.nx);
-        const int64_t r = i / d.nx;
-        const int32_t y = (int32_t)(r % d.ny), z = (int32_t)(r / d.ny);
-        bricks[brick_byte(x, y, z)] = remap[dense[i]];
-    }
+    const uint32_t t = (((v & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v) & 0x80808080u;
+    return ((t >> 7) * 0x10204080u) >> 28;
 }
 
-/* occ64[b] for block b = bx + kx*(by + ky*bz): bit (x + 4y + 16z) set when
- * local voxel (x, y, z) of the block is occupied.  The block's 64 slot bytes
- * are one Morton-ordered run inside its brick. */
-__global__ __launch_bounds__(256) void block_masks_kernel(BrickDims d, const uint8_t* __restrict__ bricks,
-                                                          uint64_t* __restrict__ occ64)
+/* One thread per 4x4x4 block of the padded block grid, consecutive threads
+ * along x.  A block's 64 slots are one Morton-ordered 64-byte line of its
+ * brick: dword z0 + 2 x1 + 4 y1 + 8 z1 holds the voxels (x0, y0) of a 2x2
+ * square.  From a dense grid (SRC 1 offsets, 2 ids) a thread reads the block's
+ * 16 rows of four voxels (a wave's rows are contiguous), writes the line and
+ * forms the mask from the same registers, so the grid is read once and the
+ * bricks are not read back.  Voxels outside the grid are set in the masks, the
+ * padding's masks are all set.  Bound by memory: 256^3 offsets (64 MB read, 21
+ * MB written) in 27 us, where the conversion into bricks alone took 68 and the
+ * padded masks and two passes of bits 25 more.  From the bricks 5 us (512^3,
+ * 35; the masks alone took 48 and 30 for two separate layouts). */
+template <int SRC>
+__global__ __launch_bounds__(256) void blocks_kernel(BrickDims d, const void* __restrict__ dense,
+                                                     const uint8_t* __restrict__ lut, uint8_t* __restrict__ bricks,
+                                                     BlockLevels L)
 {
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < d.n_blocks;
-         w += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t bx = (uint32_t)(w % (uint64_t)d.kx);
-        const uint64_t r = w / (uint64_t)d.kx;
-        const uint32_t by = (uint32_t)(r % (uint64_t)d.ky), bz = (uint32_t)(r / (uint64_t)d.ky);
-        const uint32_t sb = (bx & 1u) | ((by & 1u) << 1) | ((bz & 1u) << 2);
-        const uint4* p = (const uint4*)(bricks + (uint64_t)brick_morton(bx >> 1, by >> 1, bz >> 1) * 512u + sb * 64u);
-        uint64_t m = 0;
+    const uint32_t px = (uint32_t)d.px, py = (uint32_t)d.py;
+    const uint32_t n = (uint32_t)d.n_padded;  /* at most 1028 * 1026^2 */
+    const bool rows4 = (d.nx & 3) == 0;       /* every row of four voxels aligned */
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+        const uint32_t w = base + threadIdx.x;
+        const uint32_t r = w / px, bx = w - r * px;
+        const uint32_t bz = r / py, by = r - bz * py;
+        uint64_t m = ~0ull;
+        if (w < n && bx - 1u < (uint32_t)d.kx && by - 1u < (uint32_t)d.ky && bz - 1u < (uint32_t)d.kz) {
+            const uint32_t gx = bx - 1u, gy = by - 1u, gz = bz - 1u;
+            const int32_t x0 = (int32_t)(4u * gx), y0 = (int32_t)(4u * gy), z0 = (int32_t)(4u * gz);
+            uint4* line = (uint4*)(bricks + (uint64_t)brick_morton(gx >> 1, gy >> 1, gz >> 1) * 512u +
+                                   ((gx & 1u) | ((gy & 1u) << 1) | ((gz & 1u) << 2)) * 64u);
+            m = 0ull;
+            if (SRC == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint4 v = p[q];
-            const uint32_t wd[4] = { v.x, v.y, v.z, v.w };
+                for (int q = 0; q < 4; ++q) {
+                    const uint4 v = line[q];
+                    const uint32_t wd[4] = { v.x, v.y, v.z, v.w };
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const uint32_t mo = (uint32_t)(q * 16 + k * 4 + b);   /* Morton index in the block */
-                    const uint32_t bit = (mo & 1u) | ((mo >> 2) & 2u) |            /* x bits 0, 3 */
-                                         (((mo >> 1) & 1u) << 2) | (((mo >> 4) & 1u) << 3) |   /* y */
-                                         (((mo >> 2) & 1u) << 4) | (((mo >> 5) & 1u) << 5);    /* z */
-                    if ((wd[k] >> (8 * b)) & 0xffu) m |= 1ull << bit;
+                    for (int k = 0; k < 4; ++k) {
+                        const int i = 4 * q + k;
+                        const uint32_t f = nonzero_bytes(wd[k]);
+                        m |= (uint64_t)((f & 3u) | ((f & 12u) << 2))
+                             << (2 * ((i >> 1) & 1) + 8 * ((i >> 2) & 1) + 16 * ((i & 1) + 2 * (i >> 3)));
+                    }
                 }
+            } else {
+                uint32_t row[16];             /* slots of row (y, z) at 4 z + y */
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int32_t y = y0 + (i & 3), z = z0 + (i >> 2);
+                    row[i] = 0u;
+                    if (y >= d.ny || z >= d.nz) continue;
+                    const uint64_t at = (uint64_t)x0 + (uint64_t)d.nx * ((uint64_t)y + (uint64_t)d.ny * (uint64_t)z);
+                    if (SRC == 1) {
+                        const int32_t* p = (const int32_t*)dense + at;
+                        int32_t o[4] = { -1, -1, -1, -1 };
+                        if (rows4) {
+                            const int4 v = *(const int4*)p;
+                            o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                if (x0 + k < d.nx) o[k] = p[k];
+                        }
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if (o[k] >= 0) row[i] |= (uint32_t)lut[o[k]] << (8 * k);
+                    } else {
+                        const uint8_t* p = (const uint8_t*)dense + at;
+                        if (rows4) {
+                            const uint32_t v = *(const uint32_t*)p;
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) row[i] |= (uint32_t)lut[(v >> (8 * k)) & 0xffu] << (8 * k);
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                if (x0 + k < d.nx) row[i] |= (uint32_t)lut[p[k]] << (8 * k);
+                        }
+                    }
+                    m |= (uint64_t)nonzero_bytes(row[i]) << (4 * (i & 3) + 16 * (i >> 2));
+                }
+                uint32_t out[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int x1 = (i >> 1) & 1, y1 = (i >> 2) & 1, z = (i & 1) + 2 * (i >> 3);
+                    out[i] = ((row[4 * z + 2 * y1] >> (16 * x1)) & 0xffffu) |
+                             (((row[4 * z + 2 * y1 + 1] >> (16 * x1)) & 0xffffu) << 16);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) line[q] = make_uint4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+            }
+            if (x0 + 4 > d.nx || y0 + 4 > d.ny || z0 + 4 > d.nz)
+                for (int l = 0; l < 64; ++l)
+                    if (x0 + (l & 3) >= d.nx || y0 + ((l >> 2) & 3) >= d.ny || z0 + (l >> 4) >= d.nz) m |= 1ull << l;
         }
-        occ64[w] = m;
+        /* a wave's 64 blocks are two words of bits */
+        const unsigned long long bits = __ballot(w < n && m != 0ull);
+        if (w < n) {
+            L.occp[w] = m;
+            if (L.occr) L.occr[w] = __builtin_bitreverse64(m);
+            if ((threadIdx.x & 31u) == 0u) L.bitsp[w >> 5] = (uint32_t)(bits >> (threadIdx.x & 32u));
+        }
     }
 }
 
-/* bits[i] bit k = (occ64[32i + k] != 0). */
-__global__ __launch_bounds__(256) void block_bits_kernel(uint64_t n_blocks, const uint64_t* __restrict__ occ64,
-                                                         uint32_t* __restrict__ bits)
-{
-    const uint64_t n_words = (n_blocks + 31) / 32;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t v = 0;
-        for (uint32_t k = 0; k < 32u && i * 32u + k < n_blocks; ++k)
-            if (occ64[i * 32u + k]) v |= 1u << k;
-        bits[i] = v;
-    }
-}
-
-/* occp over the padded block grid (kx+2) x (ky+2) x (kz+2): border blocks
- * all set; interior block (bx, by, bz) = grid block (bx-1, by-1, bz-1)
- * with the bits of its voxels outside the grid set (grids whose extents
- * are not multiples of 4). */
-__global__ __launch_bounds__(256) void block_masks_padded_kernel(BrickDims d, const uint64_t* __restrict__ occ64,
-                                                                 uint64_t* __restrict__ occp)
-{
-    const uint32_t px = (uint32_t)d.kx + 2u, py = (uint32_t)d.ky + 2u, pz = (uint32_t)d.kz + 2u;
-    const uint64_t n = (uint64_t)px * py * pz;
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < n; w += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t bx = (uint32_t)(w % px);
-        const uint64_t r = w / px;
-        const uint32_t by = (uint32_t)(r % py), bz = (uint32_t)(r / py);
-        if (bx == 0 || by == 0 || bz == 0 || bx == px - 1u || by == py - 1u || bz == pz - 1u) {
-            occp[w] = ~0ull;
-            continue;
-        }
-        const uint32_t gx = bx - 1u, gy = by - 1u, gz = bz - 1u;
-        uint64_t m = occ64[gx + (uint64_t)d.kx * (gy + (uint64_t)d.ky * gz)];
-        for (uint32_t l = 0; l < 64u; ++l) {
-            const int32_t x = (int32_t)(4u * gx + (l & 3u)), y = (int32_t)(4u * gy + ((l >> 2) & 3u)),
-                          z = (int32_t)(4u * gz + (l >> 4));
-            if (x >= d.nx || y >= d.ny || z >= d.nz) m |= 1ull << l;
-        }
-        occp[w] = m;
-    }
-}
-
-/* occr: occp with each mask's bits reversed (voxel l of the block at bit
- * 63 - l): the packed march tests a voxel by shifting its bit into the sign. */
-__global__ __launch_bounds__(256) void block_masks_reversed_kernel(const uint64_t* __restrict__ occp,
-                                                                   uint64_t* __restrict__ occr, uint64_t n)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        occr[i] = __builtin_bitreverse64(occp[i]);
-}
-
-/* Bytes of the jump march's codes: one workgroup per aligned cube of the
- * largest size (2^T cells an edge), one thread per cell, eight consecutive
- * threads per 2x2x2 cells.  A cell is taken as occupied when any of its
- * voxels is occupied or lies outside the grid (occp has those bits set), so
- * no coded cube reaches past the grid.  codes bytes: see GridView::codes. */
+#define CODE_BYTES 8
+/* Codes of the jump march: one workgroup per R x R rows of cells (R = 2^T, the
+ * largest coded cube's edge) and 8 bytes of each row.  A row's bytes begin one
+ * cell before the grid's, so a workgroup reads the cubes of one more R in x.
+ * A cell is full when it has an occupied voxel or one outside the grid, or
+ * lies outside the cell grid itself: no coded cube reaches past the grid.
+ * Bound by the latency of its loads, which are independent (a thread per
+ * cell): 8.4 us at 256^3, 24 at 512^3; a row of cells per workgroup, with the
+ * loads of one y after the other, took 15 and 47. */
 template <int T>
-__global__ __launch_bounds__(1 << (3 * T)) void cell_codes_kernel(BrickDims d, const uint64_t* __restrict__ occp,
-                                                                  uint32_t cg, int32_t ncx, int32_t ncy, int32_t ncz,
-                                                                  uint8_t* __restrict__ cells)
+__global__ __launch_bounds__(256) void cell_codes_kernel(BrickDims d, const uint64_t* __restrict__ occp, uint32_t cg,
+                                                         int32_t ncx, int32_t ncy, int32_t ncz, uint32_t ccx,
+                                                         uint32_t ccy, uint8_t* __restrict__ codes)
 {
-    const uint32_t t = threadIdx.x;
-    /* local cell: bit k of each coordinate from bits 3k, 3k+1, 3k+2 of the thread */
-    int32_t l[3] = { 0, 0, 0 };
-#pragma unroll
-    for (int k = 0; k < T; ++k)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) l[c] |= (int32_t)((t >> (3 * k + c)) & 1u) << k;
-    const int32_t cx = (int32_t)(blockIdx.x << T) + l[0], cy = (int32_t)(blockIdx.y << T) + l[1],
-                  cz = (int32_t)(blockIdx.z << T) + l[2];
-    const bool in = cx < ncx && cy < ncy && cz < ncz;
-    bool full = true;
-    if (in) {
-        const int32_t e = 1 << (cg - 2u);     /* 4x4x4 blocks per cell edge */
-        const int32_t x0 = cx * e, y0 = cy * e, z0 = cz * e;
-        full = x0 + e > d.kx || y0 + e > d.ky || z0 + e > d.kz;
-        const uint64_t px = (uint64_t)(d.kx + 2), py = (uint64_t)(d.ky + 2);
-        for (int32_t z = z0; z < z0 + e && !full; ++z)
-            for (int32_t y = y0; y < y0 + e && !full; ++y)
-                for (int32_t x = x0; x < x0 + e; ++x)
-                    full = full || occp[(uint64_t)(x + 1) + px * ((uint64_t)(y + 1) + py * (uint64_t)(z + 1))] != 0ull;
+    constexpr int R = 1 << T, H = R / 2, QB = CODE_BYTES, W = 4 * QB + R;
+    __shared__ uint8_t full[R * R * W], pair[H * H * (W / 2)], top[W / R];
+    const int32_t cy0 = (int32_t)blockIdx.x * R, cz0 = (int32_t)blockIdx.y * R, q0 = (int32_t)blockIdx.z * QB;
+    const int32_t cx0 = 4 * q0 - R;
+    const int32_t e = 1 << (cg - 2u);               /* 4x4x4 blocks per cell edge */
+    const uint64_t px = (uint64_t)d.px, py = (uint64_t)d.py;
+    for (int32_t i = threadIdx.x; i < R * R * W; i += blockDim.x) {
+        const int32_t cx = cx0 + i % W, cy = cy0 + i / W % R, cz = cz0 + i / (W * R);
+        const int32_t bx = cx * e, by = cy * e, bz = cz * e;
+        bool occ = cx < 0 || cx >= ncx || cy >= ncy || cz >= ncz || bx + e > d.kx || by + e > d.ky || bz + e > d.kz;
+        if (!occ) {
+            uint64_t m = 0ull;
+            for (int32_t z = bz; z < bz + e; ++z)
+                for (int32_t y = by; y < by + e; ++y)
+                    for (int32_t x = bx; x < bx + e; ++x)
+                        m |= occp[(uint64_t)(x + 1) + px * ((uint64_t)(y + 1) + py * (uint64_t)(z + 1))];
+            occ = m != 0ull;
+        }
+        full[i] = occ ? 1u : 0u;
     }
-    const unsigned long long m = __ballot(full);
-    const bool oct_full = ((m >> (t & 56u)) & 0xffull) != 0ull;
-    const bool top_full = T == 2 ? m != 0ull : __syncthreads_or(full) != 0;
-    if (in)
-        cells[(uint64_t)(cx + 1) + (uint64_t)(ncx + 2) * ((uint64_t)(cy + 1) + (uint64_t)(ncy + 2) * (uint64_t)(cz + 1))] =
-            full ? 0 : !top_full ? 3 : !oct_full ? 2 : 1;
-}
-
-/* 16 cell bytes -> one word of two-bit codes. */
-__global__ __launch_bounds__(256) void pack_codes_kernel(const uint4* __restrict__ cells, uint32_t n_words,
-                                                         uint32_t* __restrict__ codes)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_words) return;
-    const uint4 v = cells[i];
-    const uint32_t wd[4] = { v.x, v.y, v.z, v.w };
-    uint32_t out = 0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) out |= ((wd[k >> 2] >> (8 * (k & 3))) & 3u) << (2 * k);
-    codes[i] = out;
+    for (int32_t i = threadIdx.x; i < W / R; i += blockDim.x) top[i] = 0u;
+    __syncthreads();
+    for (int32_t i = threadIdx.x; i < H * H * (W / 2); i += blockDim.x) {
+        const int32_t x = i % (W / 2), y = i / (W / 2) % H, z = i / (W / 2 * H);
+        const uint8_t* p = full + 2 * x + W * (2 * y + R * (2 * z));
+        const uint32_t o = p[0] | p[1] | p[W] | p[W + 1] | p[W * R] | p[W * R + 1] | p[W * R + W] | p[W * R + W + 1];
+        pair[i] = (uint8_t)o;
+        if (o) top[x / H] = 1u;                     /* every writer writes 1 */
+    }
+    __syncthreads();
+    const int32_t row_bytes = (int32_t)(ccx / 4u);
+    for (int32_t i = threadIdx.x; i < R * R * QB; i += blockDim.x) {
+        const int32_t q = q0 + i % QB, y = i / QB % R, z = i / (QB * R);
+        if (q >= row_bytes || cy0 + y >= ncy || cz0 + z >= ncz) continue;
+        uint32_t out = 0u;
+        for (int k = 0; k < 4; ++k) {
+            const int32_t x = 4 * q + k - 1 - cx0;
+            const uint32_t c = full[x + W * (y + R * z)]                         ? 0u
+                               : !top[x / R]                                     ? 3u
+                               : !pair[x / 2 + W / 2 * (y / 2 + H * (z / 2))]    ? 2u
+                                                                                 : 1u;
+            out |= c << (2 * k);
+        }
+        codes[(uint64_t)q + (uint64_t)row_bytes * ((uint64_t)(cy0 + y + 1) + (uint64_t)ccy * (uint64_t)(cz0 + z + 1))] =
+            (uint8_t)out;
+    }
 }
 
 __global__ __launch_bounds__(256) void dense_from_bricks_kernel(BrickDims d, const uint8_t* __restrict__ bricks,
@@ -253,45 +295,58 @@ static unsigned grid_for(uint64_t n)
     return (unsigned)b;
 }
 
-hipError_t launch_brick_from_offsets(const BrickDims& d, const int32_t* dense, const uint8_t* lut, int32_t lut_n,
-                                     uint8_t* bricks, uint32_t* bad, hipStream_t s)
+hipError_t launch_scan_offsets(const int32_t* dense, uint64_t n, int32_t lut_n, uint8_t* used, unsigned long long* bad,
+                               hipStream_t s)
 {
-    brick_from_offsets_kernel<<<grid_for((uint64_t)d.nx * d.ny * d.nz), 256, 0, s>>>(d, dense, lut, lut_n, bricks, bad);
+    const unsigned g = grid_for(n / 16u + 1u);    /* four int4 a thread */
+    scan_offsets_kernel<<<g, 256, 0, s>>>(dense, n, lut_n, used, bad);
     return hipGetLastError();
 }
 
-hipError_t launch_brick_from_ids(const BrickDims& d, const uint8_t* dense, const uint8_t* remap, uint8_t* bricks,
-                                 hipStream_t s)
+hipError_t launch_check_emissive(const int32_t* emissive, int32_t n, uint64_t n_vox, const int32_t* offsets,
+                                 const uint8_t* ids, const uint8_t* remap, uint32_t* bad, hipStream_t s)
 {
-    brick_from_ids_kernel<<<grid_for((uint64_t)d.nx * d.ny * d.nz), 256, 0, s>>>(d, dense, remap, bricks);
+    if (n <= 0) return hipSuccess;
+    check_emissive_kernel<<<grid_for((uint64_t)n), 256, 0, s>>>(emissive, n, n_vox, offsets, ids, remap, bad);
     return hipGetLastError();
 }
 
-hipError_t launch_block_masks(const BrickDims& d, const uint8_t* bricks, uint64_t* occ64, uint32_t* bits,
-                              uint64_t* occp, uint32_t* bitsp, uint64_t* occr, hipStream_t s)
+static unsigned blocks_grid(const BrickDims& d)
 {
-    block_masks_kernel<<<grid_for(d.n_blocks), 256, 0, s>>>(d, bricks, occ64);
-    block_bits_kernel<<<grid_for((d.n_blocks + 31) / 32), 256, 0, s>>>(d.n_blocks, occ64, bits);
-    const uint64_t np = (uint64_t)(d.kx + 2) * (uint64_t)(d.ky + 2) * (uint64_t)(d.kz + 2);
-    block_masks_padded_kernel<<<grid_for(np), 256, 0, s>>>(d, occ64, occp);
-    block_bits_kernel<<<grid_for((np + 31) / 32), 256, 0, s>>>(np, occp, bitsp);
-    if (occr) block_masks_reversed_kernel<<<grid_for(np), 256, 0, s>>>(occp, occr, np);
+    return grid_for(d.n_padded);
+}
+
+hipError_t launch_blocks_from_bricks(const BrickDims& d, const uint8_t* bricks, const BlockLevels& L, hipStream_t s)
+{
+    blocks_kernel<0><<<blocks_grid(d), 256, 0, s>>>(d, nullptr, nullptr, const_cast<uint8_t*>(bricks), L);
     return hipGetLastError();
 }
 
-hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint8_t* cells,
-                             uint64_t n_cells, uint32_t* codes, hipStream_t s)
+hipError_t launch_blocks_from_offsets(const BrickDims& d, const int32_t* dense, const uint8_t* lut, uint8_t* bricks,
+                                      const BlockLevels& L, hipStream_t s)
+{
+    blocks_kernel<1><<<blocks_grid(d), 256, 0, s>>>(d, dense, lut, bricks, L);
+    return hipGetLastError();
+}
+
+hipError_t launch_blocks_from_ids(const BrickDims& d, const uint8_t* dense, const uint8_t* remap, uint8_t* bricks,
+                                  const BlockLevels& L, hipStream_t s)
+{
+    blocks_kernel<2><<<blocks_grid(d), 256, 0, s>>>(d, dense, remap, bricks, L);
+    return hipGetLastError();
+}
+
+hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint32_t ccx,
+                             uint32_t ccy, uint32_t* codes, hipStream_t s)
 {
     const int32_t e = 1 << cg;
     const int32_t nx = (d.nx + e - 1) / e, ny = (d.ny + e - 1) / e, nz = (d.nz + e - 1) / e;
-    const uint32_t c = 1u << top;
-    const dim3 grid(((uint32_t)nx + c - 1) / c, ((uint32_t)ny + c - 1) / c, ((uint32_t)nz + c - 1) / c);
+    const uint32_t r = 1u << top;
+    const dim3 grid(((uint32_t)ny + r - 1) / r, ((uint32_t)nz + r - 1) / r, (ccx / 4u + CODE_BYTES - 1) / CODE_BYTES);
     if (top == 2u)
-        cell_codes_kernel<2><<<grid, 64, 0, s>>>(d, occp, cg, nx, ny, nz, cells);
+        cell_codes_kernel<2><<<grid, 256, 0, s>>>(d, occp, cg, nx, ny, nz, ccx, ccy, (uint8_t*)codes);
     else
-        cell_codes_kernel<3><<<grid, 512, 0, s>>>(d, occp, cg, nx, ny, nz, cells);
-    const uint32_t words = (uint32_t)((n_cells + 15) / 16);
-    pack_codes_kernel<<<(words + 255) / 256, 256, 0, s>>>((const uint4*)cells, words, codes);
+        cell_codes_kernel<3><<<grid, 256, 0, s>>>(d, occp, cg, nx, ny, nz, ccx, ccy, (uint8_t*)codes);
     return hipGetLastError();
 }
 
