@@ -726,8 +726,12 @@ __device__ __forceinline__ int DdaState::advance_wave_packed(const GridView& g, 
  * limits below (non-finite or far from unit directions) is marched step by
  * step instead.
  *
- * Full-shading scene (256^3, 99 DDA steps a ray): 12 iterations a ray, 99.9 %
- * of the rays within 69 (the steps: 580). */
+ * In a cell with an occupied voxel the cube is the aligned 2x2x2 around the
+ * position when the mask shows it empty: 42 % of the iterations are in such
+ * cells, and one shift and one AND there save 12-15 % of all iterations.
+ *
+ * Full-shading scene (256^3, 99 DDA steps a ray): 10.7 iterations a ray (12.1
+ * without the cubes of 2), 99.9 % of the rays within 56 (69; the steps: 580). */
 #define VT_JUMP_A_MIN 9.765625e-4f        /* 2^-10 */
 #define VT_JUMP_A_MAX 2.0e5f
 #define VT_ULP24 5.9604644775390625e-8f   /* 2^-24 */
@@ -832,8 +836,11 @@ struct JumpState {
                 bi = index3<UNI>((ux - k) >> 2, (uy - k) >> 2, (uz - k) >> 2, g.bxp, g.byp);
             }
             const uint64_t m = load_mask(g.occp, bi);
-            if (voxel_bit(m, ux, uy, uz)) return false;
-            if (!FINE && m == 0ull) edge = 3;
+            /* the 2x2x2 voxels around the position, then the voxel itself */
+            const uint32_t b = local_bit(ux, uy, uz);
+            const uint32_t t = (uint32_t)(m >> (b & 0x2au));
+            if ((t & 0x00330033u) == 0u) edge = !FINE && m == 0ull ? 3 : 1;
+            else if (((t >> (b & 0x15u)) & 1u) != 0u) return false;
         }
         return true;
     }
@@ -842,14 +849,14 @@ struct JumpState {
     {
         return ((const __attribute__((address_space(1))) uint64_t*)occp)[i];
     }
-    /* bit (x & 3) + 4 (y & 3) + 16 (z & 3) of m */
-    static __device__ __forceinline__ bool voxel_bit(uint64_t m, uint32_t vx, uint32_t vy, uint32_t vz)
+    /* (x & 3) + 4 (y & 3) + 16 (z & 3): a voxel's bit in its block's mask */
+    static __device__ __forceinline__ uint32_t local_bit(uint32_t vx, uint32_t vy, uint32_t vz)
     {
         uint32_t b = vy << 2;
         asm("v_bfi_b32 %0, 3, %1, %2" : "=v"(b) : "v"(vx), "v"(b));
         uint32_t c = vz << 4;
         asm("v_bfi_b32 %0, 15, %1, %2" : "=v"(c) : "v"(b), "v"(c));
-        return ((m >> (c & 63u)) & 1ull) != 0ull;
+        return c & 63u;
     }
     /* Whether the voxel at mirrored (px, py, pz), inside the grid or one past
      * it, is occupied or outside the grid. */
@@ -857,7 +864,8 @@ struct JumpState {
     __device__ __forceinline__ bool blocked(const GridView& g, int32_t px, int32_t py, int32_t pz) const
     {
         const uint32_t vx = xor_add<false>(px, fx, 4u), vy = xor_add<false>(py, fy, 4u), vz = xor_add<false>(pz, fz, 4u);
-        return voxel_bit(load_mask(g.occp, index3<UNI>(vx >> 2, vy >> 2, vz >> 2, g.bxp, g.byp)), vx, vy, vz);
+        const uint64_t m = load_mask(g.occp, index3<UNI>(vx >> 2, vy >> 2, vz >> 2, g.bxp, g.byp));
+        return ((m >> local_bit(vx, vy, vz)) & 1ull) != 0ull;
     }
 
     /* (a ^ b) + c in one instruction; c is wave-uniform with UNI */

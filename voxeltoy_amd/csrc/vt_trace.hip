@@ -605,13 +605,13 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  *
  * Bound by vector issue (0.86 wave-instructions a CU and cycle, 48 % of the
  * lanes at work, full-shading scene) and, in the later launches, by the chain
- * of its longest rays (up to 160 jumps of about a microsecond).  That scene at
- * 1024^2, 16 passes, 8 bounces (90 M rays, 9 launches): 10.1 ms stepping voxel
- * by voxel, 7.0 ms with the jump march and one queue counter (of that, 4.6 ms
- * at least in the counter's 352 k updates), 5.3 ms dealt, 4.5 ms with the
- * undecided steps settled by the voxels they could skip; one pass at
- * 1920x1080: 3.15, 2.4, 1.1, 0.81 ms; 512^3 mesh scene at 1920x1080, 8 passes:
- * 5.26, 2.9, 2.05, 1.45 ms. */
+ * of its longest rays (up to 115 jumps of about half a microsecond).  That
+ * scene at 1024^2, 16 passes, 8 bounces (90 M rays, 9 launches): 10.1 ms
+ * stepping voxel by voxel, 7.0 ms with the jump march and one queue counter (of
+ * that, 4.6 ms at least in the counter's 352 k updates), 5.3 ms dealt, 4.7 ms
+ * with the undecided steps settled by the voxels they could skip, 4.4 ms with
+ * the cubes of 2 voxels; one pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78 ms;
+ * 512^3 mesh scene at 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38 ms. */
 #define WF_TRAVERSE_THREADS 1024
 #define WF_TAKEN_BYTES 16u      /* LDS of a traversal workgroup's list counter */
 
