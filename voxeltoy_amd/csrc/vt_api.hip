@@ -387,7 +387,7 @@ void choose_cells(vt_context* c)
     c->code_top = std::max(ex, std::max(ey, ez)) > 56 && cg < 6 ? 3u : 2u;   /* an edge of at most 256: cedge holds bytes */
     c->cell_ex = (uint32_t)((ex + 5) / 4 * 4);      /* rows of whole bytes; dims.px for cells of one block */
     c->cell_ey = (uint32_t)ey + 2;
-    c->code_words = (uint32_t)(((uint64_t)c->cell_ex * c->cell_ey * (ez + 2) + 15) / 16);
+    c->code_words = (uint32_t)(((uint64_t)c->cell_ex * c->cell_ey * (ez + 2) + 63) / 64 * 4);   /* whole uint4 */
 }
 
 int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const float* mat_data, int32_t mat_size,
@@ -424,7 +424,7 @@ int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const
         VT_HIP(hipMalloc(&c->d_bricks, d.n_bricks * 512u));
         const uint64_t np = d.n_padded;
         VT_HIP(hipMalloc(&c->d_occp, np * 8u));
-        c->bit_words_p = (uint32_t)((np + 31) / 32);
+        c->bit_words_p = (uint32_t)((np + 127) / 128 * 4);      /* whole uint4 */
         VT_HIP(hipMalloc(&c->d_bitsp, (size_t)c->bit_words_p * 4u));
         if (nx <= VT_PACKED_MAX_EXTENT && ny <= VT_PACKED_MAX_EXTENT && nz <= VT_PACKED_MAX_EXTENT)
             VT_HIP(hipMalloc(&c->d_occr, np * 8u));

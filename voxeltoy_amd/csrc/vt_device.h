@@ -820,13 +820,16 @@ struct JumpState {
      * single voxel; false when the voxel is occupied or outside the grid.
      * FINE: cells are the 4x4x4 blocks.  UNI: one grid for the whole wave. */
     template <bool FINE, bool UNI>
-    __device__ __forceinline__ bool lookup(const GridView& g, const uint32_t* __restrict__ codes, int32_t& edge) const
+    __device__ __forceinline__ bool lookup(const GridView& g, int32_t& edge) const
     {
         const uint32_t cg = FINE ? 2u : g.cg;
         const uint32_t pad = 1u << cg;
         const uint32_t ux = xor_add<UNI>(x, fx, pad), uy = xor_add<UNI>(y, fy, pad), uz = xor_add<UNI>(z, fz, pad);
         const uint32_t ci = index3<UNI>(ux >> cg, uy >> cg, uz >> cg, g.ccx, g.ccy);
-        const uint32_t word = UNI ? codes[ci >> 4] : ((const __attribute__((address_space(1))) uint32_t*)codes)[ci >> 4];
+        /* UNI: the codes are at the start of the workgroup's LDS (an address
+         * of its own would cost an add) */
+        const uint32_t word = UNI ? *(const __attribute__((address_space(3))) uint32_t*)(ci >> 4 << 2)
+                                  : ((const __attribute__((address_space(1))) uint32_t*)g.codes)[ci >> 4];
         const uint32_t c = field<2, false>(word, ci << 1);
         edge = (int32_t)field<8, UNI>(g.cedge, c << 3);
         if (c == 0u) {
@@ -839,8 +842,9 @@ struct JumpState {
             /* the 2x2x2 voxels around the position, then the voxel itself */
             const uint32_t b = local_bit(ux, uy, uz);
             const uint32_t t = (uint32_t)(m >> (b & 0x2au));
-            if ((t & 0x00330033u) == 0u) edge = !FINE && m == 0ull ? 3 : 1;
-            else if (((t >> (b & 0x15u)) & 1u) != 0u) return false;
+            edge = (t & 0x00330033u) == 0u ? 1 : 0;
+            if (!FINE && m == 0ull) edge = 3;
+            return ((t >> (b & 0x15u)) & 1u) == 0u;
         }
         return true;
     }
@@ -901,38 +905,58 @@ struct JumpState {
         return r;
     }
 
-    /* Leave the cube of lookup(); false, with the position unchanged, when
-     * the order of two steps is undecided and matters. */
-    template <bool UNI>
+    /* Leave the cube of lookup(); false, with the position unchanged, when a
+     * second axis is within the bound of a step. */
     __device__ __forceinline__ bool jump(const GridView& g, int32_t edge)
+    {
+        float px, py, pz;
+        const float del2 = 2.0f * leave(g, edge, px, py, pz);
+        if (__builtin_amdgcn_fmed3f(__builtin_amdgcn_fractf(px), __builtin_amdgcn_fractf(py),
+                                    __builtin_amdgcn_fractf(pz)) < del2)
+            return false;
+        x = floor_i32(px); y = floor_i32(py); z = floor_i32(pz);
+        return true;
+    }
+
+    /* The position (plus the bound, which it returns) at the value that leaves
+     * the cube. */
+    __device__ __forceinline__ float leave(const GridView& g, int32_t edge, float& px, float& py, float& pz) const
     {
         const int32_t bx = x | edge, by = y | edge, bz = z | edge;
         const float m = min3f(__builtin_fmaf((float)(bx - x0), ax, X0), __builtin_fmaf((float)(by - y0), ay, Y0),
                               __builtin_fmaf((float)(bz - z0), az, Z0));
         const float del = bound(g, m);
-        const float px = __builtin_fmaf(m, ix, q_x) + del, py = __builtin_fmaf(m, iy, q_y) + del,
-                    pz = __builtin_fmaf(m, iz, q_z) + del;
+        px = __builtin_fmaf(m, ix, q_x) + del;
+        py = __builtin_fmaf(m, iy, q_y) + del;
+        pz = __builtin_fmaf(m, iz, q_z) + del;
+        return del;
+    }
+
+    /* The jump that jump() declined: false, with the position unchanged, when
+     * the order of two steps is undecided and matters. */
+    template <bool UNI>
+    __device__ __forceinline__ bool near_jump(const GridView& g, int32_t edge)
+    {
+        float px, py, pz;
+        const float del2 = 2.0f * leave(g, edge, px, py, pz);
         const float rx = __builtin_amdgcn_fractf(px), ry = __builtin_amdgcn_fractf(py), rz = __builtin_amdgcn_fractf(pz);
-        const float del2 = del + del;
         const int32_t tx = floor_i32(px), ty = floor_i32(py), tz = floor_i32(pz);
-        if (__builtin_amdgcn_fmed3f(rx, ry, rz) < del2) {
-            /* steps ahead only: one that is behind was taken before */
-            const bool mx = tx > x, my = ty > y, mz = tz > z;
-            const bool nx = rx < del2 && mx, ny = ry < del2 && my, nz = rz < del2 && mz;
-            if (nx && ny && nz) return false;
-            if ((nx && ny) || (ny && nz) || (nz && nx)) {
-                const float am = fmaxf(fmaxf(nx ? ax : 0.0f, ny ? ay : 0.0f), nz ? az : 0.0f);
-                const float ex = del2 * __builtin_fmaf(am, ix, 1.0f), ey = del2 * __builtin_fmaf(am, iy, 1.0f),
-                            ez = del2 * __builtin_fmaf(am, iz, 1.0f);
-                if (!(fmaxf(fmaxf(ex, ey), ez) < 0.4f)) return false;
-                if ((!nx && ((mx && rx < ex) || rx > 1.0f - ex)) || (!ny && ((my && ry < ey) || ry > 1.0f - ey)) ||
-                    (!nz && ((mz && rz < ez) || rz > 1.0f - ez)))
-                    return false;
-                /* the voxels where one of the two steps is missing */
-                if (nx && blocked<UNI>(g, tx - 1, ty, tz)) return false;
-                if (ny && blocked<UNI>(g, tx, ty - 1, tz)) return false;
-                if (nz && blocked<UNI>(g, tx, ty, tz - 1)) return false;
-            }
+        /* steps ahead only: one that is behind was taken before */
+        const bool mx = tx > x, my = ty > y, mz = tz > z;
+        const bool nx = rx < del2 && mx, ny = ry < del2 && my, nz = rz < del2 && mz;
+        if (nx && ny && nz) return false;
+        if ((nx && ny) || (ny && nz) || (nz && nx)) {
+            const float am = fmaxf(fmaxf(nx ? ax : 0.0f, ny ? ay : 0.0f), nz ? az : 0.0f);
+            const float ex = del2 * __builtin_fmaf(am, ix, 1.0f), ey = del2 * __builtin_fmaf(am, iy, 1.0f),
+                        ez = del2 * __builtin_fmaf(am, iz, 1.0f);
+            if (!(fmaxf(fmaxf(ex, ey), ez) < 0.4f)) return false;
+            if ((!nx && ((mx && rx < ex) || rx > 1.0f - ex)) || (!ny && ((my && ry < ey) || ry > 1.0f - ey)) ||
+                (!nz && ((mz && rz < ez) || rz > 1.0f - ez)))
+                return false;
+            /* the voxels where one of the two steps is missing */
+            if (nx && blocked<UNI>(g, tx - 1, ty, tz)) return false;
+            if (ny && blocked<UNI>(g, tx, ty - 1, tz)) return false;
+            if (nz && blocked<UNI>(g, tx, ty, tz - 1)) return false;
         }
         x = tx; y = ty; z = tz;
         return true;
@@ -945,7 +969,7 @@ struct JumpState {
         return r;
     }
 
-    /* The jump that jump() left undecided: the smallest value that leaves the
+    /* The jump that near_jump() left undecided: the smallest value that leaves the
      * cube from the FP32 sums, then on each axis the steps up to it, the last
      * one checked against its sum where the real line leaves it open. */
     __device__ __forceinline__ void resolve(const GridView& g, int32_t edge)

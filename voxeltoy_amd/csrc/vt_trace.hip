@@ -603,15 +603,16 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * takes about 13 ns an update.  Workgroups of 1024 threads share one
  * LDS copy of the empty-cube codes (of the block occupancy bits with STATS).
  *
- * Bound by vector issue (0.86 wave-instructions a CU and cycle, 48 % of the
+ * Bound by vector issue (0.85 wave-instructions a CU and cycle, 48 % of the
  * lanes at work, full-shading scene) and, in the later launches, by the chain
- * of its longest rays (up to 115 jumps of about half a microsecond).  That
- * scene at 1024^2, 16 passes, 8 bounces (90 M rays, 9 launches): 10.1 ms
- * stepping voxel by voxel, 7.0 ms with the jump march and one queue counter (of
- * that, 4.6 ms at least in the counter's 352 k updates), 5.3 ms dealt, 4.7 ms
- * with the undecided steps settled by the voxels they could skip, 4.4 ms with
- * the cubes of 2 voxels; one pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78 ms;
- * 512^3 mesh scene at 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38 ms. */
+ * of its longest rays (up to 115 jumps of about 0.4 microseconds).  That scene
+ * at 1024^2, 16 passes, 8 bounces (90 M rays, 9 launches): 10.1 ms stepping
+ * voxel by voxel, 7.0 ms with the jump march and one queue counter (of that,
+ * 4.6 ms at least in the counter's 352 k updates), 5.3 ms dealt, 4.7 ms with
+ * the undecided steps settled by the voxels they could skip, 4.4 ms with the
+ * cubes of 2 voxels, 4.0 ms with the march as one loop of the whole wave; one
+ * pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78, 0.65 ms; 512^3 mesh scene at
+ * 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38, 1.23 ms. */
 #define WF_TRAVERSE_THREADS 1024
 #define WF_TAKEN_BYTES 16u      /* LDS of a traversal workgroup's list counter */
 
@@ -626,24 +627,24 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * (swept from 6 to 42 lanes: within 2 % from 18 on) */
 #define VT_JUMP_REFILL 3u
 
-/* The jump march of the calling lanes: at most `jumps` jumps, until fewer than
- * `keep` of them still march.  `stop`: the position is the ray's last voxel;
- * `und`: its next jump needs a resolve. */
+/* The jump march of the wave's `live` lanes: at most `jumps` jumps, until
+ * fewer than `keep` of them still march.  A lane is live no longer at its
+ * ray's last voxel, or where a jump needs more than JumpState::jump (`near`).
+ * The loop is the whole wave's: with lanes that leave it one by one the
+ * compiler copies the position twice in every iteration. */
 template <bool FINE, bool UNI>
-__device__ __forceinline__ void jump_march(JumpState& J, const GridView& g, const uint32_t* __restrict__ codes,
-                                           int jumps, int keep, bool& stop, bool& und)
+__device__ __forceinline__ void jump_march(JumpState& J, const GridView& g, int jumps, int keep, bool& live, bool& near)
 {
     do {
-        int32_t edge;
-        if (!J.lookup<FINE, UNI>(g, codes, edge)) {
-            stop = true;
-            break;
+        if (live) {
+            int32_t edge;
+            live = J.lookup<FINE, UNI>(g, edge);
+            if (live) {
+                live = J.jump(g, edge);
+                near = !live;
+            }
         }
-        if (!J.jump<UNI>(g, edge)) {
-            und = true;
-            break;
-        }
-    } while (--jumps > 0 && __popcll(__builtin_amdgcn_ballot_w64(true)) >= keep);
+    } while (--jumps > 0 && __popcll(__builtin_amdgcn_ballot_w64(live)) >= keep);
 }
 
 /* A ray marched step by step (DdaState::advance): hit record. */
@@ -686,9 +687,18 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
     uint32_t* taken = (uint32_t*)smem + words;     /* of the workgroup's list; after the table, whose reads then need no base */
     if (threadIdx.x == 0) *taken = 0u;
     if (STAGE) {
-        uint32_t* sb = (uint32_t*)smem;
-        for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) sb[i] = bits[i];
-        bits = sb;
+        /* four words a thread, four of these in flight (the tables are
+         * allocated, and the counter placed, to whole fours) */
+        const uint4* from = (const uint4*)bits;
+        uint4* to = (uint4*)smem;
+        const uint32_t n4 = words / 4u, T = WF_TRAVERSE_THREADS;
+        uint32_t i = threadIdx.x;
+        for (; i + 3u * T < n4; i += 4u * T) {
+            const uint4 v0 = from[i], v1 = from[i + T], v2 = from[i + 2u * T], v3 = from[i + 3u * T];
+            to[i] = v0; to[i + T] = v1; to[i + 2u * T] = v2; to[i + 3u * T] = v3;
+        }
+        for (; i < n4; i += T) to[i] = from[i];
+        bits = (const uint32_t*)smem;
     }
     __syncthreads();
     const float4* qa = sel ? P.qa1 : P.qa0;
@@ -768,23 +778,20 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
                 }
             }
         } else {
-            if (has) {
-                /* march on until a refill is due, or to the end */
-                const int keep = done ? 1 : 65 - (int)refill_min;
-                bool stop = false, und = false;
-                jump_march<LDSB, !BATCH>(J, G, BATCH ? G.codes : bits, budget, keep, stop, und);
-                if (und) {
-                    int32_t edge;
-                    (void)J.lookup<LDSB, !BATCH>(G, BATCH ? G.codes : bits, edge);
-                    J.resolve(G, edge);
-                }
-                if (stop) {
-                    const int32_t x = J.gx(), y = J.gy(), z = J.gz();
-                    const bool inside = (uint32_t)x < (uint32_t)G.nx && (uint32_t)y < (uint32_t)G.ny &&
-                                        (uint32_t)z < (uint32_t)G.nz;
-                    P.hit[jq] = pack_hit(x, y, z, inside ? KIND_VOXEL : (y < 0 ? KIND_GROUND : KIND_MISS));
-                    has = false;
-                }
+            /* march on until a refill is due, or to the end */
+            const int keep = done ? 1 : 65 - (int)refill_min;
+            bool live = has, near = false;
+            jump_march<LDSB, !BATCH>(J, G, budget, keep, live, near);
+            if (near) {
+                int32_t edge;
+                (void)J.lookup<LDSB, !BATCH>(G, edge);
+                if (!J.near_jump<!BATCH>(G, edge)) J.resolve(G, edge);
+            } else if (has && !live) {
+                const int32_t x = J.gx(), y = J.gy(), z = J.gz();
+                const bool inside = (uint32_t)x < (uint32_t)G.nx && (uint32_t)y < (uint32_t)G.ny &&
+                                    (uint32_t)z < (uint32_t)G.nz;
+                P.hit[jq] = pack_hit(x, y, z, inside ? KIND_VOXEL : (y < 0 ? KIND_GROUND : KIND_MISS));
+                has = false;
             }
         }
     }
