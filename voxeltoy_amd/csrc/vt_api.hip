@@ -99,42 +99,48 @@ struct DevTmp {
 }  // namespace
 
 /* ---- staging memory of vt_trace_rays_noalloc -------------------------------------
- * A fixed device array, one copy per device, held until the process ends:
- * origins (VT_NOALLOC_MAX_RAYS x 12 B), directions (x 12 B) and hit records
- * (x 32 B).  Its host-side name is a stand-in, not a device address, so host
- * code uses only the address that hipGetSymbolAddress returns for each
- * device (looked up once per device by vt_create, with that device current). */
+ * A fixed array of pinned host memory, one per device, made by the device's
+ * first vt_create and held until the process ends: origins
+ * (VT_NOALLOC_MAX_RAYS x 12 B), directions (x 12 B), hit records (x 32 B) and
+ * the word in which the kernel reports its end.  The kernel reads and writes it
+ * over the link: three copies of a few bytes and a wait for the stream took 50
+ * us a call. */
 #define VT_STR_(x) #x
 #define VT_STR(x) VT_STR_(x)
 namespace {
 constexpr size_t VT_NOALLOC_O = 0;
 constexpr size_t VT_NOALLOC_D = (size_t)VT_NOALLOC_MAX_RAYS * 12u;
 constexpr size_t VT_NOALLOC_R = (size_t)VT_NOALLOC_MAX_RAYS * 24u;
-constexpr size_t VT_NOALLOC_BYTES = (size_t)VT_NOALLOC_MAX_RAYS * 56u;
+constexpr size_t VT_NOALLOC_FLAG = (size_t)VT_NOALLOC_MAX_RAYS * 56u;
+constexpr size_t VT_NOALLOC_BYTES = VT_NOALLOC_FLAG + 64u;
 constexpr int VT_MAX_DEVICES = 64;
 static_assert(VT_NOALLOC_R % 256 == 0, "record staging must stay aligned");
 
+struct RayStage {
+    unsigned char* host = nullptr;
+    uint32_t* count = nullptr;                   /* device: finished workgroups */
+    uint32_t seq = 0;
+};
 std::mutex g_noalloc_lock;                       /* guards the table and serializes calls */
-void* g_noalloc_ptr[VT_MAX_DEVICES] = {};
+RayStage g_noalloc[VT_MAX_DEVICES];
 
-/* Device address of the current device's copy of `scratch`. */
-int noalloc_lookup(int device);
-}  // namespace
-
-static __device__ __align__(256) unsigned char scratch[VT_NOALLOC_BYTES];
-
-namespace {
+/* The current device's staging memory, once per device. */
 int noalloc_lookup(int device)
 {
     std::lock_guard<std::mutex> lk(g_noalloc_lock);
-    if (g_noalloc_ptr[device]) return VT_OK;
-    void* ptr = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !ptr) {
+    RayStage& st = g_noalloc[device];
+    if (st.host) return VT_OK;
+    void* host = nullptr;
+    const uint32_t zero = 0;
+    hipError_t e = st.count ? hipSuccess : hipMalloc(&st.count, sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemcpy(st.count, &zero, sizeof(zero), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipHostMalloc(&host, VT_NOALLOC_BYTES, hipHostMallocDefault);
+    if (e != hipSuccess) {
         (void)hipGetLastError();
-        return fail(VT_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
+        return fail(VT_ERR_HIP, std::string("staging memory of picking: ") + hipGetErrorString(e));
     }
-    g_noalloc_ptr[device] = ptr;
+    std::memset((unsigned char*)host + VT_NOALLOC_FLAG, 0, 64);
+    st.host = (unsigned char*)host;
     return VT_OK;
 }
 }  // namespace
@@ -2135,6 +2141,32 @@ int vt_trace_first_hit(vt_context* c, uint64_t seed, uint32_t frame, int32_t* re
     });
 }
 
+namespace {
+/* n <= VT_NOALLOC_MAX_RAYS rays through the device's staging memory, with
+ * g_noalloc_lock held.  The host reads the kernel's word for as long as a pick
+ * takes on an idle stream; behind other work it waits for the stream. */
+int trace_rays_staged(vt_context* c, int32_t n, const float* o, const float* dir, int32_t* rec)
+{
+    RayStage& st = g_noalloc[c->device];
+    if (!st.host) return fail(VT_ERR_STATE, "staging array of the device was not looked up");
+    uint32_t* const flag = (uint32_t*)(st.host + VT_NOALLOC_FLAG);
+    const uint32_t seq = ++st.seq;
+    std::memcpy(st.host + VT_NOALLOC_O, o, (size_t)n * 12);
+    std::memcpy(st.host + VT_NOALLOC_D, dir, (size_t)n * 12);
+    VT_HIP(vt::launch_trace_rays(trace_args(c), n, (const float*)(st.host + VT_NOALLOC_O),
+                                 (const float*)(st.host + VT_NOALLOC_D), (int32_t*)(st.host + VT_NOALLOC_R), st.count, flag,
+                                 seq, c->stream));
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    while (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != seq)
+        if (std::chrono::steady_clock::now() > until) {
+            VT_HIP(hipStreamSynchronize(c->stream));
+            break;
+        }
+    std::memcpy(rec, st.host + VT_NOALLOC_R, (size_t)n * 32);
+    return VT_OK;
+}
+}  // namespace
+
 int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, int32_t* rec)
 {
     return no_throw([&]() -> int {
@@ -2142,6 +2174,10 @@ int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, in
         if (!c->has_volume) return fail(VT_ERR_STATE, "no volume");
         if (n == 0) return VT_OK;
         VT_HIP(hipSetDevice(c->device));
+        if (n <= VT_NOALLOC_MAX_RAYS) {
+            std::unique_lock<std::mutex> lk(g_noalloc_lock, std::try_to_lock);
+            if (lk.owns_lock()) return trace_rays_staged(c, n, o, dir, rec);
+        }
         vt::TraceArgs a = trace_args(c);
         WorkSpace ws;
         const size_t dir_at = aligned((size_t)n * 12), rec_at = 2 * dir_at;
@@ -2151,7 +2187,7 @@ int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, in
         VT_HIP(to_device(c, work, o, (size_t)n * 12));
         VT_HIP(to_device(c, work + dir_at, dir, (size_t)n * 12));
         VT_HIP(vt::launch_trace_rays(a, n, (const float*)work, (const float*)(work + dir_at), (int32_t*)(work + rec_at),
-                                     c->stream));
+                                     nullptr, nullptr, 0u, c->stream));
         VT_HIP(to_host(c, rec, work + rec_at, (size_t)n * 32));
         return VT_OK;
     });
@@ -2170,18 +2206,7 @@ int vt_trace_rays_noalloc(vt_context* c, int32_t n, const float* o, const float*
         /* one call at a time uses the device's staging array; a call returns only
          * after its records are back on the host */
         std::lock_guard<std::mutex> lk(g_noalloc_lock);
-        unsigned char* base = (unsigned char*)g_noalloc_ptr[c->device];
-        if (!base) return fail(VT_ERR_STATE, "staging array of the device was not looked up");
-        float* d_o = (float*)(base + VT_NOALLOC_O);
-        float* d_d = (float*)(base + VT_NOALLOC_D);
-        int32_t* d_r = (int32_t*)(base + VT_NOALLOC_R);
-        vt::TraceArgs a = trace_args(c);
-        VT_HIP(hipMemcpyAsync(d_o, o, (size_t)n * 12, hipMemcpyHostToDevice, c->stream));
-        VT_HIP(hipMemcpyAsync(d_d, dir, (size_t)n * 12, hipMemcpyHostToDevice, c->stream));
-        VT_HIP(vt::launch_trace_rays(a, n, d_o, d_d, d_r, c->stream));
-        VT_HIP(hipMemcpyAsync(rec, d_r, (size_t)n * 32, hipMemcpyDeviceToHost, c->stream));
-        VT_HIP(hipStreamSynchronize(c->stream));
-        return VT_OK;
+        return trace_rays_staged(c, n, o, dir, rec);
     });
 }
 

@@ -181,6 +181,20 @@ __device__ __forceinline__ float aabb(f3 o, f3 d, f3 bmin, f3 bmax)
  * Returns 1 on hit, 0 when the march ended without a hit (position written),
  * -1 when the start point lies outside the grid (position not written).
  * `slot` receives the hit voxel's material slot. */
+/* Accesses to pinned host memory that pass the L2s by: a buffer that the host
+ * and kernels use in turn without a barrier in the stream shows its current
+ * contents, and a store is on its way to the host when it is done. */
+template <class T>
+__device__ __forceinline__ T load_system(const T* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+template <class T>
+__device__ __forceinline__ void store_system(T* p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct Hit { int32_t x, y, z, steps; uint32_t slot; };
 
 /* Smallest of three floats in one instruction.  The DDA's distances are
@@ -718,8 +732,8 @@ __device__ __forceinline__ int DdaState::advance_wave_packed(const GridView& g, 
  * not matter.  That holds when no other step can fall between the two, which
  * are at most 2 del a apart (a: the longer step of the two axes): the third
  * axis must be 2 del (1 + a / its step) from an integer on either side.
- * Otherwise (10-19 % of the undecided jumps) jump() leaves the position
- * unchanged and resolve() compares the FP32 sums themselves.
+ * jump() leaves such a jump to near_jump(), which leaves the rest (10-19 % of
+ * the undecided jumps) to resolve(), which compares the FP32 sums themselves.
  *
  * Axes are mirrored (x ^ -1) so that every step is +1 and the far face of an
  * aligned cube is x | (edge - 1).  A ray whose set-up leaves the range of the
@@ -1022,6 +1036,67 @@ __device__ __forceinline__ int dda(const GridView& g, const uint32_t* __restrict
         return -1;
     }
     const int status = D.advance<COUNT>(g, bits, g.max_steps, visits);
+    D.finish(g, status, h);
+    return status == 1 ? 1 : 0;
+}
+
+/* dda() through the codes of the jump march, for single rays: the march's
+ * latency is that of its dependent loads, one code and one mask a cube of empty
+ * voxels here, both in flight together, where DdaState::advance loads a bit and
+ * then a mask a block.  Inside a cube it steps in registers (the step count is
+ * part of the record).  Steps, their order and the end are those of advance. */
+__device__ __forceinline__ int32_t room(int32_t x, int32_t st, uint32_t edge)
+{
+    const int32_t in = x & (int32_t)edge;
+    return st > 0 ? (int32_t)edge - in : st < 0 ? in : 0x3fffffff;
+}
+__device__ __forceinline__ int dda_cubes(const GridView& g, f3 o, f3 d, Hit& h)
+{
+    DdaState D;
+    if (!D.init(g, o, d)) {
+        h.steps = -1;
+        return -1;
+    }
+    const uint32_t pad = 1u << g.cg;
+    for (;;) {
+        const uint32_t ux = (uint32_t)D.x + pad, uy = (uint32_t)D.y + pad, uz = (uint32_t)D.z + pad;
+        const uint32_t ci = JumpState::index3<true>(ux >> g.cg, uy >> g.cg, uz >> g.cg, g.ccx, g.ccy);
+        const uint32_t k = pad - 4u;
+        const uint32_t bi = JumpState::index3<true>((ux - k) >> 2, (uy - k) >> 2, (uz - k) >> 2, g.bxp, g.byp);
+        uint32_t word = g.codes[ci >> 4];
+        uint64_t m = JumpState::load_mask(g.occp, bi);
+        asm volatile("" : "+v"(word), "+v"(m));         /* both in flight together */
+        const uint32_t c = (word >> (2u * (ci & 15u))) & 3u;
+        uint32_t edge = (g.cedge >> (8u * c)) & 0xffu;
+        if (c == 0u) {
+            const uint32_t b = JumpState::local_bit(ux, uy, uz);
+            const uint32_t t = (uint32_t)(m >> (b & 0x2au));
+            if (((t >> (b & 0x15u)) & 1u) != 0u) break;
+            edge = m == 0ull ? 3u : (t & 0x00330033u) == 0u ? 1u : 0u;
+        }
+        if (D.steps >= g.max_steps) break;
+        /* steps of each axis, and of all, that stay in the cube and the limit */
+        const int32_t rx = room(D.x, D.stx, edge), ry = room(D.y, D.sty, edge), rz = room(D.z, D.stz, edge);
+        const int32_t rs = g.max_steps - D.steps - 1;
+        int32_t dx = rx, dy = ry, dz = rz, ds = rs;
+        do {
+            const float t = min3f(D.disx, D.disy, D.disz);
+            const bool mx = D.disx == t, my = D.disy == t, mz = D.disz == t;
+            D.disx = D.disx + (mx ? D.ax : 0.0f);
+            D.disy = D.disy + (my ? D.ay : 0.0f);
+            D.disz = D.disz + (mz ? D.az : 0.0f);
+            dx -= mx ? 1 : 0;
+            dy -= my ? 1 : 0;
+            dz -= mz ? 1 : 0;
+            ds -= 1;
+        } while ((dx | dy | dz | ds) >= 0);
+        D.x += D.stx * (rx - dx);
+        D.y += D.sty * (ry - dy);
+        D.z += D.stz * (rz - dz);
+        D.steps += rs - ds;
+    }
+    const bool inside = (uint32_t)D.x < (uint32_t)g.nx && (uint32_t)D.y < (uint32_t)g.ny && (uint32_t)D.z < (uint32_t)g.nz;
+    const int status = D.steps < g.max_steps && inside ? 1 : 2;
     D.finish(g, status, h);
     return status == 1 ? 1 : 0;
 }

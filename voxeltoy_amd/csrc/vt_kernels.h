@@ -162,7 +162,7 @@ hipError_t launch_render(const TraceArgs& a, int grid, hipStream_t s, bool stats
 int render_blocks_per_cu(const TraceArgs& a, bool stats);
 hipError_t launch_first_hit(const TraceArgs& a, int32_t* out, hipStream_t s);
 hipError_t launch_trace_rays(const TraceArgs& a, int32_t n, const float* o, const float* d, int32_t* out,
-                             hipStream_t s);
+                             uint32_t* count, uint32_t* flag, uint32_t seq, hipStream_t s);
 hipError_t launch_reset_counter(uint32_t* c, unsigned long long* stats, hipStream_t s);
 hipError_t launch_device_math(int32_t fn, int32_t n, const float* a, const float* b, float* out, hipStream_t s);
 

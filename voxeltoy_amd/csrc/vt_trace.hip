@@ -1218,14 +1218,13 @@ hipError_t launch_light_table(const GridView& g, int4* out, hipStream_t s)
     return hipGetLastError();
 }
 
-/* First hit of the primary ray of every pixel (the parity probe). */
-__device__ __forceinline__ void hit_record(const GridView& g, const uint32_t* bits, f3 o, f3 d, f3 basis_o,
-                                           int32_t* rec)
+/* Record of a ray's first hit (8 words). */
+__device__ __forceinline__ void hit_record(const GridView& g, f3 o, f3 d, f3 basis_o, int32_t* rec)
 {
     Hit h;
     h.x = h.y = h.z = 0;
-    uint32_t dummy = 0;
-    const int kind = traverse<false>(g, bits, o, d, h, dummy);
+    const int r = dda_cubes(g, o, d, h);
+    const int kind = r == 1 ? KIND_VOXEL : r == 0 && h.y < 0 ? KIND_GROUND : KIND_MISS;
     rec[1] = h.x; rec[2] = h.y; rec[3] = h.z; rec[4] = h.steps;
     if (h.steps < 0) { rec[1] = rec[2] = rec[3] = 0; }
     rec[5] = rec[6] = rec[7] = 0;
@@ -1235,6 +1234,7 @@ __device__ __forceinline__ void hit_record(const GridView& g, const uint32_t* bi
     rec[5] = (int32_t)B.n.x; rec[6] = (int32_t)B.n.y; rec[7] = (int32_t)B.n.z;
 }
 
+/* First hit of the primary ray of every pixel (the parity probe). */
 __global__ __launch_bounds__(256) void first_hit_kernel(TraceArgs a, int32_t* out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1253,17 +1253,56 @@ __global__ __launch_bounds__(256) void first_hit_kernel(TraceArgs a, int32_t* ou
         for (int k = 0; k < 8; ++k) rec[k] = 0;
         return;
     }
-    hit_record(g, g.bitsp, o + d * t, d, o, rec);
+    hit_record(g, o + d * t, d, o, rec);
 }
 
-__global__ __launch_bounds__(256) void trace_rays_kernel(TraceArgs a, int32_t n, const float* orig, const float* dir,
-                                                         int32_t* out)
+/* Injected rays, one wave a workgroup.  Rays and records may lie in pinned host
+ * memory: they pass through LDS so that a wave moves whole lines over the link,
+ * with accesses of system scope, and *flag = seq (when not null) tells the host
+ * that the records are there; `count` is a zeroed device word that the kernel
+ * leaves zero.  One ray against a 126x20x126 grid (72
+ * steps): 47 us a call with three copies, a wait for the stream and a march by
+ * blocks, 27 with the staging memory and the march by cubes, 23 with its loop
+ * cut to the remaining steps of the cube. */
+__global__ __launch_bounds__(64) void trace_rays_kernel(TraceArgs a, int32_t n, const float* orig, const float* dir,
+                                                        int32_t* out, uint32_t* count, uint32_t* flag, uint32_t seq)
 {
-    const int32_t i = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n) return;
-    const f3 o = mk(orig[3 * i], orig[3 * i + 1], orig[3 * i + 2]);
-    const f3 d = mk(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]);
-    hit_record(a.g, a.g.bitsp, o, d, o, out + 8 * (size_t)i);
+    __shared__ __align__(16) uint32_t st[64 * 8];
+    const int32_t lane = (int32_t)threadIdx.x, base = (int32_t)blockIdx.x * 64;
+    const int32_t m = n - base < 64 ? n - base : 64;
+    const float* po = orig + 3 * (size_t)base;
+    const float* pd = dir + 3 * (size_t)base;
+    uint32_t v[6];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int32_t i = 64 * k + lane;
+        v[k] = v[k + 3] = 0u;
+        if (i < 3 * m) {
+            v[k] = load_system((const uint32_t*)po + i);
+            v[k + 3] = load_system((const uint32_t*)pd + i);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) st[64 * k + lane] = v[k];
+    __syncthreads();
+    const float* so = (const float*)st + 3 * lane;
+    const f3 o = mk(so[0], so[1], so[2]), d = mk(so[192], so[193], so[194]);
+    __syncthreads();
+    if (lane < m) hit_record(a.g, o, d, o, (int32_t*)st + 8 * lane);
+    __syncthreads();
+    uint64_t* to = (uint64_t*)(out + 8 * (size_t)base);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int32_t i = 64 * k + lane;
+        if (i < 4 * m) store_system(to + i, ((const uint64_t*)st)[i]);
+    }
+    if (!flag) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    /* the wave's records are written */
+    if (lane == 0 &&
+        __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u) {
+        __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 __global__ void reset_counter_kernel(uint32_t* c, unsigned long long* stats)
@@ -1330,9 +1369,9 @@ hipError_t launch_first_hit(const TraceArgs& a, int32_t* out, hipStream_t s)
 }
 
 hipError_t launch_trace_rays(const TraceArgs& a, int32_t n, const float* o, const float* d, int32_t* out,
-                             hipStream_t s)
+                             uint32_t* count, uint32_t* flag, uint32_t seq, hipStream_t s)
 {
-    trace_rays_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(a, n, o, d, out);
+    trace_rays_kernel<<<(unsigned)((n + 63) / 64), 64, 0, s>>>(a, n, o, d, out, count, flag, seq);
     return hipGetLastError();
 }
 

@@ -277,16 +277,6 @@ __global__ __launch_bounds__(256) void copy_kernel(const uint4* __restrict__ src
  * accesses between two system-scope fences 41.4 (fences of one wave a
  * workgroup) or 47 (of every wave), with an event after the kernel 45. */
 #define CHUNK_COPY_BLOCKS 64
-template <class T>
-__device__ __forceinline__ T load_system(const T* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-template <class T>
-__device__ __forceinline__ void store_system(T* p, T v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 __global__ __launch_bounds__(256) void copy_chunk_kernel(const uint64_t* src, uint64_t* dst, uint32_t bytes,
                                                          uint32_t* count, uint32_t* flag, uint32_t seq)
 {
