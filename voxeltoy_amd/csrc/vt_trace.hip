@@ -613,7 +613,11 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * cubes of 2 voxels, 4.0 ms with the march as one loop of the whole wave; one
  * pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78, 0.65 ms; 512^3 mesh scene at
  * 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38, 1.23 ms. */
-#define WF_TRAVERSE_THREADS 1024
+/* Batch launches without statistics keep each lane's grid in registers (72),
+ * which leaves 6 waves a SIMD: workgroups of 256 threads use them all, those of
+ * 1024 only 4.  They stage nothing in LDS.  16 scenes of 32^3 to 200^3: 1.33 ms
+ * with 1024 threads, 1.15 with 256 (5 launches). */
+constexpr uint32_t wf_traverse_threads(bool stats, bool batch) { return batch && !stats ? 256u : 1024u; }
 #define WF_TAKEN_BYTES 16u      /* LDS of a traversal workgroup's list counter */
 
 /* SGPRs are allocated in steps of 16.  A build of this kernel whose
@@ -664,7 +668,7 @@ __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r
  * codes (always staged in LDS, except in batch launches) are the 4x4x4
  * blocks. */
 template <bool STATS, bool LDSB, bool BATCH>
-__global__ __launch_bounds__(WF_TRAVERSE_THREADS) __attribute__((amdgpu_num_sgpr(WF_TRAVERSE_SGPRS)))
+__global__ __launch_bounds__(wf_traverse_threads(STATS, BATCH)) __attribute__((amdgpu_num_sgpr(WF_TRAVERSE_SGPRS)))
 void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
 {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -691,7 +695,7 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
          * allocated, and the counter placed, to whole fours) */
         const uint4* from = (const uint4*)bits;
         uint4* to = (uint4*)smem;
-        const uint32_t n4 = words / 4u, T = WF_TRAVERSE_THREADS;
+        const uint32_t n4 = words / 4u, T = wf_traverse_threads(STATS, BATCH);
         uint32_t i = threadIdx.x;
         for (; i + 3u * T < n4; i += 4u * T) {
             const uint4 v0 = from[i], v1 = from[i + T], v2 = from[i + 2u * T], v3 = from[i + 3u * T];
@@ -1054,7 +1058,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
     const size_t lds_t = WF_TAKEN_BYTES + (BATCH ? 0u : STATS ? (LDSB ? (size_t)a.g.bit_words_p * 4u : 0u)
                                                           : (size_t)a.g.code_words * 4u);
     const size_t lds_s = BATCH ? 0 : 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
-    const int bt = blocks_per_cu(wf_traverse_kernel<STATS, LDSB, BATCH>, WF_TRAVERSE_THREADS, lds_t);
+    const int bt = blocks_per_cu(wf_traverse_kernel<STATS, LDSB, BATCH>, wf_traverse_threads(STATS, BATCH), lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<STATS, PH_PRIMARY, BATCH>, WF_SHADE_THREADS, lds_s);
     const int bs1 = blocks_per_cu(wf_shade_kernel<STATS, PH_COMB, BATCH>, WF_SHADE_THREADS, lds_s);
     for (uint64_t g0 = 0; g0 < total; g0 += P.cap) {
@@ -1071,7 +1075,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used], s);
                 if (e != hipSuccess) return e;
             }
-            wf_traverse_kernel<STATS, LDSB, BATCH><<<cus * bt, WF_TRAVERSE_THREADS, lds_t, s>>>(a, B, P, sel);
+            wf_traverse_kernel<STATS, LDSB, BATCH><<<cus * bt, wf_traverse_threads(STATS, BATCH), lds_t, s>>>(a, B, P, sel);
             if (timed) {
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used + 1], s);
                 if (e != hipSuccess) return e;
@@ -1148,7 +1152,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0 };
     const size_t lds_t = WF_TAKEN_BYTES + (size_t)a.g.code_words * 4u;
     const size_t lds_s = 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
-    const int bt = blocks_per_cu(wf_traverse_kernel<false, LDSB, false>, WF_TRAVERSE_THREADS, lds_t);
+    const int bt = blocks_per_cu(wf_traverse_kernel<false, LDSB, false>, wf_traverse_threads(false, false), lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<false, PH_PRIMARY, false, true>, WF_SHADE_THREADS, lds_s);
     const int bs1 = blocks_per_cu(wf_shade_kernel<false, PH_COMB, false, true>, WF_SHADE_THREADS, lds_s);
     const uint64_t WH = (uint64_t)a.W * (uint64_t)a.H;
@@ -1167,7 +1171,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     wf_generate_kernel<false, false, true><<<gg, WF_GENERATE_THREADS, 0, s>>>(a, B, P, 0, n, C);
     int sel = 0;
     for (int r = 0; r < rounds; ++r) {
-        wf_traverse_kernel<false, LDSB, false><<<cus * bt, WF_TRAVERSE_THREADS, lds_t, s>>>(a, B, P, sel);
+        wf_traverse_kernel<false, LDSB, false><<<cus * bt, wf_traverse_threads(false, false), lds_t, s>>>(a, B, P, sel);
         if (r == 0)
             wf_shade_kernel<false, PH_PRIMARY, false, true><<<cus * bs0, WF_SHADE_THREADS, lds_s, s>>>(a, B, P, sel, C);
         else
