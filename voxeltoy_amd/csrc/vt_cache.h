@@ -30,7 +30,7 @@ enum {
     MLP_TPACK_HID = 4 * 4 * 64 * 4, MLP_TPACK_OUT = 4 * 64,
     MLP_TPACK = 4 * MLP_TPACK_HID + MLP_TPACK_OUT,
     /* training: column blocks of the weight-gradient GEMM, K splits */
-    MLP_GRAD_ITEMS = 15, MLP_GRAD_SPLITS = 64,
+    MLP_GRAD_ITEMS = 10, MLP_GRAD_SPLITS = 56,
 };
 
 /* Offsets of each layer's weights and biases in the parameter vector. */

@@ -289,86 +289,137 @@ __global__ __launch_bounds__(FB_THREADS) void mlp_train_fb_kernel(const h8* __re
     if (lane == 0 && lsum != 0.0f) atomicAdd(S.loss, lsum);
 }
 
+#define GRAD_THREADS 512
+
 /* Column blocks of the weight-gradient GEMM: (layer, first 16-column tile,
- * tiles); column `in` of a layer is its bias (input 1). */
+ * tiles); the light one last. */
 __device__ __forceinline__ void grad_item(int item, int& layer, int& nt0, int& nts)
 {
-    if (item < 5) { layer = 0; nt0 = 4 * item; nts = item < 4 ? 4 : 3; return; }
-    layer = 1 + (item - 5) / 2;
-    const int k = (item - 5) % 2;
-    nt0 = 4 * k;
-    nts = k == 0 ? 4 : 1;
+    layer = item < 5 ? 0 : item - 4;
+    nt0 = item < 5 ? (item < 4 ? 4 * item : 15) : 0;
+    nts = item == 3 || item == 4 ? 3 : 4;
 }
 
-/* part[split][param] = sum over the split's samples of dZ[o][q] * A[i][q]
- * (A[in][q] = 1 for the bias), FP32 MFMA with 16 samples per K step. */
-__global__ __launch_bounds__(64) void mlp_train_grad_kernel(TrainBatch b, TrainScratch S)
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+/* acc[m][c] += dZ[16 m + ..][q] * A[16 (nt0 + c) + ..][q] and bsum[m] +=
+ * dZ[16 m + r][q] over the samples q of tiles t, t + step, ...; the next tile's
+ * operands are loaded before the current one's products. */
+template <int MTS, int NTS>
+__device__ __forceinline__ void grad_tiles(const float* __restrict__ D, size_t dstride, const _Float16* __restrict__ A,
+                                           size_t astride, int rows, uint32_t t, uint32_t t1, uint32_t step, int r,
+                                           f4 (&acc)[4][4], float (&bsum)[4])
 {
+    f4 dv[MTS];
+    h4 ah[NTS];
+    auto load = [&](uint32_t at) {
+#pragma unroll
+        for (int m = 0; m < MTS; ++m)
+            dv[m] = 16 * m + r < rows ? *(const f4*)(D + (size_t)at * dstride + 16 * (16 * m + r))
+                                      : (f4){ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int c = 0; c < NTS; ++c) ah[c] = *(const h4*)(A + (size_t)at * astride + 16 * (16 * c + r));
+    };
+    if (t < t1) load(t);
+    while (t < t1) {
+        f4 d[MTS];
+        h4 a[NTS];
+#pragma unroll
+        for (int m = 0; m < MTS; ++m) d[m] = dv[m];
+#pragma unroll
+        for (int c = 0; c < NTS; ++c) a[c] = ah[c];
+        t += step;
+        if (t < t1) load(t);
+#pragma unroll
+        for (int m = 0; m < MTS; ++m) bsum[m] += (d[m][0] + d[m][1]) + (d[m][2] + d[m][3]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float av[NTS];
+#pragma unroll
+            for (int c = 0; c < NTS; ++c) av[c] = (float)a[c][u];
+#pragma unroll
+            for (int m = 0; m < MTS; ++m)
+#pragma unroll
+                for (int c = 0; c < NTS; ++c)
+                    acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[m][u], av[c], acc[m][c], 0, 0, 0);
+        }
+    }
+}
+
+/* part[split][param] = sum over the split's samples of dZ[o][q] * A[i][q], FP32
+ * MFMA with 16 samples per K step, and of dZ[o][q] for the bias.  Eight waves
+ * share a split's tiles and add up in LDS, in a fixed order: 56 splits of 9 like
+ * items and a light one are two workgroups a CU, 4 waves a SIMD.  Bound by the
+ * matrix units (1.76 M products of 32 cycles for 50001 samples, 23 us) and by
+ * the reads of dZ, 5 times for layer 0 (177 MB in all): 48 us, where one wave per item
+ * and split, with nothing to hide its loads behind, took 121. */
+__global__ __launch_bounds__(GRAD_THREADS, 4) void mlp_train_grad_kernel(TrainBatch b, TrainScratch S)
+{
+    __shared__ f4 red[4 * 16 * 64];
     const uint32_t n = batch_count(b);
     if (n == 0u) return;
     int layer, nt0, nts;
-    grad_item(blockIdx.x, layer, nt0, nts);
-    const int split = blockIdx.y, splits = gridDim.y;
+    grad_item(blockIdx.y, layer, nt0, nts);
+    const int split = blockIdx.x, splits = gridDim.x;
     const int in = layer == 0 ? MLP_IN : MLP_W, out = layer == 5 ? MLP_OUT : MLP_W;
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, wave = threadIdx.x >> 6;
     /* per-tile strides and the layer's first row inside a tile */
     const size_t dstride = layer == 5 ? MLP_OUT * 16 : 5 * MLP_W * 16;
     const size_t astride = layer == 0 ? MLP_IN * 16 : 5 * MLP_W * 16;
-    const float* D = layer == 5 ? S.DY : S.DZ + (size_t)layer * MLP_W * 16;
-    const _Float16* A = layer == 0 ? S.X : S.H + (size_t)(layer - 1) * MLP_W * 16;
-    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    const float* D = (layer == 5 ? S.DY : S.DZ + (size_t)layer * MLP_W * 16) + 4 * g;
+    const _Float16* A = (layer == 0 ? S.X : S.H + (size_t)(layer - 1) * MLP_W * 16) + 16 * 16 * nt0 + 4 * g;
     const uint32_t tiles = (n + 15u) / 16u;
     const uint32_t per = (tiles + splits - 1) / splits;
     const uint32_t t0 = split * per, t1 = t0 + per < tiles ? t0 + per : tiles;
     f4 acc[4][4];
+    float bsum[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[m][c] = (f4){ 0.0f, 0.0f, 0.0f, 0.0f };
-    const int mts = out > 16 ? 4 : 1;
-    for (uint32_t t = t0; t < t1; ++t) {
-        const float* Dt = D + (size_t)t * dstride + 4 * g;
-        const _Float16* At = A + (size_t)t * astride + 4 * g;
-        f4 dv[4], av[4];
+    constexpr uint32_t W = GRAD_THREADS / 64;
+    if (layer == 5) grad_tiles<1, 4>(D, dstride, A, astride, out, t0 + wave, t1, W, r, acc, bsum);
+    else if (nts == 4) grad_tiles<4, 4>(D, dstride, A, astride, out, t0 + wave, t1, W, r, acc, bsum);
+    else grad_tiles<4, 3>(D, dstride, A, astride, out, t0 + wave, t1, W, r, acc, bsum);
+    /* waves 4..7 onto 0..3, then four terms an element */
+    f4* mine = red + (wave & 3) * 16 * 64 + lane;
+    if (wave >= 4)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const int row = 16 * m + r;
-            dv[m] = (m < mts && row < out) ? *(const f4*)(Dt + 16 * row) : (f4){ 0.0f, 0.0f, 0.0f, 0.0f };
-        }
+        for (int p = 0; p < 16; ++p) mine[64 * p] = acc[p >> 2][p & 3];
+    __syncthreads();
+    if (wave < 4)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int col = 16 * (nt0 + c) + r;
-            if (c < nts && col < in) {
-                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                const h4 h = *(const h4*)(At + 16 * col);
-                av[c] = (f4){ (float)h[0], (float)h[1], (float)h[2], (float)h[3] };
-            } else {
-                const float one = (c < nts && col == in) ? 1.0f : 0.0f;
-                av[c] = (f4){ one, one, one, one };
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if (m < mts && c < nts)
-                        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(dv[m][u], av[c][u], acc[m][c], 0, 0, 0);
-    }
+        for (int p = 0; p < 16; ++p) mine[64 * p] = acc[p >> 2][p & 3] + mine[64 * p];
+    __syncthreads();
     float* part = S.part + (size_t)split * MLP_N_PARAMS;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int k = 0; k < 2; ++k) {
+        const int p = 2 * wave + k, m = p >> 2, c = p & 3;
+        const f4* q = red + 64 * p + lane;
+        const f4 sum = (q[0] + q[16 * 64]) + (q[2 * 16 * 64] + q[3 * 16 * 64]);
+        const int i = 16 * (nt0 + c) + r;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (m >= mts || c >= nts) continue;
-            const int i = 16 * (nt0 + c) + r;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int o = 16 * m + 4 * g + v;
-                if (o >= out || i > in) continue;
-                part[i < in ? mlp_w_off(layer) + o * in + i : mlp_b_off(layer) + o] = acc[m][c][v];
-            }
+        for (int v = 0; v < 4; ++v) {
+            const int o = 16 * m + 4 * g + v;
+            if (c < nts && o < out) part[mlp_w_off(layer) + o * in + i] = sum[v];
         }
+    }
+    if (nt0 != 0) return;
+    __syncthreads();
+    float* bias = (float*)red;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        float t = bsum[m];
+        t += __shfl_xor(t, 16, 64);
+        t += __shfl_xor(t, 32, 64);
+        if (g == 0) bias[wave * MLP_W + 16 * m + r] = t;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < out) {
+        float t = 0.0f;
+        for (uint32_t w = 0; w < W; ++w) t += bias[w * MLP_W + threadIdx.x];
+        part[mlp_b_off(layer) + threadIdx.x] = t;
+    }
 }
 
 /* Sum of the split partials (fixed order); then either the gradient out or
@@ -492,7 +543,7 @@ hipError_t launch_mlp_train_fb(const _Float16* pack, const float* bias, const fl
 hipError_t launch_mlp_train_grad(const TrainBatch& b, const TrainScratch& S, hipStream_t s)
 {
     if (b.batch == 0u || 16ull * S.tiles < b.batch) return hipErrorInvalidValue;
-    mlp_train_grad_kernel<<<dim3(MLP_GRAD_ITEMS, MLP_GRAD_SPLITS), 64, 0, s>>>(b, S);
+    mlp_train_grad_kernel<<<dim3(MLP_GRAD_SPLITS, MLP_GRAD_ITEMS), GRAD_THREADS, 0, s>>>(b, S);
     return hipGetLastError();
 }
 
