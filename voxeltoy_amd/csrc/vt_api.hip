@@ -556,7 +556,7 @@ vt::TraceArgs trace_args(const vt_context* c)
     a.cdfv_lds_bytes = c->env.use_image ? ((c->env.cdf_v_n * 4 + 15) / 16) * 16 : 0;
     const size_t base = 256 * sizeof(vt::MatRec) + (size_t)a.cdfv_lds_bytes;
     a.lds_bits = (base + (size_t)c->bit_words_p * 4u <= c->lds_limit) ? 1 : 0;
-    a.lds_bits_p = ((size_t)c->bit_words_p * 4u + 16u <= c->lds_limit) ? 1 : 0;   /* and the list counter */
+    a.lds_bits_p = ((size_t)c->bit_words_p * 4u + vt::WF_TAKEN_BYTES <= c->lds_limit) ? 1 : 0;
     a.dda_budget = c->dda_budget;
     a.refill_min = c->refill_min;
     a.refill_chunk = c->refill_chunk;
@@ -582,7 +582,7 @@ int alloc_paths(vt::WfPaths& P, uint64_t& alloc, uint64_t slots)
 {
     if (alloc >= slots) { P.cap = slots; return VT_OK; }
     free_paths(P, alloc);
-    const size_t n = (size_t)slots;
+    const size_t n = (size_t)vt::queue_positions(slots);
     for (vt::PathBuf& B : P.s) {
         VT_HIP(hipMalloc(&B.o, n * 16)); VT_HIP(hipMalloc(&B.nd, n * 16)); VT_HIP(hipMalloc(&B.thr, n * 16));
         VT_HIP(hipMalloc(&B.rad, n * 16)); VT_HIP(hipMalloc(&B.dir, n * 16)); VT_HIP(hipMalloc(&B.fac, n * 16));
@@ -593,7 +593,7 @@ int alloc_paths(vt::WfPaths& P, uint64_t& alloc, uint64_t slots)
     VT_HIP(hipMalloc(&P.smp, n * 16));
     VT_HIP(hipMalloc(&P.qa0, 2 * n * 16)); VT_HIP(hipMalloc(&P.qb0, 2 * n * 8)); VT_HIP(hipMalloc(&P.qt0, 2 * n * 4));
     VT_HIP(hipMalloc(&P.qa1, 2 * n * 16)); VT_HIP(hipMalloc(&P.qb1, 2 * n * 8)); VT_HIP(hipMalloc(&P.qt1, 2 * n * 4));
-    VT_HIP(hipMalloc(&P.cnt, 16));
+    VT_HIP(hipMalloc(&P.cnt, 2 * vt::QUEUE_PARTS * vt::QUEUE_COUNT_STRIDE * 4));
     P.cap = slots;
     alloc = slots;
     return VT_OK;

@@ -82,6 +82,36 @@ __device__ __forceinline__ int32_t unpack_hit(uint2 r, Hit& h)
     return (int32_t)(r.y >> 16);
 }
 
+/* A queue of paths has QUEUE_PARTS parts with a length of their own, in lines
+ * of their own: a length that workgroups of all XCDs add to takes 13 ns an
+ * addition, which bound the kernels that append (65 k additions a launch).  The
+ * positions of the parts are interleaved by runs of QUEUE_RUN paths, so a part
+ * needs no share of the arrays of its own; part s holds its m-th path at
+ * queue_position(s, m).  Work units of one size (threads of a workgroup) append
+ * to parts in turn (queue_part), every 16 units in another order, so that a
+ * pattern of the image does not fill one part more than another.  Positions up
+ * to the longest part's end are visited, those past a part's length are empty. */
+enum : uint32_t { QUEUE_PARTS = 16, QUEUE_RUN = 64, QUEUE_COUNT_STRIDE = 32 };
+__host__ __device__ inline uint32_t queue_position(uint32_t s, uint32_t m)
+{
+    return (m / QUEUE_RUN * QUEUE_PARTS + s) * QUEUE_RUN + m % QUEUE_RUN;
+}
+__host__ __device__ inline uint32_t queue_part(uint32_t unit)
+{
+    return (unit + ((unit / QUEUE_PARTS * 0x9e3779b1u) >> 28)) % QUEUE_PARTS;
+}
+/* Positions that a chunk of `paths` paths needs in any round, for units of at
+ * most 1024 paths: QUEUE_PARTS units that are full, rounded up to the next run
+ * of rounds' units (queue_part gives each part one of QUEUE_PARTS units). */
+inline uint64_t queue_positions(uint64_t paths)
+{
+    return (paths + QUEUE_PARTS * 1024u - 1u) / (QUEUE_PARTS * 1024u) * (QUEUE_PARTS * 1024u);
+}
+
+/* LDS of a traversal workgroup after its table: the list counter and the
+ * lengths of the queue's parts. */
+enum : uint32_t { WF_TAKEN_BYTES = 16 + QUEUE_PARTS * 4 };
+
 struct WfPaths {
     PathBuf s[2];     /* state of the paths in queue 0 / queue 1 */
     uint2* hit;       /* traversal result per queue entry (pack_hit): x, y, z (each + 1), kind */
@@ -93,7 +123,7 @@ struct WfPaths {
     float4* qa1;      /* ray queue 1 */
     float2* qb1;
     uint32_t* qt1;
-    uint32_t* cnt;    /* queue lengths: cnt[0] for q0, cnt[1] for q1 */
+    uint32_t* cnt;    /* paths in each part of queue 0, then of queue 1 (queue_count) */
     uint64_t cap;     /* slots */
 };
 

@@ -438,16 +438,17 @@ __device__ __forceinline__ void flush_counters(unsigned long long* stats, const 
 }
 
 /* Append the ray (o, d) for the threads with `keep` to a ray queue (length
- * counter *n) and return each such thread's position; the queue stores the
+ * counters cnt, work unit `unit`) and return each such thread's position; the queue stores the
  * rays themselves, already prepared for the march (prepare_ray, 24 bytes in
  * qa and qb) and, when qt is given (batch launches), the scene index `tag`,
  * so the traversal reads them in queue order.  One atomic per workgroup of NT
- * threads: every queue counter is a single device address that all XCDs
- * contend for.  Every thread of the workgroup must call it. */
+ * threads, on the length of the unit's part of the queue.  Every thread of the
+ * workgroup must call it. */
 template <int NT>
 __device__ __forceinline__ uint32_t block_append(bool keep, uint32_t tag, f3 o, f3 d, float4* qa, float2* qb,
-                                                 uint32_t* qt, uint32_t* n)
+                                                 uint32_t* qt, uint32_t* cnt, uint32_t unit)
 {
+    const uint32_t part = queue_part(unit);
     __shared__ uint32_t wsum[NT / 64];
     __shared__ uint32_t bbase;
     const unsigned long long mask = __ballot(keep);
@@ -457,10 +458,10 @@ __device__ __forceinline__ uint32_t block_append(bool keep, uint32_t tag, f3 o, 
     if (threadIdx.x == 0) {
         uint32_t t = 0;
         for (int w = 0; w < NT / 64; ++w) { const uint32_t c = wsum[w]; wsum[w] = t; t += c; }
-        bbase = t ? atomicAdd(n, t) : 0u;
+        bbase = t ? atomicAdd(cnt + part * QUEUE_COUNT_STRIDE, t) : 0u;
     }
     __syncthreads();
-    const uint32_t j = bbase + wsum[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+    const uint32_t j = queue_position(part, bbase + wsum[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)));
     if (keep) {
         const PreRay r = prepare_ray(o, d);
         qa[j] = queue_a(r);
@@ -471,13 +472,39 @@ __device__ __forceinline__ uint32_t block_append(bool keep, uint32_t tag, f3 o, 
     return j;
 }
 
+/* Counters of queue sel. */
+__device__ __forceinline__ uint32_t* queue_count(const WfPaths& P, int sel)
+{
+    return P.cnt + (uint32_t)sel * QUEUE_PARTS * QUEUE_COUNT_STRIDE;
+}
+/* Every wave: the queue's lengths into LDS (one wave would do, but all then
+ * need no barrier to know the result), returns the positions to visit. */
+__device__ __forceinline__ uint32_t queue_extent(const uint32_t* cnt, uint32_t* lengths)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t m = 0u;
+    if (lane < QUEUE_PARTS) lengths[lane] = m = cnt[lane * QUEUE_COUNT_STRIDE];
+    for (uint32_t k = QUEUE_PARTS / 2u; k > 0u; k >>= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)m, (int)k, 64);
+        m = o > m ? o : m;
+    }
+    m = (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+    return (m + QUEUE_RUN - 1u) / QUEUE_RUN * (QUEUE_RUN * QUEUE_PARTS);
+}
+/* Whether position p holds a path. */
+__device__ __forceinline__ bool queue_holds(const uint32_t* lengths, uint32_t p)
+{
+    return p / (QUEUE_RUN * QUEUE_PARTS) * QUEUE_RUN + p % QUEUE_RUN < lengths[p / QUEUE_RUN % QUEUE_PARTS];
+}
+
 /* The same with two rays per thread with `keep`, sharing the origin o (a
  * shadow ray along d0 and a continuation ray along d1): they take queue
  * entries 2k and 2k + 1, k being the returned position. */
 template <int NT>
 __device__ __forceinline__ uint32_t block_append2(bool keep, uint32_t tag, f3 o, f3 d0, f3 d1, float4* qa,
-                                                  float2* qb, uint32_t* qt, uint32_t* n)
+                                                  float2* qb, uint32_t* qt, uint32_t* cnt, uint32_t unit)
 {
+    const uint32_t part = queue_part(unit);
     __shared__ uint32_t wsum2[NT / 64];
     __shared__ uint32_t bbase2;
     const unsigned long long mask = __ballot(keep);
@@ -487,10 +514,10 @@ __device__ __forceinline__ uint32_t block_append2(bool keep, uint32_t tag, f3 o,
     if (threadIdx.x == 0) {
         uint32_t t = 0;
         for (int w = 0; w < NT / 64; ++w) { const uint32_t c = wsum2[w]; wsum2[w] = t; t += c; }
-        bbase2 = t ? atomicAdd(n, 2u * t) / 2u : 0u;
+        bbase2 = t ? atomicAdd(cnt + part * QUEUE_COUNT_STRIDE, t) : 0u;
     }
     __syncthreads();
-    const uint32_t k = bbase2 + wsum2[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+    const uint32_t k = queue_position(part, bbase2 + wsum2[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)));
     if (keep) {
         const PreRay r0 = prepare_ray(o, d0), r1 = prepare_ray(o, d1);
         qa[2 * k] = queue_a(r0);
@@ -587,7 +614,8 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
             gtag = tag;
         }
         const uint32_t q =
-            block_append<WF_GENERATE_THREADS>(keep, sid, ro, rd, P.qa0, P.qb0, BATCH ? P.qt0 : nullptr, &P.cnt[0]);
+            block_append<WF_GENERATE_THREADS>(keep, sid, ro, rd, P.qa0, P.qb0, BATCH ? P.qt0 : nullptr, queue_count(P, 0),
+                                              base / WF_GENERATE_THREADS);
         if (keep) store_generated<BATCH || CACHE>(P.s[0], q, G, gpix, i, gtag);
     }
     flush_counters<STATS>(BATCH ? B.stats : a0.stats, cnt);
@@ -618,7 +646,6 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * 1024 only 4.  They stage nothing in LDS.  16 scenes of 32^3 to 200^3: 1.33 ms
  * with 1024 threads, 1.15 with 256 (5 launches). */
 constexpr uint32_t wf_traverse_threads(bool stats, bool batch) { return batch && !stats ? 256u : 1024u; }
-#define WF_TAKEN_BYTES 16u      /* LDS of a traversal workgroup's list counter */
 
 /* SGPRs are allocated in steps of 16.  A build of this kernel whose
  * allocation rose from 80 to 96 SGPRs, with its hot loop unchanged
@@ -669,11 +696,18 @@ __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r
  * blocks. */
 template <bool STATS, bool LDSB, bool BATCH>
 __global__ __launch_bounds__(wf_traverse_threads(STATS, BATCH)) __attribute__((amdgpu_num_sgpr(WF_TRAVERSE_SGPRS)))
-void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
+void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t two)
 {
     extern __shared__ __align__(16) uint8_t smem[];
-    const uint32_t n = P.cnt[sel];
-    if (blockIdx.x == 0 && threadIdx.x == 0) P.cnt[sel ^ 1] = 0u;
+    /* the march reads the padded block bits, or the codes */
+    constexpr bool STAGE = !BATCH && (LDSB || !STATS);
+    const uint32_t* bits = STATS ? a.g.bitsp : a.g.codes;
+    const uint32_t words = !STAGE ? 0u : STATS ? a.g.bit_words_p : a.g.code_words;
+    uint32_t* taken = (uint32_t*)smem + words;     /* of the workgroup's list; after the table, whose reads then need no base */
+    uint32_t* lengths = taken + 4;                 /* of the queue's parts */
+    /* ray positions: a path's one ray, or (two = 1) its two */
+    const uint32_t n = queue_extent(queue_count(P, sel), lengths) << two;
+    if (blockIdx.x == 0 && threadIdx.x < QUEUE_PARTS) queue_count(P, sel ^ 1)[threadIdx.x * QUEUE_COUNT_STRIDE] = 0u;
     /* Segment: a power of two, at most what deals every workgroup its share,
      * at least a ray per lane of a wave.  A short queue leaves workgroups
      * without a segment. */
@@ -684,11 +718,6 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
     if (blockIdx.x >= n_seg) return;
     /* entries of the workgroup's own list, its segments one after another */
     const uint32_t mine = ((n_seg - blockIdx.x + gridDim.x - 1u) / gridDim.x) << seg_log;
-    /* the march reads the padded block bits, or the codes */
-    constexpr bool STAGE = !BATCH && (LDSB || !STATS);
-    const uint32_t* bits = STATS ? a.g.bitsp : a.g.codes;
-    const uint32_t words = !STAGE ? 0u : STATS ? a.g.bit_words_p : a.g.code_words;
-    uint32_t* taken = (uint32_t*)smem + words;     /* of the workgroup's list; after the table, whose reads then need no base */
     if (threadIdx.x == 0) *taken = 0u;
     if (STAGE) {
         /* four words a thread, four of these in flight (the tables are
@@ -731,12 +760,12 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel)
             if (!has) {
                 v += (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
                 uint32_t j = ((((v >> seg_log) * gridDim.x + blockIdx.x)) << seg_log) + (v & ((1u << seg_log) - 1u));
-                if (v < mine && j < n) {
+                j = n - 1u - j;
+                if (v < mine && j < n && queue_holds(lengths, j >> two)) {
                     /* the queue is taken from its end: paths are queued in
                      * pixel order, and the last rows (towards the horizon)
                      * hold the longest rays, which then start first instead
                      * of prolonging the end of the launch */
-                    j = n - 1u - j;
                     float4 o = qa[j];
                     float2 d = qb[j];
                     /* both parts of the entry in flight together: one
@@ -865,7 +894,9 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
     uint32_t* qto = BATCH ? (sel ? P.qt0 : P.qt1) : nullptr;
     const PathBuf& Bc = P.s[sel];
     const PathBuf& Bn = P.s[sel ^ 1];
-    const uint32_t n = PHASE == PH_PRIMARY ? P.cnt[sel] : P.cnt[sel] / 2u;
+    __shared__ uint32_t lengths[QUEUE_PARTS];
+    const uint32_t n = queue_extent(queue_count(P, sel), lengths);
+    __syncthreads();
     Counters cnt = { 0, 0, 0, 0, 0, 0 };
     /* Shadow and continuation rounds: each batch of a workgroup's paths is
      * sorted so that the paths whose continuation ray left the grid (the sky
@@ -885,7 +916,7 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
         uint4 hraw = make_uint4(0u, 0u, 0u, 0u);
         if (SORT) {
             uint32_t cls = 2u;                              /* no path */
-            if (j < n) {
+            if (queue_holds(lengths, j)) {
                 hraw = ((const uint4*)P.hit)[j];
                 Hit hh;
                 cls = unpack_hit(make_uint2(hraw.z, hraw.w), hh) == KIND_MISS ? 1u : 0u;
@@ -915,7 +946,7 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
         float vraw[12];
         PathState S;
         uint4 me = make_uint4(0u, 0u, 0u, 0u);
-        if (j < n) {
+        if (queue_holds(lengths, j)) {
             load_phase<PHASE == PH_PRIMARY ? PH_PRIMARY : PH_SHADOW, BATCH || CACHE>(Bc, j, S, me);
             if (BATCH) sid = me.w;
             const TraceArgs& a = BATCH ? B.tab[sid] : a0;
@@ -981,7 +1012,8 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
                 C.q_thr[qi] = make_float4(S.throughput.x, S.throughput.y, S.throughput.z, 0.0f);
             }
         }
-        const uint32_t k = block_append2<WF_SHADE_THREADS>(keep, sid, ro, rd, rn, qao, qbo, qto, &P.cnt[sel ^ 1]);
+        const uint32_t k = block_append2<WF_SHADE_THREADS>(keep, sid, ro, rd, rn, qao, qbo, qto, queue_count(P, sel ^ 1),
+                                                           base / WF_SHADE_THREADS);
         if (keep) store_cont<BATCH || CACHE>(Bn, k, S, me);
     }
     flush_counters<STATS>(BATCH ? B.stats : a0.stats, cnt);
@@ -1035,7 +1067,7 @@ __global__ __launch_bounds__(256) void wf_accumulate_kernel(TraceArgs a0, BatchT
 
 __global__ void wf_reset_kernel(uint32_t* cnt)
 {
-    if (threadIdx.x < 4) cnt[threadIdx.x] = 0u;
+    if (threadIdx.x < 2u * QUEUE_PARTS) cnt[threadIdx.x * QUEUE_COUNT_STRIDE] = 0u;
 }
 
 /* Resident workgroups per CU of a kernel (at least 1). */
@@ -1075,7 +1107,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used], s);
                 if (e != hipSuccess) return e;
             }
-            wf_traverse_kernel<STATS, LDSB, BATCH><<<cus * bt, wf_traverse_threads(STATS, BATCH), lds_t, s>>>(a, B, P, sel);
+            wf_traverse_kernel<STATS, LDSB, BATCH><<<cus * bt, wf_traverse_threads(STATS, BATCH), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
             if (timed) {
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used + 1], s);
                 if (e != hipSuccess) return e;
@@ -1171,7 +1203,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     wf_generate_kernel<false, false, true><<<gg, WF_GENERATE_THREADS, 0, s>>>(a, B, P, 0, n, C);
     int sel = 0;
     for (int r = 0; r < rounds; ++r) {
-        wf_traverse_kernel<false, LDSB, false><<<cus * bt, wf_traverse_threads(false, false), lds_t, s>>>(a, B, P, sel);
+        wf_traverse_kernel<false, LDSB, false><<<cus * bt, wf_traverse_threads(false, false), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
         if (r == 0)
             wf_shade_kernel<false, PH_PRIMARY, false, true><<<cus * bs0, WF_SHADE_THREADS, lds_s, s>>>(a, B, P, sel, C);
         else
