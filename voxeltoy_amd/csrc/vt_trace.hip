@@ -553,7 +553,12 @@ __device__ __forceinline__ uint32_t block_reserve(bool want, uint32_t* counter)
     return idx;
 }
 
-#define WF_GENERATE_THREADS 1024
+/* Bound by its writes (80 bytes a path that enters the grid's box, 16 one that
+ * does not).  A workgroup waits three times for its slowest wave, so small ones
+ * are better now that appending is cheap: 16.7 M paths in 243 us with 1024
+ * threads, 192 with 256. */
+#define WF_GENERATE_THREADS 256
+#define WF_GENERATE_BLOCKS 10u  /* a CU: 5 are resident */
 #define WF_SHADE_THREADS 256
 
 /* Scene of global path index gi in a batch: base[s] <= gi < base[s + 1]. */
@@ -1098,7 +1103,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
         const uint32_t n = (uint32_t)(g1 - g0);
         wf_reset_kernel<<<1, 64, 0, s>>>(P.cnt);
         const uint32_t gn = (n + WF_GENERATE_THREADS - 1) / WF_GENERATE_THREADS;
-        const unsigned gg = (unsigned)(gn < (uint32_t)cus * 2u ? gn : (uint32_t)cus * 2u);
+        const unsigned gg = (unsigned)(gn < (uint32_t)cus * WF_GENERATE_BLOCKS ? gn : (uint32_t)cus * WF_GENERATE_BLOCKS);
         wf_generate_kernel<STATS, BATCH><<<gg, WF_GENERATE_THREADS, 0, s>>>(a, B, P, g0, n);
         int sel = 0;
         for (int r = 0; r < rounds; ++r) {
@@ -1199,7 +1204,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     if (qround >= 0 && tround >= 0) rounds = std::min(rounds, 1 + std::max(qround, tround));
     wf_reset_kernel<<<1, 64, 0, s>>>(P.cnt);
     const uint32_t gn = (n + WF_GENERATE_THREADS - 1) / WF_GENERATE_THREADS;
-    const unsigned gg = (unsigned)(gn < (uint32_t)cus * 2u ? gn : (uint32_t)cus * 2u);
+    const unsigned gg = (unsigned)(gn < (uint32_t)cus * WF_GENERATE_BLOCKS ? gn : (uint32_t)cus * WF_GENERATE_BLOCKS);
     wf_generate_kernel<false, false, true><<<gg, WF_GENERATE_THREADS, 0, s>>>(a, B, P, 0, n, C);
     int sel = 0;
     for (int r = 0; r < rounds; ++r) {
