@@ -350,7 +350,8 @@ int32_t vt_prune_emissive(const int32_t* material_offsets, int32_t nx, int32_t n
 /* ---- diagnostics (not part of the renderer's interface) -------------------
  * Device evaluation of the elementary functions used by the kernels, for
  * checking that device and host arithmetic agree bit for bit.  fn: 0 sqrt,
- * 1 a/b, 2 sin, 3 cos, 4 acos, 5 atan2(a,b), 6 log2, 7 exp2, 8 pow(a,b). */
+ * 1 a/b, 2 sin, 3 cos, 4 acos, 5 atan2(a,b), 6 log2, 7 exp2, 8 pow(a,b),
+ * 9 1/a, 10 1/sqrt(a), 11 a/pi, 12 a/(2 pi). */
 int vt_device_math(vt_context* ctx, int32_t fn, int32_t n, const float* a, const float* b, float* out);
 
 /* Diagnostic: streaming copy of `bytes` bytes between two device buffers,

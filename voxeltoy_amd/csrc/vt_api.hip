@@ -279,6 +279,8 @@ vt::MatRec decode(const std::vector<float>& m, int32_t off)
         r.r[k] = mat_at(m, (int64_t)off + 4 + k);
     }
     r.rough = mat_at(m, (int64_t)off + 7);
+    for (int k = 0; k < 3; ++k) r.r_pi[k] = r.r[k] / VT_PI_F;
+    r.pad = 0.0f;
     return r;
 }
 

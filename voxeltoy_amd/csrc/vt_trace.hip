@@ -163,7 +163,7 @@ __device__ __forceinline__ int shade_step(const TraceArgs& a, const MatRec* recs
         if (STATS) cnt.env_samples++;
     } else {
         const float y = u[1];
-        const float r = sqrtf(vt_maxf(0.0f, 1.0f - y * y));
+        const float r = root(vt_maxf(0.0f, 1.0f - y * y));
         const float phi = (u[2] * 2.0f) * VT_PI_F;
         float sn, cs;
         vt_sincosf(phi, &sn, &cs);
@@ -235,7 +235,7 @@ __device__ __forceinline__ void stage_lds(const TraceArgs& a, uint8_t* smem, Mat
 {
     uint32_t* w = (uint32_t*)smem;
     const uint32_t* src = (const uint32_t*)a.recs;
-    for (int i = threadIdx.x; i < 256 * 8; i += blockDim.x) w[i] = src[i];
+    for (int i = threadIdx.x; i < (int)(256 * sizeof(MatRec) / 4); i += blockDim.x) w[i] = src[i];
     recs = (MatRec*)smem;
     float* cv = (float*)(smem + 256 * sizeof(MatRec));
     if (a.e.use_image) {
@@ -1359,7 +1359,7 @@ __global__ void device_math_kernel(int32_t fn, int32_t n, const float* a, const 
     const float x = a[i], y = b[i];
     float r = 0.0f, s, c;
     switch (fn) {
-        case 0: r = sqrtf(x); break;
+        case 0: r = root(x); break;
         case 1: r = x / y; break;
         case 2: vt_sincosf(x, &s, &c); r = s; break;
         case 3: vt_sincosf(x, &s, &c); r = c; break;
@@ -1368,6 +1368,10 @@ __global__ void device_math_kernel(int32_t fn, int32_t n, const float* a, const 
         case 6: r = vt_log2f(x); break;
         case 7: r = vt_exp2f(x); break;
         case 8: r = vt_powf(x, y); break;
+        case 9: r = recip(x); break;
+        case 10: r = recip_root(x); break;
+        case 11: r = over_pi<0>(x); break;
+        case 12: r = over_pi<1>(x); break;
         default: r = 0.0f; break;
     }
     out[i] = r;
