@@ -1066,7 +1066,8 @@ int vt_render(vt_context* c, uint64_t seed, uint32_t n0, uint32_t count, uint32_
         vt::TraceArgs a = trace_args(c);
         a.seed = seed; a.n0 = n0; a.count = count; a.rng_frame_max = rng_frame_max;
         a.stats = c->stats_enabled ? c->d_stats : nullptr;
-        VT_HIP(vt::launch_reset_counter(c->d_tile, a.stats, c->stream));
+        /* the tile counter of mode 0, and the statistics */
+        if (c->render_mode != 1 || a.stats) VT_HIP(vt::launch_reset_counter(c->d_tile, a.stats, c->stream));
         if (c->render_mode == 1) {
             const uint64_t total = (uint64_t)c->W * c->H * count;
             c->lt_used = 0;
