@@ -901,10 +901,10 @@ struct JumpState {
     }
 
     /* Edge minus one of the empty aligned cube around the position, 0 for a
-     * single voxel; false when the voxel is occupied or outside the grid.
+     * single voxel; -1 when the voxel is occupied or outside the grid.
      * FINE: cells are the 4x4x4 blocks.  UNI: one grid for the whole wave. */
     template <bool FINE, bool UNI>
-    __device__ __forceinline__ bool lookup(const GridView& g, int32_t& edge) const
+    __device__ __forceinline__ int32_t lookup(const GridView& g) const
     {
         const uint32_t cg = FINE ? 2u : g.cg;
         const uint32_t pad = 1u << cg;
@@ -915,7 +915,7 @@ struct JumpState {
         const uint32_t word = UNI ? *(const __attribute__((address_space(3))) uint32_t*)(ci >> 4 << 2)
                                   : ((const __attribute__((address_space(1))) uint32_t*)g.codes)[ci >> 4];
         const uint32_t c = field<2, false>(word, ci << 1);
-        edge = (int32_t)field<8, UNI>(g.cedge, c << 3);
+        int32_t edge = (int32_t)field<8, UNI>(g.cedge, c << 3);
         if (c == 0u) {
             uint32_t bi = ci;
             if (!FINE) {
@@ -928,9 +928,17 @@ struct JumpState {
             const uint32_t t = (uint32_t)(m >> (b & 0x2au));
             edge = (t & 0x00330033u) == 0u ? 1 : 0;
             if (!FINE && m == 0ull) edge = 3;
-            return ((t >> (b & 0x15u)) & 1u) == 0u;
+            edge |= bit_mask(t, b & 0x15u);
         }
-        return true;
+        return edge;
+    }
+
+    /* -1 when bit (at & 31) of v is set, else 0 */
+    static __device__ __forceinline__ int32_t bit_mask(uint32_t v, uint32_t at)
+    {
+        int32_t r;
+        asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(r) : "v"(v), "v"(at));
+        return r;
     }
 
     static __device__ __forceinline__ uint64_t load_mask(const uint64_t* occp, uint32_t i)
@@ -989,17 +997,19 @@ struct JumpState {
         return r;
     }
 
-    /* Leave the cube of lookup(); false, with the position unchanged, when a
-     * second axis is within the bound of a step. */
+    /* Leave the cube of lookup(); false, with the position unchanged, when
+     * there is none or a second axis is within the bound of a step. */
     __device__ __forceinline__ bool jump(const GridView& g, int32_t edge)
     {
         float px, py, pz;
         const float del2 = 2.0f * leave(g, edge, px, py, pz);
-        if (__builtin_amdgcn_fmed3f(__builtin_amdgcn_fractf(px), __builtin_amdgcn_fractf(py),
-                                    __builtin_amdgcn_fractf(pz)) < del2)
-            return false;
-        x = floor_i32(px); y = floor_i32(py); z = floor_i32(pz);
-        return true;
+        const float r = __builtin_amdgcn_fmed3f(__builtin_amdgcn_fractf(px), __builtin_amdgcn_fractf(py),
+                                                __builtin_amdgcn_fractf(pz));
+        const bool ok = (int)!(r < del2) & (int)(edge >= 0);
+        if (ok) {
+            x = floor_i32(px); y = floor_i32(py); z = floor_i32(pz);
+        }
+        return ok;
     }
 
     /* The position (plus the bound, which it returns) at the value that leaves

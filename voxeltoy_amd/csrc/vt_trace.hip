@@ -643,9 +643,10 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * voxel by voxel, 7.0 ms with the jump march and one queue counter (of that,
  * 4.6 ms at least in the counter's 352 k updates), 5.3 ms dealt, 4.7 ms with
  * the undecided steps settled by the voxels they could skip, 4.4 ms with the
- * cubes of 2 voxels, 4.0 ms with the march as one loop of the whole wave; one
- * pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78, 0.65 ms; 512^3 mesh scene at
- * 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38, 1.23 ms. */
+ * cubes of 2 voxels, 4.0 ms with the march as one loop of the whole wave, 3.9
+ * with one mask in it; one pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78, 0.65,
+ * 0.64 ms; 512^3 mesh scene at 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38,
+ * 1.23, 1.18 ms. */
 /* Batch launches without statistics keep each lane's grid in registers (72),
  * which leaves 6 waves a SIMD: workgroups of 256 threads use them all, those of
  * 1024 only 4.  They stage nothing in LDS.  16 scenes of 32^3 to 200^3: 1.33 ms
@@ -665,20 +666,17 @@ constexpr uint32_t wf_traverse_threads(bool stats, bool batch) { return batch &&
 
 /* The jump march of the wave's `live` lanes: at most `jumps` jumps, until
  * fewer than `keep` of them still march.  A lane is live no longer at its
- * ray's last voxel, or where a jump needs more than JumpState::jump (`near`).
- * The loop is the whole wave's: with lanes that leave it one by one the
- * compiler copies the position twice in every iteration. */
+ * ray's last voxel (edge -1), or where leaving the cube of `edge` needs more
+ * than JumpState::jump.  The loop is the whole wave's, with one mask: lanes that
+ * leave it one by one make the compiler copy the position twice in every
+ * iteration, and every further flag costs a merge. */
 template <bool FINE, bool UNI>
-__device__ __forceinline__ void jump_march(JumpState& J, const GridView& g, int jumps, int keep, bool& live, bool& near)
+__device__ __forceinline__ void jump_march(JumpState& J, const GridView& g, int jumps, int keep, bool& live, int32_t& edge)
 {
     do {
         if (live) {
-            int32_t edge;
-            live = J.lookup<FINE, UNI>(g, edge);
-            if (live) {
-                live = J.jump(g, edge);
-                near = !live;
-            }
+            edge = J.lookup<FINE, UNI>(g);
+            live = J.jump(g, edge);
         }
     } while (--jumps > 0 && __popcll(__builtin_amdgcn_ballot_w64(live)) >= keep);
 }
@@ -818,11 +816,10 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
         } else {
             /* march on until a refill is due, or to the end */
             const int keep = done ? 1 : 65 - (int)refill_min;
-            bool live = has, near = false;
-            jump_march<LDSB, !BATCH>(J, G, budget, keep, live, near);
-            if (near) {
-                int32_t edge;
-                (void)J.lookup<LDSB, !BATCH>(G, edge);
+            bool live = has;
+            int32_t edge = 0;
+            jump_march<LDSB, !BATCH>(J, G, budget, keep, live, edge);
+            if (has && !live && edge >= 0) {
                 if (!J.near_jump<!BATCH>(G, edge)) J.resolve(G, edge);
             } else if (has && !live) {
                 const int32_t x = J.gx(), y = J.gy(), z = J.gz();
