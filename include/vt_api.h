@@ -145,10 +145,12 @@ int vt_set_stats(vt_context* ctx, int32_t enabled);
  * Default 1. */
 int vt_set_render_mode(vt_context* ctx, int32_t mode, uint64_t max_paths);
 /* Wavefront traversal tuning (results are identical for every value):
- * dda_budget   DDA steps a lane takes between refill checks (1..4096),
- * refill_min   idle lanes of a 64-lane wave that trigger a refill (1..64),
- * refill_chunk queue entries a wave reserves per atomic (64..65536, or -1
- *              for exactly the idle lanes);
+ * dda_budget   jumps (with statistics: DDA steps) a lane takes between
+ *              refill checks (1..4096),
+ * refill_min   idle lanes of a 64-lane wave that trigger a refill (1..64;
+ *              without statistics three times as many, at most 64),
+ * refill_chunk queue entries that are dealt to a workgroup at a time, rounded
+ *              down to a power of two (64..65536, or -1 for 64);
  * 0 selects the default of each.  No counterpart in the reference (its
  * traversal is one fragment-shader loop). */
 int vt_set_traversal_tuning(vt_context* ctx, int32_t dda_budget, int32_t refill_min, int32_t refill_chunk);

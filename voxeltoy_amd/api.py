@@ -375,9 +375,9 @@ class Context:
         _check(lib().vt_set_render_mode(self._c, mode, max_paths))
 
     def set_traversal_tuning(self, dda_budget: int = 0, refill_min: int = 0, refill_chunk: int = 0):
-        """Wavefront traversal: DDA steps between refill checks, idle lanes
-        per wave that trigger a refill, queue entries reserved per atomic
-        (-1 = exactly the idle lanes); 0 = default.  Images are identical."""
+        """Wavefront traversal: jumps (or DDA steps) between refill checks, idle
+        lanes per wave that trigger a refill, queue entries dealt to a
+        workgroup at a time (-1 = 64); 0 = default.  Images are identical."""
         _check(lib().vt_set_traversal_tuning(self._c, dda_budget, refill_min, refill_chunk))
 
     def autotune(self, passes: int = 1) -> dict:

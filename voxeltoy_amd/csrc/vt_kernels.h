@@ -25,9 +25,9 @@ struct TraceArgs {
     int32_t lds_bits;            /* stage occupancy bits in LDS */
     int32_t lds_bits_p;          /* wavefront traversal with statistics: stage the padded block bits in LDS */
     int32_t cdfv_lds_bytes;
-    int32_t dda_budget;          /* wavefront traversal: DDA steps between refill checks */
+    int32_t dda_budget;          /* wavefront traversal: jumps or DDA steps between refill checks */
     int32_t refill_min;          /* wavefront traversal: idle lanes that trigger a refill */
-    int32_t refill_chunk;        /* wavefront traversal: queue entries a wave reserves per atomic */
+    int32_t refill_chunk;        /* wavefront traversal: queue entries dealt to a workgroup at a time */
 };
 
 struct Counters {

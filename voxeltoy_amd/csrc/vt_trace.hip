@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256) void render_kernel(TraceArgs a)
  * chunk of paths; after the camera rays, each round traces every path's
  * shadow ray and continuation ray together.  The traversal kernel only runs the DDA, so it needs few
  * registers and keeps many waves resident; shading consumes the hits and
- * appends surviving paths to the next queue with one atomic per wave. */
+ * appends surviving paths to the next queue with one atomic per workgroup. */
 
 /* Path state in HBM, by queue position (PathBuf).  Every path of a
  * traversal round is in the same phase (round 0 PRIMARY, odd rounds SHADOW,
