@@ -134,7 +134,7 @@ int noalloc_lookup(int device)
     const uint32_t zero = 0;
     hipError_t e = st.count ? hipSuccess : hipMalloc(&st.count, sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemcpy(st.count, &zero, sizeof(zero), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipHostMalloc(&host, VT_NOALLOC_BYTES, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc(&host, VT_NOALLOC_BYTES, hipHostMallocCoherent);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return fail(VT_ERR_HIP, std::string("staging memory of picking: ") + hipGetErrorString(e));

@@ -172,10 +172,10 @@ private:
     bool make()
     {
         if (made_) return true;
-        bool ok = hipHostMalloc((void**)&flags_, SLOTS * FLAG_STRIDE * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess &&
+        bool ok = hipHostMalloc((void**)&flags_, SLOTS * FLAG_STRIDE * sizeof(uint32_t), hipHostMallocCoherent) == hipSuccess &&
                   hipMalloc((void**)&count_, sizeof(uint32_t)) == hipSuccess &&
                   hipEventCreateWithFlags(&last_, hipEventDisableTiming) == hipSuccess;
-        for (int k = 0; k < SLOTS && ok; ++k) ok = hipHostMalloc(&slot_[k], CHUNK, hipHostMallocDefault) == hipSuccess;
+        for (int k = 0; k < SLOTS && ok; ++k) ok = hipHostMalloc(&slot_[k], CHUNK, hipHostMallocCoherent) == hipSuccess;
         const uint32_t zero = 0;
         ok = ok && hipMemcpy(count_, &zero, sizeof(zero), hipMemcpyHostToDevice) == hipSuccess;
         if (!ok) {
