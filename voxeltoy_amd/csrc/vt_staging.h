@@ -223,14 +223,14 @@ private:
         chunks_ = (int)((bytes + CHUNK - 1) / CHUNK);
         pieces_ = (int64_t)((bytes + PIECE - 1) / PIECE);
         for (int k = 0; k < SLOTS; ++k) copied_[k].store(0, std::memory_order_relaxed);
+        open_.store(0, std::memory_order_relaxed);
         next_.store(0, std::memory_order_relaxed);
         done_.store(0, std::memory_order_relaxed);
-        open_.store(0, std::memory_order_relaxed);
         abandon_.store(false, std::memory_order_relaxed);
         {
             std::lock_guard<std::mutex> g(wake_lock_);
             ++job_;
-            active_.store(true, std::memory_order_release);
+            active_ = true;
         }
         wake_.notify_all();
     }
@@ -255,11 +255,16 @@ private:
     }
 
     /* every piece that was taken is copied (all of them, unless abandoned),
-     * and no thread looks at the job any more */
+     * and no thread looks at the job any more: a worker joins a job under the
+     * lock, so it has either joined before the job is closed here, and is in
+     * busy_, or finds it closed */
     void finish()
     {
         while (!abandon_.load(std::memory_order_acquire) && done_.load(std::memory_order_acquire) < pieces_) help();
-        active_.store(false, std::memory_order_release);
+        {
+            std::lock_guard<std::mutex> g(wake_lock_);
+            active_ = false;
+        }
         while (busy_.load(std::memory_order_acquire) != 0) std::this_thread::yield();
     }
 
@@ -272,13 +277,12 @@ private:
                 wake_.wait(g, [&] { return quit_ || job_ != seen; });
                 if (quit_) return;
                 seen = job_;
+                if (!active_) continue;                 /* woken too late */
                 busy_.fetch_add(1, std::memory_order_acq_rel);
             }
             /* a copy is at most some milliseconds long: look for pieces until
-             * all are taken (a thread that wakes late finds no active job, or
-             * the next one, which waits for it as well) */
-            while (active_.load(std::memory_order_acquire) && !abandon_.load(std::memory_order_acquire) &&
-                   next_.load(std::memory_order_relaxed) < pieces_)
+             * all are taken */
+            while (!abandon_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < pieces_)
                 if (!help()) std::this_thread::yield();
             busy_.fetch_sub(1, std::memory_order_acq_rel);
         }
@@ -302,12 +306,12 @@ private:
     std::atomic<int> copied_[SLOTS];
     std::atomic<int64_t> next_{ 0 }, done_{ 0 };
     std::atomic<int> open_{ 0 };
-    std::atomic<bool> abandon_{ false }, active_{ false };
-    std::atomic<int> busy_{ 0 };
-    std::mutex wake_lock_;
+    std::atomic<bool> abandon_{ false };
+    std::atomic<int> busy_{ 0 };        /* workers in the job */
+    std::mutex wake_lock_;              /* guards the three below */
     std::condition_variable wake_;
     uint64_t job_ = 0;
-    bool quit_ = false;
+    bool active_ = false, quit_ = false;
 };
 
 }  // namespace vt
