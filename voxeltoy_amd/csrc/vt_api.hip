@@ -59,7 +59,6 @@ int no_throw(F&& f) noexcept
 #define VT_DEFAULT_REFILL_MIN 8
 #define VT_DEFAULT_REFILL_CHUNK 256
 #define VT_WORK_KEEP (256ull << 20)  /* workspace kept on a context */
-#define VT_CODE_LDS_BYTES 80640ull  /* half a CU's LDS but one 1280-byte allocation unit */
 /* (x, y) columns above which the voxelizer gives a triangle a whole wave */
 #define VT_VOX_BIG_AREA 32
 /* paths from which a scene of a batch gets its own launches */
@@ -202,8 +201,7 @@ struct vt_context {
     uint32_t* d_bitsp = nullptr;
     uint32_t bit_words_p = 0;
     uint32_t* d_codes = nullptr;    /* the jump march's codes */
-    uint32_t code_words = 0;
-    uint32_t cell_shift = 2, code_top = 2, cell_ex = 0, cell_ey = 0;
+    vt::CellLayout cells{};
     int32_t* d_emissive = nullptr;
     int32_t n_emissive = 0;
     int4* d_lights = nullptr;       /* emissive entries decoded: x, y, z, slot */
@@ -301,8 +299,7 @@ vt::TraceArgs trace_args(const vt_context* c);
  * codes and the emissive light table. */
 int refresh_codes(vt_context* c)
 {
-    VT_HIP(vt::launch_cell_codes(c->dims, c->d_occp, c->cell_shift, c->code_top, c->cell_ex, c->cell_ey, c->d_codes,
-                                 c->stream));
+    VT_HIP(vt::launch_cell_codes(c->dims, c->d_occp, c->cells, c->d_codes, c->stream));
     if (c->n_emissive > 0 && c->d_emissive) {
         if (c->lights_cap < c->n_emissive) {
             dfree(c->d_lights);
@@ -347,22 +344,6 @@ private:
 };
 size_t aligned(size_t bytes) { return (bytes + 255u) & ~(size_t)255u; }
 
-vt::BrickDims make_dims(int32_t nx, int32_t ny, int32_t nz)
-{
-    vt::BrickDims d;
-    d.nx = nx; d.ny = ny; d.nz = nz;
-    d.bx = (nx + 7) / 8; d.by = (ny + 7) / 8; d.bz = (nz + 7) / 8;
-    int32_t m = std::max(d.bx, std::max(d.by, d.bz));
-    int32_t p = 1;
-    while (p < m) p <<= 1;
-    d.bdim = p;
-    d.n_bricks = (uint64_t)p * p * p;
-    d.kx = (nx + 3) / 4; d.ky = (ny + 3) / 4; d.kz = (nz + 3) / 4;
-    d.px = (d.kx + 5) / 4 * 4; d.py = d.ky + 2; d.pz = d.kz + 2;
-    d.n_padded = (uint64_t)d.px * d.py * d.pz;
-    return d;
-}
-
 /* Reference bounds (renderer.cpp:845-850): cubic voxels, longest axis 1000. */
 void reference_bounds(int32_t nx, int32_t ny, int32_t nz, float* bmin, float* bmax)
 {
@@ -375,36 +356,13 @@ void reference_bounds(int32_t nx, int32_t ny, int32_t nz, float* bmin, float* bm
     }
 }
 
-/* Cells of the jump march: the smallest power-of-two edge, from 4 voxels,
- * whose padded two-bit codes let two traversal workgroups share a CU's
- * 160 KiB LDS (4 up to about 266 voxels an axis, 8 up to about 530).  The
- * coded cubes are 1, 2 and 8 cells an edge, or 1, 2 and 4 where the grid has
- * at most 56 cells an axis: iterations a ray 12.1 against 13.0 on a 256^3
- * terrain, 8.9 against 9.9 the other way on a 64^3 one. */
-void choose_cells(vt_context* c)
-{
-    const vt::BrickDims& d = c->dims;
-    uint32_t cg = 2;
-    uint64_t ex, ey, ez;
-    for (;; ++cg) {
-        const uint64_t e = 1ull << cg;
-        ex = ((uint64_t)d.nx + e - 1) / e; ey = ((uint64_t)d.ny + e - 1) / e; ez = ((uint64_t)d.nz + e - 1) / e;
-        if (((ex + 5) / 4 * 4) * (ey + 2) * (ez + 2) <= VT_CODE_LDS_BYTES * 4u) break;
-    }
-    c->cell_shift = cg;
-    c->code_top = std::max(ex, std::max(ey, ez)) > 56 && cg < 6 ? 3u : 2u;   /* an edge of at most 256: cedge holds bytes */
-    c->cell_ex = (uint32_t)((ex + 5) / 4 * 4);      /* rows of whole bytes; dims.px for cells of one block */
-    c->cell_ey = (uint32_t)ey + 2;
-    c->code_words = (uint32_t)(((uint64_t)c->cell_ex * c->cell_ey * (ez + 2) + 63) / 64 * 4);   /* whole uint4 */
-}
-
 int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const float* mat_data, int32_t mat_size,
                         const float* bmin, const float* bmax)
 {
     if (nx <= 0 || ny <= 0 || nz <= 0 || nx > 4096 || ny > 4096 || nz > 4096)
         return fail(VT_ERR_ARG, "volume resolution must be in [1, 4096] per axis");
     if (mat_size < 0 || (mat_size > 0 && !mat_data)) return fail(VT_ERR_ARG, "bad material data");
-    const vt::BrickDims d = make_dims(nx, ny, nz);
+    const vt::BrickDims d = vt::make_dims(nx, ny, nz);
     c->has_volume = false;
     /* a grid of the same extents keeps its buffers */
     const bool keep = c->d_bricks && c->d_occp && c->d_bitsp && c->d_codes && c->dims.nx == nx && c->dims.ny == ny &&
@@ -436,11 +394,11 @@ int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const
         VT_HIP(hipMalloc(&c->d_bitsp, (size_t)c->bit_words_p * 4u));
         if (nx <= VT_PACKED_MAX_EXTENT && ny <= VT_PACKED_MAX_EXTENT && nz <= VT_PACKED_MAX_EXTENT)
             VT_HIP(hipMalloc(&c->d_occr, np * 8u));
-        choose_cells(c);
-        VT_HIP(hipMalloc(&c->d_codes, (size_t)c->code_words * 4u));
+        c->cells = vt::cell_layout(d);
+        VT_HIP(hipMalloc(&c->d_codes, (size_t)c->cells.words * 4u));
         /* what the conversions never write: the bricks' voxels outside the
          * grid and the codes' padding */
-        VT_HIP(vt::launch_fill_u8((uint8_t*)c->d_codes, (uint64_t)c->code_words * 4u, 0, c->stream));
+        VT_HIP(vt::launch_fill_u8((uint8_t*)c->d_codes, (uint64_t)c->cells.words * 4u, 0, c->stream));
         VT_HIP(vt::launch_fill_u8(c->d_bricks, d.n_bricks * 512u, 0, c->stream));
     }
     return VT_OK;
@@ -502,18 +460,18 @@ vt::GridView grid_view(const vt_context* c)
     }
     g.bricks = c->d_bricks;
     g.bxp = (uint32_t)c->dims.px;
-    g.byp = (uint32_t)c->dims.ky + 2u;
+    g.byp = (uint32_t)c->dims.py;
     g.occp = c->d_occp;
     g.bitsp = c->d_bitsp;
     g.bit_words_p = c->bit_words_p;
     g.occr = c->d_occr;
     g.wide = c->dims.n_padded > (1ull << 29);
     g.codes = c->d_codes;
-    g.code_words = c->code_words;
-    g.ccx = c->cell_ex;
-    g.ccy = c->cell_ey;
-    g.cg = c->cell_shift;
-    g.cedge = ((1u << g.cg) - 1u) << 8 | ((2u << g.cg) - 1u) << 16 | ((1u << (g.cg + c->code_top)) - 1u) << 24;
+    g.code_words = c->cells.words;
+    g.ccx = c->cells.ex;
+    g.ccy = c->cells.ey;
+    g.cg = c->cells.shift;
+    g.cedge = c->cells.edges();
     g.jc0 = VT_ULP24 * (float)(2 * std::max(g.nx, std::max(g.ny, g.nz)) + 32);
     g.n_emissive = c->n_emissive;
     g.emissive = c->d_emissive;
@@ -618,6 +576,7 @@ int vt_create(int device, vt_context** out)
         if (device < 0 || device >= n) return fail(VT_ERR_ARG, "no such device");
         if (device >= VT_MAX_DEVICES) return fail(VT_ERR_LIMIT, "device index beyond the library's table");
         VT_HIP(hipSetDevice(device));
+        VT_HIP(vt::check_lds_base());
         if (int r = noalloc_lookup(device)) return r;
         vt_context* c = new vt_context();
         c->device = device;

@@ -5,6 +5,7 @@
 #pragma once
 
 #include "vt_device.h"
+#include "vt_layout.h"
 
 namespace vt {
 
@@ -190,26 +191,16 @@ hipError_t launch_render_wavefront(const TraceArgs& a, const WfPaths& P, int cus
                                    const LaunchTimer* timer = nullptr, hipEvent_t acc_wait = nullptr);
 hipError_t launch_render(const TraceArgs& a, int grid, hipStream_t s, bool stats);
 int render_blocks_per_cu(const TraceArgs& a, bool stats);
+/* The jump march of a single grid reads its codes from LDS address 0, where a
+ * kernel's dynamic LDS begins if it has no other: an error if one has. */
+hipError_t check_lds_base();
 hipError_t launch_first_hit(const TraceArgs& a, int32_t* out, hipStream_t s);
 hipError_t launch_trace_rays(const TraceArgs& a, int32_t n, const float* o, const float* d, int32_t* out,
                              uint32_t* count, uint32_t* flag, uint32_t seq, hipStream_t s);
 hipError_t launch_reset_counter(uint32_t* c, unsigned long long* stats, hipStream_t s);
 hipError_t launch_device_math(int32_t fn, int32_t n, const float* a, const float* b, float* out, hipStream_t s);
 
-/* ---- volume layout --------------------------------------------------------------------- */
-struct BrickDims {
-    int32_t nx, ny, nz;          /* voxels */
-    int32_t bx, by, bz;          /* bricks per axis */
-    int32_t bdim;                /* power-of-two cube edge in bricks (Morton range) */
-    uint64_t n_bricks;           /* bdim^3 */
-    int32_t kx, ky, kz;          /* 4x4x4 blocks per axis (ceil(n/4)) */
-    /* the block grid padded by one block on every side, rows to a multiple of
-     * four blocks (rows of the jump march's codes are whole bytes, and with
-     * cells of one block both have one index) */
-    int32_t px, py, pz;
-    uint64_t n_padded;           /* px*py*pz */
-};
-
+/* ---- volume layout (BrickDims: vt_layout.h) --------------------------------------------- */
 /* Which material offsets a dense int32 grid uses: used[o] = 1 for every o in
  * [0, lut_n) that occurs (used zero at launch); *bad = the smallest index of
  * an offset >= lut_n (all ones at launch). */
@@ -234,12 +225,11 @@ hipError_t launch_blocks_from_offsets(const BrickDims& d, const int32_t* dense, 
                                       const BlockLevels& L, hipStream_t s);
 hipError_t launch_blocks_from_ids(const BrickDims& d, const uint8_t* dense, const uint8_t* remap, uint8_t* bricks,
                                   const BlockLevels& L, hipStream_t s);
-/* The jump march's codes (GridView::codes) from the padded masks, for cells of
- * 2^cg voxels in rows of ccx and layers of ccx ccy cells.  The largest coded
- * cube has 2^top cells an edge (top 2 or 3), the next 2, the smallest 1.  The
- * codes of the padding are not written (zero). */
-hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint32_t ccx,
-                             uint32_t ccy, uint32_t* codes, hipStream_t s);
+/* The jump march's codes (GridView::codes) from the padded masks.  The largest
+ * coded cube has 2^top cells an edge (top 2 or 3), the next 2, the smallest 1.
+ * The codes of the padding are not written (zero). */
+hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, const CellLayout& c, uint32_t* codes,
+                             hipStream_t s);
 /* Bricked slots -> dense int32 offsets via slot_off[256]. */
 hipError_t launch_dense_from_bricks(const BrickDims& d, const uint8_t* bricks, const int32_t* slot_off, int32_t* dense,
                                     hipStream_t s);

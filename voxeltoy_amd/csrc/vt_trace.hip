@@ -1082,6 +1082,18 @@ static int blocks_per_cu(K kernel, int threads, size_t lds)
     return b;
 }
 
+hipError_t check_lds_base()
+{
+    for (const void* k : { (const void*)wf_traverse_kernel<false, false, false>,
+                           (const void*)wf_traverse_kernel<false, true, false> }) {
+        hipFuncAttributes at;
+        const hipError_t e = hipFuncGetAttributes(&at, k);
+        if (e != hipSuccess) return e;
+        if (at.sharedSizeBytes != 0) return hipErrorInvalidKernelFile;
+    }
+    return hipSuccess;
+}
+
 /* generate -> (traverse -> shade) x rounds -> accumulate per chunk of at
  * most P.cap paths.  `a` describes the single scene (or, in a batch, carries
  * the traversal tuning and the LDS sizes of scene 0). */

@@ -357,17 +357,17 @@ hipError_t launch_blocks_from_ids(const BrickDims& d, const uint8_t* dense, cons
     return hipGetLastError();
 }
 
-hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, uint32_t cg, uint32_t top, uint32_t ccx,
-                             uint32_t ccy, uint32_t* codes, hipStream_t s)
+hipError_t launch_cell_codes(const BrickDims& d, const uint64_t* occp, const CellLayout& c, uint32_t* codes,
+                             hipStream_t s)
 {
-    const int32_t e = 1 << cg;
+    const int32_t e = 1 << c.shift;
     const int32_t nx = (d.nx + e - 1) / e, ny = (d.ny + e - 1) / e, nz = (d.nz + e - 1) / e;
-    const uint32_t r = 1u << top;
-    const dim3 grid(((uint32_t)ny + r - 1) / r, ((uint32_t)nz + r - 1) / r, (ccx / 4u + CODE_BYTES - 1) / CODE_BYTES);
-    if (top == 2u)
-        cell_codes_kernel<2><<<grid, 256, 0, s>>>(d, occp, cg, nx, ny, nz, ccx, ccy, (uint8_t*)codes);
+    const uint32_t r = 1u << c.top;
+    const dim3 grid(((uint32_t)ny + r - 1) / r, ((uint32_t)nz + r - 1) / r, (c.ex / 4u + CODE_BYTES - 1) / CODE_BYTES);
+    if (c.top == 2u)
+        cell_codes_kernel<2><<<grid, 256, 0, s>>>(d, occp, c.shift, nx, ny, nz, c.ex, c.ey, (uint8_t*)codes);
     else
-        cell_codes_kernel<3><<<grid, 256, 0, s>>>(d, occp, cg, nx, ny, nz, ccx, ccy, (uint8_t*)codes);
+        cell_codes_kernel<3><<<grid, 256, 0, s>>>(d, occp, c.shift, nx, ny, nz, c.ex, c.ey, (uint8_t*)codes);
     return hipGetLastError();
 }
 
