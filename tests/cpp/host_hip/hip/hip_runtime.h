@@ -2,8 +2,22 @@
  * headers under test use.  Streams, copies and kernels are the test's own. */
 #pragma once
 
+#include <math.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <string.h>
+
+#define __device__
+#define __host__
+#define __forceinline__ inline
+
+struct float2 { float x, y; };
+struct float4 { float x, y, z, w; };
+struct int4 { int32_t x, y, z, w; };
+inline uint32_t __float_as_uint(float v) { uint32_t u; memcpy(&u, &v, 4); return u; }
+inline float __uint_as_float(uint32_t u) { float v; memcpy(&v, &u, 4); return v; }
+inline uint32_t min(uint32_t a, uint32_t b) { return b < a ? b : a; }
+inline uint32_t max(uint32_t a, uint32_t b) { return b > a ? b : a; }
 
 typedef enum { hipSuccess = 0, hipErrorNotReady = 600, hipErrorUnknown = 999 } hipError_t;
 typedef struct test_stream* hipStream_t;

@@ -472,7 +472,7 @@ vt::GridView grid_view(const vt_context* c)
     g.ccy = c->cells.ey;
     g.cg = c->cells.shift;
     g.cedge = c->cells.edges();
-    g.jc0 = VT_ULP24 * (float)(2 * std::max(g.nx, std::max(g.ny, g.nz)) + 32);
+    g.jc0 = vt::jump_bound0(std::max(g.nx, std::max(g.ny, g.nz)));
     g.n_emissive = c->n_emissive;
     g.emissive = c->d_emissive;
     g.lights = c->d_lights;

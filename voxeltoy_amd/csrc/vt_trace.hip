@@ -664,23 +664,6 @@ constexpr uint32_t wf_traverse_threads(bool stats, bool batch) { return batch &&
  * (swept from 6 to 42 lanes: within 2 % from 18 on) */
 #define VT_JUMP_REFILL 3u
 
-/* The jump march of the wave's `live` lanes: at most `jumps` jumps, until
- * fewer than `keep` of them still march.  A lane is live no longer at its
- * ray's last voxel (edge -1), or where leaving the cube of `edge` needs more
- * than JumpState::jump.  The loop is the whole wave's, with one mask: lanes that
- * leave it one by one make the compiler copy the position twice in every
- * iteration, and every further flag costs a merge. */
-template <bool FINE, bool UNI>
-__device__ __forceinline__ void jump_march(JumpState& J, const GridView& g, int jumps, int keep, bool& live, int32_t& edge)
-{
-    do {
-        if (live) {
-            edge = J.lookup<FINE, UNI>(g);
-            live = J.jump(g, edge);
-        }
-    } while (--jumps > 0 && __popcll(__builtin_amdgcn_ballot_w64(live)) >= keep);
-}
-
 /* A ray marched step by step (DdaState::advance): hit record. */
 __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r)
 {
