@@ -113,3 +113,25 @@ def test_cubes_inside_blocks(exe, tmp_path, orc, edge, at):
         occ[z:z + edge, y:y + 1 + at, x:x + 1] = True
     o, d = rays_of(rng, np.full(3, -500.0), np.full(3, 500.0), (48, 48, 48), 24000)
     compare(exe, tmp_path, orc, occ, o, d, 10000)
+
+
+@pytest.mark.parametrize("wall", [3970, 3971, 3972, 4092])
+def test_far_end_of_the_longest_grid(exe, tmp_path, orc, wall):
+    """4096 voxels an axis: the error bound passes one voxel near the 3970th
+    step.  Rays along x whose y and z step together right before the step
+    into a wall."""
+    res = np.array([4096, 6, 6])
+    occ = np.zeros(res[::-1], bool)
+    occ[:, :, wall] = True
+    rng = np.random.default_rng(wall)
+    n = 4000
+    hi = 500.0 * res / 4096
+    vs = 1000.0 / 4096
+    p = np.concatenate([rng.uniform(0, 1, (n, 1)), rng.uniform(2, 3, (n, 2))], 1)
+    p[::2, 2] = p[::2, 1]
+    rest = wall - p[:, 0] - 10.0 ** rng.uniform(-5, -2, n)
+    slope = (np.ceil(p[:, 1:]) - p[:, 1:]) / rest[:, None]
+    d = np.concatenate([np.ones((n, 1)), slope], 1)
+    d *= rng.uniform(0.7, 1.4, (n, 1))                  # steps that are no round numbers
+    o = p * vs - hi - np.sign(d) * 0.001
+    compare(exe, tmp_path, orc, occ, o.astype(F), d.astype(F), n // 2)

@@ -183,10 +183,11 @@ __device__ __forceinline__ int lanes_with(bool p) { return p ? 1 : 0; }
  * the FP32 sums is off by at most half an ulp, so with M = m / (smallest a) the
  * two sequences that a decision compares are together off their lines by at
  * most 2^-24 (M^2 + 3M) steps, and the evaluation itself by 2^-24 (3M + 2
- * extent + 8); del = 2^-24 (1.06 (M + 4)^2 + 2 extent + 32) covers both.  With q the real-valued position (an integer where an axis
- * steps), floor(q + del) is the exact position unless q lies within del of an
- * integer; on the axis that leaves the cube it always does, and it is then
- * right as well.  When a second axis is that near an integer the order of the
+ * extent + 8); del = 2^-24 (1.06 (M + 4)^2 + 2 extent + 32) covers both.
+ * With q the real-valued position (an integer where an axis steps), floor(q +
+ * del) is the exact position unless q lies within del of an integer; on the
+ * axis that leaves the cube it always does, and it is then right as well as
+ * long as del stays below 1 (3970 steps).  When a second axis is that near an integer the order of the
  * two steps is undecided (0.1-0.3 % of the jumps).  Both orders and a common
  * step end in the same voxel, by way of one of the two voxels where one of the
  * steps is still missing: if both are empty the ray passes and the order does
@@ -373,7 +374,9 @@ struct JumpState {
         /* steps ahead only: one that is behind was taken before */
         const bool mx = tx > x, my = ty > y, mz = tz > z;
         const bool nx = rx < del2 && mx, ny = ry < del2 && my, nz = rz < del2 && mz;
-        if (nx && ny && nz) return false;
+        /* a bound near 1 (from about 3860 steps) no longer tells the step that
+         * leaves the cube from the one after it */
+        if ((nx && ny && nz) || del2 > 1.9f) return false;
         if ((nx && ny) || (ny && nz) || (nz && nx)) {
             const float am = fmaxf(fmaxf(nx ? ax : 0.0f, ny ? ay : 0.0f), nz ? az : 0.0f);
             const float ex = del2 * __builtin_fmaf(am, ix, 1.0f), ey = del2 * __builtin_fmaf(am, iy, 1.0f),
