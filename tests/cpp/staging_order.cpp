@@ -102,7 +102,7 @@ int main(int argc, char** argv)
 {
     const int jobs = argc > 1 ? std::atoi(argv[1]) : 400;
     caller_ = std::this_thread::get_id();
-    vt::StagingRing* ring = new vt::StagingRing();
+    vt::Staging* ring = new vt::Staging();
     test_stream s;
     const size_t most = 3u << 20;
     std::vector<unsigned char> dev(most + 64), host(most + 64);

@@ -137,6 +137,7 @@ hipError_t hipEventSynchronize(hipEvent_t e)
     if (e->s) device_.wait(e->s);
     return hipSuccess;
 }
+hipError_t hipEventQuery(hipEvent_t e) { return !e->s || device_.idle(e->s) ? hipSuccess : hipErrorNotReady; }
 hipError_t hipGetLastError() { return hipSuccess; }
 
 namespace vt {

@@ -29,3 +29,8 @@ def test_ring_has_no_data_race(tmp_path):
     r = run(tmp_path, "staging_order.cpp", "120", cxx=CLANG, flags=("-g", "-fsanitize=thread"))
     assert "ThreadSanitizer" not in r.stderr, r.stderr[-4000:]
     assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+
+
+def test_copy_behind_a_long_kernel_sleeps_and_leaves_the_ring(tmp_path):
+    r = run(tmp_path, "staging_busy.cpp")
+    assert r.returncode == 0, r.stdout + r.stderr

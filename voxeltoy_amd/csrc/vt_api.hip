@@ -145,17 +145,17 @@ int noalloc_lookup(int device)
 }  // namespace
 
 /* Staging rings (vt_staging.h) and the contexts that share them, per device.
- * A ring object is never destroyed, only emptied: the process may end with
+ * The object is never destroyed, only emptied: the process may end with
  * contexts alive. */
 namespace {
 std::mutex g_ring_lock;
-vt::StagingRing* g_ring[VT_MAX_DEVICES] = {};
+vt::Staging* g_ring[VT_MAX_DEVICES] = {};
 int g_ring_users[VT_MAX_DEVICES] = {};
 
 void ring_join(int device)
 {
     std::lock_guard<std::mutex> lk(g_ring_lock);
-    if (!g_ring[device]) g_ring[device] = new vt::StagingRing();
+    if (!g_ring[device]) g_ring[device] = new vt::Staging();
     ++g_ring_users[device];
 }
 
@@ -173,7 +173,7 @@ struct vt_context {
     std::vector<vt_batch*> batches;
     std::vector<vt_cache*> caches;
     int device = 0;
-    vt::StagingRing* ring = nullptr;   /* the device's, for large copies */
+    vt::Staging* ring = nullptr;   /* the device's rings, for large copies */
     int cus = 0;
     size_t lds_limit = 65536;       /* dynamic LDS per workgroup */
     hipStream_t stream = nullptr;
@@ -252,13 +252,13 @@ namespace {
  * the host memory free on return. */
 hipError_t to_host(vt_context* c, void* dst, const void* src, size_t bytes)
 {
-    if (bytes >= vt::StagingRing::MIN_BYTES) return c->ring->read(dst, src, bytes, c->stream);
+    if (bytes >= vt::Staging::MIN_BYTES) return c->ring->read(dst, src, bytes, c->stream);
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
     return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
 }
 hipError_t to_device(vt_context* c, void* dst, const void* src, size_t bytes)
 {
-    if (bytes >= vt::StagingRing::MIN_BYTES) return c->ring->write(dst, src, bytes, c->stream);
+    if (bytes >= vt::Staging::MIN_BYTES) return c->ring->write(dst, src, bytes, c->stream);
     return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream);
 }
 

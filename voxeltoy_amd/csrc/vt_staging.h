@@ -12,10 +12,10 @@
  * the host that its chunk is done, by a word of pinned memory: with an event
  * after every kernel the link stood still for 5.6 us of every 45.
  *
- * One ring and its threads per device, shared by the device's contexts: made
- * by the first large copy, given back when the last context is destroyed.  A
- * copy that finds the ring in use by another thread, or whose ring could not
- * be made, takes the runtime's path.
+ * A ring and its threads belong to a device, whose contexts share it: made by
+ * the first large copy, given back when the last context is destroyed.  A copy
+ * that finds both of the device's rings in use by other threads, or whose ring
+ * could not be made, takes the runtime's path.
  */
 #pragma once
 
@@ -48,18 +48,31 @@ public:
     static constexpr int WORKERS = 3;              /* besides the calling thread */
     static constexpr size_t MIN_BYTES = 1u << 20;  /* smaller copies take the runtime's path */
 
+    static constexpr int POLL_MS = 2;
     static constexpr int PIECES = (int)(CHUNK / PIECE);
+
+    /* Whether a copy on stream s may use the ring; it then holds `lk`.  Chunks
+     * of the last write may still be on their way out of it, behind whatever
+     * their stream holds: on the same stream the kernels of a read come after
+     * them, a write waits for them, and other streams go without the ring. */
+    bool take(std::unique_lock<std::mutex>& lk, hipStream_t s, bool to_device)
+    {
+        lk = std::unique_lock<std::mutex>(use_, std::try_to_lock);
+        if (lk.owns_lock() && made_ && in_flight_) {
+            if (stream_ == s ? to_device : hipEventQuery(last_) != hipSuccess) {
+                (void)hipGetLastError();
+                if (stream_ != s || hipEventSynchronize(last_) != hipSuccess) lk.unlock();
+            }
+            if (lk.owns_lock()) in_flight_ = false;
+        }
+        if (lk.owns_lock() && !make()) lk.unlock();
+        return lk.owns_lock();
+    }
 
     /* Device to host; complete when it returns. */
     hipError_t read(void* dst, const void* src, size_t bytes, hipStream_t s)
     {
-        std::unique_lock<std::mutex> lk(use_, std::try_to_lock);
-        if (!lk.owns_lock() || !make()) {
-            const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-            return e != hipSuccess ? e : hipStreamSynchronize(s);
-        }
-        hipError_t err = settle();
-        if (err != hipSuccess) return err;
+        hipError_t err = hipSuccess;
         begin((char*)dst, bytes, false);
         const int n = chunks_;
         int issued = 0, arrived = 0;
@@ -73,7 +86,7 @@ public:
                 if (err == hipSuccess) ++issued;
             }
             if (err != hipSuccess) break;
-            if (arrived < issued && complete(arrived)) open_.store(++arrived, std::memory_order_release);
+            if (arrived < issued && complete(arrived)) open(++arrived);
             else if (!help()) err = stalled(arrived, issued, s);
         }
         if (err != hipSuccess) abandon_.store(true, std::memory_order_release);
@@ -86,14 +99,11 @@ public:
      * when it returns. */
     hipError_t write(void* dst, const void* src, size_t bytes, hipStream_t s)
     {
-        std::unique_lock<std::mutex> lk(use_, std::try_to_lock);
-        if (!lk.owns_lock() || !make()) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
-        hipError_t err = settle();
-        if (err != hipSuccess) return err;
+        hipError_t err = hipSuccess;
         begin((char*)const_cast<void*>(src), bytes, true);
         const int n = chunks_;
         int issued = 0, drained = 0;
-        open_.store(n < SLOTS ? n : SLOTS, std::memory_order_release);
+        open(n < SLOTS ? n : SLOTS);
         while (issued < n && err == hipSuccess) {
             if (issued < open_.load(std::memory_order_relaxed) &&
                 copied_[issued % SLOTS].load(std::memory_order_acquire) == goal(issued)) {
@@ -102,7 +112,7 @@ public:
             } else if (drained < issued && open_.load(std::memory_order_relaxed) < n && complete(drained)) {
                 copied_[drained % SLOTS].store(0, std::memory_order_relaxed);
                 ++drained;
-                open_.store(drained + SLOTS < n ? drained + SLOTS : n, std::memory_order_release);
+                open(drained + SLOTS < n ? drained + SLOTS : n);
             } else if (!help()) {
                 err = stalled(drained, issued, s);
             }
@@ -110,7 +120,7 @@ public:
         if (err != hipSuccess) abandon_.store(true, std::memory_order_release);
         finish();
         if (err == hipSuccess) err = hipEventRecord(last_, s);
-        if (err == hipSuccess) in_flight_ = true;
+        if (err == hipSuccess) in_flight_ = true, stream_ = s;
         else (void)hipStreamSynchronize(s);
         return err;
     }
@@ -120,7 +130,8 @@ public:
     {
         std::lock_guard<std::mutex> lk(use_);
         if (!made_) return;
-        (void)settle();
+        if (in_flight_) (void)hipEventSynchronize(last_);
+        in_flight_ = false;
         {
             std::lock_guard<std::mutex> g(wake_lock_);
             quit_ = true;
@@ -152,20 +163,16 @@ private:
         return __atomic_load_n(flag(chunk), __ATOMIC_ACQUIRE) == seq_[chunk % SLOTS];
     }
 
-    /* Nothing to copy now.  Once a millisecond the stream is asked whether
-     * the chunk that is waited for (when one was issued) can still come. */
+    /* Nothing to copy now: chunk `waiting` is waited for.  It is polled for a
+     * frame's time, since a wait that sleeps comes back later; behind longer
+     * work the thread sleeps until the chunks that were issued are done. */
     hipError_t stalled(int waiting, int issued, hipStream_t s)
     {
         std::this_thread::yield();
         const auto now = std::chrono::steady_clock::now();
-        if (now - asked_ < std::chrono::milliseconds(1)) return hipSuccess;
-        asked_ = now;
-        if (waiting >= issued) return hipSuccess;
-        const hipError_t e = hipStreamQuery(s);
-        if (e == hipErrorNotReady) {
-            (void)hipGetLastError();
-            return hipSuccess;
-        }
+        if (waiting != stalled_at_) stalled_at_ = waiting, since_ = now;
+        if (now - since_ < std::chrono::milliseconds(POLL_MS) || waiting >= issued) return hipSuccess;
+        const hipError_t e = hipStreamSynchronize(s);
         return e != hipSuccess ? e : complete(waiting) ? hipSuccess : hipErrorUnknown;
     }
 
@@ -207,14 +214,6 @@ private:
         last_ = nullptr;
     }
 
-    /* the last write's chunks have left the ring */
-    hipError_t settle()
-    {
-        if (!in_flight_) return hipSuccess;
-        in_flight_ = false;
-        return hipEventSynchronize(last_);
-    }
-
     void begin(char* host, size_t bytes, bool to_ring)
     {
         host_ = host;
@@ -227,12 +226,25 @@ private:
         next_.store(0, std::memory_order_relaxed);
         done_.store(0, std::memory_order_relaxed);
         abandon_.store(false, std::memory_order_relaxed);
+        stalled_at_ = -1;
         {
             std::lock_guard<std::mutex> g(wake_lock_);
             ++job_;
             active_ = true;
         }
         wake_.notify_all();
+    }
+
+    /* Chunks up to n may be copied now. */
+    void open(int n)
+    {
+        bool asleep;
+        {
+            std::lock_guard<std::mutex> g(wake_lock_);
+            open_.store(n, std::memory_order_release);
+            asleep = asleep_ > 0;
+        }
+        if (asleep) wake_.notify_all();
     }
 
     /* One piece of an open chunk; false when there is none now. */
@@ -261,10 +273,13 @@ private:
     void finish()
     {
         while (!abandon_.load(std::memory_order_acquire) && done_.load(std::memory_order_acquire) < pieces_) help();
+        bool asleep;
         {
             std::lock_guard<std::mutex> g(wake_lock_);
             active_ = false;
+            asleep = asleep_ > 0;
         }
+        if (asleep) wake_.notify_all();
         while (busy_.load(std::memory_order_acquire) != 0) std::this_thread::yield();
     }
 
@@ -280,10 +295,25 @@ private:
                 if (!active_) continue;                 /* woken too late */
                 busy_.fetch_add(1, std::memory_order_acq_rel);
             }
-            /* a copy is at most some milliseconds long: look for pieces until
-             * all are taken */
-            while (!abandon_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < pieces_)
-                if (!help()) std::this_thread::yield();
+            /* Look for pieces until all are taken: with yields for a frame's
+             * time, then asleep until a chunk opens (behind a render of
+             * seconds every worker would keep a core busy). */
+            auto last = std::chrono::steady_clock::now();
+            while (!abandon_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < pieces_) {
+                if (help()) {
+                    last = std::chrono::steady_clock::now();
+                    continue;
+                }
+                std::this_thread::yield();
+                if (std::chrono::steady_clock::now() - last < std::chrono::milliseconds(POLL_MS)) continue;
+                std::unique_lock<std::mutex> g(wake_lock_);
+                ++asleep_;
+                wake_.wait(g, [&] {
+                    const int64_t p = next_.load(std::memory_order_relaxed);
+                    return !active_ || p >= pieces_ || p / PIECES < open_.load(std::memory_order_relaxed);
+                });
+                --asleep_;
+            }
             busy_.fetch_sub(1, std::memory_order_acq_rel);
         }
     }
@@ -291,11 +321,13 @@ private:
     std::mutex use_;
     bool made_ = false, in_flight_ = false;
     void* slot_[SLOTS] = {};
-    hipEvent_t last_ = nullptr;         /* after the last write */
+    hipEvent_t last_ = nullptr;         /* after the last write, on stream_ */
+    hipStream_t stream_ = nullptr;
     uint32_t* flags_ = nullptr;         /* pinned: a slot's last finished chunk */
     uint32_t* count_ = nullptr;         /* device: the copy kernel's finished workgroups */
     uint32_t seq_[SLOTS] = {}, last_seq_ = 0;
-    std::chrono::steady_clock::time_point asked_{};
+    int stalled_at_ = -1;               /* chunk that the caller waits for, since when */
+    std::chrono::steady_clock::time_point since_{};
     std::vector<std::thread> threads_;
     /* the copy in progress */
     char* host_ = nullptr;
@@ -308,10 +340,41 @@ private:
     std::atomic<int> open_{ 0 };
     std::atomic<bool> abandon_{ false };
     std::atomic<int> busy_{ 0 };        /* workers in the job */
-    std::mutex wake_lock_;              /* guards the three below */
+    std::mutex wake_lock_;              /* guards the four below */
     std::condition_variable wake_;
     uint64_t job_ = 0;
+    int asleep_ = 0;                    /* workers that wait for a chunk */
     bool active_ = false, quit_ = false;
+};
+
+/* The copies of a device's contexts.  The second ring is for a copy that finds
+ * the first in use: a read of another context may hold it behind a render. */
+class Staging {
+public:
+    static constexpr size_t MIN_BYTES = StagingRing::MIN_BYTES;
+
+    hipError_t read(void* dst, const void* src, size_t bytes, hipStream_t s)
+    {
+        std::unique_lock<std::mutex> lk;
+        for (StagingRing& r : ring_)
+            if (r.take(lk, s, false)) return r.read(dst, src, bytes, s);
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        return e != hipSuccess ? e : hipStreamSynchronize(s);
+    }
+    hipError_t write(void* dst, const void* src, size_t bytes, hipStream_t s)
+    {
+        std::unique_lock<std::mutex> lk;
+        for (StagingRing& r : ring_)
+            if (r.take(lk, s, true)) return r.write(dst, src, bytes, s);
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+    }
+    void release()
+    {
+        for (StagingRing& r : ring_) r.release();
+    }
+
+private:
+    StagingRing ring_[2];
 };
 
 }  // namespace vt
