@@ -74,6 +74,7 @@ struct late_atomic {
         if (this_thread::get_id() != caller_ && chance(4)) pause_us((int)(dice_ >> 24));
         return pending_.drain(), v.fetch_add(x);
     }
+    T fetch_or(T x, memory_order = memory_order_seq_cst) { return pending_.drain(), v.fetch_or(x); }
     T fetch_sub(T x, memory_order = memory_order_seq_cst) { return pending_.drain(), v.fetch_sub(x); }
     bool compare_exchange_weak(T& e, T x, memory_order = memory_order_seq_cst)
     {

@@ -34,3 +34,8 @@ def test_ring_has_no_data_race(tmp_path):
 def test_copy_behind_a_long_kernel_sleeps_and_leaves_the_ring(tmp_path):
     r = run(tmp_path, "staging_busy.cpp")
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_one_small_copy_makes_no_ring(tmp_path):
+    r = run(tmp_path, "staging_first.cpp")
+    assert r.returncode == 0, r.stdout + r.stderr

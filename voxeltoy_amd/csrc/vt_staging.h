@@ -13,7 +13,7 @@
  * after every kernel the link stood still for 5.6 us of every 45.
  *
  * A ring and its threads belong to a device, whose contexts share it: made by
- * the first large copy, given back when the last context is destroyed.  A copy
+ * the second large copy (the first from 16 MiB), given back when the last context is destroyed.  A copy
  * that finds both of the device's rings in use by other threads, or whose ring
  * could not be made, takes the runtime's path.
  */
@@ -356,25 +356,36 @@ public:
     hipError_t read(void* dst, const void* src, size_t bytes, hipStream_t s)
     {
         std::unique_lock<std::mutex> lk;
-        for (StagingRing& r : ring_)
-            if (r.take(lk, s, false)) return r.read(dst, src, bytes, s);
+        if (pays(bytes))
+            for (StagingRing& r : ring_)
+                if (r.take(lk, s, false)) return r.read(dst, src, bytes, s);
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     }
     hipError_t write(void* dst, const void* src, size_t bytes, hipStream_t s)
     {
         std::unique_lock<std::mutex> lk;
-        for (StagingRing& r : ring_)
-            if (r.take(lk, s, true)) return r.write(dst, src, bytes, s);
+        if (pays(bytes))
+            for (StagingRing& r : ring_)
+                if (r.take(lk, s, true)) return r.write(dst, src, bytes, s);
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
     }
     void release()
     {
         for (StagingRing& r : ring_) r.release();
+        copies_.store(0, std::memory_order_relaxed);
     }
 
 private:
+    /* Making a ring and giving it back take 300 us, as much as a copy of 12 to
+     * 16 MiB gains (8 MiB from the device: 0.60 ms by the runtime, 0.34 by the
+     * ring, 0.76 by one made for it): a program's only copy, unless it is
+     * larger, goes without. */
+    static constexpr size_t ALONE_BYTES = 16u << 20;
+    bool pays(size_t bytes) { return copies_.fetch_or(1, std::memory_order_relaxed) != 0 || bytes >= ALONE_BYTES; }
+
     StagingRing ring_[2];
+    std::atomic<int> copies_{ 0 };      /* 1 after the first */
 };
 
 }  // namespace vt
