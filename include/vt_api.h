@@ -312,8 +312,9 @@ int vt_trace_rays(vt_context* ctx, int32_t n, const float* origins, const float*
  * as vt_trace_rays for n <= VT_NOALLOC_MAX_RAYS (VT_ERR_LIMIT beyond, nothing
  * launched).  Rays and records are staged in a fixed array of pinned host
  * memory of VT_NOALLOC_MAX_RAYS x 56 bytes (896 KiB), one per device, that the
- * library holds until the process ends; calls that would overlap on one device take
- * turns on it (each returns after its records are on the host). */
+ * library holds until the process ends (vt_trace_rays has another); calls that
+ * would overlap on one device take turns on it (each returns after its records
+ * are on the host). */
 #define VT_NOALLOC_MAX_RAYS 16384
 int vt_trace_rays_noalloc(vt_context* ctx, int32_t n, const float* origins, const float* dirs, int32_t* rec);
 

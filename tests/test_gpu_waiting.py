@@ -29,3 +29,33 @@ def test_readback_behind_a_render_leaves_the_cores_idle(ctx):
     assert np.isfinite(img[..., 3]).all()
     assert wall > 0.2
     assert cpu < 1.8 * wall, (cpu, wall)      # the caller, if the runtime's wait spins; not four threads
+
+
+def test_pick_behind_a_render_holds_up_no_other_context(ctx, vtapi):
+    """vt_trace_rays on a context whose render goes on, and meanwhile a pick
+    through vt_trace_rays_noalloc on another context."""
+    import threading
+    from voxeltoy_amd import workloads
+    o = np.array([[0.0, 400.0, 0.0]], np.float32)
+    d = np.array([[0.1, -0.99, 0.1]], np.float32)
+    with vtapi.Context(0) as other:
+        workloads.load(other, workloads.small(1))
+        want = other.trace_rays(o, d)
+        long_render(ctx, 1.0)
+        took = {}
+
+        def behind():
+            t = time.perf_counter()
+            ctx.trace_rays(o, d)
+            took["behind"] = time.perf_counter() - t
+
+        th = threading.Thread(target=behind)
+        th.start()
+        time.sleep(0.05)
+        t = time.perf_counter()
+        got = other.trace_rays_noalloc(o, d)
+        took["other"] = time.perf_counter() - t
+        th.join(60)
+        assert np.array_equal(got, want)
+        assert took["behind"] > 0.5
+        assert took["other"] < 0.5 * took["behind"], took

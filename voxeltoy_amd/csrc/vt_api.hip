@@ -97,13 +97,15 @@ struct DevTmp {
 
 }  // namespace
 
-/* ---- staging memory of vt_trace_rays_noalloc -------------------------------------
- * A fixed array of pinned host memory, one per device, made by the device's
+/* ---- staging memory of picking ---------------------------------------------------
+ * Fixed arrays of pinned host memory, two per device, made by the device's
  * first vt_create and held until the process ends: origins
  * (VT_NOALLOC_MAX_RAYS x 12 B), directions (x 12 B), hit records (x 32 B) and
  * the word in which the kernel reports its end.  The kernel reads and writes it
  * over the link: three copies of a few bytes and a wait for the stream took 50
- * us a call. */
+ * us a call.  vt_trace_rays_noalloc calls take turns on the first;
+ * vt_trace_rays has one of its own, since a call may hold its array behind a
+ * render of its context, and goes without when that one is in use. */
 #define VT_STR_(x) #x
 #define VT_STR(x) VT_STR_(x)
 namespace {
@@ -116,18 +118,17 @@ constexpr int VT_MAX_DEVICES = 64;
 static_assert(VT_NOALLOC_R % 256 == 0, "record staging must stay aligned");
 
 struct RayStage {
+    std::mutex lock;                             /* held by the call that uses it */
     unsigned char* host = nullptr;
     uint32_t* count = nullptr;                   /* device: finished workgroups */
     uint32_t seq = 0;
 };
-std::mutex g_noalloc_lock;                       /* guards the table and serializes calls */
-RayStage g_noalloc[VT_MAX_DEVICES];
+RayStage g_stage_noalloc[VT_MAX_DEVICES], g_stage_trace[VT_MAX_DEVICES];
 
-/* The current device's staging memory, once per device. */
-int noalloc_lookup(int device)
+/* The current device's memory for `st`, once. */
+int stage_make(RayStage& st)
 {
-    std::lock_guard<std::mutex> lk(g_noalloc_lock);
-    RayStage& st = g_noalloc[device];
+    std::lock_guard<std::mutex> lk(st.lock);
     if (st.host) return VT_OK;
     void* host = nullptr;
     const uint32_t zero = 0;
@@ -577,7 +578,8 @@ int vt_create(int device, vt_context** out)
         if (device >= VT_MAX_DEVICES) return fail(VT_ERR_LIMIT, "device index beyond the library's table");
         VT_HIP(hipSetDevice(device));
         VT_HIP(vt::check_lds_base());
-        if (int r = noalloc_lookup(device)) return r;
+        if (int r = stage_make(g_stage_noalloc[device])) return r;
+        if (int r = stage_make(g_stage_trace[device])) return r;
         vt_context* c = new vt_context();
         c->device = device;
         ring_join(device);
@@ -2104,12 +2106,11 @@ int vt_trace_first_hit(vt_context* c, uint64_t seed, uint32_t frame, int32_t* re
 }
 
 namespace {
-/* n <= VT_NOALLOC_MAX_RAYS rays through the device's staging memory, with
- * g_noalloc_lock held.  The host reads the kernel's word for as long as a pick
+/* n <= VT_NOALLOC_MAX_RAYS rays through staging memory of the context's
+ * device, with its lock held.  The host reads the kernel's word for as long as a pick
  * takes on an idle stream; behind other work it waits for the stream. */
-int trace_rays_staged(vt_context* c, int32_t n, const float* o, const float* dir, int32_t* rec)
+int trace_rays_staged(vt_context* c, RayStage& st, int32_t n, const float* o, const float* dir, int32_t* rec)
 {
-    RayStage& st = g_noalloc[c->device];
     if (!st.host) return fail(VT_ERR_STATE, "staging array of the device was not looked up");
     uint32_t* const flag = (uint32_t*)(st.host + VT_NOALLOC_FLAG);
     const uint32_t seq = ++st.seq;
@@ -2137,8 +2138,9 @@ int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, in
         if (n == 0) return VT_OK;
         VT_HIP(hipSetDevice(c->device));
         if (n <= VT_NOALLOC_MAX_RAYS) {
-            std::unique_lock<std::mutex> lk(g_noalloc_lock, std::try_to_lock);
-            if (lk.owns_lock()) return trace_rays_staged(c, n, o, dir, rec);
+            RayStage& st = g_stage_trace[c->device];
+            std::unique_lock<std::mutex> lk(st.lock, std::try_to_lock);
+            if (lk.owns_lock()) return trace_rays_staged(c, st, n, o, dir, rec);
         }
         vt::TraceArgs a = trace_args(c);
         WorkSpace ws;
@@ -2167,8 +2169,9 @@ int vt_trace_rays_noalloc(vt_context* c, int32_t n, const float* o, const float*
         VT_HIP(hipSetDevice(c->device));
         /* one call at a time uses the device's staging array; a call returns only
          * after its records are back on the host */
-        std::lock_guard<std::mutex> lk(g_noalloc_lock);
-        return trace_rays_staged(c, n, o, dir, rec);
+        RayStage& st = g_stage_noalloc[c->device];
+        std::lock_guard<std::mutex> lk(st.lock);
+        return trace_rays_staged(c, st, n, o, dir, rec);
     });
 }
 
