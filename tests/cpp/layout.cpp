@@ -16,6 +16,8 @@ static void one(int nx, int ny, int nz)
     const vt::CellLayout c = vt::cell_layout(d);
     check(d.px >= d.kx + 2 && d.py >= d.ky + 2 && d.pz >= d.kz + 2, "blocks without padding", d);
     check(d.n_padded == (uint64_t)d.px * d.py * d.pz && d.n_padded < (1ull << 31), "padded blocks", d);
+    const uint64_t blocks = (uint64_t)d.kx * d.ky * d.kz;
+    check((uint64_t)vt::own_bit_words(d) * 32 >= blocks && (uint64_t)vt::own_bit_words(d) * 32 < blocks + 32, "own bits", d);
     const int e = 1 << c.shift;
     const uint64_t cx = (nx + e - 1) / e, cy = (ny + e - 1) / e, cz = (nz + e - 1) / e;
     check(c.ex >= cx + 2 && c.ey >= cy + 2 && c.ex % 4 == 0, "rows of cells", d);

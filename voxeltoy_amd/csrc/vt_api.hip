@@ -201,6 +201,7 @@ struct vt_context {
     uint64_t* d_occr = nullptr;     /* padded masks with reversed bits, for the packed march */
     uint32_t* d_bitsp = nullptr;
     uint32_t bit_words_p = 0;
+    uint32_t* d_bits = nullptr;     /* bits of the grid's own blocks, when the megakernel has run */
     uint32_t* d_codes = nullptr;    /* the jump march's codes */
     vt::CellLayout cells{};
     int32_t* d_emissive = nullptr;
@@ -372,6 +373,7 @@ int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const
         dfree(c->d_bricks);
         dfree(c->d_occp);
         dfree(c->d_bitsp);
+        dfree(c->d_bits);
         dfree(c->d_occr);
         dfree(c->d_codes);
     }
@@ -465,6 +467,8 @@ vt::GridView grid_view(const vt_context* c)
     g.occp = c->d_occp;
     g.bitsp = c->d_bitsp;
     g.bit_words_p = c->bit_words_p;
+    g.bits = c->d_bits;
+    g.bit_words = vt::own_bit_words(c->dims);
     g.occr = c->d_occr;
     g.wide = c->dims.n_padded > (1ull << 29);
     g.codes = c->d_codes;
@@ -515,8 +519,8 @@ vt::TraceArgs trace_args(const vt_context* c)
     a.tiles_x = (c->W + 7) / 8;
     a.n_tiles = a.tiles_x * ((c->H + 7) / 8);
     a.cdfv_lds_bytes = c->env.use_image ? ((c->env.cdf_v_n * 4 + 15) / 16) * 16 : 0;
-    const size_t base = 256 * sizeof(vt::MatRec) + (size_t)a.cdfv_lds_bytes;
-    a.lds_bits = (base + (size_t)c->bit_words_p * 4u <= c->lds_limit) ? 1 : 0;
+    const size_t base = 256 * sizeof(vt::MatBase) + (size_t)a.cdfv_lds_bytes;
+    a.lds_bits = (base + (size_t)a.g.bit_words * 4u <= c->lds_limit) ? 1 : 0;
     a.lds_bits_p = ((size_t)c->bit_words_p * 4u + vt::WF_TAKEN_BYTES <= c->lds_limit) ? 1 : 0;
     a.dda_budget = c->dda_budget;
     a.refill_min = c->refill_min;
@@ -620,7 +624,7 @@ void vt_destroy(vt_context* c)
     while (!c->batches.empty()) batch_release(c->batches.back());
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    dfree(c->d_bricks); dfree(c->d_occp); dfree(c->d_bitsp); dfree(c->d_occr); dfree(c->d_codes); dfree(c->d_work); dfree(c->d_emissive); dfree(c->d_lights); dfree(c->d_recs);
+    dfree(c->d_bricks); dfree(c->d_occp); dfree(c->d_bitsp); dfree(c->d_bits); dfree(c->d_occr); dfree(c->d_codes); dfree(c->d_work); dfree(c->d_emissive); dfree(c->d_lights); dfree(c->d_recs);
     dfree(c->d_img); dfree(c->d_quad); dfree(c->d_cdfu); dfree(c->d_cdfv);
     dfree(c->d_accum); dfree(c->d_sum64); dfree(c->d_tile); dfree(c->d_stats);
     free_wavefront(c);
@@ -1027,8 +1031,7 @@ int vt_render(vt_context* c, uint64_t seed, uint32_t n0, uint32_t count, uint32_
         vt::TraceArgs a = trace_args(c);
         a.seed = seed; a.n0 = n0; a.count = count; a.rng_frame_max = rng_frame_max;
         a.stats = c->stats_enabled ? c->d_stats : nullptr;
-        /* the tile counter of mode 0, and the statistics */
-        if (c->render_mode != 1 || a.stats) VT_HIP(vt::launch_reset_counter(c->d_tile, a.stats, c->stream));
+        if (c->render_mode == 1 && a.stats) VT_HIP(vt::launch_reset_counter(c->d_tile, a.stats, c->stream));
         if (c->render_mode == 1) {
             const uint64_t total = (uint64_t)c->W * c->H * count;
             c->lt_used = 0;
@@ -1069,6 +1072,9 @@ int vt_render(vt_context* c, uint64_t seed, uint32_t n0, uint32_t count, uint32_
                 VT_HIP(hipEventRecord(c->ev1, c->stream));
             }
         } else {
+            if (a.lds_bits && !c->d_bits) VT_HIP(hipMalloc(&c->d_bits, (size_t)a.g.bit_words * 4u));
+            a.g.bits = c->d_bits;
+            VT_HIP(vt::launch_render_setup(a.g, a.lds_bits ? c->d_bits : nullptr, c->d_tile, a.stats, c->stream));
             const int per_cu = vt::render_blocks_per_cu(a, c->stats_enabled);
             const int grid = std::max(1, c->cus * per_cu);
             VT_HIP(hipEventRecord(c->ev0, c->stream));

@@ -128,14 +128,20 @@ __device__ __forceinline__ void mat4_mul(const float* m, float x, float y, float
 }
 
 /* ---- views ------------------------------------------------------------------ */
-struct MatRec {                 /* one decoded material record (48 bytes) */
+/* A decoded material record.  The megakernel, whose LDS also holds the block
+ * bits, stages the first 32 bytes of each; the wavefront's shading takes the
+ * quotients by pi ready-made. */
+struct MatBase {
     int32_t type;               /* 0 matte, 1 metal, 2 plastic, -1 none */
     float e[3];                 /* emission */
     float r[3];                 /* albedo / reflectance */
     float rough;                /* Blinn exponent (the reference uses roughness unmapped) */
+};
+struct MatRec : MatBase {
     float r_pi[3];              /* r / pi, the matte BSDF */
     float pad;
 };
+static_assert(sizeof(MatBase) == 32 && sizeof(MatRec) == 48, "records are copied by words");
 
 struct EnvView {
     int32_t use_image;
@@ -315,15 +321,18 @@ struct DdaState {
      * lessThanEqual(dis, min(dis.yzx, dis.zxy)); dis is a running FP32 sum
      * replayed step by step.  Lanes that stop keep their state and step no
      * further (predicated updates), so the loop has one wave-uniform exit and
-     * no divergent branches except the block reload. */
-    template <bool COUNT>
+     * no divergent branches except the block reload.  OWN: `bits` are of the
+     * grid's own blocks (GridView::bits), else of the padded ones. */
+    template <bool COUNT, bool OWN>
     __device__ __forceinline__ int advance(const GridView& g, const uint32_t* __restrict__ bits, int budget,
                                            uint32_t& visits)
     {
         const int32_t limit = budget < g.max_steps - steps ? steps + budget : g.max_steps;
         bool done = false;
-        /* block-grid strides held in vector registers across the loop */
-        uint32_t bxp = g.bxp, byp = g.byp, first = 1u + g.bxp + g.bxp * g.byp;   /* padded index of block (0, 0, 0) */
+        /* strides of the bits held in vector registers across the loop, and the
+         * index of block (0, 0, 0) */
+        uint32_t bxp = g.bxp, byp = g.byp, first = 1u + g.bxp + g.bxp * g.byp;
+        if (OWN) bxp = ((uint32_t)g.nx + 3u) / 4u, byp = ((uint32_t)g.ny + 3u) / 4u, first = 0u;
         asm volatile("" : "+v"(bxp), "+v"(byp), "+v"(first));
         for (;;) {
             const bool inside = (uint32_t)x < (uint32_t)g.nx && (uint32_t)y < (uint32_t)g.ny &&
@@ -334,7 +343,9 @@ struct DdaState {
             const uint32_t bk = mad24(mad24((uint32_t)z >> 2, byp, (uint32_t)y >> 2), bxp, (uint32_t)x >> 2) + first;
             if (inside && bk != key) {
                 key = bk;
-                mask = ((bits[bk >> 5] >> (bk & 31u)) & 1u) ? g.occp[bk] : 0ull;
+                uint32_t bm = bk;
+                if (OWN) bm = mad24(mad24(((uint32_t)z >> 2) + 1u, g.byp, ((uint32_t)y >> 2) + 1u), g.bxp, ((uint32_t)x >> 2) + 1u);
+                mask = ((bits[bk >> 5] >> (bk & 31u)) & 1u) ? g.occp[bm] : 0ull;
             }
             /* the voxel test only when some lane's block has an occupied voxel
              * (a wave-uniform branch: rays in empty space skip it) */
@@ -730,7 +741,7 @@ __device__ __forceinline__ int DdaState::advance_wave_packed(const GridView& g, 
  * Returns 1 on hit, 0 when the march ended without a hit (position written),
  * -1 when the start point lies outside the grid (position not written).
  * `slot` receives the hit voxel's material slot. */
-template <bool COUNT>
+template <bool COUNT, bool OWN>
 __device__ __forceinline__ int dda(const GridView& g, const uint32_t* __restrict__ bits, f3 o, f3 d, Hit& h,
                                    uint32_t& visits)
 {
@@ -739,7 +750,7 @@ __device__ __forceinline__ int dda(const GridView& g, const uint32_t* __restrict
         h.steps = -1;
         return -1;
     }
-    const int status = D.advance<COUNT>(g, bits, g.max_steps, visits);
+    const int status = D.advance<COUNT, OWN>(g, bits, g.max_steps, visits);
     D.finish(g, status, h);
     return status == 1 ? 1 : 0;
 }
@@ -808,10 +819,10 @@ __device__ __forceinline__ int dda_cubes(const GridView& g, f3 o, f3 d, Hit& h)
 /* traverse (dda.h:63-79): 2 voxel hit, 3 ground hit (final y < 0), 0 miss. */
 enum { KIND_MISS = 0, KIND_VOXEL = 2, KIND_GROUND = 3 };
 
-template <bool COUNT>
+template <bool COUNT, bool OWN>
 __device__ __forceinline__ int traverse(const GridView& g, const uint32_t* bits, f3 o, f3 d, Hit& h, uint32_t& visits)
 {
-    const int r = dda<COUNT>(g, bits, o, d, h, visits);
+    const int r = dda<COUNT, OWN>(g, bits, o, d, h, visits);
     if (r > 0) return KIND_VOXEL;
     if (r < 0) return KIND_MISS;
     return h.y < 0 ? KIND_GROUND : KIND_MISS;
@@ -819,7 +830,7 @@ __device__ __forceinline__ int traverse(const GridView& g, const uint32_t* bits,
 
 /* Slot of a voxel position: texelFetch semantics, outside the grid reads
  * offset 0, which is record index 0 of the decoded table. */
-__device__ __forceinline__ uint32_t fetch_slot(const GridView& g, const uint32_t* bits, int32_t x, int32_t y, int32_t z)
+__device__ __forceinline__ uint32_t fetch_slot(const GridView& g, int32_t x, int32_t y, int32_t z)
 {
     if ((uint32_t)x >= (uint32_t)g.nx || (uint32_t)y >= (uint32_t)g.ny || (uint32_t)z >= (uint32_t)g.nz) return 0u;
     const uint32_t bm = brick_morton((uint32_t)x >> 3, (uint32_t)y >> 3, (uint32_t)z >> 3);
@@ -1035,13 +1046,16 @@ __device__ __forceinline__ void eval_microfacet(f3 refl, float e, f3 wo, f3 wi, 
     f = f * k;
 }
 
-__device__ __forceinline__ f3 rec_r(const MatRec& m) { return mk(m.r[0], m.r[1], m.r[2]); }
+__device__ __forceinline__ f3 rec_r(const MatBase& m) { return mk(m.r[0], m.r[1], m.r[2]); }
+__device__ __forceinline__ f3 rec_r_pi(const MatRec& m) { return mk(m.r_pi[0], m.r_pi[1], m.r_pi[2]); }
+__device__ __forceinline__ f3 rec_r_pi(const MatBase& m) { return mk(over_pi<0>(m.r[0]), over_pi<0>(m.r[1]), over_pi<0>(m.r[2])); }
 
-__device__ __forceinline__ void eval_material(const MatRec& m, f3 wo, f3 wi, f3& f, float& pdf)
+template <class Rec>
+__device__ __forceinline__ void eval_material(const Rec& m, f3 wo, f3 wi, f3& f, float& pdf)
 {
     if (m.type == 0) {
         pdf = over_pi<0>(wi.y);
-        f = mk(m.r_pi[0], m.r_pi[1], m.r_pi[2]);
+        f = rec_r_pi(m);
     } else if (m.type == 1) {
         eval_microfacet(rec_r(m), m.rough, wo, wi, f, pdf);
     } else if (m.type == 2) {
@@ -1054,7 +1068,8 @@ __device__ __forceinline__ void eval_material(const MatRec& m, f3 wo, f3 wi, f3&
 
 /* sampleMaterialBSDF (materials.h:30-43).  Draws one rand() except for an
  * unknown material type. */
-__device__ __forceinline__ f3 sample_material(const MatRec& m, f3 wo, vt_pcg32& rng, f3& f, float& pdf)
+template <class Rec>
+__device__ __forceinline__ f3 sample_material(const Rec& m, f3 wo, vt_pcg32& rng, f3& f, float& pdf)
 {
     if (m.type < 0) { f = mk(0.0f, 0.0f, 0.0f); pdf = 0.0f; return mk(0.0f, 0.0f, 0.0f); }
     float u[4];
@@ -1065,7 +1080,7 @@ __device__ __forceinline__ f3 sample_material(const MatRec& m, f3 wo, vt_pcg32& 
         vt_sincosf((2.0f * VT_PI_F) * u[1], &sn, &cs);
         const float px = r * cs, py = r * sn;
         const float y = root(vt_maxf(0.0f, (1.0f - px * px) - py * py));
-        f = mk(m.r_pi[0], m.r_pi[1], m.r_pi[2]);
+        f = rec_r_pi(m);
         pdf = over_pi<0>(y);
         return mk(px, y, py);
     }

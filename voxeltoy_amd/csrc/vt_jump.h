@@ -30,6 +30,11 @@ struct GridView {
     const uint64_t* occp;
     const uint32_t* bitsp;
     uint32_t bit_words_p;
+    /* the bits of the grid's own blocks (x + kx (y + ky z), kx = ceil(nx / 4),
+     * ...), which the megakernel stages: in LDS the padding counts.  Written
+     * before each of its launches (launch_render_setup) */
+    const uint32_t* bits;
+    uint32_t bit_words;
     /* occp with each mask's bits reversed (voxel l of the block at bit
      * 63 - l), for the packed-coordinate march; null when an extent of the
      * grid exceeds VT_PACKED_MAX_EXTENT */

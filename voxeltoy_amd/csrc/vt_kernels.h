@@ -198,6 +198,8 @@ hipError_t launch_first_hit(const TraceArgs& a, int32_t* out, hipStream_t s);
 hipError_t launch_trace_rays(const TraceArgs& a, int32_t n, const float* o, const float* d, int32_t* out,
                              uint32_t* count, uint32_t* flag, uint32_t seq, hipStream_t s);
 hipError_t launch_reset_counter(uint32_t* c, unsigned long long* stats, hipStream_t s);
+/* The same, and the megakernel's block bits (GridView::bits) unless null. */
+hipError_t launch_render_setup(const GridView& g, uint32_t* bits, uint32_t* c, unsigned long long* stats, hipStream_t s);
 hipError_t launch_device_math(int32_t fn, int32_t n, const float* a, const float* b, float* out, hipStream_t s);
 
 /* ---- volume layout (BrickDims: vt_layout.h) --------------------------------------------- */

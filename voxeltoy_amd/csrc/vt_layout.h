@@ -40,6 +40,12 @@ inline BrickDims make_dims(int32_t nx, int32_t ny, int32_t nz)
     return d;
 }
 
+/* Words of a bit per block of the grid itself. */
+inline uint32_t own_bit_words(const BrickDims& d)
+{
+    return (uint32_t)(((uint64_t)d.kx * d.ky * d.kz + 31) / 32);
+}
+
 /* Cells of the jump march: the smallest power-of-two edge, from 4 voxels,
  * whose padded two-bit codes let two traversal workgroups share a CU's
  * 160 KiB LDS (4 up to about 266 voxels an axis, 8 up to about 530).  The

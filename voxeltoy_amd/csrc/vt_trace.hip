@@ -65,9 +65,8 @@ __device__ __forceinline__ bool start_path(const TraceArgs& a, int32_t px, int32
  * with *vrec set, taken after the bounce-0 emission and before any random
  * draw; when the vertex is at bounce `cache_bounce` the step returns 2
  * there instead (the path ends into the cache). */
-template <bool STATS, bool VERT = false>
-__device__ __forceinline__ int shade_step(const TraceArgs& a, const MatRec* recs, const uint32_t* bits,
-                                          const float* cdfv, PathState& S, const Hit& h, int kind, Counters& cnt,
+template <bool STATS, bool VERT = false, class Rec>
+__device__ __forceinline__ int shade_step(const TraceArgs& a, const Rec* recs, const float* cdfv, PathState& S, const Hit& h, int kind, Counters& cnt,
                                           int cache_bounce = -1, float* vraw = nullptr, bool* vrec = nullptr)
 {
     const GridView& g = a.g;
@@ -105,7 +104,7 @@ __device__ __forceinline__ int shade_step(const TraceArgs& a, const MatRec* recs
     /* ---- shade the vertex (pathTracer.fs:214-280) ---- */
     if (STATS) cnt.interactions++;
     const Basis B = voxel_basis(g, (float)h.x, (float)h.y, (float)h.z, S.basis_o, S.ray_d);
-    const MatRec& m = recs[h.slot];   /* ground hits carry slot 0 = record of offset 0 */
+    const Rec& m = recs[h.slot];   /* ground hits carry slot 0 = record of offset 0 */
     if (h.x == st.sel[0] && h.y == st.sel[1] && h.z == st.sel[2]) {
         S.radiance = S.radiance + mk(1.0f, 0.0f, 0.0f);
         return false;
@@ -141,7 +140,7 @@ __device__ __forceinline__ int shade_step(const TraceArgs& a, const MatRec* recs
         /* the emissive list entry decoded once per grid (light_table_kernel) */
         const int4 lt = g.lights[li];
         S.ex = lt.x; S.ey = lt.y; S.ez = lt.z;
-        const MatRec& me = recs[lt.w];
+        const Rec& me = recs[lt.w];
         L = mk(me.e[0], me.e[1], me.e[2]) * 10.0f;
         const f3 vsE = mk((float)S.ex, (float)S.ey, (float)S.ez);
         const f3 bmin = mk(g.bmin[0], g.bmin[1], g.bmin[2]), bmax = mk(g.bmax[0], g.bmax[1], g.bmax[2]);
@@ -210,8 +209,8 @@ __device__ __forceinline__ f3 tonemap(const Settings& st, f3 r)
 }
 
 /* One pass of one pixel, start to finish (megakernel form). */
-template <bool STATS>
-__device__ __forceinline__ f3 trace_sample(const TraceArgs& a, const MatRec* recs, const uint32_t* bits,
+template <bool STATS, bool OWN>
+__device__ __forceinline__ f3 trace_sample(const TraceArgs& a, const MatBase* recs, const uint32_t* bits,
                                            const float* cdfv, int32_t px, int32_t py, uint32_t rng_frame,
                                            Counters& cnt)
 {
@@ -219,47 +218,50 @@ __device__ __forceinline__ f3 trace_sample(const TraceArgs& a, const MatRec* rec
     if (start_path<STATS>(a, px, py, rng_frame, S, cnt)) {
         for (;;) {
             Hit h;
-            const int kind = traverse<STATS>(a.g, bits, S.ray_o, S.ray_d, h, cnt.visits);
-            if (!shade_step<STATS>(a, recs, bits, cdfv, S, h, kind, cnt)) break;
+            const int kind = traverse<STATS, OWN>(a.g, bits, S.ray_o, S.ray_d, h, cnt.visits);
+            if (!shade_step<STATS>(a, recs, cdfv, S, h, kind, cnt)) break;
         }
     }
     return tonemap(a.s, S.radiance);
 }
 
-/* Stage records, CDF marginal and (when LDSB) the brick occupancy bits in
- * LDS.  LDSB is a template parameter so the traversal's bit reads compile to
- * LDS instructions rather than generic (flat) loads. */
-template <bool LDSB>
-__device__ __forceinline__ void stage_lds(const TraceArgs& a, uint8_t* smem, MatRec*& recs, float*& cdfv,
-                                          const uint32_t*& bits)
+/* Stage records and CDF marginal in LDS; `end` receives the LDS after them. */
+template <class Rec>
+__device__ __forceinline__ void stage_lds(const TraceArgs& a, uint8_t* smem, Rec*& recs, float*& cdfv, uint8_t*& end)
 {
+    constexpr int W = (int)(sizeof(Rec) / 4), WS = (int)(sizeof(MatRec) / 4);
     uint32_t* w = (uint32_t*)smem;
     const uint32_t* src = (const uint32_t*)a.recs;
-    for (int i = threadIdx.x; i < (int)(256 * sizeof(MatRec) / 4); i += blockDim.x) w[i] = src[i];
-    recs = (MatRec*)smem;
-    float* cv = (float*)(smem + 256 * sizeof(MatRec));
+    for (int i = threadIdx.x; i < 256 * W; i += blockDim.x) w[i] = src[i / W * WS + i % W];
+    recs = (Rec*)smem;
+    float* cv = (float*)(smem + 256 * sizeof(Rec));
     if (a.e.use_image) {
         for (int i = threadIdx.x; i < a.e.cv_n; i += blockDim.x) cv[i] = a.e.cdfv[i];
     }
     cdfv = cv;
-    if (LDSB) {
-        uint32_t* sb = (uint32_t*)(smem + 256 * sizeof(MatRec) + a.cdfv_lds_bytes);
-        for (uint32_t i = threadIdx.x; i < a.g.bit_words_p; i += blockDim.x) sb[i] = a.g.bitsp[i];
-        bits = sb;
-    } else {
-        bits = a.g.bitsp;
-    }
-    __syncthreads();
+    end = (uint8_t*)cv + a.cdfv_lds_bytes;
 }
 
+/* LDSB: the block bits are staged in LDS, those of the grid's own blocks (rows
+ * and layers of padding would take 8 to 11 % more, which at some sizes is a
+ * workgroup a CU: 320^3 at 640x480, two passes, 3.09 ms against 2.91).  A
+ * template parameter so that the traversal's bit reads compile to LDS
+ * instructions rather than generic (flat) loads. */
 template <bool STATS, bool LDSB>
 __global__ __launch_bounds__(256) void render_kernel(TraceArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem[];
-    MatRec* recs;
+    MatBase* recs;
     float* cdfv;
-    const uint32_t* bits;
-    stage_lds<LDSB>(a, smem, recs, cdfv, bits);
+    uint8_t* end;
+    stage_lds(a, smem, recs, cdfv, end);
+    const uint32_t* bits = a.g.bitsp;
+    if (LDSB) {
+        uint32_t* sb = (uint32_t*)end;
+        for (uint32_t i = threadIdx.x; i < a.g.bit_words; i += blockDim.x) sb[i] = a.g.bits[i];
+        bits = sb;
+    }
+    __syncthreads();
     const int lane = threadIdx.x & 63;
     Counters cnt = { 0, 0, 0, 0, 0, 0 };
     uint64_t tot[6] = { 0, 0, 0, 0, 0, 0 };
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) void render_kernel(TraceArgs a)
             for (uint32_t k = 0; k < a.count; ++k) {
                 const uint32_t n = a.n0 + k;
                 const uint32_t rf = n < a.rng_frame_max ? n : a.rng_frame_max;
-                const f3 c = trace_sample<STATS>(a, recs, bits, cdfv, px, py, rf, cnt);
+                const f3 c = trace_sample<STATS, LDSB>(a, recs, bits, cdfv, px, py, rf, cnt);
                 /* accumulation.fs:17, one pass at a time (the running mean
                  * stays in memory between passes, as the ping-pong textures do) */
                 const float fn = (float)n, fn1 = (float)(n + 1u);
@@ -672,7 +674,7 @@ __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r
     /* with no finite distance the ray never moves: its start voxel decides */
     const bool stuck = D.disx != D.disx && D.disy != D.disy && D.disz != D.disz;
     uint32_t dummy = 0;
-    const int status = D.advance<false>(g, g.bitsp, stuck ? 1 : g.max_steps, dummy);
+    const int status = D.advance<false, false>(g, g.bitsp, stuck ? 1 : g.max_steps, dummy);
     return pack_hit(D.x, D.y, D.z, status == 1 ? KIND_VOXEL : (D.y < 0 ? KIND_GROUND : KIND_MISS));
 }
 
@@ -872,8 +874,11 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
     extern __shared__ __align__(16) uint8_t smem[];
     MatRec* recs0 = nullptr;
     float* cdfv0 = nullptr;
-    const uint32_t* bits0 = nullptr;
-    if (!BATCH) stage_lds<false>(a0, smem, recs0, cdfv0, bits0);
+    if (!BATCH) {
+        uint8_t* end;
+        stage_lds(a0, smem, recs0, cdfv0, end);
+        __syncthreads();
+    }
     float4* qao = sel ? P.qa0 : P.qa1;
     float2* qbo = sel ? P.qb0 : P.qb1;
     uint32_t* qto = BATCH ? (sel ? P.qt0 : P.qt1) : nullptr;
@@ -938,7 +943,6 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
             const TraceArgs& a = BATCH ? B.tab[sid] : a0;
             const MatRec* recs = BATCH ? a.recs : recs0;
             const float* cdfv = BATCH ? a.e.cdfv : cdfv0;
-            const uint32_t* bits = BATCH ? a.g.bitsp : bits0;
             const uint32_t slot1 = CACHE ? me.w : 0u;   /* training slot + 1 */
             Hit h;
             h.steps = 0;
@@ -961,9 +965,9 @@ __global__ __launch_bounds__(WF_SHADE_THREADS) __attribute__((amdgpu_waves_per_e
             const int kind = unpack_hit(hv, h);
             /* the hit voxel's material slot is read here, where occupancy
              * hides the load, not by the traversal (ground: slot 0) */
-            h.slot = kind == KIND_VOXEL ? fetch_slot(a.g, bits, h.x, h.y, h.z) : 0u;
+            h.slot = kind == KIND_VOXEL ? fetch_slot(a.g, h.x, h.y, h.z) : 0u;
             bool vrec = false;
-            const int st = shade_step<STATS, CACHE>(a, recs, bits, cdfv, S, h, kind, cnt,
+            const int st = shade_step<STATS, CACHE>(a, recs, cdfv, S, h, kind, cnt,
                                                     slot1 ? C.train_bounce : C.cache_bounce, vraw, &vrec);
             /* a training path records its vertices, except the one where it
              * ends into the cache (whose target would be the prediction) */
@@ -1240,7 +1244,7 @@ __global__ __launch_bounds__(256) void light_table_kernel(GridView g, int4* __re
         idx -= z * dz;
         const int32_t y = idx / dy;
         idx -= y * dy;
-        out[i] = make_int4(idx, y, z, (int32_t)fetch_slot(g, g.bitsp, idx, y, z));
+        out[i] = make_int4(idx, y, z, (int32_t)fetch_slot(g, idx, y, z));
     }
 }
 
@@ -1339,6 +1343,34 @@ __global__ __launch_bounds__(64) void trace_rays_kernel(TraceArgs a, int32_t n, 
     }
 }
 
+/* Before a launch of the megakernel: the tile counter and the statistics, and
+ * (words > 0) the bits of the grid's own blocks out of the padded ones, a word
+ * a thread. */
+__global__ __launch_bounds__(256) void render_setup_kernel(GridView g, uint32_t* bits, uint32_t words, uint32_t* c,
+                                                           unsigned long long* stats)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i == 0u) *c = 0u;
+    if (stats && i < 6u) stats[i] = 0ull;
+    if (i >= words) return;
+    const uint32_t kx = ((uint32_t)g.nx + 3u) / 4u, ky = ((uint32_t)g.ny + 3u) / 4u, kz = ((uint32_t)g.nz + 3u) / 4u;
+    const uint32_t row = 32u * i / kx;
+    uint32_t x = 32u * i - row * kx, y = row % ky, z = row / ky, v = 0u;
+    for (uint32_t have = 0u; have < 32u && z < kz;) {
+        /* the part of a row that the word holds */
+        const uint32_t n = kx - x < 32u - have ? kx - x : 32u - have;
+        const uint32_t p = x + 1u + g.bxp * (y + 1u + g.byp * (z + 1u)), sh = p & 31u;
+        uint32_t part = g.bitsp[p >> 5] >> sh;
+        if (sh + n > 32u) part |= g.bitsp[(p >> 5) + 1u] << (32u - sh);
+        if (n < 32u) part &= (1u << n) - 1u;
+        v |= part << have;
+        have += n;
+        x = 0u;
+        if (++y == ky) y = 0u, ++z;
+    }
+    bits[i] = v;
+}
+
 __global__ void reset_counter_kernel(uint32_t* c, unsigned long long* stats)
 {
     if (threadIdx.x == 0) *c = 0u;
@@ -1373,7 +1405,7 @@ __global__ void device_math_kernel(int32_t fn, int32_t n, const float* a, const 
 /* ---- launchers ------------------------------------------------------------------ */
 size_t render_lds_bytes(const TraceArgs& a)
 {
-    return 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes + (a.lds_bits ? (size_t)a.g.bit_words_p * 4u : 0u);
+    return 256 * sizeof(MatBase) + (size_t)a.cdfv_lds_bytes + (a.lds_bits ? (size_t)a.g.bit_words * 4u : 0u);
 }
 
 static void (*render_ptr(bool stats, bool ldsb))(TraceArgs)
@@ -1416,6 +1448,13 @@ hipError_t launch_trace_rays(const TraceArgs& a, int32_t n, const float* o, cons
 hipError_t launch_reset_counter(uint32_t* c, unsigned long long* stats, hipStream_t s)
 {
     reset_counter_kernel<<<1, 64, 0, s>>>(c, stats);
+    return hipGetLastError();
+}
+
+hipError_t launch_render_setup(const GridView& g, uint32_t* bits, uint32_t* c, unsigned long long* stats, hipStream_t s)
+{
+    const uint32_t words = bits ? g.bit_words : 0u;
+    render_setup_kernel<<<words / 256u + 1u, 256, 0, s>>>(g, bits, words, c, stats);
     return hipGetLastError();
 }
 
