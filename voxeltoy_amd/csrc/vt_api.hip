@@ -11,6 +11,7 @@
 #include "vt_kernels.h"
 #include "vt_cache.h"
 #include "vt_staging.h"
+#include "vt_work.h"
 #include "../host/vt_host_algos.h"
 
 #include <algorithm>
@@ -58,7 +59,6 @@ int no_throw(F&& f) noexcept
 #define VT_DEFAULT_DDA_BUDGET 32
 #define VT_DEFAULT_REFILL_MIN 8
 #define VT_DEFAULT_REFILL_CHUNK 256
-#define VT_WORK_KEEP (256ull << 20)  /* workspace kept on a context */
 /* (x, y) columns above which the voxelizer gives a triangle a whole wave */
 #define VT_VOX_BIG_AREA 32
 /* paths from which a scene of a batch gets its own launches */
@@ -76,6 +76,19 @@ int no_throw(F&& f) noexcept
             return fail(VT_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));  \
         }                                                                                 \
     } while (0)
+
+constexpr int VT_MAX_DEVICES = 64;
+vt::DeviceWork g_work[VT_MAX_DEVICES];
+
+/* hipMalloc on the current device, with the memory of its kept workspace if
+ * there is no other. */
+template <typename T>
+hipError_t dmalloc(T** p, size_t bytes)
+{
+    int device = 0;
+    const hipError_t e = hipGetDevice(&device);
+    return e != hipSuccess ? e : device < VT_MAX_DEVICES ? g_work[device].alloc((void**)p, bytes) : hipMalloc(p, bytes);
+}
 
 template <typename T>
 void dfree(T*& p)
@@ -114,7 +127,6 @@ constexpr size_t VT_NOALLOC_D = (size_t)VT_NOALLOC_MAX_RAYS * 12u;
 constexpr size_t VT_NOALLOC_R = (size_t)VT_NOALLOC_MAX_RAYS * 24u;
 constexpr size_t VT_NOALLOC_FLAG = (size_t)VT_NOALLOC_MAX_RAYS * 56u;
 constexpr size_t VT_NOALLOC_BYTES = VT_NOALLOC_FLAG + 64u;
-constexpr int VT_MAX_DEVICES = 64;
 static_assert(VT_NOALLOC_R % 256 == 0, "record staging must stay aligned");
 
 struct RayStage {
@@ -132,7 +144,7 @@ int stage_make(RayStage& st)
     if (st.host) return VT_OK;
     void* host = nullptr;
     const uint32_t zero = 0;
-    hipError_t e = st.count ? hipSuccess : hipMalloc(&st.count, sizeof(uint32_t));
+    hipError_t e = st.count ? hipSuccess : dmalloc(&st.count, sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemcpy(st.count, &zero, sizeof(zero), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipHostMalloc(&host, VT_NOALLOC_BYTES, hipHostMallocCoherent);
     if (e != hipSuccess) {
@@ -163,7 +175,9 @@ void ring_join(int device)
 void ring_leave(int device)
 {
     std::lock_guard<std::mutex> lk(g_ring_lock);
-    if (--g_ring_users[device] == 0) g_ring[device]->release();
+    if (--g_ring_users[device] != 0) return;
+    g_ring[device]->release();
+    (void)g_work[device].give_back();
 }
 }  // namespace
 
@@ -208,9 +222,6 @@ struct vt_context {
     int32_t n_emissive = 0;
     int4* d_lights = nullptr;       /* emissive entries decoded: x, y, z, slot */
     int32_t emissive_cap = 0, lights_cap = 0;   /* entries allocated */
-    std::mutex work_lock;           /* the kept workspace is one call's at a time (WorkSpace) */
-    uint8_t* d_work = nullptr;
-    size_t work_cap = 0;
     std::vector<float> mat;
     int32_t slot_off[256];
     int32_t n_slots = 0;            /* slots 1..n_slots used */
@@ -289,7 +300,7 @@ int upload_records(vt_context* c)
     vt::MatRec recs[256];
     recs[0] = decode(c->mat, 0);
     for (int s = 1; s < 256; ++s) recs[s] = decode(c->mat, c->slot_off[s] < 0 ? 0 : c->slot_off[s]);
-    if (!c->d_recs) VT_HIP(hipMalloc(&c->d_recs, sizeof(recs)));
+    if (!c->d_recs) VT_HIP(dmalloc(&c->d_recs, sizeof(recs)));
     VT_HIP(hipMemcpyAsync(c->d_recs, recs, sizeof(recs), hipMemcpyHostToDevice, c->stream));
     VT_HIP(hipStreamSynchronize(c->stream));
     return VT_OK;
@@ -306,7 +317,7 @@ int refresh_codes(vt_context* c)
         if (c->lights_cap < c->n_emissive) {
             dfree(c->d_lights);
             c->lights_cap = 0;
-            VT_HIP(hipMalloc(&c->d_lights, (size_t)c->n_emissive * 16u));
+            VT_HIP(dmalloc(&c->d_lights, (size_t)c->n_emissive * 16u));
             c->lights_cap = c->n_emissive;
         }
         const vt::TraceArgs a = trace_args(c);
@@ -317,33 +328,6 @@ int refresh_codes(vt_context* c)
 
 vt::BlockLevels block_levels(const vt_context* c) { return { c->d_occp, c->d_occr, c->d_bitsp }; }
 
-/* Device workspace of one call, which waits for its work before it returns.
- * The context keeps up to VT_WORK_KEEP bytes for the next call; a larger one,
- * or one of a second thread that meets the context busy, is allocated for the
- * call and freed with it. */
-struct WorkSpace {
-    uint8_t* p = nullptr;
-    int take(vt_context* c, size_t bytes)
-    {
-        if (bytes <= VT_WORK_KEEP) lock = std::unique_lock<std::mutex>(c->work_lock, std::try_to_lock);
-        if (!lock.owns_lock()) {
-            VT_HIP(hipMalloc(&own.p, bytes));
-            p = own.p;
-            return VT_OK;
-        }
-        if (c->work_cap < bytes) {
-            dfree(c->d_work);
-            c->work_cap = 0;
-            VT_HIP(hipMalloc(&c->d_work, bytes));
-            c->work_cap = bytes;
-        }
-        p = c->d_work;
-        return VT_OK;
-    }
-private:
-    std::unique_lock<std::mutex> lock;
-    DevTmp<uint8_t> own;
-};
 size_t aligned(size_t bytes) { return (bytes + 255u) & ~(size_t)255u; }
 
 /* Reference bounds (renderer.cpp:845-850): cubic voxels, longest axis 1000. */
@@ -390,15 +374,15 @@ int common_volume_setup(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const
     for (int i = 0; i < 256; ++i) c->slot_off[i] = -1;
     c->n_slots = 0;
     if (!keep) {
-        VT_HIP(hipMalloc(&c->d_bricks, d.n_bricks * 512u));
+        VT_HIP(dmalloc(&c->d_bricks, d.n_bricks * 512u));
         const uint64_t np = d.n_padded;
-        VT_HIP(hipMalloc(&c->d_occp, np * 8u));
+        VT_HIP(dmalloc(&c->d_occp, np * 8u));
         c->bit_words_p = (uint32_t)((np + 127) / 128 * 4);      /* whole uint4 */
-        VT_HIP(hipMalloc(&c->d_bitsp, (size_t)c->bit_words_p * 4u));
+        VT_HIP(dmalloc(&c->d_bitsp, (size_t)c->bit_words_p * 4u));
         if (nx <= VT_PACKED_MAX_EXTENT && ny <= VT_PACKED_MAX_EXTENT && nz <= VT_PACKED_MAX_EXTENT)
-            VT_HIP(hipMalloc(&c->d_occr, np * 8u));
+            VT_HIP(dmalloc(&c->d_occr, np * 8u));
         c->cells = vt::cell_layout(d);
-        VT_HIP(hipMalloc(&c->d_codes, (size_t)c->cells.words * 4u));
+        VT_HIP(dmalloc(&c->d_codes, (size_t)c->cells.words * 4u));
         /* what the conversions never write: the bricks' voxels outside the
          * grid and the codes' padding */
         VT_HIP(vt::launch_fill_u8((uint8_t*)c->d_codes, (uint64_t)c->cells.words * 4u, 0, c->stream));
@@ -414,7 +398,7 @@ int upload_emissive(vt_context* c, const int32_t* emissive, int32_t n)
     if (c->emissive_cap < n) {
         dfree(c->d_emissive);
         c->emissive_cap = 0;
-        VT_HIP(hipMalloc(&c->d_emissive, (size_t)n * 4u));
+        VT_HIP(dmalloc(&c->d_emissive, (size_t)n * 4u));
         c->emissive_cap = n;
     }
     VT_HIP(to_device(c, c->d_emissive, emissive, (size_t)n * 4u));
@@ -549,16 +533,16 @@ int alloc_paths(vt::WfPaths& P, uint64_t& alloc, uint64_t slots)
     free_paths(P, alloc);
     const size_t n = (size_t)vt::queue_positions(slots);
     for (vt::PathBuf& B : P.s) {
-        VT_HIP(hipMalloc(&B.o, n * 16)); VT_HIP(hipMalloc(&B.nd, n * 16)); VT_HIP(hipMalloc(&B.thr, n * 16));
-        VT_HIP(hipMalloc(&B.rad, n * 16)); VT_HIP(hipMalloc(&B.dir, n * 16)); VT_HIP(hipMalloc(&B.fac, n * 16));
-        VT_HIP(hipMalloc(&B.meta, n * 16)); VT_HIP(hipMalloc(&B.rng, n * 8));
+        VT_HIP(dmalloc(&B.o, n * 16)); VT_HIP(dmalloc(&B.nd, n * 16)); VT_HIP(dmalloc(&B.thr, n * 16));
+        VT_HIP(dmalloc(&B.rad, n * 16)); VT_HIP(dmalloc(&B.dir, n * 16)); VT_HIP(dmalloc(&B.fac, n * 16));
+        VT_HIP(dmalloc(&B.meta, n * 16)); VT_HIP(dmalloc(&B.rng, n * 8));
     }
     /* queues and hits: two entries (shadow and continuation ray) per path */
-    VT_HIP(hipMalloc(&P.hit, 2 * n * 8));
-    VT_HIP(hipMalloc(&P.smp, n * 16));
-    VT_HIP(hipMalloc(&P.qa0, 2 * n * 16)); VT_HIP(hipMalloc(&P.qb0, 2 * n * 8)); VT_HIP(hipMalloc(&P.qt0, 2 * n * 4));
-    VT_HIP(hipMalloc(&P.qa1, 2 * n * 16)); VT_HIP(hipMalloc(&P.qb1, 2 * n * 8)); VT_HIP(hipMalloc(&P.qt1, 2 * n * 4));
-    VT_HIP(hipMalloc(&P.cnt, 2 * vt::QUEUE_PARTS * vt::QUEUE_COUNT_STRIDE * 4));
+    VT_HIP(dmalloc(&P.hit, 2 * n * 8));
+    VT_HIP(dmalloc(&P.smp, n * 16));
+    VT_HIP(dmalloc(&P.qa0, 2 * n * 16)); VT_HIP(dmalloc(&P.qb0, 2 * n * 8)); VT_HIP(dmalloc(&P.qt0, 2 * n * 4));
+    VT_HIP(dmalloc(&P.qa1, 2 * n * 16)); VT_HIP(dmalloc(&P.qb1, 2 * n * 8)); VT_HIP(dmalloc(&P.qt1, 2 * n * 4));
+    VT_HIP(dmalloc(&P.cnt, 2 * vt::QUEUE_PARTS * vt::QUEUE_COUNT_STRIDE * 4));
     P.cap = slots;
     alloc = slots;
     return VT_OK;
@@ -594,7 +578,7 @@ int vt_create(int device, vt_context** out)
         c->lds_limit = prop.sharedMemPerBlock;
         if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
-            hipMalloc(&c->d_tile, 4) != hipSuccess || hipMalloc(&c->d_stats, 6 * sizeof(unsigned long long)) != hipSuccess) {
+            dmalloc(&c->d_tile, 4) != hipSuccess || dmalloc(&c->d_stats, 6 * sizeof(unsigned long long)) != hipSuccess) {
             vt_destroy(c);
             return fail(VT_ERR_HIP, "context resource creation failed");
         }
@@ -624,7 +608,7 @@ void vt_destroy(vt_context* c)
     while (!c->batches.empty()) batch_release(c->batches.back());
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    dfree(c->d_bricks); dfree(c->d_occp); dfree(c->d_bitsp); dfree(c->d_bits); dfree(c->d_occr); dfree(c->d_codes); dfree(c->d_work); dfree(c->d_emissive); dfree(c->d_lights); dfree(c->d_recs);
+    dfree(c->d_bricks); dfree(c->d_occp); dfree(c->d_bitsp); dfree(c->d_bits); dfree(c->d_occr); dfree(c->d_codes); dfree(c->d_emissive); dfree(c->d_lights); dfree(c->d_recs);
     dfree(c->d_img); dfree(c->d_quad); dfree(c->d_cdfu); dfree(c->d_cdfv);
     dfree(c->d_accum); dfree(c->d_sum64); dfree(c->d_tile); dfree(c->d_stats);
     free_wavefront(c);
@@ -663,11 +647,10 @@ int vt_set_volume(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const int32
         const int64_t nvox = (int64_t)nx * ny * nz;
         const size_t lut_n = (size_t)std::max(mat_size, 1);
         /* workspace: dense grid, offsets in use, LUT, {first bad voxel, first bad emissive entry} */
-        WorkSpace ws;
+        vt::WorkSpace ws(g_work[c->device], c->stream);
         const size_t used_at = aligned((size_t)nvox * 4u), bad_at = used_at + aligned(lut_n), lut_at = bad_at + 256;
-        r = ws.take(c, lut_at + lut_n);
-        if (r != VT_OK) return r;
-        uint8_t* const work = ws.p;
+        VT_HIP(ws.take(lut_at + lut_n));
+        uint8_t* const work = ws.p();
         const int32_t* d_dense = (const int32_t*)work;
         unsigned long long* d_bad = (unsigned long long*)(work + bad_at);
         VT_HIP(to_device(c, work, offsets, (size_t)nvox * 4u));
@@ -702,7 +685,9 @@ int vt_set_volume(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const int32
         if (r != VT_OK) return r;
         VT_HIP(to_device(c, work + lut_at, lut.data(), lut_n));
         VT_HIP(vt::launch_blocks_from_offsets(c->dims, d_dense, work + lut_at, c->d_bricks, block_levels(c), c->stream));
-        return finish_volume(c, n_emissive);
+        r = finish_volume(c, n_emissive);
+        if (r == VT_OK) ws.waited();
+        return r;
     });
 }
 
@@ -728,11 +713,10 @@ int vt_set_volume_u8(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const ui
         }
         c->n_slots = ns;
         const int64_t nvox = (int64_t)nx * ny * nz;
-        WorkSpace ws;
+        vt::WorkSpace ws(g_work[c->device], c->stream);
         const size_t remap_at = aligned((size_t)nvox), bad_at = remap_at + 256;
-        r = ws.take(c, bad_at + 4);
-        if (r != VT_OK) return r;
-        uint8_t* const work = ws.p;
+        VT_HIP(ws.take(bad_at + 4));
+        uint8_t* const work = ws.p();
         VT_HIP(to_device(c, work, ids, (size_t)nvox));
         VT_HIP(to_device(c, work + remap_at, remap, 256));
         uint32_t bad_entry = 0xffffffffu;
@@ -747,7 +731,9 @@ int vt_set_volume_u8(vt_context* c, int32_t nx, int32_t ny, int32_t nz, const ui
         r = emissive_error(emissive, n_emissive, nvox, bad_entry);
         if (r != VT_OK) return r;
         VT_HIP(vt::launch_blocks_from_ids(c->dims, work, work + remap_at, c->d_bricks, block_levels(c), c->stream));
-        return finish_volume(c, n_emissive);
+        r = finish_volume(c, n_emissive);
+        if (r == VT_OK) ws.waited();
+        return r;
     });
 }
 
@@ -774,14 +760,14 @@ int vt_read_volume(vt_context* c, int32_t* offsets)
         int32_t table[256];
         table[0] = -1;
         for (int s = 1; s < 256; ++s) table[s] = c->slot_off[s];
-        WorkSpace ws;
+        vt::WorkSpace ws(g_work[c->device], c->stream);
         const size_t table_at = aligned((size_t)nvox * 4u);
-        const int r = ws.take(c, table_at + sizeof(table));
-        if (r != VT_OK) return r;
-        uint8_t* const work = ws.p;
+        VT_HIP(ws.take(table_at + sizeof(table)));
+        uint8_t* const work = ws.p();
         VT_HIP(to_device(c, work + table_at, table, sizeof(table)));
         VT_HIP(vt::launch_dense_from_bricks(c->dims, c->d_bricks, (const int32_t*)(work + table_at), (int32_t*)work, c->stream));
         VT_HIP(to_host(c, offsets, work, (size_t)nvox * 4u));
+        ws.waited();
         return VT_OK;
     });
 }
@@ -842,10 +828,10 @@ int vt_set_environment(vt_context* c, const vt_environment* env)
         float* cdfv = nullptr;
         if (e.use_image) {
             const size_t ni = (size_t)e.image_w * e.image_h * 3, nu = (size_t)e.cdf_u_w * e.cdf_u_h;
-            hipError_t he = hipMalloc(&img, ni * 4);
-            if (he == hipSuccess) he = hipMalloc(&cdfu, nu * 4);
-            if (he == hipSuccess) he = hipMalloc(&cdfv, (size_t)e.cdf_v_n * 4);
-            if (he == hipSuccess) he = hipMalloc(&quad, (size_t)(e.image_w + 1) * (size_t)(e.image_h + 1) * 64);
+            hipError_t he = dmalloc(&img, ni * 4);
+            if (he == hipSuccess) he = dmalloc(&cdfu, nu * 4);
+            if (he == hipSuccess) he = dmalloc(&cdfv, (size_t)e.cdf_v_n * 4);
+            if (he == hipSuccess) he = dmalloc(&quad, (size_t)(e.image_w + 1) * (size_t)(e.image_h + 1) * 64);
             if (he == hipSuccess) he = to_device(c, img, e.image_rgb, ni * 4);
             if (he == hipSuccess) he = to_device(c, cdfu, e.cdf_u, nu * 4);
             if (he == hipSuccess)
@@ -895,8 +881,8 @@ int vt_set_frame(vt_context* c, int32_t w, int32_t h, int32_t fp64)
         VT_HIP(hipStreamSynchronize(c->stream));
         dfree(c->d_accum); dfree(c->d_sum64);
         c->W = w; c->H = h;
-        VT_HIP(hipMalloc(&c->d_accum, (size_t)w * h * sizeof(float4)));
-        if (fp64) VT_HIP(hipMalloc(&c->d_sum64, (size_t)w * h * 3 * sizeof(double)));
+        VT_HIP(dmalloc(&c->d_accum, (size_t)w * h * sizeof(float4)));
+        if (fp64) VT_HIP(dmalloc(&c->d_sum64, (size_t)w * h * 3 * sizeof(double)));
         return vt_reset_accum(c);
     });
 }
@@ -1072,7 +1058,7 @@ int vt_render(vt_context* c, uint64_t seed, uint32_t n0, uint32_t count, uint32_
                 VT_HIP(hipEventRecord(c->ev1, c->stream));
             }
         } else {
-            if (a.lds_bits && !c->d_bits) VT_HIP(hipMalloc(&c->d_bits, (size_t)a.g.bit_words * 4u));
+            if (a.lds_bits && !c->d_bits) VT_HIP(dmalloc(&c->d_bits, (size_t)a.g.bit_words * 4u));
             a.g.bits = c->d_bits;
             VT_HIP(vt::launch_render_setup(a.g, a.lds_bits ? c->d_bits : nullptr, c->d_tile, a.stats, c->stream));
             const int per_cu = vt::render_blocks_per_cu(a, c->stats_enabled);
@@ -1134,9 +1120,9 @@ int vt_batch_create(vt_context* const* ctxs, int32_t n, vt_batch** out)
         b->h_base.resize(2 * ((size_t)n + 1));
         for (vt_context* c : b->ctxs)
             if (std::find(c->batches.begin(), c->batches.end(), b) == c->batches.end()) c->batches.push_back(b);
-        if (hipMalloc(&b->d_tab, sizeof(vt::TraceArgs) * (size_t)n) != hipSuccess ||
-            hipMalloc(&b->d_base, sizeof(uint64_t) * b->h_base.size()) != hipSuccess ||
-            hipMalloc(&b->d_stats, 6 * sizeof(unsigned long long)) != hipSuccess ||
+        if (dmalloc(&b->d_tab, sizeof(vt::TraceArgs) * (size_t)n) != hipSuccess ||
+            dmalloc(&b->d_base, sizeof(uint64_t) * b->h_base.size()) != hipSuccess ||
+            dmalloc(&b->d_stats, 6 * sizeof(unsigned long long)) != hipSuccess ||
             hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess ||
             hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -1226,8 +1212,8 @@ int vt_autotune_batch(vt_batch* b, const uint64_t* seeds, const uint32_t* n0, co
             Saved v = { c, nullptr, nullptr, (size_t)c->W * c->H * sizeof(float4),
                         c->d_sum64 ? (size_t)c->W * c->H * 3 * sizeof(double) : 0 };
             hipError_t he = hipStreamSynchronize(c->stream);
-            if (he == hipSuccess) he = hipMalloc(&v.acc, v.acc_b);
-            if (he == hipSuccess && v.sum_b) he = hipMalloc(&v.sum, v.sum_b);
+            if (he == hipSuccess) he = dmalloc(&v.acc, v.acc_b);
+            if (he == hipSuccess && v.sum_b) he = dmalloc(&v.sum, v.sum_b);
             if (he == hipSuccess) he = hipMemcpyAsync(v.acc, c->d_accum, v.acc_b, hipMemcpyDeviceToDevice, c->stream);
             if (he == hipSuccess && v.sum_b) he = hipMemcpyAsync(v.sum, c->d_sum64, v.sum_b, hipMemcpyDeviceToDevice, c->stream);
             saved.push_back(v);
@@ -1559,10 +1545,10 @@ int cache_train_scratch(vt_cache* c, uint32_t batch)
     dfree(c->d_X); dfree(c->d_H); dfree(c->d_DZ); dfree(c->d_DY);
     c->tiles = 0;
     const size_t t16 = (size_t)tiles * 16u;
-    VT_HIP(hipMalloc(&c->d_X, t16 * vt::MLP_IN * 2));
-    VT_HIP(hipMalloc(&c->d_H, t16 * 5 * vt::MLP_W * 2));
-    VT_HIP(hipMalloc(&c->d_DZ, t16 * 5 * vt::MLP_W * 4));
-    VT_HIP(hipMalloc(&c->d_DY, t16 * vt::MLP_OUT * 4));
+    VT_HIP(dmalloc(&c->d_X, t16 * vt::MLP_IN * 2));
+    VT_HIP(dmalloc(&c->d_H, t16 * 5 * vt::MLP_W * 2));
+    VT_HIP(dmalloc(&c->d_DZ, t16 * 5 * vt::MLP_W * 4));
+    VT_HIP(dmalloc(&c->d_DY, t16 * vt::MLP_OUT * 4));
     c->tiles = tiles;
     return VT_OK;
 }
@@ -1574,8 +1560,8 @@ int cache_upload_samples(vt_cache* c, int64_t n, const float* raw, const float* 
     if (n > c->cap) {
         dfree(c->d_raw); dfree(c->d_tgt);
         c->cap = 0;
-        VT_HIP(hipMalloc(&c->d_raw, (size_t)n * vt::MLP_RAW * 4));
-        VT_HIP(hipMalloc(&c->d_tgt, (size_t)n * vt::MLP_OUT * 4));
+        VT_HIP(dmalloc(&c->d_raw, (size_t)n * vt::MLP_RAW * 4));
+        VT_HIP(dmalloc(&c->d_tgt, (size_t)n * vt::MLP_OUT * 4));
         c->cap = n;
     }
     VT_HIP(to_device(c->ctx, c->d_raw, raw, (size_t)n * vt::MLP_RAW * 4));
@@ -1661,14 +1647,14 @@ int vt_cache_create(vt_context* ctx, uint64_t seed, vt_cache** out)
                 return fail(VT_ERR_STATE, "internal error: FP32 weight pack mapping is not invertible");
             }
         }
-        if (hipMalloc(&c->d_params, pb) != hipSuccess || hipMalloc(&c->d_grad, pb) != hipSuccess ||
-            hipMalloc(&c->d_m, pb) != hipSuccess || hipMalloc(&c->d_v, pb) != hipSuccess ||
-            hipMalloc(&c->d_pack, (size_t)vt::MLP_PACK * 2) != hipSuccess ||
-            hipMalloc(&c->d_bias, (size_t)vt::MLP_BIAS * 4) != hipSuccess ||
-            hipMalloc(&c->d_tpack, (size_t)vt::MLP_TPACK * 4) != hipSuccess ||
-            hipMalloc(&c->d_part, (size_t)vt::MLP_GRAD_SPLITS * vt::MLP_N_PARAMS * 4) != hipSuccess ||
-            hipMalloc(&c->d_loss, VT_CACHE_LOSS_SLOTS * 4) != hipSuccess || hipMalloc(&c->d_steps, 4) != hipSuccess ||
-            hipMalloc(&c->d_nsamp, 4) != hipSuccess || hipMalloc(&c->d_tally, 16) != hipSuccess) {
+        if (dmalloc(&c->d_params, pb) != hipSuccess || dmalloc(&c->d_grad, pb) != hipSuccess ||
+            dmalloc(&c->d_m, pb) != hipSuccess || dmalloc(&c->d_v, pb) != hipSuccess ||
+            dmalloc(&c->d_pack, (size_t)vt::MLP_PACK * 2) != hipSuccess ||
+            dmalloc(&c->d_bias, (size_t)vt::MLP_BIAS * 4) != hipSuccess ||
+            dmalloc(&c->d_tpack, (size_t)vt::MLP_TPACK * 4) != hipSuccess ||
+            dmalloc(&c->d_part, (size_t)vt::MLP_GRAD_SPLITS * vt::MLP_N_PARAMS * 4) != hipSuccess ||
+            dmalloc(&c->d_loss, VT_CACHE_LOSS_SLOTS * 4) != hipSuccess || dmalloc(&c->d_steps, 4) != hipSuccess ||
+            dmalloc(&c->d_nsamp, 4) != hipSuccess || dmalloc(&c->d_tally, 16) != hipSuccess) {
             vt_cache_destroy(c);
             return fail(VT_ERR_HIP, "cache allocation failed");
         }
@@ -1770,8 +1756,8 @@ int vt_cache_infer(vt_cache* c, int64_t n, const float* raw, float* out)
         if (n > c->icap) {
             dfree(c->d_iraw); dfree(c->d_iout);
             c->icap = 0;
-            VT_HIP(hipMalloc(&c->d_iraw, (size_t)n * vt::MLP_RAW * 4));
-            VT_HIP(hipMalloc(&c->d_iout, (size_t)n * vt::MLP_OUT * 4));
+            VT_HIP(dmalloc(&c->d_iraw, (size_t)n * vt::MLP_RAW * 4));
+            VT_HIP(dmalloc(&c->d_iout, (size_t)n * vt::MLP_OUT * 4));
             c->icap = n;
         }
         VT_HIP(to_device(c->ctx, c->d_iraw, raw, (size_t)n * vt::MLP_RAW * 4));
@@ -1824,22 +1810,22 @@ int vt_render_cached(vt_context* c, vt_cache* k, uint64_t seed, uint32_t n0, uin
         if (k->qcap < WH) {
             dfree(k->d_qraw); dfree(k->d_qout); dfree(k->d_qmeta); dfree(k->d_qrad); dfree(k->d_qthr);
             k->qcap = 0;
-            VT_HIP(hipMalloc(&k->d_qraw, WH * 12 * 4));
-            VT_HIP(hipMalloc(&k->d_qout, WH * 3 * 4));
-            VT_HIP(hipMalloc(&k->d_qmeta, WH * 16));
-            VT_HIP(hipMalloc(&k->d_qrad, WH * 16));
-            VT_HIP(hipMalloc(&k->d_qthr, WH * 16));
+            VT_HIP(dmalloc(&k->d_qraw, WH * 12 * 4));
+            VT_HIP(dmalloc(&k->d_qout, WH * 3 * 4));
+            VT_HIP(dmalloc(&k->d_qmeta, WH * 16));
+            VT_HIP(dmalloc(&k->d_qrad, WH * 16));
+            VT_HIP(dmalloc(&k->d_qthr, WH * 16));
             k->qcap = WH;
         }
-        if (!k->d_counts) VT_HIP(hipMalloc(&k->d_counts, 16));
+        if (!k->d_counts) VT_HIP(dmalloc(&k->d_counts, 16));
         const uint32_t maxv = (uint32_t)std::max(1, c->st.max_bounces);
         const uint32_t stride = train_paths ? (uint32_t)std::max<uint64_t>(1, WH / train_paths) : (uint32_t)WH + 1u;
         const uint64_t slots = train_paths ? (WH + stride - 1) / stride : 0;
         if (k->vcap < slots * maxv || k->vslots < slots) {
             dfree(k->d_vrec); dfree(k->d_vrec_n);
             k->vcap = k->vslots = 0;
-            VT_HIP(hipMalloc(&k->d_vrec, std::max<uint64_t>(1, slots * maxv) * 18 * 4));
-            VT_HIP(hipMalloc(&k->d_vrec_n, std::max<uint64_t>(1, slots) * 4));
+            VT_HIP(dmalloc(&k->d_vrec, std::max<uint64_t>(1, slots * maxv) * 18 * 4));
+            VT_HIP(dmalloc(&k->d_vrec_n, std::max<uint64_t>(1, slots) * 4));
             k->vcap = slots * maxv;
             k->vslots = slots;
         }
@@ -1847,8 +1833,8 @@ int vt_render_cached(vt_context* c, vt_cache* k, uint64_t seed, uint32_t n0, uin
         if (k->scap < scap) {
             dfree(k->d_sraw); dfree(k->d_stgt);
             k->scap = 0;
-            VT_HIP(hipMalloc(&k->d_sraw, scap * 12 * 4));
-            VT_HIP(hipMalloc(&k->d_stgt, scap * 3 * 4));
+            VT_HIP(dmalloc(&k->d_sraw, scap * 12 * 4));
+            VT_HIP(dmalloc(&k->d_stgt, scap * 3 * 4));
             k->scap = scap;
         }
         if (scap > 0xffffffffull) return fail(VT_ERR_LIMIT, "too many training samples per pass");
@@ -1950,8 +1936,8 @@ int vt_autotune(vt_context* c, uint32_t passes, vt_tuning* out)
         DevTmp<void> save_acc;
         DevTmp<void> save_sum;
         {
-            hipError_t he = hipMalloc(&save_acc.p, acc_bytes);
-            if (he == hipSuccess && sum_bytes) he = hipMalloc(&save_sum.p, sum_bytes);
+            hipError_t he = dmalloc(&save_acc.p, acc_bytes);
+            if (he == hipSuccess && sum_bytes) he = dmalloc(&save_sum.p, sum_bytes);
             if (he == hipSuccess)
                 he = hipMemcpyAsync(save_acc.p, c->d_accum, acc_bytes, hipMemcpyDeviceToDevice, c->stream);
             if (he == hipSuccess && sum_bytes)
@@ -2101,12 +2087,12 @@ int vt_trace_first_hit(vt_context* c, uint64_t seed, uint32_t frame, int32_t* re
         vt::TraceArgs a = trace_args(c);
         a.seed = seed; a.n0 = frame;
         const size_t bytes = (size_t)c->W * c->H * 8 * 4;
-        WorkSpace ws;
-        const int r = ws.take(c, bytes);
-        if (r != VT_OK) return r;
-        uint8_t* const work = ws.p;
+        vt::WorkSpace ws(g_work[c->device], c->stream);
+        VT_HIP(ws.take(bytes));
+        uint8_t* const work = ws.p();
         VT_HIP(vt::launch_first_hit(a, (int32_t*)work, c->stream));
         VT_HIP(to_host(c, rec, work, bytes));
+        ws.waited();
         return VT_OK;
     });
 }
@@ -2149,16 +2135,16 @@ int vt_trace_rays(vt_context* c, int32_t n, const float* o, const float* dir, in
             if (lk.owns_lock()) return trace_rays_staged(c, st, n, o, dir, rec);
         }
         vt::TraceArgs a = trace_args(c);
-        WorkSpace ws;
+        vt::WorkSpace ws(g_work[c->device], c->stream);
         const size_t dir_at = aligned((size_t)n * 12), rec_at = 2 * dir_at;
-        const int r = ws.take(c, rec_at + (size_t)n * 32);
-        if (r != VT_OK) return r;
-        uint8_t* const work = ws.p;
+        VT_HIP(ws.take(rec_at + (size_t)n * 32));
+        uint8_t* const work = ws.p();
         VT_HIP(to_device(c, work, o, (size_t)n * 12));
         VT_HIP(to_device(c, work + dir_at, dir, (size_t)n * 12));
         VT_HIP(vt::launch_trace_rays(a, n, (const float*)work, (const float*)(work + dir_at), (int32_t*)(work + rec_at),
                                      nullptr, nullptr, 0u, c->stream));
         VT_HIP(to_host(c, rec, work + rec_at, (size_t)n * 32));
+        ws.waited();
         return VT_OK;
     });
 }
@@ -2216,14 +2202,11 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
         const int64_t nvox = (int64_t)c->dims.nx * c->dims.ny * c->dims.nz;
         /* workspace: vertices, indices, the list of large triangles (a wave
          * each) and its counter, the dense occupancy */
-        WorkSpace ws;
+        vt::WorkSpace ws(g_work[c->device], c->stream);
         const size_t idx_at = aligned((size_t)nv * 12), big_at = idx_at + aligned((size_t)ntri * 12),
                      occ_at = big_at + aligned(((size_t)ntri + 1) * 4);
-        {
-            const int r = ws.take(c, occ_at + (occupancy ? (size_t)nvox : 0u));
-            if (r != VT_OK) return r;
-        }
-        uint8_t* const work = ws.p;
+        VT_HIP(ws.take(occ_at + (occupancy ? (size_t)nvox : 0u)));
+        uint8_t* const work = ws.p();
         if (ntri > 0) {
             VT_HIP(to_device(c, work, verts, (size_t)nv * 12));
             VT_HIP(to_device(c, work + idx_at, idx, (size_t)ntri * 12));
@@ -2251,6 +2234,7 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
         }
         if (occupancy) VT_HIP(to_host(c, occupancy, work + occ_at, (size_t)nvox));
         VT_HIP(hipStreamSynchronize(c->stream));
+        ws.waited();
         return VT_OK;
     });
 }
@@ -2311,9 +2295,9 @@ int vt_device_math(vt_context* c, int32_t fn, int32_t n, const float* a, const f
         if (n == 0) return VT_OK;
         VT_HIP(hipSetDevice(c->device));
         DevTmp<float> da, db, dout;
-        VT_HIP(hipMalloc(&da.p, (size_t)n * 4));
-        VT_HIP(hipMalloc(&db.p, (size_t)n * 4));
-        VT_HIP(hipMalloc(&dout.p, (size_t)n * 4));
+        VT_HIP(dmalloc(&da.p, (size_t)n * 4));
+        VT_HIP(dmalloc(&db.p, (size_t)n * 4));
+        VT_HIP(dmalloc(&dout.p, (size_t)n * 4));
         VT_HIP(hipMemcpyAsync(da.p, a, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
         VT_HIP(hipMemcpyAsync(db.p, b, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
         VT_HIP(vt::launch_device_math(fn, n, da.p, db.p, dout.p, c->stream));
@@ -2329,8 +2313,8 @@ int vt_copy_probe(vt_context* c, uint64_t bytes, int32_t iters, double* kernel_m
         if (!c || bytes < 16 || bytes % 16 || iters < 1 || !kernel_ms) return fail(VT_ERR_ARG, "bad argument");
         VT_HIP(hipSetDevice(c->device));
         DevTmp<uint8_t> a, b;
-        VT_HIP(hipMalloc(&a.p, bytes));
-        VT_HIP(hipMalloc(&b.p, bytes));
+        VT_HIP(dmalloc(&a.p, bytes));
+        VT_HIP(dmalloc(&b.p, bytes));
         VT_HIP(vt::launch_fill_u8(a.p, bytes, 1, c->stream));
         VT_HIP(vt::launch_copy(a.p, b.p, bytes, c->stream));
         VT_HIP(hipEventRecord(c->ev0, c->stream));
