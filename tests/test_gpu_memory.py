@@ -65,3 +65,16 @@ def test_calls_that_share_the_workspace(vtapi, orc):
     for t in ts:
         t.join(60)
     assert not bad and not any(t.is_alive() for t in ts)
+
+
+def test_vertices_without_triangles_take_no_memory(ctx, vtapi):
+    """More vertices than the device could hold, none of them read."""
+    off = np.full((8, 8, 8), -1, np.int32)
+    off[0] = 0
+    ctx.set_volume(off, np.array([0, 0, 0, 0, .5, .5, .5, 0], np.float32))
+    occ = np.full((8, 8, 8), 7, np.uint8)
+    rc = vtapi.lib().vt_voxelize(ctx._c, np.zeros(3, np.float32), 1 << 40, np.zeros(0, np.uint32), 0,
+                                 np.eye(4, dtype=np.float32).reshape(-1), 0, 0, occ.ctypes.data)
+    assert rc == 0, vtapi.lib().vt_last_error()
+    assert not occ.any()
+    assert np.array_equal(ctx.read_volume(), off)

@@ -2203,7 +2203,7 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
         /* workspace: vertices, indices, the list of large triangles (a wave
          * each) and its counter, the dense occupancy */
         vt::WorkSpace ws(g_work[c->device], c->stream);
-        const size_t idx_at = aligned((size_t)nv * 12), big_at = idx_at + aligned((size_t)ntri * 12),
+        const size_t idx_at = ntri > 0 ? aligned((size_t)nv * 12) : 0, big_at = idx_at + aligned((size_t)ntri * 12),
                      occ_at = big_at + aligned(((size_t)ntri + 1) * 4);
         VT_HIP(ws.take(occ_at + (occupancy ? (size_t)nvox : 0u)));
         uint8_t* const work = ws.p();
