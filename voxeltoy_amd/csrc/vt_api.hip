@@ -505,6 +505,7 @@ vt::TraceArgs trace_args(const vt_context* c)
     a.cdfv_lds_bytes = c->env.use_image ? ((c->env.cdf_v_n * 4 + 15) / 16) * 16 : 0;
     const size_t base = 256 * sizeof(vt::MatBase) + (size_t)a.cdfv_lds_bytes;
     a.lds_bits = (base + (size_t)a.g.bit_words * 4u <= c->lds_limit) ? 1 : 0;
+    a.step = vt::step_march(c->dims) ? 1 : 0;
     a.lds_bits_p = ((size_t)c->bit_words_p * 4u + vt::WF_TAKEN_BYTES <= c->lds_limit) ? 1 : 0;
     a.dda_budget = c->dda_budget;
     a.refill_min = c->refill_min;
@@ -1388,8 +1389,11 @@ int vt_batch_render(vt_batch* b, const uint64_t* seeds, const uint32_t* n0, cons
         B.n = (uint32_t)m;
         B.stats = stats ? b->d_stats : nullptr;
         B.packed = 1;
-        for (size_t k = 0; k < m; ++k)
+        B.step = 0;
+        for (size_t k = 0; k < m; ++k) {
             if (!b->h_tab[k].g.occr) B.packed = 0;
+            if (b->h_tab[k].step) B.step = 1;
+        }
         vt::TraceArgs a0 = trace_args(L);
         if (b->dda_budget) a0.dda_budget = b->dda_budget;
         if (b->refill_min) a0.refill_min = b->refill_min;
@@ -1418,7 +1422,7 @@ int vt_batch_render(vt_batch* b, const uint64_t* seeds, const uint32_t* n0, cons
             std::vector<uint64_t> key = { (uint64_t)m, total, pixels, b->wf.cap, (uint64_t)max_bounces,
                                           (uint64_t)stats, (uint64_t)a0.dda_budget, (uint64_t)a0.refill_min,
                                           (uint64_t)a0.refill_chunk, (uint64_t)(uintptr_t)b->wf.s[0].o,
-                                          (uint64_t)B.packed };
+                                          (uint64_t)B.packed, (uint64_t)B.step };
             key.insert(key.end(), merged.begin(), merged.end());
             for (const auto& sa : solo) {
                 const vt_context* c = b->ctxs[sa.first];

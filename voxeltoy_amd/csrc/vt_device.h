@@ -14,8 +14,9 @@
  * (set when any voxel of the block is occupied or outside the grid), staged in
  * LDS when it fits, and one 64-bit voxel mask per block (bit x + 4y + 16z for
  * local voxel (x, y, z)).  Entering a block costs one bit test; only non-empty
- * blocks load their 8-byte mask.  Renders without statistics read codes of
- * empty cubes instead of the bits (the jump march, vt_jump.h).
+ * blocks load their 8-byte mask.  Renders without statistics, unless the grid is
+ * a long one, read codes of empty cubes instead of the bits (the jump march,
+ * vt_jump.h).
  *
  * The traversal replays the reference 3D-DDA (src/shaders/shared/dda.h:7-100)
  * step by step: `dis` is a running FP32 sum, so empty space skips the loads

@@ -24,7 +24,8 @@ struct TraceArgs {
     uint32_t* tile_counter;
     int32_t tiles_x, n_tiles;
     int32_t lds_bits;            /* stage occupancy bits in LDS */
-    int32_t lds_bits_p;          /* wavefront traversal with statistics: stage the padded block bits in LDS */
+    int32_t step;                /* wavefront traversal marches step by step (step_march) */
+    int32_t lds_bits_p;          /* step-by-step wavefront traversal: stage the padded block bits in LDS */
     int32_t cdfv_lds_bytes;
     int32_t dda_budget;          /* wavefront traversal: jumps or DDA steps between refill checks */
     int32_t refill_min;          /* wavefront traversal: idle lanes that trigger a refill */
@@ -138,6 +139,7 @@ struct BatchTable {
     uint32_t n;
     unsigned long long* stats;   /* 6 counters or null */
     int32_t packed;              /* every scene has packed-march masks (GridView::occr) */
+    int32_t step;                /* a scene marches step by step, so all do */
 };
 
 /* Radiance-cache rendering of one pass: paths that are not training paths

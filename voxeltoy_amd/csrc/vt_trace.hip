@@ -629,14 +629,14 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
 }
 
 /* Persistent traversal: each lane marches its ray a few jumps (a.dda_budget
- * DDA steps with STATS) at a time; whenever enough lanes of the wave are idle
+ * DDA steps with STEP) at a time; whenever enough lanes of the wave are idle
  * they take the next entries of the workgroup's list, so lanes stay busy until
  * the list is used up instead of idling behind the longest ray of their wave.
  * The queue, from its end, is dealt to the workgroups in segments of
  * a.refill_chunk entries in turn, and a workgroup's waves share its segments
  * through a counter in LDS: a counter for the whole queue, hit from all XCDs,
  * takes about 13 ns an update.  Workgroups of 1024 threads share one
- * LDS copy of the empty-cube codes (of the block occupancy bits with STATS).
+ * LDS copy of the empty-cube codes (of the block occupancy bits with STEP).
  *
  * Bound by vector issue (0.85 wave-instructions a CU and cycle, 48 % of the
  * lanes at work, full-shading scene) and, in the later launches, by the chain
@@ -649,11 +649,11 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * with one mask in it; one pass at 1920x1080: 3.15, 2.4, 1.1, 0.81, 0.78, 0.65,
  * 0.64 ms; 512^3 mesh scene at 1920x1080, 8 passes: 5.26, 2.9, 2.05, 1.54, 1.38,
  * 1.23, 1.18 ms. */
-/* Batch launches without statistics keep each lane's grid in registers (72),
+/* Batch launches of the jump march keep each lane's grid in registers (72),
  * which leaves 6 waves a SIMD: workgroups of 256 threads use them all, those of
  * 1024 only 4.  They stage nothing in LDS.  16 scenes of 32^3 to 200^3: 1.33 ms
  * with 1024 threads, 1.15 with 256 (5 launches). */
-constexpr uint32_t wf_traverse_threads(bool stats, bool batch) { return batch && !stats ? 256u : 1024u; }
+constexpr uint32_t wf_traverse_threads(bool step, bool batch) { return batch && !step ? 256u : 1024u; }
 
 /* SGPRs are allocated in steps of 16.  A build of this kernel whose
  * allocation rose from 80 to 96 SGPRs, with its hot loop unchanged
@@ -678,19 +678,19 @@ __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r
     return pack_hit(D.x, D.y, D.z, status == 1 ? KIND_VOXEL : (D.y < 0 ? KIND_GROUND : KIND_MISS));
 }
 
-/* STATS: the step-by-step march, which counts voxel visits.  LDSB: with
- * STATS, the padded block bits are staged in LDS; without, the cells of the
- * codes (always staged in LDS, except in batch launches) are the 4x4x4
- * blocks. */
-template <bool STATS, bool LDSB, bool BATCH>
-__global__ __launch_bounds__(wf_traverse_threads(STATS, BATCH)) __attribute__((amdgpu_num_sgpr(WF_TRAVERSE_SGPRS)))
+/* STEP: the step-by-step march, of renders with statistics, which count voxel
+ * visits, and of grids with long axes (TraceArgs::step).  LDSB: with STEP, the
+ * padded block bits are staged in LDS; without, the cells of the codes (always
+ * staged in LDS, except in batch launches) are the 4x4x4 blocks. */
+template <bool STATS, bool LDSB, bool BATCH, bool STEP>
+__global__ __launch_bounds__(wf_traverse_threads(STEP, BATCH)) __attribute__((amdgpu_num_sgpr(WF_TRAVERSE_SGPRS)))
 void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t two)
 {
     extern __shared__ __align__(16) uint8_t smem[];
     /* the march reads the padded block bits, or the codes */
-    constexpr bool STAGE = !BATCH && (LDSB || !STATS);
-    const uint32_t* bits = STATS ? a.g.bitsp : a.g.codes;
-    const uint32_t words = !STAGE ? 0u : STATS ? a.g.bit_words_p : a.g.code_words;
+    constexpr bool STAGE = !BATCH && (LDSB || !STEP);
+    const uint32_t* bits = STEP ? a.g.bitsp : a.g.codes;
+    const uint32_t words = !STAGE ? 0u : STEP ? a.g.bit_words_p : a.g.code_words;
     uint32_t* taken = (uint32_t*)smem + words;     /* of the workgroup's list; after the table, whose reads then need no base */
     uint32_t* lengths = taken + 4;                 /* of the queue's parts */
     /* ray positions: a path's one ray, or (two = 1) its two */
@@ -712,7 +712,7 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
          * allocated, and the counter placed, to whole fours) */
         const uint4* from = (const uint4*)bits;
         uint4* to = (uint4*)smem;
-        const uint32_t n4 = words / 4u, T = wf_traverse_threads(STATS, BATCH);
+        const uint32_t n4 = words / 4u, T = wf_traverse_threads(STEP, BATCH);
         uint32_t i = threadIdx.x;
         for (; i + 3u * T < n4; i += 4u * T) {
             const uint4 v0 = from[i], v1 = from[i + T], v2 = from[i + 2u * T], v3 = from[i + 3u * T];
@@ -727,7 +727,7 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
     const uint32_t* qt = sel ? P.qt1 : P.qt0;
     Counters cnt = { 0, 0, 0, 0, 0, 0 };
     const uint32_t lane = threadIdx.x & 63u;
-    uint32_t refill_min = (uint32_t)a.refill_min * (STATS ? 1u : VT_JUMP_REFILL);
+    uint32_t refill_min = (uint32_t)a.refill_min * (STEP ? 1u : VT_JUMP_REFILL);
     if (refill_min > 64u) refill_min = 64u;
     const int budget = a.dda_budget;
     DdaState D;
@@ -761,7 +761,7 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
                     asm volatile("" : "+v"(o.x), "+v"(o.y), "+v"(o.z), "+v"(o.w), "+v"(d.x), "+v"(d.y));
                     jq = j;
                     if (BATCH) gl = B.tab[qt[j]].g;
-                    if constexpr (STATS) {
+                    if constexpr (STEP) {
                         has = D.init(G, unpack_ray(o, d));
                         if (!has) P.hit[j] = pack_hit(0, 0, 0, KIND_MISS);
                     } else {
@@ -778,7 +778,7 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
             if (done) break;
             continue;
         }
-        if constexpr (STATS) {
+        if constexpr (STEP) {
             if (has) {
                 /* per-lane grids (batch) and grids whose padded masks span 4 GiB
                  * address the masks with 64-bit per-lane arithmetic */
@@ -1071,8 +1071,8 @@ static int blocks_per_cu(K kernel, int threads, size_t lds)
 
 hipError_t check_lds_base()
 {
-    for (const void* k : { (const void*)wf_traverse_kernel<false, false, false>,
-                           (const void*)wf_traverse_kernel<false, true, false> }) {
+    for (const void* k : { (const void*)wf_traverse_kernel<false, false, false, false>,
+                           (const void*)wf_traverse_kernel<false, true, false, false> }) {
         hipFuncAttributes at;
         const hipError_t e = hipFuncGetAttributes(&at, k);
         if (e != hipSuccess) return e;
@@ -1084,15 +1084,15 @@ hipError_t check_lds_base()
 /* generate -> (traverse -> shade) x rounds -> accumulate per chunk of at
  * most P.cap paths.  `a` describes the single scene (or, in a batch, carries
  * the traversal tuning and the LDS sizes of scene 0). */
-template <bool STATS, bool LDSB, bool BATCH>
+template <bool STATS, bool LDSB, bool BATCH, bool STEP>
 static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths& P, uint64_t total,
                          uint64_t n_pixels, int rounds, int cus, hipStream_t s, const LaunchTimer* timer = nullptr,
                          hipEvent_t acc_wait = nullptr)
 {
-    const size_t lds_t = WF_TAKEN_BYTES + (BATCH ? 0u : STATS ? (LDSB ? (size_t)a.g.bit_words_p * 4u : 0u)
-                                                          : (size_t)a.g.code_words * 4u);
+    const size_t lds_t = WF_TAKEN_BYTES + (BATCH ? 0u : STEP ? (LDSB ? (size_t)a.g.bit_words_p * 4u : 0u)
+                                                         : (size_t)a.g.code_words * 4u);
     const size_t lds_s = BATCH ? 0 : 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
-    const int bt = blocks_per_cu(wf_traverse_kernel<STATS, LDSB, BATCH>, wf_traverse_threads(STATS, BATCH), lds_t);
+    const int bt = blocks_per_cu(wf_traverse_kernel<STATS, LDSB, BATCH, STEP>, wf_traverse_threads(STEP, BATCH), lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<STATS, PH_PRIMARY, BATCH>, WF_SHADE_THREADS, lds_s);
     const int bs1 = blocks_per_cu(wf_shade_kernel<STATS, PH_COMB, BATCH>, WF_SHADE_THREADS, lds_s);
     for (uint64_t g0 = 0; g0 < total; g0 += P.cap) {
@@ -1109,7 +1109,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used], s);
                 if (e != hipSuccess) return e;
             }
-            wf_traverse_kernel<STATS, LDSB, BATCH><<<cus * bt, wf_traverse_threads(STATS, BATCH), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
+            wf_traverse_kernel<STATS, LDSB, BATCH, STEP><<<cus * bt, wf_traverse_threads(STEP, BATCH), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
             if (timed) {
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used + 1], s);
                 if (e != hipSuccess) return e;
@@ -1135,24 +1135,29 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
 hipError_t launch_render_wavefront(const TraceArgs& a, const WfPaths& P, int cus, hipStream_t s, bool stats,
                                    const LaunchTimer* timer, hipEvent_t acc_wait)
 {
-    const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0 };
+    const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0, 0 };
     const uint64_t WH = (uint64_t)a.W * (uint64_t)a.H;
     const uint64_t total = WH * a.count;
     const int rounds = 1 + (a.s.max_bounces > 0 ? a.s.max_bounces : 0);
-    const bool lds_bits = stats ? a.lds_bits_p != 0 : a.g.cg == 2u;
+    const bool step = stats || a.step != 0;
+    const bool lds_bits = step ? a.lds_bits_p != 0 : a.g.cg == 2u;
     if (stats)
-        return lds_bits ? wf_run<true, true, false>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait)
-                        : wf_run<true, false, false>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait);
-    return lds_bits ? wf_run<false, true, false>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait)
-                    : wf_run<false, false, false>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait);
+        return lds_bits ? wf_run<true, true, false, true>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait)
+                        : wf_run<true, false, false, true>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait);
+    if (step)
+        return lds_bits ? wf_run<false, true, false, true>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait)
+                        : wf_run<false, false, false, true>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait);
+    return lds_bits ? wf_run<false, true, false, false>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait)
+                    : wf_run<false, false, false, false>(a, B, P, total, WH, rounds, cus, s, timer, acc_wait);
 }
 
 hipError_t launch_render_batch(const TraceArgs& a0, const BatchTable& B, const WfPaths& P, uint64_t total_paths,
                                uint64_t total_pixels, int max_bounces, int cus, hipStream_t s, bool stats)
 {
     const int rounds = 1 + (max_bounces > 0 ? max_bounces : 0);
-    if (stats) return wf_run<true, false, true>(a0, B, P, total_paths, total_pixels, rounds, cus, s);
-    return wf_run<false, false, true>(a0, B, P, total_paths, total_pixels, rounds, cus, s);
+    if (stats) return wf_run<true, false, true, true>(a0, B, P, total_paths, total_pixels, rounds, cus, s);
+    if (B.step) return wf_run<false, false, true, true>(a0, B, P, total_paths, total_pixels, rounds, cus, s);
+    return wf_run<false, false, true, false>(a0, B, P, total_paths, total_pixels, rounds, cus, s);
 }
 
 /* Paths that ended into the cache since the last apply (queries
@@ -1179,14 +1184,14 @@ __global__ void cache_mark_kernel(CacheRender C)
     if (threadIdx.x == 0) *C.q_done = *C.q_count;
 }
 
-template <bool LDSB>
+template <bool LDSB, bool STEP>
 static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const CacheRender& C, const void* pack,
                                 const float* bias, int cus, hipStream_t s)
 {
-    const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0 };
-    const size_t lds_t = WF_TAKEN_BYTES + (size_t)a.g.code_words * 4u;
+    const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0, 0 };
+    const size_t lds_t = WF_TAKEN_BYTES + (!STEP ? (size_t)a.g.code_words * 4u : LDSB ? (size_t)a.g.bit_words_p * 4u : 0u);
     const size_t lds_s = 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
-    const int bt = blocks_per_cu(wf_traverse_kernel<false, LDSB, false>, wf_traverse_threads(false, false), lds_t);
+    const int bt = blocks_per_cu(wf_traverse_kernel<false, LDSB, false, STEP>, wf_traverse_threads(STEP, false), lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<false, PH_PRIMARY, false, true>, WF_SHADE_THREADS, lds_s);
     const int bs1 = blocks_per_cu(wf_shade_kernel<false, PH_COMB, false, true>, WF_SHADE_THREADS, lds_s);
     const uint64_t WH = (uint64_t)a.W * (uint64_t)a.H;
@@ -1205,7 +1210,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     wf_generate_kernel<false, false, true><<<gg, WF_GENERATE_THREADS, 0, s>>>(a, B, P, 0, n, C);
     int sel = 0;
     for (int r = 0; r < rounds; ++r) {
-        wf_traverse_kernel<false, LDSB, false><<<cus * bt, wf_traverse_threads(false, false), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
+        wf_traverse_kernel<false, LDSB, false, STEP><<<cus * bt, wf_traverse_threads(STEP, false), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
         if (r == 0)
             wf_shade_kernel<false, PH_PRIMARY, false, true><<<cus * bs0, WF_SHADE_THREADS, lds_s, s>>>(a, B, P, sel, C);
         else
@@ -1228,8 +1233,11 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
 hipError_t launch_render_cached(const TraceArgs& a, const WfPaths& P, const CacheRender& C, const void* pack,
                                 const float* bias, int cus, hipStream_t s)
 {
-    return a.g.cg == 2u ? wf_run_cached<true>(a, P, C, pack, bias, cus, s)
-                        : wf_run_cached<false>(a, P, C, pack, bias, cus, s);
+    if (a.step)
+        return a.lds_bits_p ? wf_run_cached<true, true>(a, P, C, pack, bias, cus, s)
+                            : wf_run_cached<false, true>(a, P, C, pack, bias, cus, s);
+    return a.g.cg == 2u ? wf_run_cached<true, false>(a, P, C, pack, bias, cus, s)
+                        : wf_run_cached<false, false>(a, P, C, pack, bias, cus, s);
 }
 
 /* Emissive list entry i -> (x, y, z, material slot) of its voxel: the
