@@ -48,7 +48,7 @@ public:
     static constexpr int WORKERS = 3;              /* besides the calling thread */
     static constexpr size_t MIN_BYTES = 1u << 20;  /* smaller copies take the runtime's path */
 
-    static constexpr int POLL_MS = 2;
+    static constexpr int WORKER_POLL_MS = 2, CALLER_POLL_MS = 20;
     static constexpr int PIECES = (int)(CHUNK / PIECE);
 
     /* Whether a copy on stream s may use the ring; it then holds `lk`.  Chunks
@@ -171,7 +171,7 @@ private:
         std::this_thread::yield();
         const auto now = std::chrono::steady_clock::now();
         if (waiting != stalled_at_) stalled_at_ = waiting, since_ = now;
-        if (now - since_ < std::chrono::milliseconds(POLL_MS) || waiting >= issued) return hipSuccess;
+        if (now - since_ < std::chrono::milliseconds(CALLER_POLL_MS) || waiting >= issued) return hipSuccess;
         const hipError_t e = hipStreamSynchronize(s);
         return e != hipSuccess ? e : complete(waiting) ? hipSuccess : hipErrorUnknown;
     }
@@ -305,7 +305,7 @@ private:
                     continue;
                 }
                 std::this_thread::yield();
-                if (std::chrono::steady_clock::now() - last < std::chrono::milliseconds(POLL_MS)) continue;
+                if (std::chrono::steady_clock::now() - last < std::chrono::milliseconds(WORKER_POLL_MS)) continue;
                 std::unique_lock<std::mutex> g(wake_lock_);
                 ++asleep_;
                 wake_.wait(g, [&] {
