@@ -297,11 +297,14 @@ vt::MatRec decode(const std::vector<float>& m, int32_t off)
 
 int upload_records(vt_context* c)
 {
+    /* the slots in use: no voxel holds another (all 256, with 48 bytes each,
+     * took 20 us a call where 32 bytes had taken 18) */
+    const int n = c->n_slots + 1;
     vt::MatRec recs[256];
     recs[0] = decode(c->mat, 0);
-    for (int s = 1; s < 256; ++s) recs[s] = decode(c->mat, c->slot_off[s] < 0 ? 0 : c->slot_off[s]);
+    for (int s = 1; s < n; ++s) recs[s] = decode(c->mat, c->slot_off[s] < 0 ? 0 : c->slot_off[s]);
     if (!c->d_recs) VT_HIP(dmalloc(&c->d_recs, sizeof(recs)));
-    VT_HIP(hipMemcpyAsync(c->d_recs, recs, sizeof(recs), hipMemcpyHostToDevice, c->stream));
+    VT_HIP(hipMemcpyAsync(c->d_recs, recs, sizeof(recs[0]) * (size_t)n, hipMemcpyHostToDevice, c->stream));
     VT_HIP(hipStreamSynchronize(c->stream));
     return VT_OK;
 }
