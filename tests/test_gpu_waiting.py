@@ -59,3 +59,40 @@ def test_pick_behind_a_render_holds_up_no_other_context(ctx, vtapi):
         assert np.array_equal(got, want)
         assert took["behind"] > 0.5
         assert took["other"] < 0.5 * took["behind"], took
+
+
+def test_large_copies_of_others_while_one_waits(ctx, vtapi):
+    """A readback behind a long render holds a ring; other contexts copy to and
+    from the device meanwhile, and the readback itself comes back whole.  (Frames
+    are set before: freeing one waits for the device.)"""
+    import threading
+    rng = np.random.default_rng(2)
+    others = [vtapi.Context(0) for _ in range(2)]
+    bad, got = [], {}
+
+    def copies(c, k, w):
+        for _ in range(3):
+            a = rng.integers(0, 1 << 32, (1, w, 4), dtype=np.uint32).view(np.float32)
+            c.write_accum(a)
+            if not np.array_equal(c.read_accum().view(np.uint32), a.view(np.uint32)):
+                bad.append((k, w))
+
+    def behind():
+        got["img"] = ctx.read_accum()
+
+    for k, c in enumerate(others):
+        c.set_frame((200000, 1 << 20)[k], 1)
+        copies(c, k, (200000, 1 << 20)[k])
+    long_render(ctx, 1.0)
+    th = threading.Thread(target=behind)
+    th.start()
+    ts = [threading.Thread(target=copies, args=(c, k, (200000, 1 << 20)[k])) for k, c in enumerate(others)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(60)
+    th.join(60)
+    for c in others:
+        c.close()
+    assert not bad
+    assert np.array_equal(got["img"].view(np.uint32), ctx.read_accum().view(np.uint32))
