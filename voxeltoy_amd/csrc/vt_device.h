@@ -54,10 +54,12 @@ __device__ __forceinline__ f3 cross(f3 a, f3 b)
  * The compiler's IEEE division takes 11 instructions, its square root 15, since
  * they scale for every exponent.  Where scaling is not needed the hardware's
  * approximation and one step of Newton's iteration with a fused residual give
- * the same, correctly rounded result: each function below was compared bit by
- * bit with the operator it replaces, for all 2^32 arguments, over the range its
- * test admits.  Other arguments (zero, denormals, the largest, infinities, NaN)
- * take the operator.  Shading issues vector instructions three quarters of its
+ * the same, correctly rounded result over the range that each function below
+ * tests for.  The GPU test compares every significand at both parities of the
+ * exponent (steps by a power of four scale every operation exactly), random bit
+ * patterns and the edges of the ranges with IEEE arithmetic, bit by bit; a sweep
+ * over all 2^32 arguments, which is no test, found no difference either.  Other
+ * arguments (zero, denormals, the largest, infinities, NaN) take the operator.  Shading issues vector instructions three quarters of its
  * time, and its code holds 11 roots and 78 quotients: 9 % fewer instructions,
  * 1024^2 x 16 passes of the full-shading scene 7.72 -> 7.57 ms. */
 #define VT_MIN_NORMAL 1.17549435e-38f     /* 2^-126 */

@@ -58,8 +58,12 @@ inline uint32_t own_bit_words(const BrickDims& d)
  * whose padded two-bit codes let two traversal workgroups share a CU's
  * 160 KiB LDS (4 up to about 266 voxels an axis, 8 up to about 530).  The
  * coded cubes are 1, 2 and 8 cells an edge, or 1, 2 and 4 where the grid has
- * at most 56 cells an axis: iterations a ray 12.1 against 13.0 on a 256^3
- * terrain, 8.9 against 9.9 the other way on a 64^3 one. */
+ * at most 56 cells an axis.  Iterations a ray: 12.1 against 13.0 on a 256^3
+ * terrain, 9.9 against 8.9 on a 64^3 one; the line lies below the larger of the
+ * two and is not sharp, since the time hardly tells them apart.  With largest
+ * cubes of 8 and of 4 cells, us a call (800x500, 4 passes, or 640x400, 2): full
+ * scene 64^3 630 / 637, 128^3 746 / 739, 224^3 812 / 809, 256^3 867 / 871, 300^3
+ * 1006 / 983; mesh in 512^3 579 / 578, 800^3 899 / 877; terrain of 512 977 / 975. */
 struct CellLayout {
     uint32_t shift, top;         /* cells of 2^shift voxels; the largest coded cube has 2^top of them an edge */
     uint32_t ex, ey;             /* padded cells a row, rows a layer */

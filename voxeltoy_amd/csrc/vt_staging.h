@@ -46,8 +46,10 @@ public:
     static constexpr int SLOTS = 6;
     static constexpr int FLAG_STRIDE = 16;         /* words: a cache line a flag */
     static constexpr int WORKERS = 3;              /* besides the calling thread */
-    static constexpr size_t MIN_BYTES = 1u << 20;  /* smaller copies take the runtime's path */
-
+    /* Smaller copies take the runtime's path.  Runtime / ring, us: to the device
+     * 512 KiB 26 / 35, 1008 44 / 48, 2048 80 / 72; from it into fresh pages 512 34 /
+     * 43, 896 53 / 55, 1008 58 / 61, 1024 (two transfers of the runtime's) 82 / 62. */
+    static constexpr size_t MIN_BYTES = 1u << 20;
     static constexpr int WORKER_POLL_MS = 2, CALLER_POLL_MS = 20;
     static constexpr int PIECES = (int)(CHUNK / PIECE);
 
@@ -230,21 +232,26 @@ private:
         {
             std::lock_guard<std::mutex> g(wake_lock_);
             ++job_;
-            active_ = true;
+            active_.store(true);
         }
+        wake_.notify_all();
+    }
+
+    /* Wakes the workers that sleep in the job, after a sequentially consistent
+     * store to open_ or active_: a worker raises asleep_ and then reads both
+     * under the lock, so it is seen here or sees the store. */
+    void rouse()
+    {
+        if (asleep_.load() == 0) return;
+        { std::lock_guard<std::mutex> g(wake_lock_); }
         wake_.notify_all();
     }
 
     /* Chunks up to n may be copied now. */
     void open(int n)
     {
-        bool asleep;
-        {
-            std::lock_guard<std::mutex> g(wake_lock_);
-            open_.store(n, std::memory_order_release);
-            asleep = asleep_ > 0;
-        }
-        if (asleep) wake_.notify_all();
+        open_.store(n);
+        rouse();
     }
 
     /* One piece of an open chunk; false when there is none now. */
@@ -267,20 +274,16 @@ private:
     }
 
     /* every piece that was taken is copied (all of them, unless abandoned),
-     * and no thread looks at the job any more: a worker joins a job under the
-     * lock, so it has either joined before the job is closed here, and is in
-     * busy_, or finds it closed */
+     * and no thread looks at the job any more: a worker raises busy_ and then
+     * reads active_, both in one order with the store and the load here, so it
+     * is either seen or finds the job closed.  (No lock: the workers that leave
+     * would queue for it with the caller.) */
     void finish()
     {
         while (!abandon_.load(std::memory_order_acquire) && done_.load(std::memory_order_acquire) < pieces_) help();
-        bool asleep;
-        {
-            std::lock_guard<std::mutex> g(wake_lock_);
-            active_ = false;
-            asleep = asleep_ > 0;
-        }
-        if (asleep) wake_.notify_all();
-        while (busy_.load(std::memory_order_acquire) != 0) std::this_thread::yield();
+        active_.store(false);
+        rouse();
+        while (busy_.load() != 0) std::this_thread::yield();
     }
 
     void work()
@@ -292,14 +295,14 @@ private:
                 wake_.wait(g, [&] { return quit_ || job_ != seen; });
                 if (quit_) return;
                 seen = job_;
-                if (!active_) continue;                 /* woken too late */
-                busy_.fetch_add(1, std::memory_order_acq_rel);
+                busy_.fetch_add(1);
             }
             /* Look for pieces until all are taken: with yields for a frame's
              * time, then asleep until a chunk opens (behind a render of
              * seconds every worker would keep a core busy). */
             auto last = std::chrono::steady_clock::now();
-            while (!abandon_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < pieces_) {
+            while (active_.load() && !abandon_.load(std::memory_order_acquire) &&
+                   next_.load(std::memory_order_relaxed) < pieces_) {
                 if (help()) {
                     last = std::chrono::steady_clock::now();
                     continue;
@@ -307,12 +310,12 @@ private:
                 std::this_thread::yield();
                 if (std::chrono::steady_clock::now() - last < std::chrono::milliseconds(WORKER_POLL_MS)) continue;
                 std::unique_lock<std::mutex> g(wake_lock_);
-                ++asleep_;
+                asleep_.fetch_add(1);
                 wake_.wait(g, [&] {
                     const int64_t p = next_.load(std::memory_order_relaxed);
-                    return !active_ || p >= pieces_ || p / PIECES < open_.load(std::memory_order_relaxed);
+                    return !active_.load() || p >= pieces_ || p / PIECES < open_.load();
                 });
-                --asleep_;
+                asleep_.fetch_sub(1);
             }
             busy_.fetch_sub(1, std::memory_order_acq_rel);
         }
@@ -338,13 +341,13 @@ private:
     std::atomic<int> copied_[SLOTS];
     std::atomic<int64_t> next_{ 0 }, done_{ 0 };
     std::atomic<int> open_{ 0 };
-    std::atomic<bool> abandon_{ false };
+    std::atomic<bool> abandon_{ false }, active_{ false };
     std::atomic<int> busy_{ 0 };        /* workers in the job */
-    std::mutex wake_lock_;              /* guards the four below */
+    std::atomic<int> asleep_{ 0 };      /* of them, waiting for a chunk */
+    std::mutex wake_lock_;              /* guards the two below */
     std::condition_variable wake_;
     uint64_t job_ = 0;
-    int asleep_ = 0;                    /* workers that wait for a chunk */
-    bool active_ = false, quit_ = false;
+    bool quit_ = false;
 };
 
 /* The copies of a device's contexts.  The second ring is for a copy that finds

@@ -638,7 +638,7 @@ __global__ __launch_bounds__(WF_GENERATE_THREADS) void wf_generate_kernel(TraceA
  * takes about 13 ns an update.  Workgroups of 1024 threads share one
  * LDS copy of the empty-cube codes (of the block occupancy bits with STEP).
  *
- * Bound by vector issue (0.85 wave-instructions a CU and cycle, 48 % of the
+ * Bound by vector issue (0.95 wave-instructions a CU and cycle, 49 % of the
  * lanes at work, full-shading scene) and, in the later launches, by the chain
  * of its longest rays (up to 115 jumps of about 0.4 microseconds).  That scene
  * at 1024^2, 16 passes, 8 bounces (90 M rays, 9 launches): 10.1 ms stepping
