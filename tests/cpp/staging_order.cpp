@@ -1,7 +1,7 @@
 /* The ring's hand-over between the calling thread and its workers, with the
  * reordering that x86 and C++ allow: a store that is not sequentially
- * consistent may become visible only after the thread's next load of another
- * variable.  std::atomic and std::mutex inside vt_staging.h are replaced by
+ * consistent may become visible only after the thread's next loads of other
+ * variables.  std::atomic and std::mutex inside vt_staging.h are replaced by
  * ones that do this, pausing in between, so that what is a matter of
  * nanoseconds on a processor happens in every run.
  *
@@ -61,7 +61,7 @@ struct late_atomic {
         const T x = v.load();
         if (pending_.at) {
             if (chance(2)) pause_us(30);
-            pending_.drain();
+            if (chance(2)) pending_.drain();            /* or it waits behind another load */
         } else if (sizeof(T) == 1 && chance(4)) {
             pause_us(50);
         }
