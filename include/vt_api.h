@@ -17,7 +17,13 @@
  *     thread;
  *   - images are in GL row order: row 0 is the bottom row;
  *   - matrices are row-major float[16] (m[r*4+c]), as Imath stores them
- *     and as the reference uploads them with transpose = GL_TRUE.
+ *     and as the reference uploads them with transpose = GL_TRUE;
+ *   - per device, and shared by its contexts, the library keeps between calls
+ *     one device workspace of at most 256 MiB (given back with the last
+ *     context, and to an allocation of its own that finds no memory), up to two
+ *     pinned rings of 12 MiB with three threads each for host copies of 1 MiB
+ *     and more (given back with the last context), and two pinned arrays of
+ *     896 KiB for picking (held until the process ends).
  */
 #ifndef VT_API_H_
 #define VT_API_H_
@@ -141,14 +147,15 @@ int vt_set_stats(vt_context* ctx, int32_t enabled);
 /* Kernel organisation of vt_render (results are identical):
  *   0 = persistent megakernel (one lane renders a pixel's passes start to end)
  *   1 = wavefront (generate / traverse / shade kernels over ray queues; at
- *       most max_paths paths in flight, 0 = default 16M).
+ *       most max_paths paths in flight, 0 = default 16M, whose storage of
+ *       384 bytes a path is rounded up to 16 384 paths).
  * Default 1. */
 int vt_set_render_mode(vt_context* ctx, int32_t mode, uint64_t max_paths);
 /* Wavefront traversal tuning (results are identical for every value):
- * dda_budget   jumps (with statistics: DDA steps) a lane takes between
- *              refill checks (1..4096),
+ * dda_budget   jumps a lane takes between refill checks (with statistics, and
+ *              in grids of more than 900 voxels an axis, DDA steps) (1..4096),
  * refill_min   idle lanes of a 64-lane wave that trigger a refill (1..64;
- *              without statistics three times as many, at most 64),
+ *              where lanes jump three times as many, at most 64),
  * refill_chunk queue entries that are dealt to a workgroup at a time, rounded
  *              down to a power of two (64..65536, or -1 for 64);
  * 0 selects the default of each.  No counterpart in the reference (its

@@ -352,7 +352,7 @@ __device__ __forceinline__ void grad_tiles(const float* __restrict__ D, size_t d
  * items and a light one are two workgroups a CU, 4 waves a SIMD.  Bound by the
  * matrix units (1.75 M products of 32 cycles for 50001 samples, 23 us, 42 % of
  * the time) and by the reads of dZ, 5 times for layer 0 (177 MB by the loads, 132
- * MB past the L2s, 3.3 TB/s): 40 us, where one wave per item and split, with
+ * MB past the L2s, at 3.3 TB/s): 40 us, where one wave per item and split, with
  * nothing to hide its loads behind, took 121. */
 __global__ __launch_bounds__(GRAD_THREADS, 4) void mlp_train_grad_kernel(TrainBatch b, TrainScratch S)
 {
