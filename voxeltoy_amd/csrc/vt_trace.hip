@@ -678,11 +678,14 @@ __device__ __forceinline__ uint2 stepwise_hit(const GridView& g, const PreRay& r
     return pack_hit(D.x, D.y, D.z, status == 1 ? KIND_VOXEL : (D.y < 0 ? KIND_GROUND : KIND_MISS));
 }
 
-/* STEP: the step-by-step march, of renders with statistics, which count voxel
- * visits, and of grids with long axes (TraceArgs::step).  LDSB: with STEP, the
- * padded block bits are staged in LDS; without, the cells of the codes (always
- * staged in LDS, except in batch launches) are the 4x4x4 blocks. */
-template <bool STATS, bool LDSB, bool BATCH, bool STEP>
+/* STEP: the step-by-step march, of renders with statistics and of grids with long
+ * axes (TraceArgs::step); it counts voxel visits in either case and adds them up
+ * when there are statistics (1000x300x1000 at 1280x800, 2 passes: 2.76 ms, in
+ * kernels that do not count 2.72; flat grids the same).
+ * LDSB: with STEP, the padded block bits are staged in LDS; without, the cells of
+ * the codes (always staged in LDS, except in batch launches) are the 4x4x4
+ * blocks. */
+template <bool STEP, bool LDSB, bool BATCH>
 __global__ __launch_bounds__(wf_traverse_threads(STEP, BATCH)) __attribute__((amdgpu_num_sgpr(WF_TRAVERSE_SGPRS)))
 void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t two)
 {
@@ -784,13 +787,13 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
                  * address the masks with 64-bit per-lane arithmetic */
                 int status;
                 if (BATCH && B.packed)
-                    status = D.advance_wave_packed<STATS, false, false>(G, nullptr, budget, cnt.visits);
+                    status = D.advance_wave_packed<STEP, false, false>(G, nullptr, budget, cnt.visits);
                 else if (BATCH || G.wide)
-                    status = D.advance_wave<STATS, false, false>(G, G.bitsp, budget, cnt.visits);
+                    status = D.advance_wave<STEP, false, false>(G, G.bitsp, budget, cnt.visits);
                 else if (LDSB && G.occr)
-                    status = D.advance_wave_packed<STATS, true, true>(G, bits, budget, cnt.visits);
+                    status = D.advance_wave_packed<STEP, true, true>(G, bits, budget, cnt.visits);
                 else
-                    status = D.advance_wave<STATS, LDSB, true>(G, bits, budget, cnt.visits);
+                    status = D.advance_wave<STEP, LDSB, true>(G, bits, budget, cnt.visits);
                 if (status) {
                     /* kind and voxel only: the shade kernel reads the material slot */
                     const int kind = status == 1 ? KIND_VOXEL : (D.y < 0 ? KIND_GROUND : KIND_MISS);
@@ -815,7 +818,8 @@ void wf_traverse_kernel(TraceArgs a, BatchTable B, WfPaths P, int sel, uint32_t 
             }
         }
     }
-    flush_counters<STATS>(BATCH ? B.stats : a.stats, cnt);
+    unsigned long long* const stats = BATCH ? B.stats : a.stats;
+    if (STEP && stats) flush_counters<STEP>(stats, cnt);
 }
 
 /* Largest training target kept: above it a sample is an outlier of the
@@ -1071,8 +1075,8 @@ static int blocks_per_cu(K kernel, int threads, size_t lds)
 
 hipError_t check_lds_base()
 {
-    for (const void* k : { (const void*)wf_traverse_kernel<false, false, false, false>,
-                           (const void*)wf_traverse_kernel<false, true, false, false> }) {
+    for (const void* k : { (const void*)wf_traverse_kernel<false, false, false>,
+                           (const void*)wf_traverse_kernel<false, true, false> }) {
         hipFuncAttributes at;
         const hipError_t e = hipFuncGetAttributes(&at, k);
         if (e != hipSuccess) return e;
@@ -1092,7 +1096,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
     const size_t lds_t = WF_TAKEN_BYTES + (BATCH ? 0u : STEP ? (LDSB ? (size_t)a.g.bit_words_p * 4u : 0u)
                                                          : (size_t)a.g.code_words * 4u);
     const size_t lds_s = BATCH ? 0 : 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
-    const int bt = blocks_per_cu(wf_traverse_kernel<STATS, LDSB, BATCH, STEP>, wf_traverse_threads(STEP, BATCH), lds_t);
+    const int bt = blocks_per_cu(wf_traverse_kernel<STEP, LDSB, BATCH>, wf_traverse_threads(STEP, BATCH), lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<STATS, PH_PRIMARY, BATCH>, WF_SHADE_THREADS, lds_s);
     const int bs1 = blocks_per_cu(wf_shade_kernel<STATS, PH_COMB, BATCH>, WF_SHADE_THREADS, lds_s);
     for (uint64_t g0 = 0; g0 < total; g0 += P.cap) {
@@ -1109,7 +1113,7 @@ static hipError_t wf_run(const TraceArgs& a, const BatchTable& B, const WfPaths&
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used], s);
                 if (e != hipSuccess) return e;
             }
-            wf_traverse_kernel<STATS, LDSB, BATCH, STEP><<<cus * bt, wf_traverse_threads(STEP, BATCH), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
+            wf_traverse_kernel<STEP, LDSB, BATCH><<<cus * bt, wf_traverse_threads(STEP, BATCH), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
             if (timed) {
                 const hipError_t e = hipEventRecord(timer->ev[2 * *timer->used + 1], s);
                 if (e != hipSuccess) return e;
@@ -1191,7 +1195,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     const BatchTable B = { nullptr, nullptr, nullptr, 0u, nullptr, 0, 0 };
     const size_t lds_t = WF_TAKEN_BYTES + (!STEP ? (size_t)a.g.code_words * 4u : LDSB ? (size_t)a.g.bit_words_p * 4u : 0u);
     const size_t lds_s = 256 * sizeof(MatRec) + (size_t)a.cdfv_lds_bytes;
-    const int bt = blocks_per_cu(wf_traverse_kernel<false, LDSB, false, STEP>, wf_traverse_threads(STEP, false), lds_t);
+    const int bt = blocks_per_cu(wf_traverse_kernel<STEP, LDSB, false>, wf_traverse_threads(STEP, false), lds_t);
     const int bs0 = blocks_per_cu(wf_shade_kernel<false, PH_PRIMARY, false, true>, WF_SHADE_THREADS, lds_s);
     const int bs1 = blocks_per_cu(wf_shade_kernel<false, PH_COMB, false, true>, WF_SHADE_THREADS, lds_s);
     const uint64_t WH = (uint64_t)a.W * (uint64_t)a.H;
@@ -1210,7 +1214,7 @@ static hipError_t wf_run_cached(const TraceArgs& a, const WfPaths& P, const Cach
     wf_generate_kernel<false, false, true><<<gg, WF_GENERATE_THREADS, 0, s>>>(a, B, P, 0, n, C);
     int sel = 0;
     for (int r = 0; r < rounds; ++r) {
-        wf_traverse_kernel<false, LDSB, false, STEP><<<cus * bt, wf_traverse_threads(STEP, false), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
+        wf_traverse_kernel<STEP, LDSB, false><<<cus * bt, wf_traverse_threads(STEP, false), lds_t, s>>>(a, B, P, sel, r == 0 ? 0u : 1u);
         if (r == 0)
             wf_shade_kernel<false, PH_PRIMARY, false, true><<<cus * bs0, WF_SHADE_THREADS, lds_s, s>>>(a, B, P, sel, C);
         else
