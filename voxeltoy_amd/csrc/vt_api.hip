@@ -2239,8 +2239,10 @@ int vt_voxelize(vt_context* c, const float* verts, int64_t nv, const uint32_t* i
             int r = refresh_codes(c);
             if (r != VT_OK) return r;
         }
+        /* either waits for all of the call's work (the other wait after the copy
+         * would cost a marker of its own, 15 us) */
         if (occupancy) VT_HIP(to_host(c, occupancy, work + occ_at, (size_t)nvox));
-        VT_HIP(hipStreamSynchronize(c->stream));
+        else VT_HIP(hipStreamSynchronize(c->stream));
         ws.waited();
         return VT_OK;
     });
